@@ -425,6 +425,24 @@ def test_float32_product_of_few_rows_has_the_bits_of_the_product_of_many(n, k):
             assert torch.equal(few, many[11:11 + rows]), f"{rows} rows, tile-major copy {tiles is not None}"
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 2048, 16384), (129, 2048, 2064), (333, 2560, 2048), (200, 30, 4100), (128, 513, 520),
+                                   (300, 70, 500), (520, 4096, 1536)])
+def test_float32_product_of_many_rows_has_the_same_bits_with_its_k_axis_cut(m, n, k):
+    """More than 64 rows in float32: tiles of any size, and a K axis whose segments several workgroups take (with sums
+    of their own, added by a further kernel in the same order), leave the bits that 64 rows at a time give.  Odd
+    columns, a K axis that ends inside a segment and inside a chunk of 16 keys, one segment and many."""
+    torch.manual_seed(19)
+    x = torch.randn(m, k, device=DEV)
+    w = torch.randn(n, k, device=DEV) / math.sqrt(k)
+    out = torch.full((m + 1, n), 7.0, device=DEV)
+    ops.linear(x, w, out[:m])
+    rows = torch.empty((m, n), device=DEV)
+    for r in range(0, m, 64):
+        ops.linear(x[r:r + 64], w, rows[r:r + 64])
+    assert torch.equal(out[:m], rows) and bool((out[m] == 7.0).all())
+    close(out[:m], x.double() @ w.double().T, torch.float32, "product")
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 2048, 16384), (5, 2560, 2048), (16, 1000, 8192), (1, 777, 516), (3, 40000, 2048),
                                    (40, 2048, 4096), (64, 1000, 2048)])
 def test_float32_linear_leaves_partial_sums_to_the_caller(m, n, k):

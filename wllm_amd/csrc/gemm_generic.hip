@@ -180,12 +180,17 @@ gemm_f32_few_rows_kernel(const float* __restrict__ x, const float* __restrict__ 
 }
 
 // More rows: a workgroup of four wavefronts (2 x 2) makes 32 WM rows by 32 WN columns; the tiles of
-// x and w of a chunk go through shared memory, the next chunk's loads in flight while this one is
+// x and w of a chunk go through shared memory, the next chunks' loads in flight while this one is
 // multiplied.  Rows of a tile are padded to 20 floats, so that the 16-byte fragment reads of 8 lanes
-// fall into different banks.
-template <int WM, int WN>
+// fall into different banks.  What lies beyond the K axis becomes zero when it is put into shared memory
+// and not when it is loaded: a choice made on a load's result waits for the load at once (with it there,
+// 4,096 x 4,096 x 4,096 ran at 109 TFLOP/s, every chunk a trip to memory).
+// SPLIT: a workgroup (blockIdx.z) takes `per_group` segments of the K axis and leaves each one's sum in
+// out[segment]; the kernel below adds them in the order in which the unsplit walk does.
+template <int WM, int WN, bool SPLIT>
 __global__ void __launch_bounds__(256, 2)
-gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K) {
+gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
+                     int per_group) {
     constexpr int TM = 32 * WM, TN = 32 * WN, kStride = kF32Chunk + 4;
     constexpr int XP = TM * 4 / 256, WP = TN * 4 / 256;       // 16-byte pieces of a chunk's tiles per thread
     static_assert(XP * 256 == TM * 4 && WP * 256 == TN * 4, "whole pieces per thread");
@@ -207,21 +212,20 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
     // multiplied, so a trip to memory has two chunks' products to hide behind
     f32x4 xr[2][XP], wr[2][WP];
     auto fetch = [&](f32x4 (&xq)[XP], f32x4 (&wq)[WP], int k0) {
-        const int k = k0 + p_k;
-        const bool live = k < K;
-        const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int k = min(k0 + p_k, K - 4);
 #pragma unroll
-        for (int p = 0; p < XP; ++p) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(xsrc[p] + min(k, K - 4));
-            xq[p] = live ? v : zero;
-        }
+        for (int p = 0; p < XP; ++p) xq[p] = *reinterpret_cast<const f32x4*>(xsrc[p] + k);
 #pragma unroll
-        for (int p = 0; p < WP; ++p) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(wsrc[p] + min(k, K - 4));
-            wq[p] = live ? v : zero;
-        }
+        for (int p = 0; p < WP; ++p) wq[p] = *reinterpret_cast<const f32x4*>(wsrc[p] + k);
     };
-    auto stage = [&](int buf, const f32x4 (&xq)[XP], const f32x4 (&wq)[WP]) {
+    auto stage = [&](int buf, f32x4 (&xq)[XP], f32x4 (&wq)[WP], int k0) {
+        if (k0 + kF32Chunk > K && k0 + p_k >= K) {
+            const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 0; p < XP; ++p) xq[p] = zero;
+#pragma unroll
+            for (int p = 0; p < WP; ++p) wq[p] = zero;
+        }
 #pragma unroll
         for (int p = 0; p < XP; ++p) *reinterpret_cast<f32x4*>(&xs[buf][(p_row + 64 * p) * kStride + p_k]) = xq[p];
 #pragma unroll
@@ -232,8 +236,29 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
     for (int jm = 0; jm < WM; ++jm)
 #pragma unroll
         for (int jn = 0; jn < WN; ++jn) acc[jm][jn] = total[jm][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int chunks = (K + kF32Chunk - 1) / kF32Chunk;
+    auto put = [&](float* to, const f32x4 (&value)[WM][WN]) {
+#pragma unroll
+        for (int jm = 0; jm < WM; ++jm) {
+            const int m = m0 + wm0 + 16 * jm + i;
+            if (m >= M) continue;
+#pragma unroll
+            for (int jn = 0; jn < WN; ++jn) {
+                const int n = n0 + wn0 + 16 * jn + 4 * g;
+                float* dst = to + static_cast<size_t>(m) * N + n;
+                if (N % 4 == 0 && n + 3 < N) {
+                    *reinterpret_cast<f32x4*>(dst) = value[jm][jn];
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < N) dst[v] = value[jm][jn][v];
+                }
+            }
+        }
+    };
     constexpr int kChunksPerSegment = kF32Segment / kF32Chunk;
+    const int all_chunks = (K + kF32Chunk - 1) / kF32Chunk;
+    const int first = SPLIT ? blockIdx.z * per_group * kChunksPerSegment : 0;
+    const int chunks = SPLIT ? min(all_chunks, first + per_group * kChunksPerSegment) : all_chunks;   // one past the last
     // chunk q: multiplied from tile q % 2 of shared memory; chunk q + 1 waits in the registers (q + 1) % 2
     // and goes to the other tile when the products of chunk q are issued; chunk q + 2 is asked for
     auto step = [&](int q, int buf, f32x4 (&x_next)[XP], f32x4 (&w_next)[WP], f32x4 (&x_ask)[XP], f32x4 (&w_ask)[WP]) {
@@ -251,54 +276,50 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
                 for (int jn = 0; jn < WN; ++jn)
                     acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[jn][t], b[jm][t], acc[jm][jn], 0, 0, 0);
         if ((q + 1) % kChunksPerSegment == 0 || q + 1 == chunks) {
-            // a segment ends: its sum joins the sums of the segments before it
-            const bool first = q < kChunksPerSegment;
+            // a segment ends: its sum joins the sums of the segments before it, or goes to its own place
+            const bool alone = q < kChunksPerSegment;
+            if (SPLIT) put(out + static_cast<size_t>(q / kChunksPerSegment) * M * N, acc);
 #pragma unroll
             for (int jm = 0; jm < WM; ++jm)
 #pragma unroll
                 for (int jn = 0; jn < WN; ++jn) {
-                    total[jm][jn] = first ? acc[jm][jn] : total[jm][jn] + acc[jm][jn];
+                    if (!SPLIT) total[jm][jn] = alone ? acc[jm][jn] : total[jm][jn] + acc[jm][jn];
                     acc[jm][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
         }
-        if (q + 1 < chunks) stage(buf ^ 1, x_next, w_next);
+        if (q + 1 < chunks) stage(buf ^ 1, x_next, w_next, (q + 1) * kF32Chunk);
         __syncthreads();
     };
-    fetch(xr[0], wr[0], 0);
-    stage(0, xr[0], wr[0]);
-    if (chunks > 1) fetch(xr[1], wr[1], kF32Chunk);
+    fetch(xr[0], wr[0], first * kF32Chunk);
+    stage(0, xr[0], wr[0], first * kF32Chunk);
+    if (first + 1 < chunks) fetch(xr[1], wr[1], (first + 1) * kF32Chunk);
     __syncthreads();
-    for (int q = 0; q < chunks; q += 2) {
+    for (int q = first; q < chunks; q += 2) {
         step(q, 0, xr[1], wr[1], xr[0], wr[0]);
         if (q + 1 < chunks) step(q + 1, 1, xr[0], wr[0], xr[1], wr[1]);
     }
-#pragma unroll
-    for (int jm = 0; jm < WM; ++jm) {
-        const int m = m0 + wm0 + 16 * jm + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int jn = 0; jn < WN; ++jn) {
-            const int n = n0 + wn0 + 16 * jn + 4 * g;
-            float* dst = out + static_cast<size_t>(m) * N + n;
-            if (N % 4 == 0 && n + 3 < N) {
-                *reinterpret_cast<f32x4*>(dst) = total[jm][jn];
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (n + v < N) dst[v] = total[jm][jn][v];
-            }
-        }
-    }
+    if (!SPLIT) put(out, total);
 }
 
-// out[i] = partial[0][i] + partial[1][i] + ... in ascending order of the segments.
+// out[i] = partial[0][i] + partial[1][i] + ... in ascending order of the segments; VEC consecutive elements a thread
+// (four where the count and the addresses allow it), eight segments asked for before the first is added.
+template <int VEC>
 __global__ void __launch_bounds__(256)
-gemm_segments_sum_kernel(const float* __restrict__ partial, float* __restrict__ out, int count, int segments) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+gemm_segments_sum_kernel(const float* __restrict__ partial, float* __restrict__ out, long long count, int segments) {
+    typedef float floats __attribute__((ext_vector_type(VEC)));
+    const long long i = (static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x) * VEC;
     if (i >= count) return;
-    float total = partial[i];
-    for (int s = 1; s < segments; ++s) total = total + partial[static_cast<size_t>(s) * count + i];
-    out[i] = total;
+    floats total = *reinterpret_cast<const floats*>(partial + i);
+    for (int s0 = 1; s0 < segments; s0 += 8) {
+        floats t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            t[j] = *reinterpret_cast<const floats*>(partial + static_cast<size_t>(min(s0 + j, segments - 1)) * count + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s0 + j < segments) total = total + t[j];
+    }
+    *reinterpret_cast<floats*>(out + i) = total;
 }
 
 namespace {
@@ -306,6 +327,55 @@ namespace {
 // of 16 columns alone are too few wavefronts to keep the memory busy.
 bool few_rows_split(int N, int K) { return K > kF32Segment && (N + 15) / 16 < 1024; }
 bool f32_by_matrix_cores(int in_bf16, int out_bf16, int K) { return !in_bf16 && !out_bf16 && K % 4 == 0 && K >= 4; }
+
+int sum_segments(const float* partial, float* out, long long count, int segments, hipStream_t stream) {
+    const bool fours = count % 4 == 0 && (reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+    const int vec = fours ? 4 : 1;
+    const long long blocks = (count / vec + 255) / 256;
+    if (blocks > 0x7fffffffLL) return -1;
+    if (vec == 4)
+        gemm_segments_sum_kernel<4><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(partial, out, count, segments);
+    else
+        gemm_segments_sum_kernel<1><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(partial, out, count, segments);
+    return launch_status();
+}
+
+// How a product of more than 64 rows is cut: tiles of 32 wm by 32 wn, and `per_group` segments of the K axis a
+// workgroup (0: all of them, no partial sums).  Every choice gives the same bits, so the cheapest by this estimate
+// is taken: a compute unit that holds two or more workgroups works off one's tile and segment in the first time
+// below, one that holds a single workgroup in the second (measured, in us: 132, 117 and 110 TFLOP/s with all
+// compute units full, 110, 92 and 75 with one workgroup each), and partial sums are written and read at
+// 4 TB/s by a further launch.  333 rows, by the estimate against tiles chosen by their number alone:
+// K 16,384 to 2,048 columns 596 to 260 us, 2,048 to 2,560 84 to 49, 2,048 to 2,048 80 to 42; 100 rows, 16,384 to
+// 2,048: 596 to 94.
+struct F32Cut {
+    int wm, wn, per_group;
+};
+constexpr long long kMostPartials = 64LL << 20;       // floats of partial sums a product may leave (256 MiB)
+
+F32Cut f32_cut(int M, int N, int K, bool may_split) {
+    constexpr struct { int wm, wn; float shared, alone; } kTiles[] = {{4, 4, 32.6f, 38.f}, {4, 2, 18.4f, 22.7f}, {2, 4, 18.4f, 22.7f}, {2, 2, 9.7f, 14.3f}};
+    constexpr int kUnits = 256;
+    const int segments = (K + kF32Segment - 1) / kF32Segment;
+    F32Cut best{4, 4, 0};
+    float least = 3.4e38f;
+    for (const auto& t : kTiles) {
+        const long long tiles = static_cast<long long>((M + 32 * t.wm - 1) / (32 * t.wm)) * ((N + 32 * t.wn - 1) / (32 * t.wn));
+        for (int per_group = segments; per_group >= 1; per_group = per_group == 1 ? 0 : (per_group + 1) / 2) {
+            const int groups = (segments + per_group - 1) / per_group;
+            const bool split = groups > 1;
+            if (split && (!may_split || groups > 65535 || static_cast<long long>(segments) * M * N > kMostPartials)) break;
+            const long long on_a_unit = (tiles * groups + kUnits - 1) / kUnits;
+            float us = per_group * ((on_a_unit & ~1LL) * t.shared + (on_a_unit & 1) * t.alone);
+            if (split) us += 4.f + 2e-6f * segments * M * N;
+            if (us < least) {
+                least = us;
+                best = F32Cut{t.wm, t.wn, split ? per_group : 0};
+            }
+        }
+    }
+    return best;
+}
 }  // namespace
 
 // The tile-major copy of a float32 weight [N, K] (K a multiple of 4): for band b of 16 rows and chunk q
@@ -341,10 +411,11 @@ WLLM_API int wllm_tile_weight_f32(const float* w, float* tiles, int N, int K, hi
 }
 
 // Into how many partial sums [segments, M, N] a float32 product of these sizes is split (1: it is not).
-// `wllm_gemm_generic` needs `partial` to hold them; with `out` null it leaves them there for a consumer
-// that adds them in ascending order.
+// `wllm_gemm_generic` needs `partial` to hold them (at most 64 rows; with more rows it runs unsplit without); with
+// `out` null it leaves them there for a consumer that adds them in ascending order.
 WLLM_API int wllm_gemm_f32_segments(int M, int N, int K) {
-    if (M < 1 || M > 64 || K % 4 != 0 || !few_rows_split(N, K)) return 1;
+    if (M < 1 || N < 1 || K < 4 || K % 4 != 0) return 1;
+    if (M <= 64 ? !few_rows_split(N, K) : f32_cut(M, N, K, true).per_group == 0) return 1;
     return (K + kF32Segment - 1) / kF32Segment;
 }
 
@@ -381,7 +452,7 @@ WLLM_API int wllm_gemm_generic(const void* x, const void* w, const void* tiles, 
                 float* pf = static_cast<float*>(partial);
                 FEW_ROWS(true, dim3(groups, segments), pf);
                 if (int err = launch_status()) return err;
-                if (of) gemm_segments_sum_kernel<<<(M * N + 255) / 256, 256, 0, stream>>>(pf, of, M * N, segments);
+                if (of) return sum_segments(pf, of, static_cast<long long>(M) * N, segments, stream);
             } else {
                 if (!of) return -1;
                 FEW_ROWS(false, dim3(groups), of);
@@ -389,18 +460,25 @@ WLLM_API int wllm_gemm_generic(const void* x, const void* w, const void* tiles, 
 #undef FEW_ROWS
             return launch_status();
         }
-        if (!of) return -1;
-        // tiles of 128 x 128 where they fill the machine, smaller ones where a product has few columns or rows
-        const long long rows128 = (M + 127) / 128, cols128 = (N + 127) / 128, cols64 = (N + 63) / 64;
-        if (rows128 > 65535 || (M + 63) / 64 > 65535) return -1;
-        if (rows128 * cols128 >= 384) {
-            gemm_f32_tile_kernel<4, 4><<<dim3(cols128, rows128), 256, 0, stream>>>(xf, wf, of, M, N, K);
-        } else if (rows128 * cols64 >= 384) {
-            gemm_f32_tile_kernel<4, 2><<<dim3(cols64, rows128), 256, 0, stream>>>(xf, wf, of, M, N, K);
-        } else {
-            gemm_f32_tile_kernel<2, 2><<<dim3(cols64, (M + 63) / 64), 256, 0, stream>>>(xf, wf, of, M, N, K);
-        }
-        return launch_status();
+        float* pf = static_cast<float*>(partial);
+        const F32Cut cut = f32_cut(M, N, K, pf != nullptr);
+        const int segments = (K + kF32Segment - 1) / kF32Segment;
+        if (!of && !cut.per_group) return -1;
+        const dim3 grid((N + 32 * cut.wn - 1) / (32 * cut.wn), (M + 32 * cut.wm - 1) / (32 * cut.wm),
+                        cut.per_group ? (segments + cut.per_group - 1) / cut.per_group : 1);
+        if (grid.y > 65535) return -1;
+#define TILES(WM, WN)                                                                                                   \
+    do {                                                                                                                \
+        if (cut.per_group) gemm_f32_tile_kernel<WM, WN, true><<<grid, 256, 0, stream>>>(xf, wf, pf, M, N, K, cut.per_group); \
+        else gemm_f32_tile_kernel<WM, WN, false><<<grid, 256, 0, stream>>>(xf, wf, of, M, N, K, 0);                     \
+    } while (0)
+        if (cut.wm == 4 && cut.wn == 4) TILES(4, 4);
+        else if (cut.wm == 4) TILES(4, 2);
+        else if (cut.wn == 4) TILES(2, 4);
+        else TILES(2, 2);
+#undef TILES
+        if (const int err = launch_status()) return err;
+        return cut.per_group && of ? sum_segments(pf, of, static_cast<long long>(M) * N, segments, stream) : 0;
     }
     const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
     if (grid.y > 65535) return -1;

@@ -462,11 +462,15 @@ class HipBackend:
                 return
             self._generic(x, weight, out, segments, tiles)
             return
-        self._generic(x, weight, out, 1)
+        # float32, more rows: the kernel says whether it cuts the K axis over workgroups
+        segments = self.lib.wllm_gemm_f32_segments(m, weight.shape[0], k) if x.dtype == torch.float32 else 1
+        partial = torch.empty(segments * m * weight.shape[0], dtype=torch.float32, device=x.device) if segments > 1 else None
+        self._generic(x, weight, out, 1, partial=partial)
 
-    def _generic(self, x, weight, out, segments: int, tiles=None) -> None:
+    def _generic(self, x, weight, out, segments: int, tiles=None, partial=None) -> None:
         m, n = x.shape[0], weight.shape[0]
-        partial = self._gemm_partial(segments * m * n, x.device) if segments > 1 else None
+        if segments > 1:
+            partial = self._gemm_partial(segments * m * n, x.device)
         self._check(self.lib.wllm_gemm_generic(
             _ptr(x), _ptr(weight), _ptr(tiles) if x.dtype == torch.float32 else c_void_p(0), int(x.dtype == torch.bfloat16),
             _ptr(out), int(out.dtype == torch.bfloat16),
