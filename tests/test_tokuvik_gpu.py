@@ -213,6 +213,41 @@ def test_the_recurrence_whole_and_token_by_token(dtype, heads, groups, n_state, 
     close(out, plain.gated_group_norm(y.double(), z[:, 2:2 + inner].double(), w.double(), parts, 1e-5), dtype, "gated norm")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,groups,n_state,p,lengths", [
+    (4, 2, 16, 16, [64, 3, 80]), (3, 1, 7, 10, [63, 64, 65]), (2, 2, 130, 72, [79, 1]), (20, 1, 64, 20, [97]), (6, 3, 200, 33, [1, 300, 1, 70]),
+    (1, 1, 256, 4, [128]), (64, 8, 128, 64, [333, 40])])
+def test_the_recurrence_over_long_segments(dtype, heads, groups, n_state, p, lengths):
+    """Segments of 64 tokens and more go over the matrix cores in chunks of 16, the ones beside them token by token: on
+    either side of that line, whole chunks and one token more or less, rows of state and columns that fill no tile, more
+    heads a group than a pass of the operands' kernel, from states that are not zero."""
+    g = torch.Generator().manual_seed(n_state + p + len(lengths))
+    inner, slots_total = heads * p, len(lengths) + 2
+    width, n = inner + 2 * groups * n_state, sum(lengths)
+    xbc = (torch.randn(n, width, generator=g) * 0.7).to(dtype)
+    dt = torch.randn(n, heads + 3, generator=g).to(dtype)
+    dt_bias, a_log, d_skip = -1.0 + torch.randn(heads, generator=g), -0.5 + 0.8 * torch.randn(heads, generator=g), 1 + 0.3 * torch.randn(heads, generator=g)
+    state0 = torch.randn(slots_total, heads * n_state * p + 9, generator=g)
+    q_len, q_start, _, slots = _segments(lengths, g, slots_total)
+    state, y = state0.to(DEV), torch.full((n, inner), 7.0, device=DEV)
+    ops.ssm_scan(xbc.to(DEV), dt.to(DEV)[:, 1:1 + heads], dt_bias.to(DEV), a_log.to(DEV), d_skip.to(DEV), state, q_start.to(DEV),
+                 q_len.to(DEV), slots.to(DEV), y, heads=heads, groups=groups, state_size=n_state, head_dim=p)
+    for i, (at, length) in enumerate(zip(q_start.tolist(), lengths)):
+        s64 = xbc[at:at + length].double()
+        first = state0[int(slots[i]), :heads * n_state * p].double().view(heads, n_state, p)
+        want, last = plain.state_space_recurrence(
+            s64[:, :inner].view(-1, heads, p), s64[:, inner:inner + groups * n_state].view(-1, groups, n_state),
+            s64[:, inner + groups * n_state:].view(-1, groups, n_state),
+            plain.softplus(dt[at:at + length, 1:1 + heads].double() + dt_bias.double()), a_log.double(), d_skip.double(), first)
+        # float32 sums of up to 256 products a token and of every token before: a few units of 2^-24 of the largest
+        close(y[at:at + length], want.reshape(-1, inner), torch.float32, f"segment {i}", scale=float(want.abs().max()))
+        kept = state[int(slots[i]), :heads * n_state * p].view(heads, n_state, p)
+        close(kept, last, torch.float32, f"the state segment {i} leaves", scale=float(last.abs().max()))
+    assert torch.equal(state[:, heads * n_state * p:].cpu(), state0[:, heads * n_state * p:]), "what lies behind the states"
+    others = [i for i in range(slots_total) if i not in slots.tolist()]
+    assert torch.equal(state[others].cpu(), state0[others]), "a state of another request changed"
+
+
 def _attention_problem(dtype, nh, nkv, d, ps, segs, seed, extra_columns):
     g = torch.Generator().manual_seed(seed)
     n = sum(q for q, _ in segs)

@@ -229,11 +229,11 @@ __global__ void __launch_bounds__(kWave * kScanWaves)
 ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int tokens,
                 const float* __restrict__ d_skip, float* __restrict__ state, long long state_stride, const int* __restrict__ seg_q_start,
                 const int* __restrict__ seg_q_len, const int* __restrict__ state_slots, float* __restrict__ y, int heads,
-                int groups, int n_state, int p_dim) {
+                int groups, int n_state, int p_dim, int shorter_than) {
     extern __shared__ __align__(16) float smem[];
     const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * kScanCols;
     const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
-    if (q_len <= 0) return;
+    if (q_len <= 0 || q_len >= shorter_than) return;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int col = lane % kScanCols, slice = wave * kScanLaneSlices + lane / kScanCols;
     const int p = p0 + col;
@@ -352,15 +352,311 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
     }
 }
 
-// `steps`: scratch of 2 * tokens * heads floats (the step sizes, then the decays).
+// ---- the same recurrence over many tokens, 16 at a time on the matrix cores.  With f_t, d_t the decay and the step of
+// a head's token t, pre_t the product of a chunk's decays up to t, and suf_s that of the decays behind s,
+//   y_t = pre_t (C_t . S0) + sum over s <= t of N_ts x_s + D x_t,   S = pre_16 S0 + B^T (suf_s d_s x_s),
+//   N_ts = (C_t . B_s) (the decays s < r <= t) d_s.
+// A product of decays is formed from the decays it is made of (never as a quotient or a difference of logarithms), so
+// the numbers are those of the walk token by token up to the order of float32 sums.  Nothing but S0 depends on the
+// tokens before, so `ssm_chunk_kernel` makes all else for every chunk at once: per (chunk, group) the rows C_t and the
+// transposed B, per (chunk, head) N, pre, suf d and pre_16; and `ssm_chunk_scan_kernel` walks a segment's chunks with
+// v_mfma_f32_16x16x4_f32 (float32 in and out), 17 of them a wavefront and chunk.  A chunk begins every 16 tokens of a
+// segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).  Chunk c of segment s lies
+// at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// The walk token by token is bound by its chain (0.27 us a token).  64 heads of 64 with 128 rows of state: 1,500 tokens
+// 410 us token by token, 13 and 90 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
+// 64 tokens 21 us against 7 and 9, which is where the line between the two ways lies. ----
+constexpr int kChunk = 16;
+constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, suf d, pre_16 (and padding)
+
+// The operands of a chunk and a group: 28 us at 8 heads a group with a thread an entry of N that multiplied its decays one
+// after the other as it read them, 7 (6 chunks) to 13 (95) with a head a wavefront, a lane's 16 decays read at once and the products C_t . B_s
+// on the matrix cores.
+typedef float ssm_float4 __attribute__((ext_vector_type(4)));
+
+template <typename T, int TILES>        // C = 64 TILES: the rows of state, padded
+__global__ void __launch_bounds__(256)
+ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long long dt_stride, const float* __restrict__ dt_bias,
+                 const float* __restrict__ a_log, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                 int segments, float* __restrict__ of_head, T* __restrict__ of_group, int heads, int groups, int n_state,
+                 int p_dim, int from) {
+    constexpr int C = 64 * TILES, kRow = C + 4;
+    __shared__ __align__(16) float b_s[kChunk * kRow], c_s[kChunk * kRow];
+    __shared__ __align__(16) float f_s[kChunk][kChunk], dt_s[kChunk][kChunk];          // [head of sixteen][token]
+    __shared__ ssm_float4 g_s[4][kWave];
+    __shared__ int found;
+    const int place = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+    if (tid == 0) found = -1;
+    __syncthreads();
+    for (int s = tid; s < segments; s += 256) {
+        const int first = seg_q_start[s] / kChunk + s, len = seg_q_len[s];
+        if (len >= from && place >= first && place < first + (len + kChunk - 1) / kChunk) found = s;
+    }
+    __syncthreads();
+    const int seg = found;
+    if (seg < 0) return;
+    const int q_start = seg_q_start[seg], local = (place - q_start / kChunk - seg) * kChunk;
+    const int count = min(kChunk, seg_q_len[seg] - local), token = q_start + local;
+    const int inner = heads * p_dim, channels = inner + 2 * groups * n_state;
+    const int b_col = inner + g * n_state, c_col = b_col + groups * n_state;
+    T* rows = of_group + (static_cast<size_t>(place) * groups + g) * 2 * kChunk * C;
+    constexpr int kEach = kChunk * C / 256;
+    T b[kEach], c[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int t = (tid + 256 * k) / C, n = (tid + 256 * k) % C;
+        const T* row = xbc + static_cast<size_t>(token + min(t, count - 1)) * channels + min(n, n_state - 1);
+        b[k] = row[b_col];
+        c[k] = row[c_col];
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int t = (tid + 256 * k) / C, n = (tid + 256 * k) % C;
+        const bool there = t < count && n < n_state;
+        const T bv = there ? b[k] : from_float<T>(0.f), cv = there ? c[k] : from_float<T>(0.f);
+        b_s[t * kRow + n] = to_float(bv);
+        c_s[t * kRow + n] = to_float(cv);
+        rows[tid + 256 * k] = cv;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int e = tid + 256 * k;
+        rows[kChunk * C + e] = from_float<T>(b_s[e % kChunk * kRow + e / kChunk]);
+    }
+    const int lane = tid % kWave, wave = tid / kWave, i = lane % 16, q = lane / 16;
+    {
+        // lane (i, q) takes what every wavefront's quarter of the rows gives of B_s . C_t for t = i, s = 4q .. 4q + 3
+        ssm_float4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) {
+            const int n = (wave * TILES + j) * 16 + 4 * q;
+            const ssm_float4 bv = *reinterpret_cast<const ssm_float4*>(b_s + i * kRow + n);
+            const ssm_float4 cv = *reinterpret_cast<const ssm_float4*>(c_s + i * kRow + n);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) part = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[u], cv[u], part, 0, 0, 0);
+        }
+        g_s[wave][lane] = part;
+    }
+    const int per_group = heads / groups;
+    for (int h0 = 0; h0 < per_group; h0 += kChunk) {
+        {
+            const int hh = tid / kChunk, t = tid % kChunk, h = g * per_group + h0 + hh;
+            float step = 0.f, decay = 1.f;
+            if (h0 + hh < per_group && t < count) {
+                step = softplus(to_float(dt_in[static_cast<size_t>(token + t) * dt_stride + h]) + dt_bias[h]);
+                decay = expf(-expf(a_log[h]) * step);
+            }
+            if (h0 > 0) __syncthreads();                  // the sixteen heads before are done with
+            dt_s[hh][t] = step;
+            f_s[hh][t] = decay;
+        }
+        __syncthreads();
+        ssm_float4 dot = g_s[0][lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) dot += g_s[w][lane];
+        for (int hh = wave; hh < min(kChunk, per_group - h0); hh += 4) {
+            float* out = of_head + (static_cast<size_t>(place) * heads + g * per_group + h0 + hh) * kChunkHeadFloats;
+            float f[kChunk];
+#pragma unroll
+            for (int r = 0; r < kChunk; r += 4) *reinterpret_cast<ssm_float4*>(f + r) = *reinterpret_cast<const ssm_float4*>(&f_s[hh][r]);
+            const ssm_float4 step = *reinterpret_cast<const ssm_float4*>(&dt_s[hh][4 * q]);
+            // the decays between s and t = i for s = 4q + 3, and from there down.  (Products in 64 bits, rounded once: a
+            // whole row of sums shares their error, where the walk token by token rounds every element for itself.)
+            double between = 1.0;
+#pragma unroll
+            for (int r = 4; r < kChunk; ++r) between *= r > 4 * q + 3 && r <= i ? f[r] : 1.f;
+            ssm_float4 n;
+#pragma unroll
+            for (int u = 3; u >= 0; --u) {
+                const int s = 4 * q + u;
+                n[u] = s <= i ? dot[u] * static_cast<float>(between * step[u]) : 0.f;
+                between *= s <= i ? f_s[hh][s] : 1.f;
+            }
+            *reinterpret_cast<ssm_float4*>(out + i * kChunk + 4 * q) = n;
+            // lanes of q = 0: the decays up to token i; of q = 1: those behind it, times its step; of q = 2: all of them
+            double v = q == 1 ? dt_s[hh][i] : 1.f;
+#pragma unroll
+            for (int r = 0; r < kChunk; ++r) v *= q == 2 || (q == 0 ? r <= i : r > i) ? f[r] : 1.f;
+            if (q < 3) out[kChunk * kChunk + q * kChunk + i] = static_cast<float>(v);
+        }
+    }
+}
+
+// A workgroup owns (head, segment, 16 columns of P); its four wavefronts cut the rows of state, each with TILES tiles of
+// 16: lane (i, g) holds the rows 4g .. 4g + 3 of a tile in column i, which is what a product leaves and, row by row, what
+// it takes (the k-th of four products takes the rows 4g + k), so the state never moves between lanes.  The wavefronts'
+// parts of y meet in shared memory (two places in turn: one barrier a chunk, which the state's own chain does not wait
+// for).  The operands of the next chunks are asked for kAhead chunks before they are used.
+template <typename T> struct alignas(4 * sizeof(T)) SsmFour { T v[4]; };
+
+template <typename T, int TILES>
+__global__ void __launch_bounds__(256)
+ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, const float* __restrict__ d_skip,
+                      float* __restrict__ state, long long state_stride, const int* __restrict__ seg_q_start,
+                      const int* __restrict__ seg_q_len, const int* __restrict__ state_slots, float* __restrict__ y, int heads,
+                      int groups, int n_state, int p_dim, int from) {
+    constexpr int C = 64 * TILES, kAhead = 4;
+    __shared__ ssm_float4 part_s[2][4][kWave];
+    const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * 16;
+    const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
+    if (q_len < from) return;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int i = lane % 16, g = lane / 16;
+    const int p = p0 + i;
+    const bool live = p < p_dim;
+    const int inner = heads * p_dim, channels = inner + 2 * groups * n_state;
+    float* s_rows = state + static_cast<size_t>(state_slots[seg]) * state_stride + static_cast<size_t>(h) * n_state * p_dim + p;
+    const int n0 = wave * 16 * TILES;
+    ssm_float4 s[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int n = n0 + 16 * j + 4 * g + u;
+            s[j][u] = live && n < n_state ? s_rows[static_cast<size_t>(n) * p_dim] : 0.f;
+        }
+    const float skip = d_skip[h];
+    struct Operands {
+        SsmFour<T> c[TILES], b[TILES];
+        ssm_float4 pre, suf;
+        float n, all;
+        T x[4];
+    };
+    const size_t first = static_cast<size_t>(q_start / kChunk + seg);
+    const float* head_first = of_head + (first * heads + h) * kChunkHeadFloats;
+    const T* group_first = of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C;
+    const T* x_first = xbc + static_cast<size_t>(q_start) * channels + h * p_dim;
+    float* y_first = y + static_cast<size_t>(q_start) * inner + h * p_dim;
+    // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
+    const unsigned c_at = i * C + n0 + 4 * g, b_at = kChunk * C + (n0 + i) * kChunk + 4 * g;
+    const unsigned n_at = i * kChunk + 4 * g + wave, pre_at = kChunk * kChunk + 4 * g;
+    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(channels);
+    auto load = [&](int c) {
+        Operands o;
+        const T* rows = group_first + static_cast<size_t>(c) * groups * 2 * kChunk * C;
+        const float* of = head_first + static_cast<size_t>(c) * heads * kChunkHeadFloats;
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) {
+            o.c[j] = *reinterpret_cast<const SsmFour<T>*>(rows + c_at + 16 * j);
+            o.b[j] = *reinterpret_cast<const SsmFour<T>*>(rows + b_at + 16 * kChunk * j);
+        }
+        o.n = of[n_at];
+        o.pre = *reinterpret_cast<const ssm_float4*>(of + pre_at);
+        o.suf = *reinterpret_cast<const ssm_float4*>(of + pre_at + kChunk);
+        o.all = of[kChunk * kChunk + 2 * kChunk];
+        const T* x_chunk = x_first + static_cast<size_t>(c) * kChunk * channels;
+        const unsigned beyond = (min(kChunk, q_len - c * kChunk) - 1) * row;          // the chunk's last token
+        // (beyond it, that token's once more: what it is multiplied by is zero)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o.x[u] = x_chunk[min((4 * g + u) * row, beyond) + col];
+        return o;
+    };
+    const int count = (q_len + kChunk - 1) / kChunk;
+    auto walk = [&](int c, const Operands& now) {
+        ssm_float4 x, read = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = c * kChunk + 4 * g + u < q_len ? to_float(now.x[u]) : 0.f;
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                read = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.c[j].v[u]), s[j][u], read, 0, 0, 0);
+        const ssm_float4 moved = x * now.suf;
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) s[j] *= now.all;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < TILES; ++j)
+                s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.b[j].v[u]), moved[u], s[j], 0, 0, 0);
+        // a wavefront's part: its rows of the state, and the chunk's own tokens 4g + wave
+        const float mine = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
+        read *= now.pre;
+        read = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, read, 0, 0, 0);
+        part_s[c % 2][wave][lane] = read;
+        // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // wavefront w writes the tokens 4g + w
+        const float* parts = reinterpret_cast<const float*>(&part_s[c % 2][0][lane]) + wave;
+        float o = parts[0];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
+        const int t = 4 * g + wave;
+        if (live && c * kChunk + t < q_len)
+            (y_first + static_cast<size_t>(c) * kChunk * inner)[t * static_cast<unsigned>(inner) + col] = fmaf(skip, mine, o);
+    };
+    // the operands of kAhead chunks in turn (beyond the last chunk: the last's once more).  The loads stay where they are
+    // written: the scratch and xbc may alias y as far as the compiler knows, and the empty statements touch memory.
+    Operands ring[kAhead];
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d) ring[d] = load(min(d, count - 1));
+    int c = 0;
+    for (; c + kAhead <= count; c += kAhead) {
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) {
+            walk(c + d, ring[d]);
+            ring[d] = load(min(c + d + kAhead, count - 1));
+            asm volatile("" ::: "memory");
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d)
+        if (c + d < count) walk(c + d, ring[d]);
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int n = n0 + 16 * j + 4 * g + u;
+            if (live && n < n_state) s_rows[static_cast<size_t>(n) * p_dim] = s[j][u];
+        }
+}
+
+// `steps`: scratch of 2 * tokens * heads floats (the step sizes, then the decays).  `from` tokens (16 at least; 0: no
+// segment) is what a segment needs to be walked in chunks, out of the scratch `chunks`: a place for every chunk of every
+// segment (tokens / 16 + segments + 1), first [place][head] of kChunkHeadFloats floats, then [place][group] of
+// 32 x (the rows of state padded to a multiple of 64) elements.
 WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stride, const float* dt_bias, const float* a_log,
                            const float* d_skip, float* state, long long state_stride, const int* seg_q_start,
                            const int* seg_q_len, const int* state_slots, float* y, float* steps, int is_bf16, int tokens,
-                           int segments, int heads, int groups, int n_state, int p_dim, hipStream_t stream) {
+                           int segments, int heads, int groups, int n_state, int p_dim, float* chunks, int from,
+                           hipStream_t stream) {
     if (segments <= 0 || tokens <= 0) return 0;
     if (!steps) return -1;
     if (heads <= 0 || groups <= 0 || heads % groups != 0 || n_state <= 0 || n_state > 16 * kScanSlices || p_dim <= 0) return -1;
     if (segments > 65535 || (p_dim + kScanCols - 1) / kScanCols > 65535) return -1;
+    const dim3 grid(heads, segments, (p_dim + kScanCols - 1) / kScanCols);
+    // (a segment of `from` tokens leaves room for the others' single tokens)
+    const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
+    if (in_chunks) {
+        if (!chunks || from < kChunk || n_state > 256 || groups > 65535 || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
+        const int places = tokens / kChunk + segments + 1;
+        const dim3 chunk_grid(places, groups);
+        float* of_group = chunks + static_cast<size_t>(places) * heads * kChunkHeadFloats;
+#define LAUNCH(T, TILES)                                                                                               \
+    do {                                                                                                               \
+        ssm_chunk_kernel<T, TILES><<<chunk_grid, 256, 0, stream>>>(                                                    \
+            static_cast<const T*>(xbc), static_cast<const T*>(dt_in), dt_stride, dt_bias, a_log, seg_q_start, seg_q_len, \
+            segments, chunks, reinterpret_cast<T*>(of_group), heads, groups, n_state, p_dim, from);                    \
+        if (const int err = launch_status()) return err;                                                               \
+        ssm_chunk_scan_kernel<T, TILES><<<grid, 256, 0, stream>>>(                                                     \
+            chunks, reinterpret_cast<const T*>(of_group), static_cast<const T*>(xbc), d_skip, state, state_stride, seg_q_start, \
+            seg_q_len, state_slots, y, heads, groups, n_state, p_dim, from);                                           \
+    } while (0)
+#define LAUNCH_TILES(T)                     \
+    if (n_state <= 64) LAUNCH(T, 1);        \
+    else if (n_state <= 128) LAUNCH(T, 2);  \
+    else if (n_state <= 192) LAUNCH(T, 3);  \
+    else LAUNCH(T, 4);
+        if (is_bf16) { LAUNCH_TILES(bf16) } else { LAUNCH_TILES(float) }
+#undef LAUNCH_TILES
+#undef LAUNCH
+        if (const int err = launch_status()) return err;
+        if (segments == 1) return 0;
+    }
+    const int shorter_than = in_chunks ? from : 0x7fffffff;
     const int r = (n_state + kScanSlices - 1) / kScanSlices;
     {
         const int total = tokens * heads, blocks = (total + 255) / 256;
@@ -373,13 +669,12 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
         if (const int err = launch_status()) return err;
     }
     const int n_pad = (n_state + 3) / 4 * 4;
-    const dim3 grid(heads, segments, (p_dim + kScanCols - 1) / kScanCols);
     const size_t smem = sizeof(float) * (2 * kScanTokens * n_pad + kScanTokens * kScanCols + 2 * kScanTokens +
                                          kScanTokens * kScanWaves * kScanCols);
 #define LAUNCH(T, R, V)                                                                                             \
     ssm_scan_kernel<T, R, (R * kScanSlices + kScanFetchers - 1) / kScanFetchers, V><<<grid, kWave * kScanWaves, smem, stream>>>( \
         static_cast<const T*>(xbc), steps, tokens, d_skip, state, state_stride, seg_q_start, seg_q_len, state_slots, y, \
-        heads, groups, n_state, p_dim)
+        heads, groups, n_state, p_dim, shorter_than)
 #define LAUNCH_R(T)                                                                          \
     if (r <= 1) LAUNCH(T, 1, false);                                                         \
     else if (r <= 2) LAUNCH(T, 2, false);                                                    \

@@ -1016,6 +1016,25 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
              state_size, head_dim, steps)
 
 
+# tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
+# on the matrix cores
+SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
+
+
+def _scan_places(tokens: int, segments: int) -> int:
+    """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
+    return tokens // SCAN_CHUNK + segments + 1 if tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
+
+
+def _ssm_chunks(xbc: torch.Tensor, segments: int, heads: int, groups: int, state_size: int) -> Optional[torch.Tensor]:
+    """The scratch of the walk in chunks, or None (a decode step has none, so a captured graph holds no address of it)."""
+    places = _scan_places(xbc.shape[0], segments)
+    if not places:
+        return None
+    rows = 2 * SCAN_CHUNK * (-(-state_size // 64) * 64) * xbc.element_size() // 4
+    return torch.empty(places * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows), dtype=torch.float32, device=xbc.device)
+
+
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
                      eps: float) -> None:
     """out = v / sqrt(mean over the part (v^2) + eps) * weight with v = y * silu(z), the row cut into
@@ -1597,12 +1616,14 @@ def _register_own() -> None:
                     weight.shape[0], int(single_tokens), stream))
     register_op("ssm_scan", entry_point="wllm_ssm_scan",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
-                          c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+                          c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                          c_int, c_void_p],
                 launch=lambda fn, stream, xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y,
                 heads, groups, state_size, head_dim, steps: fn(
                     p(xbc), p(dt), dt.stride(0), p(dt_bias), p(a_log), p(d_skip), p(state), state.stride(0), p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(steps), int(xbc.dtype == torch.bfloat16), xbc.shape[0],
-                    seg_q_start.shape[0], heads, groups, state_size, head_dim, stream))
+                    seg_q_start.shape[0], heads, groups, state_size, head_dim,
+                    p(_ssm_chunks(xbc, seg_q_start.shape[0], heads, groups, state_size)), SCAN_CHUNK_FROM, stream))
     register_op("gated_group_norm", entry_point="wllm_gated_group_norm",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
                 launch=lambda fn, stream, y, z, weight, out, groups, eps: fn(
