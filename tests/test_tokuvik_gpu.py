@@ -162,6 +162,46 @@ def test_the_convolution_whole_and_cut_with_its_carried_inputs(dtype, channels, 
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("channels,extra,lengths", [(40, 8, [1, 70, 3, 2]), (1028, 4, [64]), (42, 2, [66, 1]), (64, 3, [9, 8, 7, 6, 5, 33]), (2048, 0, [63, 1, 1])])
+def test_convolutions_of_many_tokens_have_the_bits_of_few(dtype, channels, extra, lengths):
+    """From 64 tokens on a thread walks tokens with the last inputs in registers (4 taps; channels and strides in fours, else
+    the kernel for any): the bits of the same segments in steps of fewer tokens, in both convolutions, from carried rows,
+    with segments that begin inside a thread's run of tokens."""
+    g = torch.Generator().manual_seed(channels + len(lengths))
+    n, slots_total = sum(lengths), len(lengths) + 2
+    rows = torch.randn(n, channels + extra, generator=g).to(dtype).to(DEV)
+    stream = torch.randn(n, channels, generator=g).to(DEV)
+    weight, bias = torch.randn(channels, 4, generator=g).to(DEV), torch.randn(channels, generator=g).to(DEV)
+    offset, first = 8, extra // 2        # a band that begins at a multiple of four elements, or not
+    state0 = torch.randn(slots_total, offset + 3 * channels, generator=g).to(DEV)
+    q_len, q_start, tok_seg, slots = _segments(lengths, g, slots_total)
+
+    def run(segments):
+        state_a, state_b, out = state0.clone(), state0.clone(), torch.zeros(2, n, channels, dtype=dtype, device=DEV)
+        for part in segments:
+            lo, hi = int(q_start[part[0]]), int(q_start[part[-1]] + q_len[part[-1]])
+            seg = (tok_seg[lo:hi] - part[0], q_start[part] - lo, q_len[part], slots[part])
+            seg = [t.to(torch.int32).to(DEV) for t in seg]
+            ops.causal_conv(rows[lo:hi, first:first + channels], weight, bias, state_a, offset, *seg, out[0, lo:hi])
+            ops.stream_conv(stream[lo:hi], weight.t().contiguous(), state_b, offset, *seg, out[1, lo:hi])
+        return out, state_a, state_b
+
+    def cut():
+        out, state_a, state_b = torch.zeros(2, n, channels, dtype=dtype, device=DEV), state0.clone(), state0.clone()
+        for i, length in enumerate(lengths):
+            for a in range(0, length, 20):
+                b = min(length, a + 20)
+                lo, hi = int(q_start[i]) + a, int(q_start[i]) + b
+                seg = [torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0] * (b - a), [0], [b - a], [int(slots[i])])]
+                ops.causal_conv(rows[lo:hi, first:first + channels], weight, bias, state_a, offset, *seg, out[0, lo:hi])
+                ops.stream_conv(stream[lo:hi], weight.t().contiguous(), state_b, offset, *seg, out[1, lo:hi])
+        return out, state_a, state_b
+
+    for got, want in zip(run([list(range(len(lengths)))]), cut()):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("heads,groups,n_state,p", [(4, 2, 16, 16), (3, 1, 7, 10), (2, 2, 130, 72), (6, 3, 48, 64), (1, 1, 256, 4)])
 def test_the_recurrence_whole_and_token_by_token(dtype, heads, groups, n_state, p):
     """Sequences side by side through the recurrence's kernel: whole, and cut down to single tokens, from

@@ -33,6 +33,93 @@ causal_conv_kernel(const T* __restrict__ in, long long in_stride, const float* _
     }
 }
 
+// The same sums for the many tokens of a prompt's portion and convolutions of kSlideTaps taps: a thread takes four
+// consecutive channels and walks kSlideTokens tokens with the last inputs in registers, so a row is read once and not
+// once a tap, in 8-byte (float32: 16-byte) pieces (6,144 channels of 1,500 tokens: 62 to 17 us).
+constexpr int kSlideTaps = 4, kSlideTokens = 8, kSlideFrom = 64;
+template <typename T> struct alignas(4 * sizeof(T)) ConvFour { T v[4]; };
+
+template <typename T>
+__device__ __forceinline__ float4 conv_four(const T* p) {
+    const ConvFour<T> r = *reinterpret_cast<const ConvFour<T>*>(p);
+    return make_float4(to_float(r.v[0]), to_float(r.v[1]), to_float(r.v[2]), to_float(r.v[3]));
+}
+
+// Walks `count` tokens from `token0`, four channels at `in`: calls make(token, rows) with the rows of the last
+// kSlideTaps inputs, the oldest first.  Inputs before a segment's first token are its request's carried rows.
+template <typename T, typename MAKE>
+__device__ __forceinline__ void slide(const T* in, long long in_stride, const float* state, long long state_stride,
+                                      long long carried_offset, const int* token_segment, const int* seg_q_start,
+                                      const int* state_slots, int channels, int token0, int count, MAKE make) {
+    float4 rows[kSlideTaps];
+    auto before = [&](int token, int seg, int local) {             // the rows that a token at place `local` finds
+        const float* carried = state + static_cast<size_t>(state_slots[seg]) * state_stride + carried_offset;
+#pragma unroll
+        for (int k = 1; k < kSlideTaps; ++k) {
+            const int src = local - kSlideTaps + k;
+            rows[k] = src >= 0 ? conv_four(in + static_cast<size_t>(token - local + src) * in_stride)
+                               : *reinterpret_cast<const float4*>(carried + static_cast<size_t>(kSlideTaps - 1 + src) * channels);
+        }
+    };
+    ConvFour<T> now[kSlideTokens];
+    int segs[kSlideTokens];
+#pragma unroll
+    for (int t = 0; t < kSlideTokens; ++t) {
+        const int token = token0 + min(t, count - 1);
+        now[t] = *reinterpret_cast<const ConvFour<T>*>(in + static_cast<size_t>(token) * in_stride);
+        segs[t] = token_segment[token];
+    }
+    before(token0, segs[0], token0 - seg_q_start[segs[0]]);
+#pragma unroll
+    for (int t = 0; t < kSlideTokens; ++t) {
+        if (t >= count) break;
+        if (t > 0 && segs[t] != segs[t - 1]) before(token0 + t, segs[t], 0);
+#pragma unroll
+        for (int k = 0; k + 1 < kSlideTaps; ++k) rows[k] = rows[k + 1];
+        rows[kSlideTaps - 1] = make_float4(to_float(now[t].v[0]), to_float(now[t].v[1]), to_float(now[t].v[2]), to_float(now[t].v[3]));
+        make(token0 + t, rows);
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+causal_conv_slide_kernel(const T* __restrict__ in, long long in_stride, const float* __restrict__ weight,
+                         const float* __restrict__ bias, const float* __restrict__ state, long long state_stride,
+                         long long carried_offset, const int* __restrict__ token_segment, const int* __restrict__ seg_q_start,
+                         const int* __restrict__ state_slots, T* __restrict__ out, int tokens, int channels) {
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4, token0 = blockIdx.x * kSlideTokens;
+    if (c >= channels) return;
+    float4 w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = *reinterpret_cast<const float4*>(weight + static_cast<size_t>(c + u) * kSlideTaps);
+    const float4 b = *reinterpret_cast<const float4*>(bias + c);
+    slide(in + c, in_stride, state, state_stride, carried_offset + c, token_segment, seg_q_start, state_slots, channels, token0,
+          min(kSlideTokens, tokens - token0), [&](int token, const float4 (&rows)[kSlideTaps]) {
+        float acc[4] = {b.x, b.y, b.z, b.w};
+        const float* wf = reinterpret_cast<const float*>(w);
+#pragma unroll
+        for (int k = 0; k < kSlideTaps; ++k) {
+            acc[0] = fmaf(wf[k], rows[k].x, acc[0]);
+            acc[1] = fmaf(wf[4 + k], rows[k].y, acc[1]);
+            acc[2] = fmaf(wf[8 + k], rows[k].z, acc[2]);
+            acc[3] = fmaf(wf[12 + k], rows[k].w, acc[3]);
+        }
+        ConvFour<T> r;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) r.v[u] = from_float<T>(acc[u] / (1.f + expf(-acc[u])));
+        *reinterpret_cast<ConvFour<T>*>(out + static_cast<size_t>(token) * channels + c) = r;
+    });
+}
+
+// Whether the channels and the addresses let a thread take four channels of a row at once.
+template <typename T>
+static bool in_fours(const void* in, long long in_stride, const float* weight, const float* bias, const float* state,
+                     long long state_stride, long long carried_offset, const void* out, int channels) {
+    const uintptr_t vectors = reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(state);
+    return channels % 4 == 0 && in_stride % 4 == 0 && state_stride % 4 == 0 && carried_offset % 4 == 0 && vectors % 16 == 0 &&
+           (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % (4 * sizeof(T)) == 0;
+}
+
 WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* weight, const float* bias, float* state,
                               long long state_stride, long long carried_offset, const int* token_segment,
                               const int* seg_q_start, const int* seg_q_len, const int* state_slots, void* out,
@@ -41,7 +128,18 @@ WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* 
     if (channels <= 0 || taps < 1 || taps > 64) return -1;
     const int tiles = (channels + 255) / 256 < 64 ? (channels + 255) / 256 : 64;
     const dim3 grid(tokens, tiles), carry_grid(segments, tiles);
-    if (is_bf16)
+    const dim3 slide_grid((tokens + kSlideTokens - 1) / kSlideTokens, (channels / 4 + 255) / 256);
+#define SLIDE(T)                                                                                                        \
+    causal_conv_slide_kernel<T><<<slide_grid, 256, 0, stream>>>(static_cast<const T*>(in), in_stride, weight, bias, state, \
+                                                                state_stride, carried_offset, token_segment, seg_q_start, \
+                                                                state_slots, static_cast<T*>(out), tokens, channels)
+    const bool many = taps == kSlideTaps && tokens >= kSlideFrom;
+    if (many && is_bf16 && in_fours<bf16>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
+        SLIDE(bf16);
+    else if (many && !is_bf16 && in_fours<float>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
+        SLIDE(float);
+#undef SLIDE
+    else if (is_bf16)
         causal_conv_kernel<bf16><<<grid, 256, 0, stream>>>(static_cast<const bf16*>(in), in_stride, weight, bias, state,
                                                            state_stride, carried_offset, token_segment, seg_q_start,
                                                            state_slots, static_cast<bf16*>(out), channels, taps);
@@ -106,8 +204,6 @@ stream_conv_kernel(const float* __restrict__ x, const float* __restrict__ weight
 // The same sums, four consecutive channels a thread with 16-byte loads of x and of the carried rows (a prompt's
 // portion: the kernel is bound by what it moves).  Channels, the carried rows' offset and the state's row are
 // multiples of four floats.
-template <typename T> struct alignas(4 * sizeof(T)) ConvFour { T v[4]; };
-
 template <typename T>
 __global__ void __launch_bounds__(256)
 stream_conv_four_kernel(const float* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ state,
@@ -139,6 +235,38 @@ stream_conv_four_kernel(const float* __restrict__ x, const float* __restrict__ w
     }
 }
 
+// The same for convolutions of kSlideTaps taps over many tokens: every row of x read once (see `slide`;
+// 2,048 channels of 3,001 tokens: 19.2 to 9.5 us).
+template <typename T>
+__global__ void __launch_bounds__(256)
+stream_conv_slide_kernel(const float* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ state,
+                         long long state_stride, long long carried_offset, const int* __restrict__ token_segment,
+                         const int* __restrict__ seg_q_start, const int* __restrict__ state_slots, T* __restrict__ out,
+                         int tokens, int channels) {
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4, token0 = blockIdx.x * kSlideTokens;
+    if (c >= channels) return;
+    float4 w[kSlideTaps];
+#pragma unroll
+    for (int k = 0; k < kSlideTaps; ++k) w[k] = *reinterpret_cast<const float4*>(weight + static_cast<size_t>(k) * channels + c);
+    slide(x + c, static_cast<long long>(channels), state, state_stride, carried_offset + c, token_segment, seg_q_start, state_slots,
+          channels, token0, min(kSlideTokens, tokens - token0), [&](int token, const float4 (&rows)[kSlideTaps]) {
+        float4 acc = rows[kSlideTaps - 1];
+#pragma unroll
+        for (int k = 0; k < kSlideTaps; ++k) {
+            acc.x = fmaf(w[k].x, rows[k].x, acc.x);
+            acc.y = fmaf(w[k].y, rows[k].y, acc.y);
+            acc.z = fmaf(w[k].z, rows[k].z, acc.z);
+            acc.w = fmaf(w[k].w, rows[k].w, acc.w);
+        }
+        ConvFour<T> r;
+        r.v[0] = from_float<T>(acc.x);
+        r.v[1] = from_float<T>(acc.y);
+        r.v[2] = from_float<T>(acc.z);
+        r.v[3] = from_float<T>(acc.w);
+        *reinterpret_cast<ConvFour<T>*>(out + static_cast<size_t>(token) * channels + c) = r;
+    });
+}
+
 WLLM_API int wllm_stream_conv(const float* x, const float* weight, float* state, long long state_stride,
                               long long carried_offset, const int* token_segment, const int* seg_q_start,
                               const int* seg_q_len, const int* state_slots, void* out, int out_bf16, int tokens,
@@ -154,7 +282,17 @@ WLLM_API int wllm_stream_conv(const float* x, const float* weight, float* state,
                       reinterpret_cast<uintptr_t>(out) % 16 == 0;
     if (four) {
         const dim3 grid4(tokens, (channels / 4 + 255) / 256);
-        if (out_bf16)
+        const dim3 slide_grid((tokens + kSlideTokens - 1) / kSlideTokens, (channels / 4 + 255) / 256);
+        if (taps == kSlideTaps && tokens >= kSlideFrom) {
+            if (out_bf16)
+                stream_conv_slide_kernel<bf16><<<slide_grid, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
+                                                                               token_segment, seg_q_start, state_slots,
+                                                                               static_cast<bf16*>(out), tokens, channels);
+            else
+                stream_conv_slide_kernel<float><<<slide_grid, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
+                                                                                token_segment, seg_q_start, state_slots,
+                                                                                static_cast<float*>(out), tokens, channels);
+        } else if (out_bf16)
             stream_conv_four_kernel<bf16><<<grid4, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
                                                                      token_segment, seg_q_start, state_slots,
                                                                      static_cast<bf16*>(out), channels, taps);
