@@ -241,6 +241,11 @@ class CacheManager:
                 assert popped == page
                 self.groups[gi].pool.free(page, request)
             raise
+        if num_new_tokens == 1:           # a decoded token
+            pages = [rc.tables[gi][start // ps] for gi in range(len(self.groups))]
+            if any(page < 0 for page in pages):
+                raise PageAccountingError(f"request {request!r} writes to a page it gave back")
+            return [np.array([page * ps + start % ps], dtype=np.int32) for page in pages]
         pos = np.arange(start, end, dtype=np.int64)
         out = []
         for gi in range(len(self.groups)):

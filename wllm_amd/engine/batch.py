@@ -45,16 +45,20 @@ class Workspace:
     def __init__(self, device):
         self.device = device
         self._flat: dict = {}
+        self._views: dict = {}          # the view given last under each key: the layers of a step ask for the same one
         self._frozen = False
 
     def freeze(self) -> None:
         self._frozen = True
 
     def get(self, name: str, shape: tuple, dtype: torch.dtype) -> torch.Tensor:
+        key = (name, dtype)
+        view = self._views.get(key)
+        if view is not None and view.shape == shape:
+            return view
         count = 1
         for s in shape:
             count *= s
-        key = (name, dtype)
         flat = self._flat.get(key)
         if flat is None or flat.numel() < count:
             if self._frozen:
@@ -62,7 +66,8 @@ class Workspace:
                                    "but a captured graph holds its address")
             flat = torch.empty(max(count, 1), dtype=dtype, device=self.device)
             self._flat[key] = flat
-        return flat[:count].view(shape)
+        view = self._views[key] = flat[:count].view(shape)
+        return view
 
 
 class StepContext:

@@ -4,6 +4,7 @@ on the GPU, since a host pointer handed to a kernel faults the device."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import numpy as np
@@ -25,7 +26,8 @@ _raw_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _ptr(t):
-    return c_void_p(t.data_ptr()) if t is not None else c_void_p(0)
+    # (an address as an integer: the entry points' signatures make a pointer of it)
+    return t.data_ptr() if t is not None else None
 
 
 _SIGNATURES = {
@@ -99,11 +101,11 @@ class HipBackend:
             if t is not None and not t.is_cuda:
                 raise KernelError("a kernel operand is not on the GPU")
 
-    def _stream(self) -> c_void_p:
+    def _stream(self) -> int:
         # the raw handle of torch's current stream on this process's GPU, asked for at every launch
         if _raw_current_stream is not None:
-            return c_void_p(_raw_current_stream(self._device_index))
-        return c_void_p(torch.cuda.current_stream().cuda_stream)
+            return _raw_current_stream(self._device_index)
+        return torch.cuda.current_stream().cuda_stream
 
     @staticmethod
     def _check(code: int, what: str) -> None:
@@ -305,6 +307,7 @@ class HipBackend:
             "paged_attention")
 
     @staticmethod
+    @functools.lru_cache(maxsize=4096)
     def skinny_split(n: int, k: int) -> int:
         """Over how many workgroups the K axis of a few-row product is split: enough that about
         2,000 wavefronts stream weights at once, a function of the weight's shape only."""
@@ -349,6 +352,7 @@ class HipBackend:
     TILE_GATED_MAX_ROWS = 256
 
     @staticmethod
+    @functools.lru_cache(maxsize=4096)
     def tile_splits(n: int, k: int, rows: int = 128) -> int:
         """Over how many workgroups the tiled product splits the K axis: a function of the weight's
         shape up to 640 rows, so that a row's sums do not depend on the step's other rows there.

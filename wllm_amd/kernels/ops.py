@@ -54,7 +54,11 @@ def _need(cond: bool, msg) -> None:
 
 
 def _dense(t: torch.Tensor, name: str, dtype, shape=None) -> None:
-    # the messages are made only when a check fails: this runs for every operand of every launch
+    # this runs for every operand of every launch: what passes is found out in one line, the message of what fails is
+    # made only then
+    if (isinstance(t, torch.Tensor) and (t.dtype is dtype or (type(dtype) is tuple and t.dtype in dtype)) and t.is_contiguous()
+            and (shape is None or t.shape == shape)):
+        return
     if not isinstance(t, torch.Tensor):
         raise KernelShapeError(f"{name}: expected a tensor")
     if isinstance(dtype, tuple):
@@ -330,14 +334,14 @@ def paged_attention(qkv: torch.Tensor, cache: torch.Tensor, block_tables: torch.
     """
     width = num_heads * head_dim
     _dense(qkv, "qkv", _ACT)
-    _need(qkv.dim() == 2 and qkv.shape[1] >= width,
-          lambda: f"qkv: shape {tuple(qkv.shape)}, expected [n, at least {width}]")
+    if qkv.dim() != 2 or qkv.shape[1] < width:
+        raise KernelShapeError(f"qkv: shape {tuple(qkv.shape)}, expected [n, at least {width}]")
     n = qkv.shape[0]
     _need(num_heads % num_kv_heads == 0, "num_heads must be a multiple of num_kv_heads")
     _need(softcap >= 0.0, "softcap must not be negative (0: none)")
     _dense(cache, "cache", qkv.dtype)
-    _need(cache.dim() == 4 and tuple(cache.shape[1:]) == (2, num_kv_heads, page_size * head_dim),
-          lambda: f"cache: shape {tuple(cache.shape)}, expected [pages, 2, {num_kv_heads}, {page_size * head_dim}]")
+    if cache.dim() != 4 or cache.shape[1:] != (2, num_kv_heads, page_size * head_dim):
+        raise KernelShapeError(f"cache: shape {tuple(cache.shape)}, expected [pages, 2, {num_kv_heads}, {page_size * head_dim}]")
     _dense(block_tables, "block_tables", torch.int32)
     _need(block_tables.dim() == 2, "block_tables: expected [segments, pages]")
     s = block_tables.shape[0]
@@ -430,9 +434,10 @@ def _band(t: torch.Tensor, name: str, dtype, rows: int, cols: int) -> None:
     """A tensor [rows, cols] or a band of columns of a wider contiguous one."""
     if not isinstance(t, torch.Tensor) or t.dtype != dtype:
         raise KernelShapeError(f"{name}: expected a tensor of {dtype}")
-    _need(t.dim() == 2 and tuple(t.shape) == (rows, cols), lambda: f"{name}: shape {tuple(t.shape)}, expected {(rows, cols)}")
-    _need(rows == 0 or cols == 0 or (t.stride(1) == 1 and t.stride(0) >= cols),
-          lambda: f"{name}: strides {t.stride()}: rows must be runs of consecutive elements")
+    if t.shape != (rows, cols):
+        raise KernelShapeError(f"{name}: shape {tuple(t.shape)}, expected {(rows, cols)}")
+    if rows and cols and (t.stride(1) != 1 or t.stride(0) < cols):
+        raise KernelShapeError(f"{name}: strides {t.stride()}: rows must be runs of consecutive elements")
 
 
 def sigmoid_gate(a: torch.Tensor, gate: torch.Tensor, out: torch.Tensor, per: int = 1) -> None:
@@ -559,6 +564,9 @@ def tile_weight(weight: torch.Tensor, halves: int = 1) -> Optional[torch.Tensor]
 def _check_tiles(tiles, weight, halves: int) -> None:
     if tiles is None:
         return
+    if weight.dtype is torch.bfloat16 and tiles.dtype is torch.bfloat16 and weight.shape[1] % 32 == 0 and tiles.dim() == 1 \
+            and tiles.is_contiguous() and tiles.shape[0] == halves * (-(-(weight.shape[0] // halves) // 16) * 16 * weight.shape[1]):
+        return
     if weight.dtype == torch.float32:
         _need(weight.shape[1] % 4 == 0, "tiles: float32 weights have them only with in_features % 4 == 0")
         _dense(tiles, "tiles", weight.dtype, (tiled_size(weight.shape[0], weight.shape[1], torch.float32),))
@@ -577,8 +585,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, tiles: Opti
     _dense(x, "x", _ACT)
     _need(x.dim() == 2, "x: expected [rows, in]")
     _dense(weight, "weight", x.dtype)
-    _need(weight.dim() == 2 and weight.shape[1] == x.shape[1],
-          lambda: f"weight: shape {tuple(weight.shape)}, expected [out, {x.shape[1]}]")
+    if weight.dim() != 2 or weight.shape[1] != x.shape[1]:
+        raise KernelShapeError(f"weight: shape {tuple(weight.shape)}, expected [out, {x.shape[1]}]")
     _check_tiles(tiles, weight, 1)
     if out.dim() == 3:
         s = linear_splits(x.shape[0], weight.shape[0], x.shape[1], x.dtype)
@@ -1487,7 +1495,9 @@ def moe_experts_down(act: torch.Tensor, w: torch.Tensor, plan: torch.Tensor, wei
 # ---- the framework's own operations that go through the same door as a part's ------------------
 def _register_own() -> None:
     from ctypes import c_float, c_int, c_longlong, c_void_p
-    p = pointer
+    def p(t):                       # an address as an integer, which the signatures make a pointer of
+        return t.data_ptr() if t is not None else None
+
     register_op("embed_lookup", entry_point="wllm_embed_lookup",
                 argtypes=[c_void_p, c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
                 launch=lambda fn, stream, ids, table, scale, out: fn(
