@@ -218,6 +218,57 @@ def test_segments_of_a_batch_keep_their_own_memories(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind", ["exponential", "decay", "rows"])
+@pytest.mark.parametrize("heads,d,dv,lengths", [(2, 16, 16, [64, 3, 80]), (3, 7, 10, [63, 64, 65]), (2, 130, 72, [79, 1]), (1, 256, 33, [1, 300, 1, 70]),
+                                                (16, 128, 128, [333, 40]), (5, 64, 15, [97])])
+def test_the_memory_over_long_segments(dtype, kind, heads, d, dv, lengths):
+    """Segments of 64 tokens and more go over the matrix cores in chunks of 16, the ones beside them token by token, for
+    each kind of decay: on either side of that line, whole chunks and one token more or less, channels and columns that
+    fill no tile, a normaliser's column that begins a tile or ends one, from memories that are not zero."""
+    g = torch.Generator().manual_seed(d + dv + len(lengths))
+    n, slots_total, memory = sum(lengths), len(lengths) + 2, heads * d * dv
+    qk = torch.randn(3 if kind == "rows" else 2, n, heads * d, generator=g) * d ** -0.5
+    if kind == "rows":
+        qk[2] = torch.rand(n, heads * d, generator=g)
+    v = torch.randn(n, heads * dv + 3, generator=g).to(dtype)
+    decays = 1.0 - torch.logspace(0, -4, heads)                       # from forgetting all to forgetting hardly anything
+    steps = torch.rand(3, n, heads, generator=g)
+    state0 = torch.randn(slots_total, memory + heads * d + 5, generator=g)
+    q_len, q_start, slots = _segments(lengths, g, slots_total)
+    state, y, nq = state0.to(DEV), torch.full((n, heads * dv), 7.0, device=DEV), torch.full((n, heads), 7.0, device=DEV)
+    own = kind == "exponential"
+    ops.memory_scan(qk.to(DEV), v.to(DEV)[:, 1:1 + heads * dv], steps.to(DEV) if own else None, decays.to(DEV) if kind == "decay" else None,
+                    state, q_start.to(DEV), q_len.to(DEV), slots.to(DEV), y, heads=heads, head_dim=d, value_dim=dv,
+                    nq=nq if own else None, n_offset=memory + 2 if own else 0, row_decays=kind == "rows")
+    for i, (at, length) in enumerate(zip(q_start.tolist(), lengths)):
+        row = state0[int(slots[i])].double()
+        S, norm = row[:memory].view(heads, d, dv).clone(), row[memory + 2:memory + 2 + heads * d].view(heads, d).clone()
+        want, want_nq = [], []
+        for t in range(at, at + length):
+            q, k = qk[0, t].double().view(heads, d), qk[1, t].double().view(heads, d)
+            x = v[t, 1:1 + heads * dv].double().view(heads, dv)
+            f = qk[2, t].double().view(heads, d) if kind == "rows" else (steps[0, t] if own else decays).double()[:, None].expand(heads, d)
+            k = k * steps[1, t].double()[:, None] if own else k
+            S = f[:, :, None] * S + k[:, :, None] * x[:, None]
+            norm = f * norm + k
+            want.append((S * q[:, :, None]).sum(1).reshape(-1))
+            want_nq.append((norm * q).sum(-1))
+        want = torch.stack(want)
+        # float32 sums of up to 256 products a token and of every token before: a few units of 2^-24 of the largest
+        close(y[at:at + length], want, torch.float32, f"segment {i}", scale=float(want.abs().max()))
+        kept = state[int(slots[i])]
+        close(kept[:memory].view(heads, d, dv), S, torch.float32, f"the memory segment {i} leaves", scale=float(S.abs().max()))
+        if own:
+            close(nq[at:at + length], torch.stack(want_nq), torch.float32, f"n . q of segment {i}", scale=float(torch.stack(want_nq).abs().max()))
+            close(kept[memory + 2:memory + 2 + heads * d].view(heads, d), norm, torch.float32, f"the normaliser segment {i} leaves",
+                  scale=float(norm.abs().max()))
+        behind = memory + 2 + heads * d if own else memory
+        assert torch.equal(kept[behind:].cpu(), state0[int(slots[i]), behind:]) and torch.equal(kept[memory:memory + 2].cpu(), state0[int(slots[i]), memory:memory + 2])
+    others = [i for i in range(slots_total) if i not in slots.tolist()]
+    assert torch.equal(state[others].cpu(), state0[others]), "a memory of another request changed"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,width,ff,count,top,groups,keep", [
     (1, 64, 48, 6, 2, 3, 2), (9, 128, 256, 5, 2, 1, 1), (7, 48, 24, 5, 3, 5, 5), (40, 96, 70, 8, 3, 4, 2), (300, 128, 96, 16, 4, 4, 2), (33, 36, 10, 1, 1, 1, 1),
     (90, 64, 32, 12, 1, 3, 1), (5, 256, 130, 4, 4, 2, 2), (130, 50, 16, 9, 6, 3, 2),

@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(kMemThreads)
 memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long long v_stride, const float* __restrict__ steps,
                    const float* __restrict__ decays, float* __restrict__ state, long long state_stride, long long n_offset,
                    const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len, const int* __restrict__ state_slots,
-                   float* __restrict__ y, float* __restrict__ nq, int tokens, int heads, int d, int p_dim) {
+                   float* __restrict__ y, float* __restrict__ nq, int tokens, int heads, int d, int p_dim, int shorter_than) {
     constexpr int kRow = kMemSlices * R;                   // a token's row of q (and of k) in shared memory: d and zeros
     constexpr int kPasses = kMemTokens * kRow / kMemThreads;      // elements of q (and of k) a thread stages: R
     constexpr int kRowsPass = kMemThreads / kRow;          // tokens a pass covers
@@ -211,7 +211,7 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
     __shared__ float part_s[kMemTokens * kMemWaves * kMemCols];
     const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * kMemCols;
     const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
-    if (q_len <= 0) return;
+    if (q_len <= 0 || q_len >= shorter_than) return;
     const int tid = threadIdx.x;
     const int lane = tid % kWave, wave = tid / kWave;
     const int col = lane % kMemCols, slice = wave * (kWave / kMemCols) + lane / kMemCols;
@@ -323,13 +323,267 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
     }
 }
 
+// ---- the same recurrence over many tokens, 16 at a time on the matrix cores.  Per head, with f_t the decays of token t (a
+// number a channel; the same in all channels unless the decays are a row's own) and k_t the key times its b_t,
+//   y_t = (P_t q_t) . S0 + sum over s <= t of N_ts v_s,   S = P_16 S0 + Kh^T V,   N_ts = q_t . (the decays s < r <= t) k_s,
+// P_t the product of a chunk's decays up to t, Kh_s = k_s times the decays behind s.  A product of decays is formed from
+// the decays it is made of, never as a quotient, so the numbers are those of the walk token by token up to the order of
+// float32 sums.  Nothing but S0 depends on the tokens before: `memory_chunk_kernel` makes P q, Kh, P_16 and N for every
+// chunk and head at once ([16][C], [C][16], [C], [16][16] floats, C = the channels padded to a multiple of 64), and
+// `memory_chunk_scan_kernel` walks a segment's chunks with v_mfma_f32_16x16x4_f32 (float32 in and out).  A chunk begins
+// every 16 tokens of a segment; the last one is filled with tokens that change nothing (q = k = 0, f = 1).  Chunk c of
+// segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 27 and
+// 138 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 15 and 112, with
+// exponential gates and the normaliser 297 against 15 and 110; 64 tokens 12.6 against 7 and 8, from where on a segment
+// gains.  Off the result in 64 bits: decays a head 2.0e-7 (token by token 3.1e-7), decays a row 9.6e-8 (9.2e-8). ----
+constexpr int kChunk = 16;
+typedef float memory_float4 __attribute__((ext_vector_type(4)));
+
+static __host__ __device__ __forceinline__ size_t chunk_floats(int c) { return static_cast<size_t>(2 * kChunk + 1) * c + kChunk * kChunk; }
+
+// The sum over a row of 16 lanes, in every lane.
+__device__ __forceinline__ float row_of_16_sum(float v) {
+    v += row_permuted<0x128>(v);
+    v += row_permuted<0x124>(v);
+    v += row_permuted<0x4E>(v);
+    v += row_permuted<0xB1>(v);
+    return v;
+}
+
+template <int R>        // C = 64 R
+__global__ void __launch_bounds__(256)
+memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ steps, const float* __restrict__ decays,
+                    const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len, int segments,
+                    float* __restrict__ chunks, int tokens, int heads, int d, int row_decays, int from) {
+    constexpr int C = 64 * R, kEach = kChunk * C / 256;
+    __shared__ __align__(16) float k_s[kChunk * C], q_s[kChunk * C], f_s[kChunk * C];
+    __shared__ int found;
+    const int place = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    if (tid == 0) found = -1;
+    __syncthreads();
+    for (int s = tid; s < segments; s += 256) {
+        const int first = seg_q_start[s] / kChunk + s, len = seg_q_len[s];
+        if (len >= from && place >= first && place < first + (len + kChunk - 1) / kChunk) found = s;
+    }
+    __syncthreads();
+    const int seg = found;
+    if (seg < 0) return;
+    const int q_start = seg_q_start[seg], local = (place - q_start / kChunk - seg) * kChunk;
+    const int count = min(kChunk, seg_q_len[seg] - local), token = q_start + local;
+    float* out = chunks + (static_cast<size_t>(place) * heads + h) * chunk_floats(C);
+    const size_t width = static_cast<size_t>(heads) * d, plane = static_cast<size_t>(tokens) * width;
+    float q[kEach], k[kEach], f[kEach];
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+        // (every load from a place that is there: what is not is put right below)
+        const int t = min((tid + 256 * j) / C, count - 1), i = min((tid + 256 * j) % C, d - 1);
+        const size_t at = static_cast<size_t>(token + t) * width + static_cast<size_t>(h) * d + i;
+        const size_t th = static_cast<size_t>(token + t) * heads + h;
+        q[j] = qk[at];
+        k[j] = qk[plane + at];
+        f[j] = row_decays ? qk[2 * plane + at] : steps ? steps[th] : decays[h];
+        if (steps) k[j] *= steps[static_cast<size_t>(tokens) * heads + th];
+    }
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+        const int e = tid + 256 * j;
+        const bool there = e / C < count && e % C < d;
+        q_s[e] = there ? q[j] : 0.f;
+        k_s[e] = there ? k[j] : 0.f;
+        f_s[e] = there ? f[j] : 1.f;
+    }
+    __syncthreads();
+    {
+        // N: 16 lanes hold the key of token s, which decays as t goes on
+        const int s = tid / kChunk, sl = tid % kChunk;
+        memory_float4 r[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) r[j] = *reinterpret_cast<const memory_float4*>(k_s + s * C + 64 * j + 4 * sl);
+        float mine = 0.f;                              // N of token sl and key s
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) {
+            memory_float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const int at = t * C + 64 * j + 4 * sl;
+                const memory_float4 qt = *reinterpret_cast<const memory_float4*>(q_s + at), ft = *reinterpret_cast<const memory_float4*>(f_s + at);
+                if (t > s) r[j] *= ft;
+                sum += r[j] * qt;
+            }
+            const float dot = row_of_16_sum((sum[0] + sum[1]) + (sum[2] + sum[3]));
+            if (sl == t && t >= s) mine = dot;
+        }
+        out[(2 * kChunk + 1) * C + sl * kChunk + s] = mine;
+    }
+    // the decays up to and behind every token, a channel a thread.  (Products in 64 bits, rounded once: where the decays
+    // are the head's, all channels share their error, which the walk token by token spreads over the state's elements.)
+    for (int c = tid; c < C; c += 256) {
+        double decay = 1.0, behind = 1.0;
+        float kh[kChunk];
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) {
+            decay *= f_s[t * C + c];
+            out[t * C + c] = static_cast<float>(q_s[t * C + c] * decay);
+        }
+        out[2 * kChunk * C + c] = static_cast<float>(decay);
+#pragma unroll
+        for (int t = kChunk - 1; t >= 0; --t) {
+            kh[t] = static_cast<float>(k_s[t * C + c] * behind);
+            behind *= f_s[t * C + c];
+        }
+        // (token 4u + g at place 4g + u: the u-th product of the walk then takes the tokens 4u .. 4u + 3, the oldest first)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<memory_float4*>(out + kChunk * C + c * kChunk + 4 * g) = memory_float4{kh[g], kh[4 + g], kh[8 + g], kh[12 + g]};
+    }
+}
+
+// A workgroup owns (head, segment, 16 columns of P; the column behind the last is the normaliser's, as above).  Its four
+// wavefronts cut the channels, each with TILES tiles of 16: lane (i, g) holds the channels 4g .. 4g + 3 of a tile in column
+// i, which is what a product leaves and, channel by channel, what it takes (the k-th of four products takes the channels
+// 4g + k), so the memory never moves between lanes.  The wavefronts' parts of y meet in shared memory (two places in
+// turn: one barrier a chunk, which the memory's own chain does not wait for).  The operands of a chunk are asked for
+// kAhead chunks before they are used.
+template <typename T, int TILES>
+__global__ void __launch_bounds__(256)
+memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, float* __restrict__ state, long long state_stride,
+                         long long n_offset, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                         const int* __restrict__ state_slots, float* __restrict__ y, float* __restrict__ nq, int heads, int d,
+                         int p_dim, int from) {
+    constexpr int C = 64 * TILES, kAhead = TILES <= 2 ? 4 : 2;
+    __shared__ memory_float4 part_s[2][4][kWave];
+    const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * 16;
+    const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
+    if (q_len < from) return;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int i = lane % 16, g = lane / 16;
+    const int p = p0 + i;
+    const bool norm_col = nq != nullptr && p == p_dim;
+    const bool live = p < p_dim || norm_col;
+    float* request = state + static_cast<size_t>(state_slots[seg]) * state_stride;
+    float* s_rows = norm_col ? request + n_offset + static_cast<size_t>(h) * d : request + static_cast<size_t>(h) * d * p_dim + p;
+    const size_t s_step = norm_col ? 1 : p_dim;
+    const int ch0 = wave * 16 * TILES;
+    memory_float4 s[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int ch = ch0 + 16 * j + 4 * g + u;
+            s[j][u] = live && ch < d ? s_rows[static_cast<size_t>(ch) * s_step] : 0.f;
+        }
+    struct Operands {
+        memory_float4 q[TILES], k[TILES], f[TILES];
+        float n;
+        T v[4];
+    };
+    const float* first = chunks + (static_cast<size_t>(q_start / kChunk + seg) * heads + h) * chunk_floats(C);
+    const T* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
+    // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
+    const unsigned q_at = i * C + ch0 + 4 * g, k_at = kChunk * C + (ch0 + i) * kChunk + 4 * g, f_at = 2 * kChunk * C + ch0 + 4 * g;
+    const unsigned n_at = (2 * kChunk + 1) * C + i * kChunk + 4 * wave + g;
+    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(v_stride);
+    auto load = [&](int c) {
+        Operands o;
+        const float* at = first + static_cast<size_t>(c) * heads * chunk_floats(C);
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) {
+            o.q[j] = *reinterpret_cast<const memory_float4*>(at + q_at + 16 * j);
+            o.k[j] = *reinterpret_cast<const memory_float4*>(at + k_at + 16 * kChunk * j);
+            o.f[j] = *reinterpret_cast<const memory_float4*>(at + f_at + 16 * j);
+        }
+        o.n = at[n_at];
+        const T* v_chunk = v_first + static_cast<size_t>(c) * kChunk * v_stride;
+        const unsigned beyond = (min(kChunk, q_len - c * kChunk) - 1) * row;          // the chunk's last token
+        // (beyond it, that token's once more: what it is multiplied by is zero)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[min((4 * u + g) * row, beyond) + col];
+        return o;
+    };
+    const int count = (q_len + kChunk - 1) / kChunk;
+    auto walk = [&](int c, const Operands& now) {
+        memory_float4 x, read[TILES];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            x[u] = c * kChunk + 4 * u + g < q_len ? (norm_col ? 1.f : to_float(now.v[u])) : 0.f;
+        // (a sum a tile, added in the end: short chains of products, and of roundings)
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) read[j] = memory_float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < TILES; ++j) read[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][u], s[j][u], read[j], 0, 0, 0);
+        // (the chunk's own sum first, from zero, and the memory joins it with one rounding a chunk)
+        memory_float4 own[TILES];
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) own[j] = memory_float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < TILES; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][u], x[u], own[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[j][u] = fmaf(now.f[j][u], s[j][u], own[j][u]);
+        // a wavefront's part: its channels of the memory, and four of the chunk's own tokens
+        const float mine = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
+        memory_float4 part = read[0];
+#pragma unroll
+        for (int j = 1; j < TILES; ++j) part += read[j];
+        part = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, part, 0, 0, 0);
+        part_s[c % 2][wave][lane] = part;
+        // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // wavefront w writes the tokens 4g + w
+        const float* parts = reinterpret_cast<const float*>(&part_s[c % 2][0][lane]) + wave;
+        float o = parts[0];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
+        const int t = c * kChunk + 4 * g + wave;
+        if (live && t < q_len) {
+            if (norm_col) nq[static_cast<size_t>(q_start + t) * heads + h] = o;
+            else y[static_cast<size_t>(q_start + t) * heads * p_dim + static_cast<size_t>(h) * p_dim + p] = o;
+        }
+    };
+    // the operands of kAhead chunks in turn (beyond the last chunk: the last's once more).  The loads stay where they are
+    // written: the scratch and v may alias y as far as the compiler knows, and the empty statements touch memory.
+    Operands ring[kAhead];
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) ring[a] = load(min(a, count - 1));
+    int c = 0;
+    for (; c + kAhead <= count; c += kAhead) {
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            walk(c + a, ring[a]);
+            ring[a] = load(min(c + a + kAhead, count - 1));
+            asm volatile("" ::: "memory");
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a)
+        if (c + a < count) walk(c + a, ring[a]);
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int ch = ch0 + 16 * j + 4 * g + u;
+            if (live && ch < d) s_rows[static_cast<size_t>(ch) * s_step] = s[j][u];
+        }
+}
+
 // `steps` (float32 [3, tokens, heads], of which a and b are read; then `nq` float32 [tokens, heads] takes the
 // normaliser's sums and the normaliser lies at `n_offset` of a request's row) or, if null, `decays` (float32 [heads]; b = 1),
 // or, with `row_decays`, neither: then qk has a third plane [tokens, heads * d] of decays a row and token (b = 1).
+// `from` tokens (16 at least; 0: no segment) is what a segment needs to be walked in chunks, out of the scratch `chunks`:
+// tokens / 16 + segments + 1 places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
 WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride, const float* steps, const float* decays,
                               float* state, long long state_stride, long long n_offset, const int* seg_q_start,
                               const int* seg_q_len, const int* state_slots, float* y, float* nq, int is_bf16, int tokens,
-                              int segments, int heads, int d, int p_dim, int row_decays, hipStream_t stream) {
+                              int segments, int heads, int d, int p_dim, int row_decays, float* chunks, int from,
+                              hipStream_t stream) {
     if (segments <= 0 || tokens <= 0) return 0;
     if (row_decays ? (steps || decays) : ((!steps) == (!decays) || (steps && !nq))) return -1;
     if (heads <= 0 || d <= 0 || d > 8 * kMemSlices || p_dim <= 0) return -1;
@@ -337,10 +591,38 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
     const int r = (d + kMemSlices - 1) / kMemSlices;
     const int columns = p_dim + (steps ? 1 : 0);
     const dim3 grid(heads, segments, (columns + kMemCols - 1) / kMemCols);
+    // (a segment of `from` tokens leaves room for the others' single tokens)
+    const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
+    if (in_chunks) {
+        if (!chunks || from < kChunk || d > 256 || heads > 65535 || v_stride > 0x0fffffffLL ||
+            reinterpret_cast<uintptr_t>(chunks) % 16)
+            return -1;
+        const dim3 chunk_grid(tokens / kChunk + segments + 1, heads);
+#define LAUNCH(T, R)                                                                                                   \
+    do {                                                                                                               \
+        memory_chunk_kernel<R><<<chunk_grid, 256, 0, stream>>>(qk, steps, decays, seg_q_start, seg_q_len, segments, chunks, \
+                                                               tokens, heads, d, row_decays, from);                    \
+        if (const int err = launch_status()) return err;                                                               \
+        memory_chunk_scan_kernel<T, R><<<grid, 256, 0, stream>>>(chunks, static_cast<const T*>(v), v_stride, state,    \
+                                                                 state_stride, n_offset, seg_q_start, seg_q_len,       \
+                                                                 state_slots, y, steps ? nq : nullptr, heads, d, p_dim, from); \
+    } while (0)
+#define LAUNCH_R(T)                   \
+    if (d <= 64) LAUNCH(T, 1);        \
+    else if (d <= 128) LAUNCH(T, 2);  \
+    else if (d <= 192) LAUNCH(T, 3);  \
+    else LAUNCH(T, 4);
+        if (is_bf16) { LAUNCH_R(bf16) } else { LAUNCH_R(float) }
+#undef LAUNCH_R
+#undef LAUNCH
+        if (const int err = launch_status()) return err;
+        if (segments == 1) return 0;
+    }
+    const int shorter_than = in_chunks ? from : 0x7fffffff;
 #define LAUNCH(T, R, ROWS)                                                                                          \
     memory_scan_kernel<T, R, ROWS><<<grid, kMemThreads, 0, stream>>>(qk, static_cast<const T*>(v), v_stride, steps, decays, \
                                                                      state, state_stride, n_offset, seg_q_start, seg_q_len, \
-                                                                     state_slots, y, nq, tokens, heads, d, p_dim)
+                                                                     state_slots, y, nq, tokens, heads, d, p_dim, shorter_than)
 #define LAUNCH_R(T, ROWS)                  \
     if (r <= 1) LAUNCH(T, 1, ROWS);        \
     else if (r <= 2) LAUNCH(T, 2, ROWS);   \

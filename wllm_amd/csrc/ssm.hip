@@ -692,27 +692,38 @@ ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, con
     };
     const int count = (q_len + kChunk - 1) / kChunk;
     auto walk = [&](int c, const Operands& now) {
-        ssm_float4 x, read = {0.f, 0.f, 0.f, 0.f};
+        ssm_float4 x, read[TILES];
 #pragma unroll
         for (int u = 0; u < 4; ++u) x[u] = c * kChunk + 4 * g + u < q_len ? to_float(now.x[u]) : 0.f;
+        // (a sum a tile, added in the end: short chains of products, and of roundings)
 #pragma unroll
-        for (int j = 0; j < TILES; ++j)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                read = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.c[j].v[u]), s[j][u], read, 0, 0, 0);
-        const ssm_float4 moved = x * now.suf;
-#pragma unroll
-        for (int j = 0; j < TILES; ++j) s[j] *= now.all;
+        for (int j = 0; j < TILES; ++j) read[j] = ssm_float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int j = 0; j < TILES; ++j)
-                s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.b[j].v[u]), moved[u], s[j], 0, 0, 0);
+                read[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.c[j].v[u]), s[j][u], read[j], 0, 0, 0);
+        const ssm_float4 moved = x * now.suf;
+        // (the chunk's own sum first, from zero, and the state joins it with one rounding a chunk)
+        ssm_float4 own[TILES];
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) own[j] = ssm_float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < TILES; ++j)
+                own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.b[j].v[u]), moved[u], own[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[j][u] = fmaf(now.all, s[j][u], own[j][u]);
         // a wavefront's part: its rows of the state, and the chunk's own tokens 4g + wave
         const float mine = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
-        read *= now.pre;
-        read = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, read, 0, 0, 0);
-        part_s[c % 2][wave][lane] = read;
+        ssm_float4 part = read[0];
+#pragma unroll
+        for (int j = 1; j < TILES; ++j) part += read[j];
+        part = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, part * now.pre, 0, 0, 0);
+        part_s[c % 2][wave][lane] = part;
         // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();

@@ -1043,6 +1043,15 @@ def _ssm_chunks(xbc: torch.Tensor, segments: int, heads: int, groups: int, state
     return torch.empty(places * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows), dtype=torch.float32, device=xbc.device)
 
 
+def _memory_chunks(v: torch.Tensor, segments: int, heads: int, head_dim: int) -> Optional[torch.Tensor]:
+    """The same for `memory_scan`."""
+    places = _scan_places(v.shape[0], segments)
+    if not places:
+        return None
+    c = -(-head_dim // 64) * 64
+    return torch.empty(places * heads * ((2 * SCAN_CHUNK + 1) * c + SCAN_CHUNK * SCAN_CHUNK), dtype=torch.float32, device=v.device)
+
+
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
                      eps: float) -> None:
     """out = v / sqrt(mean over the part (v^2) + eps) * weight with v = y * silu(z), the row cut into
@@ -1662,12 +1671,14 @@ def _register_own() -> None:
                     seg_q_start.shape[0], heads, stream))
     register_op("memory_scan", entry_point="wllm_memory_scan",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_longlong, c_longlong, c_void_p,
-                          c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+                          c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                          c_int, c_void_p],
                 launch=lambda fn, stream, qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads,
                 head_dim, value_dim, nq=None, n_offset=0, row_decays=False: fn(
                     p(qk), p(v), v.stride(0), p(steps), p(decays), p(state), state.stride(0), n_offset, p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(nq), bf(v), v.shape[0], seg_q_start.shape[0], heads, head_dim,
-                    value_dim, int(row_decays), stream))
+                    value_dim, int(row_decays), p(_memory_chunks(v, seg_q_start.shape[0], heads, head_dim)), SCAN_CHUNK_FROM,
+                    stream))
     register_op("head_norm_gate", entry_point="wllm_head_norm_gate",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_float, c_int,
                           c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
