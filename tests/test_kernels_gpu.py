@@ -425,6 +425,31 @@ def test_float32_product_of_few_rows_has_the_bits_of_the_product_of_many(n, k):
             assert torch.equal(few, many[11:11 + rows]), f"{rows} rows, tile-major copy {tiles is not None}"
 
 
+@pytest.mark.parametrize("n,k", [(2568, 2048), (16, 512), (777, 1024), (10304, 2048), (2048, 768), (33, 4096), (40, 16384)])
+def test_split_products_wanted_whole_have_the_bits_of_their_partial_sums(n, k):
+    """Few rows and a split K axis: a result of one axis less than the stack of partial sums is their sum in order, rounded
+    once, whichever kernel makes it (pieces that meet inside a workgroup, or a second launch), at the edges of tiles of 16
+    rows and of the rule between the two, with columns that fill no band."""
+    torch.manual_seed(21)
+    w = (torch.randn(n, k, device=DEV) / math.sqrt(k)).bfloat16()
+    tiles = ops.tile_weight(w)
+    for m in (1, 7, 16, 17, 32, 33, 48, 64):
+        x = torch.randn(m, k, device=DEV).bfloat16()
+        s = ops.linear_splits(m, n, k, torch.bfloat16)
+        assert s > 1
+        for t in (None, tiles):
+            stack = torch.full((s, m, n), 7.0, device=DEV)
+            ops.linear(x, w, stack, t)
+            want = stack[0].clone()
+            for part in stack[1:]:
+                want += part
+            for dtype in (torch.bfloat16, torch.float32):
+                out = torch.full((m + 1, n), 7.0, device=DEV, dtype=dtype)
+                ops.linear(x, w, out[:m], t)
+                assert torch.equal(out[:m], want.to(dtype)) and bool((out[m] == 7.0).all()), f"{m} rows, {dtype}, copy {t is not None}"
+    close(want, x.double() @ w.double().T, torch.float32, "product")
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 2048, 16384), (129, 2048, 2064), (333, 2560, 2048), (200, 30, 4100), (128, 513, 520),
                                    (300, 70, 500), (520, 4096, 1536)])
 def test_float32_product_of_many_rows_has_the_same_bits_with_its_k_axis_cut(m, n, k):

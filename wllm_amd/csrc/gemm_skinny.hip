@@ -250,6 +250,100 @@ WLLM_API int wllm_split_sum(const float* partial, void* out, int out_bf16, long 
     return launch_status();
 }
 
+// A split product whose result is wanted whole: a workgroup owns a band of 16 columns and its wavefronts are the pieces
+// of the K axis, so the partial sums meet in shared memory, in split order as the kernel above adds them (the same bits),
+// and no second launch adds them.  x goes from the caches straight into the lanes that multiply it (a wavefront reads its
+// piece once), every wavefront's first steps of w and x in flight at once: bound by that one trip to memory and the
+// meeting.  2,048 keys to 2,568 columns for 8 rows 5.0 us, in two launches
+// 9.1; the decode steps whose next kernel cannot add
+// partial sums itself (norms over whole projections, convolutions, gates) run three or four such products a layer.
+template <int MT, typename TO, bool TILED, int THREADS>
+__global__ void __launch_bounds__(THREADS)
+gemm_skinny_joined_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
+                          int k_per_split) {
+    extern __shared__ uint4 xs[];
+    float4_t* parts = reinterpret_cast<float4_t*>(xs);                   // [splits][MT][lanes]
+    constexpr int kBatch = MT <= 2 && THREADS <= 512 ? 8 : 4;            // steps of 32 keys on their way
+    constexpr int kStep = TILED ? 512 : 32;
+    const int lane = threadIdx.x % kWave, split = threadIdx.x / kWave, splits = blockDim.x / kWave;
+    const int i = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * 16, k_begin = split * k_per_split, steps = k_per_split / 32;
+    const bf16* wp = TILED ? w + (static_cast<size_t>(blockIdx.x) * (K / 32) + k_begin / 32) * 512 + lane * 8
+                           : w + static_cast<size_t>(min(n0 + i, N - 1)) * K + k_begin + 8 * g;
+    const bf16* xp[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xp[t] = x + static_cast<size_t>(min(16 * t + i, M - 1)) * K + k_begin + 8 * g;
+    Frag a[kBatch], b[MT][kBatch];
+    auto load_step = [&](int u, int at) {
+        at = min(at, steps - 1);                  // (beyond the last step: that one once more, and not multiplied)
+        a[u].u = load_streamed(wp + at * kStep);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) b[t][u].u = *reinterpret_cast<const uint4*>(xp[t] + at * 32);
+    };
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) load_step(u, u);
+    float4_t acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < steps; s0 += kBatch) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            if (s0 + u < steps) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u].v, b[t][u].v, acc[t], 0, 0, 0);
+                if (s0 + kBatch < steps) load_step(u, s0 + kBatch + u);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) parts[(split * MT + t) * kWave + lane] = acc[t];
+    __syncthreads();
+    // lane (i, g) of a tile holds columns n0 + 4g .. + 3 of row 16t + i
+    for (int t = split; t < MT; t += splits) {
+        float4_t sum = parts[t * kWave + lane];
+        for (int s = 1; s < splits; ++s) sum += parts[(s * MT + t) * kWave + lane];
+        const int m = 16 * t + i, n = n0 + 4 * g;
+        if (m >= M || n >= N) continue;
+        TO* o = out + static_cast<size_t>(m) * N + n;
+        if (n + 3 < N && (N % 4 == 0)) {
+            store4<TO>(o, sum);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < N) o[v] = from_float<TO>(sum[v]);
+        }
+    }
+}
+
+// out = x w^T of at most 64 rows, the K axis in `splits` (at most 16) pieces of whole steps of 32 keys, whole.  Returns 0,
+// a HIP error code, or -1 for sizes this kernel does not take.
+WLLM_API int wllm_gemm_skinny_joined(const void* x, const void* w, int tiled, void* out, int out_bf16, int M, int N, int K,
+                                     int splits, hipStream_t stream) {
+    if (M < 1 || M > 64 || N < 1 || splits < 1 || splits > 16 || K % 32 != 0 || K % splits != 0 || (K / splits) % 32 != 0 || !out)
+        return -1;
+    const int mt = (M + 15) / 16, blocks = (N + 15) / 16;
+    const size_t smem = static_cast<size_t>(splits) * mt * kWave * sizeof(float4_t);
+#define LAUNCH_T(MT, TO, T, THREADS)                                                                                    \
+    gemm_skinny_joined_kernel<MT, TO, T, THREADS><<<blocks, 64 * splits, smem, stream>>>(                               \
+        static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<TO*>(out), M, N, K, K / splits)
+#define LAUNCH(MT, TO)                                                                                        \
+    if (splits <= 8) { if (tiled) LAUNCH_T(MT, TO, true, 512); else LAUNCH_T(MT, TO, false, 512); }            \
+    else { if (tiled) LAUNCH_T(MT, TO, true, 1024); else LAUNCH_T(MT, TO, false, 1024); }
+#define BY_MT(TO)                         \
+    switch (mt) {                         \
+        case 1: LAUNCH(1, TO); break;     \
+        case 2: LAUNCH(2, TO); break;     \
+        case 3: LAUNCH(3, TO); break;     \
+        default: LAUNCH(4, TO); break;    \
+    }
+    if (out_bf16) { BY_MT(bf16) } else { BY_MT(float) }
+#undef BY_MT
+#undef LAUNCH
+#undef LAUNCH_T
+    return launch_status();
+}
+
 // Returns 0, a HIP error code, or -1 for sizes this kernel does not take.
 // `partial` must hold splits * M * N floats when splits > 1; with `out` null the partial sums
 // are the result and nothing adds them.

@@ -72,6 +72,7 @@ _SIGNATURES = {
     "wllm_sample_rows_split": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                c_int, c_int, c_void_p],
     "wllm_sample_split_row_words": [],
+    "wllm_gemm_skinny_joined": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
 }
 
 
@@ -393,6 +394,15 @@ class HipBackend:
         self._check(self.lib.wllm_tile_weight(_ptr(weight), _ptr(tiles), weight.shape[0], weight.shape[1], self._stream()),
                     "tile_weight")
 
+    @staticmethod
+    def joined_takes(rows: int, n: int, splits: int) -> bool:
+        """Where a split product whose sum the caller wants itself runs as one launch, the pieces of the K axis meeting
+        inside a workgroup (a wavefront each, at most 16).  There every band of 16 columns reads x for itself, so with
+        more rows and more columns the two launches that stage x once win: 2,048 keys to 2,568 columns 9.1 against 5.0 us
+        at 8 rows, 10.3 against 7.2 at 24, but to 2,048 columns 10.9 against 12.2 at 64; to 10,304 columns 13.9
+        against 11.1 at 8 and 15.8 against 16.3 at 24; in two pieces (768 keys to 2,048 columns) 9.9 against 6.7 at 64."""
+        return 1 < splits <= 16 and (rows <= 16 or n <= 8192 and (rows <= 32 or rows <= 64 and splits == 2))
+
     def _skinny(self, x, weight, out, tiles=None) -> None:
         m, k = x.shape
         n = weight.shape[0]
@@ -402,6 +412,10 @@ class HipBackend:
         if out.dim() == 3:      # the caller adds the partial sums later
             self._check(self.lib.wllm_gemm_skinny(_ptr(x), _ptr(w), tiled, c_void_p(0), 0, _ptr(out), m, n, k, splits,
                                                   chunk, self._stream()), "linear (few rows, partial sums)")
+            return
+        if self.joined_takes(m, n, splits):
+            self._check(self.lib.wllm_gemm_skinny_joined(_ptr(x), _ptr(w), tiled, _ptr(out), int(out.dtype == torch.bfloat16),
+                                                         m, n, k, splits, self._stream()), "linear (few rows, pieces of K joined)")
             return
         partial = self._gemm_partial(splits * m * n, x.device) if splits > 1 else None
         self._check(self.lib.wllm_gemm_skinny(_ptr(x), _ptr(w), tiled, _ptr(out), int(out.dtype == torch.bfloat16),
