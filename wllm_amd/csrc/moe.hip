@@ -516,12 +516,18 @@ WLLM_API int wllm_moe_down(const void* act, const void* w, const void* tiles, co
 // compute unit).  What differs: a tile's rows of x are gathered (row r of tile t is the assignment the plan names:
 // the token's row of x for the first product, the assignment's row of act for the second), the weights are the
 // tile's expert's, and a row's result goes where its assignment belongs.  A row's sums run over k in ascending
-// stages whatever tile it lies in.  Workgroups that share an expert's rows of w lie 8 indices apart, on one XCD.
+// stages whatever tile it lies in.
 // bfloat16; K a multiple of 64. ----
 constexpr int kBigRows = 128;
 constexpr int kBigKeys = 64;
 constexpr int kBigRowBytes = kBigKeys * 2;
 constexpr int kBigStageBytes = 2 * kBigRows * kBigRowBytes;
+// The workgroups of kBlockM tiles of rows by kBlockN tiles of columns have indices that are equal modulo 8 and follow one
+// another, so they run together on one XCD and share their rows of x and of w in its L2: the sixty-four that an XCD
+// runs at once then read some 14 MB a pass over K where one column of tiles at a time made them read 39 (every tile's
+// rows of x, and nearly every expert's rows of w), which the fabric behind the L2s had to bring for all eight XCDs.
+// 9,003 rows of 2,048 over 16 experts of 4,096: @@.
+constexpr int kBlockM = 4, kBlockN = 8;
 
 union MoeTFrag {
     uint4 u;
@@ -554,11 +560,13 @@ moe_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const in
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = lane % 16, g = lane / 16;
     const int wm = wave / 2, wn = wave % 2;
-    const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
-    const int m_tile = j % max_tiles;
-    const int n_tile = (j / max_tiles) * 8 + xcd;
+    // (see kBlockM, kBlockN)
     constexpr int kColumns = GATED ? kBigRows / 2 : kBigRows;
-    const int n_base = n_tile * kColumns;
+    const int inside = blockIdx.x / 8 % (kBlockM * kBlockN);
+    const int block = blockIdx.x / 8 / (kBlockM * kBlockN) * 8 + blockIdx.x % 8;
+    const int n_blocks = ((N + kColumns - 1) / kColumns + kBlockN - 1) / kBlockN;
+    const int m_tile = block / n_blocks * kBlockM + inside % kBlockM;
+    const int n_base = (block % n_blocks * kBlockN + inside / kBlockM) * kColumns;
     if (m_tile >= plan[0] || n_base >= N) return;
     const int e = plan[1 + m_tile];
     const int* rows = plan + 1 + max_tiles + m_tile * kBigRows;
@@ -673,7 +681,8 @@ WLLM_API int wllm_moe_tiles(const void* x, const void* w, const int* plan, int m
         return -1;
     const int columns = gated ? kBigRows / 2 : kBigRows;
     const int n_tiles = (N + columns - 1) / columns;
-    const long long blocks = static_cast<long long>((n_tiles + 7) / 8 * 8) * max_tiles;
+    const long long areas = static_cast<long long>((n_tiles + kBlockN - 1) / kBlockN) * ((max_tiles + kBlockM - 1) / kBlockM);
+    const long long blocks = (areas + 7) / 8 * 8 * kBlockM * kBlockN;
     if (blocks > 0x7fffffffLL) return -1;
     const dim3 grid(static_cast<unsigned>(blocks));
     const bf16* xp = static_cast<const bf16*>(x);
