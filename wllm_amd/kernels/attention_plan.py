@@ -36,7 +36,12 @@ KEY_CHUNK = 128
 ROWS_PER_TILE = 16
 ITEM_INTS = 8
 PREFILL_TABLE_PAGES = 1024      # pages one prefill item may span (the kernel's shared block table)
-PREFILL_MIN_PIECE = 16          # groups of 32 keys; shorter pieces cost more in partial results than they gain
+# Groups of 32 keys: shorter pieces cost more in partial results than they gain, longer ones leave compute units idle where a
+# step has few blocks of rows.  Attention and its reduce kernel with pieces of at least 8, 10 and 16 groups, 8 heads of 256
+# on one key head: 104 rows over 1,000 keys 19.1 / 21.1 / 27.4 us, 448 over 896 24.2 / 24.6 / 28.0, 700 over 700 22.4 / 23.3 /
+# 26.8, 448 over 1,000 beside 20 decoded tokens 35.4 / 36.1 / 39.9, 512 over 7,000 62.0 / 58.5 / 56.7, 300 over 300 17.3 / 17.0 /
+# 16.9 (8 cuts it in two); from 1,500 keys of their own on a prompt's blocks fill the device either way.
+PREFILL_MIN_PIECE = 10
 WORKGROUP_SLOTS = 512           # prefill workgroups a device runs at once unless the caller knows better (two a compute unit)
 PREFILL_ROWS = 64               # rows of a prefill item unless the kernel for the sizes at hand says otherwise
 
