@@ -159,8 +159,9 @@ class CacheManager:
         if not self._free_slots:
             raise OutOfSlots(f"all {self.max_requests} state slots are taken")
         slot = self._free_slots.pop()
-        for t in self.state.values():
-            t[slot].zero_()
+        if self.state:
+            # (all rows in a launch or two: a model of 18 layers may carry 24 of them)
+            torch._foreach_zero_([t[slot] for t in self.state.values()])
         self.requests[request] = RequestCache(0, slot, [[] for _ in self.groups], [0 for _ in self.groups])
         return slot
 
