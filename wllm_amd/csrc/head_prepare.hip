@@ -35,9 +35,12 @@ template <typename T> struct alignas(4 * sizeof(T)) Four { T v[4]; };
 // take kRestColumns columns each of what lies behind the query and key heads.  A decode step's few
 // tokens so fill some tens of workgroups instead of one a token, whose wavefronts would walk the heads
 // and the stack of partial sums one after the other.  FOUR: head_dim and the row's width are multiples
-// of four and the pairs are neighbours (or nothing turns), so a lane owns four consecutive elements with
-// both partners of its pairs and moves 8 or 16 bytes at a time; else a lane owns elements 64 apart and
-// finds a partner in shared memory.
+// of four, so a lane owns four consecutive elements and moves 8 or 16 bytes at a time; it holds both
+// partners of its pairs where they are neighbours, and finds the four partners of pairs rotary_dim / 2
+// apart (a multiple of four then) in shared memory.  Else a lane owns elements 64 apart and finds each
+// partner there.  A token's sines and cosines are worked out once a workgroup, a pair a thread, while the
+// heads are on their way: a sine of an angle of some thousand radians costs more than all else a lane
+// does (3,001 tokens of 8 heads and one key head of 256, half of the head turned: 37.6 to 29.5 us).
 template <typename T, bool FOUR>
 __global__ void __launch_bounds__(kWave * kPrepareWaves)
 head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict__ parts, int splits, size_t split_stride,
@@ -47,7 +50,8 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
                     int interleaved, float norm_eps, int norm_dim, int values_are_keys, int page_size, int head_pieces,
                     const float* __restrict__ pre_q, const float* __restrict__ pre_k, float pre_eps, float rot_scale,
                     float temp_coef, int temp_every) {
-    __shared__ float staged[kPrepareWaves][FOUR ? 1 : kPrepareMaxHead];
+    __shared__ __align__(16) float staged[kPrepareWaves][kPrepareMaxHead];
+    __shared__ float sines[kPrepareMaxHead / 2], cosines[kPrepareMaxHead / 2];
     const int token = blockIdx.x;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     T* row = rows + static_cast<size_t>(token) * row_width;
@@ -93,11 +97,21 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
         return;
     }
     const int head = static_cast<int>(blockIdx.y) * kPrepareWaves + wave;
-    if (head >= turned_heads) return;
-    const float pos = static_cast<float>(positions[token]);
     const int base = head * head_dim;
     const int kvh = head - num_heads;                 // >= 0: a key head
     const int half = rotary_dim / 2;
+    Four<T> loaded;                                   // FOUR: the lane's elements, asked for before the angles
+    if (FOUR && !prow && head < turned_heads && 4 * lane < head_dim) loaded = *reinterpret_cast<const Four<T>*>(row + base + 4 * lane);
+    if (inv_freq) {
+        if (static_cast<int>(threadIdx.x) < half) {
+            float sn, cs;
+            sincosf(static_cast<float>(positions[token]) * inv_freq[threadIdx.x], &sn, &cs);
+            sines[threadIdx.x] = sn * rot_scale;
+            cosines[threadIdx.x] = cs * rot_scale;
+        }
+        __syncthreads();
+    }
+    if (head >= turned_heads) return;
     float temperature = 1.f;
     if (temp_every > 0 && kvh < 0) temperature = 1.f + temp_coef * logf(static_cast<float>((positions[token] + 1) / temp_every) + 1.f);
     if (FOUR) {
@@ -124,9 +138,8 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
                     }
                 }
             } else {
-                const Four<T> t = *reinterpret_cast<const Four<T>*>(row + base + e);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = to_float(t.v[u]);
+                for (int u = 0; u < 4; ++u) v[u] = to_float(loaded.v[u]);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -147,17 +160,31 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
                 for (int u = 0; u < 4; ++u) v[u] = v[u] * pre * pw[u];
             }
         }
-        if (live) {
-            if (inv_freq) {
+        if (inv_freq && !interleaved) {
+            float* mine = staged[wave];
+            if (live) *reinterpret_cast<Four<float>*>(mine + e) = Four<float>{{v[0], v[1], v[2], v[3]}};
+            // lanes read below what other lanes of the wavefront wrote above
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+            if (e < rotary_dim) {
+                const bool first = e < half;
+                const int j = first ? e : e - half;
+                const Four<float> other = *reinterpret_cast<const Four<float>*>(mine + (first ? e + half : j));
 #pragma unroll
-                for (int u = 0; u < 4; u += 2) {
-                    if (e + u < rotary_dim) {
-                        float sn, cs, ra, rb;
-                        sincosf(pos * inv_freq[(e + u) >> 1], &sn, &cs);
-                        rotate_pair(v[u], v[u + 1], sn * rot_scale, cs * rot_scale, ra, rb);
-                        v[u] = ra;
-                        v[u + 1] = rb;
-                    }
+                for (int u = 0; u < 4; ++u) {
+                    float ra, rb;
+                    rotate_pair(first ? v[u] : other.v[u], first ? other.v[u] : v[u], sines[j + u], cosines[j + u], ra, rb);
+                    v[u] = first ? ra : rb;
+                }
+            }
+        } else if (inv_freq && live) {
+#pragma unroll
+            for (int u = 0; u < 4; u += 2) {
+                if (e + u < rotary_dim) {
+                    float ra, rb;
+                    rotate_pair(v[u], v[u + 1], sines[(e + u) >> 1], cosines[(e + u) >> 1], ra, rb);
+                    v[u] = ra;
+                    v[u + 1] = rb;
                 }
             }
         }
@@ -216,9 +243,8 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
             const int partner = interleaved ? (e ^ 1) : (first ? e + half : e - half);
             const int j = interleaved ? e >> 1 : (first ? e : e - half);
             const float other = mine[partner];
-            float sn, cs, ra, rb;
-            sincosf(pos * inv_freq[j], &sn, &cs);
-            rotate_pair(first ? v[k] : other, first ? other : v[k], sn * rot_scale, cs * rot_scale, ra, rb);
+            float ra, rb;
+            rotate_pair(first ? v[k] : other, first ? other : v[k], sines[j], cosines[j], ra, rb);
             v[k] = first ? ra : rb;
         }
         ss += v[k] * v[k];
@@ -261,7 +287,7 @@ WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const flo
     const int rest_pieces = rest ? (row_width - turned + kRestColumns - 1) / kRestColumns : 0;
     if (head_pieces + rest_pieces > 65535) return -1;
     const dim3 grid(n, head_pieces + rest_pieces);
-    const bool four = head_dim % 4 == 0 && row_width % 4 == 0 && (interleaved || rotary_dim == 0) &&
+    const bool four = head_dim % 4 == 0 && row_width % 4 == 0 && (interleaved || rotary_dim % 8 == 0) &&
                       (parts == nullptr || split_stride % 4 == 0) &&
                       reinterpret_cast<uintptr_t>(rows) % 16 == 0 && reinterpret_cast<uintptr_t>(parts) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(cache) % 16 == 0;
