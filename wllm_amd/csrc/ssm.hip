@@ -45,38 +45,63 @@ __device__ __forceinline__ float4 conv_four(const T* p) {
     return make_float4(to_float(r.v[0]), to_float(r.v[1]), to_float(r.v[2]), to_float(r.v[3]));
 }
 
-// Walks `count` tokens from `token0`, four channels at `in`: calls make(token, rows) with the rows of the last
-// kSlideTaps inputs, the oldest first.  Inputs before a segment's first token are its request's carried rows.
+// Walks the tokens of a tile of kSlideTokens from `token0`, four channels at `in`: calls make(token, rows) with the rows
+// of the last kSlideTaps inputs, the oldest first.  Inputs before a segment's first token are its request's carried rows.
+// The carried rows of a segment are read by its first three tokens only, and these always belong to the tile of the
+// first: a tile that begins at a segment's second or third token leaves them to the tile before it, which walks up to
+// kSlideOver tokens more.  So the thread that has read a request's carried rows is the only one that will, and writes
+// the new ones (the segment's last inputs) without a launch behind this one.  2,048 channels of 3,001 float32 tokens: 9.3
+// us and 3.0 in a launch behind it, now 10.0; 96 segments of one token, 6,144 channels: 8.0 and 6.4, now 10.6.
+constexpr int kSlideOver = kSlideTaps - 2;
 template <typename T, typename MAKE>
-__device__ __forceinline__ void slide(const T* in, long long in_stride, const float* state, long long state_stride,
+__device__ __forceinline__ void slide(const T* in, long long in_stride, float* state, long long state_stride,
                                       long long carried_offset, const int* token_segment, const int* seg_q_start,
-                                      const int* state_slots, int channels, int token0, int count, MAKE make) {
+                                      const int* seg_q_len, const int* state_slots, int channels, int token0, int tokens,
+                                      MAKE make) {
+    constexpr int kWalk = kSlideTokens + kSlideOver, kCarried = kSlideTaps - 1;
     float4 rows[kSlideTaps];
-    auto before = [&](int token, int seg, int local) {             // the rows that a token at place `local` finds
-        const float* carried = state + static_cast<size_t>(state_slots[seg]) * state_stride + carried_offset;
+    auto begin_segment = [&](int seg, int start) {
+        float* carried = state + static_cast<size_t>(state_slots[seg]) * state_stride + carried_offset;
+        const int len = seg_q_len[seg];
+        float4 last[kCarried];
 #pragma unroll
-        for (int k = 1; k < kSlideTaps; ++k) {
-            const int src = local - kSlideTaps + k;
-            rows[k] = src >= 0 ? conv_four(in + static_cast<size_t>(token - local + src) * in_stride)
-                               : *reinterpret_cast<const float4*>(carried + static_cast<size_t>(kSlideTaps - 1 + src) * channels);
+        for (int k = 0; k < kCarried; ++k) {
+            rows[k + 1] = *reinterpret_cast<const float4*>(carried + static_cast<size_t>(k) * channels);
+            last[k] = conv_four(in + static_cast<size_t>(start + max(len - kCarried + k, 0)) * in_stride);
+        }
+#pragma unroll
+        for (int k = 0; k < kCarried; ++k) {           // a segment of fewer tokens keeps some of the rows, moved up
+            float4 v = last[k];
+#pragma unroll
+            for (int n = 1; n < kCarried; ++n)
+                if (len == n && k + n < kCarried) v = rows[k + n + 1];
+            if (len > 0) *reinterpret_cast<float4*>(carried + static_cast<size_t>(k) * channels) = v;
         }
     };
-    ConvFour<T> now[kSlideTokens];
-    int segs[kSlideTokens];
+    ConvFour<T> now[kWalk];
+    int segs[kWalk];
 #pragma unroll
-    for (int t = 0; t < kSlideTokens; ++t) {
-        const int token = token0 + min(t, count - 1);
+    for (int t = 0; t < kWalk; ++t) {
+        const int token = min(token0 + t, tokens - 1);
         now[t] = *reinterpret_cast<const ConvFour<T>*>(in + static_cast<size_t>(token) * in_stride);
         segs[t] = token_segment[token];
     }
-    before(token0, segs[0], token0 - seg_q_start[segs[0]]);
+    const int local0 = token0 - seg_q_start[segs[0]];
+    int local = local0;
 #pragma unroll
-    for (int t = 0; t < kSlideTokens; ++t) {
-        if (t >= count) break;
-        if (t > 0 && segs[t] != segs[t - 1]) before(token0 + t, segs[t], 0);
+    for (int k = 0; k < kSlideTaps; ++k)
+        rows[k] = k > 0 && local0 - kSlideTaps + k >= 0 ? conv_four(in + static_cast<size_t>(token0 - kSlideTaps + k) * in_stride)
+                                                        : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int t = 0; t < kWalk; ++t) {
+        if (token0 + t >= tokens) break;
+        if (t > 0) local = segs[t] != segs[t - 1] ? token0 + t - seg_q_start[segs[t]] : local + 1;
+        if (t >= kSlideTokens && (local == 0 || local >= kCarried)) break;
+        if (local == 0) begin_segment(segs[t], token0 + t);
 #pragma unroll
         for (int k = 0; k + 1 < kSlideTaps; ++k) rows[k] = rows[k + 1];
         rows[kSlideTaps - 1] = make_float4(to_float(now[t].v[0]), to_float(now[t].v[1]), to_float(now[t].v[2]), to_float(now[t].v[3]));
+        if (local == t + local0 && local0 > 0 && local < kCarried) continue;       // a token of the tile before
         make(token0 + t, rows);
     }
 }
@@ -84,17 +109,18 @@ __device__ __forceinline__ void slide(const T* in, long long in_stride, const fl
 template <typename T>
 __global__ void __launch_bounds__(256)
 causal_conv_slide_kernel(const T* __restrict__ in, long long in_stride, const float* __restrict__ weight,
-                         const float* __restrict__ bias, const float* __restrict__ state, long long state_stride,
+                         const float* __restrict__ bias, float* __restrict__ state, long long state_stride,
                          long long carried_offset, const int* __restrict__ token_segment, const int* __restrict__ seg_q_start,
-                         const int* __restrict__ state_slots, T* __restrict__ out, int tokens, int channels) {
+                         const int* __restrict__ seg_q_len, const int* __restrict__ state_slots, T* __restrict__ out, int tokens,
+                         int channels) {
     const int c = (blockIdx.y * 256 + threadIdx.x) * 4, token0 = blockIdx.x * kSlideTokens;
     if (c >= channels) return;
     float4 w[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) w[u] = *reinterpret_cast<const float4*>(weight + static_cast<size_t>(c + u) * kSlideTaps);
     const float4 b = *reinterpret_cast<const float4*>(bias + c);
-    slide(in + c, in_stride, state, state_stride, carried_offset + c, token_segment, seg_q_start, state_slots, channels, token0,
-          min(kSlideTokens, tokens - token0), [&](int token, const float4 (&rows)[kSlideTaps]) {
+    slide(in + c, in_stride, state, state_stride, carried_offset + c, token_segment, seg_q_start, seg_q_len, state_slots, channels,
+          token0, tokens, [&](int token, const float4 (&rows)[kSlideTaps]) {
         float acc[4] = {b.x, b.y, b.z, b.w};
         const float* wf = reinterpret_cast<const float*>(w);
 #pragma unroll
@@ -132,14 +158,15 @@ WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* 
 #define SLIDE(T)                                                                                                        \
     causal_conv_slide_kernel<T><<<slide_grid, 256, 0, stream>>>(static_cast<const T*>(in), in_stride, weight, bias, state, \
                                                                 state_stride, carried_offset, token_segment, seg_q_start, \
-                                                                state_slots, static_cast<T*>(out), tokens, channels)
-    const bool many = taps == kSlideTaps && tokens >= kSlideFrom;
+                                                                seg_q_len, state_slots, static_cast<T*>(out), tokens, \
+                                                                channels)
+    const bool many = taps == kSlideTaps && tokens >= kSlideFrom;          // (these keep the carried rows themselves)
     if (many && is_bf16 && in_fours<bf16>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
-        SLIDE(bf16);
-    else if (many && !is_bf16 && in_fours<float>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
-        SLIDE(float);
+        return SLIDE(bf16), launch_status();
+    if (many && !is_bf16 && in_fours<float>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
+        return SLIDE(float), launch_status();
 #undef SLIDE
-    else if (is_bf16)
+    if (is_bf16)
         causal_conv_kernel<bf16><<<grid, 256, 0, stream>>>(static_cast<const bf16*>(in), in_stride, weight, bias, state,
                                                            state_stride, carried_offset, token_segment, seg_q_start,
                                                            state_slots, static_cast<bf16*>(out), channels, taps);
@@ -163,7 +190,7 @@ WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* 
 // ---- the same convolution on the residual stream itself, in front of a sublayer that reads the stream:
 // out[t, c] = x[t, c] + sum_k w[k, c] * x[t - (taps - 1) + k, c] (w a row a tap, [taps, channels]), float32 sums in this order, no bias and no
 // activation; x float32 [tokens, channels], out the activation type.  The carried rows (the request's last
-// taps - 1 rows of x, the oldest first) are kept by `conv_carry_kernel`, as above; or, CARRY (a step of single
+// taps - 1 rows of x, the oldest first) are kept by `conv_carry_kernel` (by `slide`), as above; or, CARRY (a step of single
 // tokens, where no other token of the launch reads a request's carried rows), by the token's own threads, each
 // moving its channel's rows up by one as it reads them: one launch instead of two, the same sums. ----
 template <typename T, bool CARRY>
@@ -239,17 +266,17 @@ stream_conv_four_kernel(const float* __restrict__ x, const float* __restrict__ w
 // 2,048 channels of 3,001 tokens: 19.2 to 9.5 us).
 template <typename T>
 __global__ void __launch_bounds__(256)
-stream_conv_slide_kernel(const float* __restrict__ x, const float* __restrict__ weight, const float* __restrict__ state,
+stream_conv_slide_kernel(const float* __restrict__ x, const float* __restrict__ weight, float* __restrict__ state,
                          long long state_stride, long long carried_offset, const int* __restrict__ token_segment,
-                         const int* __restrict__ seg_q_start, const int* __restrict__ state_slots, T* __restrict__ out,
-                         int tokens, int channels) {
+                         const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                         const int* __restrict__ state_slots, T* __restrict__ out, int tokens, int channels) {
     const int c = (blockIdx.y * 256 + threadIdx.x) * 4, token0 = blockIdx.x * kSlideTokens;
     if (c >= channels) return;
     float4 w[kSlideTaps];
 #pragma unroll
     for (int k = 0; k < kSlideTaps; ++k) w[k] = *reinterpret_cast<const float4*>(weight + static_cast<size_t>(k) * channels + c);
-    slide(x + c, static_cast<long long>(channels), state, state_stride, carried_offset + c, token_segment, seg_q_start, state_slots,
-          channels, token0, min(kSlideTokens, tokens - token0), [&](int token, const float4 (&rows)[kSlideTaps]) {
+    slide(x + c, static_cast<long long>(channels), state, state_stride, carried_offset + c, token_segment, seg_q_start, seg_q_len,
+          state_slots, channels, token0, tokens, [&](int token, const float4 (&rows)[kSlideTaps]) {
         float4 acc = rows[kSlideTaps - 1];
 #pragma unroll
         for (int k = 0; k < kSlideTaps; ++k) {
@@ -286,13 +313,15 @@ WLLM_API int wllm_stream_conv(const float* x, const float* weight, float* state,
         if (taps == kSlideTaps && tokens >= kSlideFrom) {
             if (out_bf16)
                 stream_conv_slide_kernel<bf16><<<slide_grid, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
-                                                                               token_segment, seg_q_start, state_slots,
+                                                                               token_segment, seg_q_start, seg_q_len, state_slots,
                                                                                static_cast<bf16*>(out), tokens, channels);
             else
                 stream_conv_slide_kernel<float><<<slide_grid, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
-                                                                                token_segment, seg_q_start, state_slots,
+                                                                                token_segment, seg_q_start, seg_q_len, state_slots,
                                                                                 static_cast<float*>(out), tokens, channels);
-        } else if (out_bf16)
+            return launch_status();
+        }
+        if (out_bf16)
             stream_conv_four_kernel<bf16><<<grid4, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
                                                                      token_segment, seg_q_start, state_slots,
                                                                      static_cast<bf16*>(out), channels, taps);
