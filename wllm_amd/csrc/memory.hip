@@ -329,18 +329,21 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
 // P_t the product of a chunk's decays up to t, Kh_s = k_s times the decays behind s.  A product of decays is formed from
 // the decays it is made of, never as a quotient, so the numbers are those of the walk token by token up to the order of
 // float32 sums.  Nothing but S0 depends on the tokens before: `memory_chunk_kernel` makes P q, Kh, P_16 and N for every
-// chunk and head at once ([16][C], [C][16], [C], [16][16] floats, C = the channels padded to a multiple of 64), and
+// chunk and head at once ([16][C], [C][16], [C], [16][16] floats, C = the channels padded to a multiple of 64; and [C][4]:
+// what the last four of a chunk's Kh, which weigh most, lost in being rounded to 32 bits), and
 // `memory_chunk_scan_kernel` walks a segment's chunks with v_mfma_f32_16x16x4_f32 (float32 in and out).  A chunk begins
-// every 16 tokens of a segment; the last one is filled with tokens that change nothing (q = k = 0, f = 1).  Chunk c of
-// segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
-// Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 27 and
-// 138 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 15 and 112, with
-// exponential gates and the normaliser 297 against 15 and 110; 64 tokens 12.6 against 7 and 8, from where on a segment
-// gains.  Off the result in 64 bits: decays a head 2.0e-7 (token by token 3.1e-7), decays a row 9.6e-8 (9.2e-8). ----
+// every 16 tokens of a segment; the last one is its last 16 tokens, those of the chunk before it as tokens that change
+// nothing (q = k = 0, f = 1).  Chunk c of segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 34 and
+// 156 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 19 and 127, with
+// exponential gates and the normaliser 297 against 19 and 125; 64 tokens 12.6 against 7 and 9, from where on a segment
+// gains.  Off the result in 64 bits (y; the memory left behind), here and token by token: decays a head 2.0e-7; 2.0e-7 and
+// 3.1e-7; 3.2e-7, decays a row 8.1e-8; 4.5e-8 and 9.1e-8; 4.5e-8, exponential gates 8.7e-8; 5.3e-8 and 9.9e-8; 5.7e-8.  With N
+// in 32 bits (27 us) and without the rest of Kh (138 us) decays a row are off by 9.4e-8; 4.8e-8, so both stay. ----
 constexpr int kChunk = 16;
 typedef float memory_float4 __attribute__((ext_vector_type(4)));
 
-static __host__ __device__ __forceinline__ size_t chunk_floats(int c) { return static_cast<size_t>(2 * kChunk + 1) * c + kChunk * kChunk; }
+static __host__ __device__ __forceinline__ size_t chunk_floats(int c) { return static_cast<size_t>(2 * kChunk + 5) * c + kChunk * kChunk; }
 
 // The sum over a row of 16 lanes, in every lane.
 __device__ __forceinline__ float row_of_16_sum(float v) {
@@ -358,6 +361,7 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
                     float* __restrict__ chunks, int tokens, int heads, int d, int row_decays, int from) {
     constexpr int C = 64 * R, kEach = kChunk * C / 256;
     __shared__ __align__(16) float k_s[kChunk * C], q_s[kChunk * C], f_s[kChunk * C];
+    __shared__ float b_s[kChunk];
     __shared__ int found;
     const int place = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     if (tid == 0) found = -1;
@@ -370,57 +374,66 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
     const int seg = found;
     if (seg < 0) return;
     const int q_start = seg_q_start[seg], local = (place - q_start / kChunk - seg) * kChunk;
-    const int count = min(kChunk, seg_q_len[seg] - local), token = q_start + local;
+    // (a segment's last chunk is its last 16 tokens, of which those that the chunk before it holds are left out)
+    const int begin = min(local, seg_q_len[seg] - kChunk), out_of = local - begin, token = q_start + begin;
     float* out = chunks + (static_cast<size_t>(place) * heads + h) * chunk_floats(C);
     const size_t width = static_cast<size_t>(heads) * d, plane = static_cast<size_t>(tokens) * width;
     float q[kEach], k[kEach], f[kEach];
 #pragma unroll
     for (int j = 0; j < kEach; ++j) {
         // (every load from a place that is there: what is not is put right below)
-        const int t = min((tid + 256 * j) / C, count - 1), i = min((tid + 256 * j) % C, d - 1);
+        const int t = (tid + 256 * j) / C, i = min((tid + 256 * j) % C, d - 1);
         const size_t at = static_cast<size_t>(token + t) * width + static_cast<size_t>(h) * d + i;
         const size_t th = static_cast<size_t>(token + t) * heads + h;
         q[j] = qk[at];
         k[j] = qk[plane + at];
         f[j] = row_decays ? qk[2 * plane + at] : steps ? steps[th] : decays[h];
-        if (steps) k[j] *= steps[static_cast<size_t>(tokens) * heads + th];
     }
+    if (tid < kChunk)
+        b_s[tid] = steps ? steps[static_cast<size_t>(tokens) * heads + static_cast<size_t>(token + tid) * heads + h] : 1.f;
 #pragma unroll
     for (int j = 0; j < kEach; ++j) {
         const int e = tid + 256 * j;
-        const bool there = e / C < count && e % C < d;
+        const bool there = e / C >= out_of && e % C < d;
         q_s[e] = there ? q[j] : 0.f;
         k_s[e] = there ? k[j] : 0.f;
         f_s[e] = there ? f[j] : 1.f;
     }
     __syncthreads();
     {
-        // N: 16 lanes hold the key of token s, which decays as t goes on
+        // N: 16 lanes hold the key of token s, which decays as t goes on (decayed keys and a lane's sums in 64 bits)
         const int s = tid / kChunk, sl = tid % kChunk;
-        memory_float4 r[R];
+        double r[R][4];
 #pragma unroll
-        for (int j = 0; j < R; ++j) r[j] = *reinterpret_cast<const memory_float4*>(k_s + s * C + 64 * j + 4 * sl);
+        for (int j = 0; j < R; ++j) {
+            const memory_float4 key = *reinterpret_cast<const memory_float4*>(k_s + s * C + 64 * j + 4 * sl);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) r[j][u] = static_cast<double>(key[u]) * b_s[s];
+        }
         float mine = 0.f;                              // N of token sl and key s
 #pragma unroll
         for (int t = 0; t < kChunk; ++t) {
-            memory_float4 sum = {0.f, 0.f, 0.f, 0.f};
+            double sum = 0.0;
 #pragma unroll
             for (int j = 0; j < R; ++j) {
                 const int at = t * C + 64 * j + 4 * sl;
                 const memory_float4 qt = *reinterpret_cast<const memory_float4*>(q_s + at), ft = *reinterpret_cast<const memory_float4*>(f_s + at);
-                if (t > s) r[j] *= ft;
-                sum += r[j] * qt;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (t > s) r[j][u] *= ft[u];
+                    sum = fma(r[j][u], static_cast<double>(qt[u]), sum);
+                }
             }
-            const float dot = row_of_16_sum((sum[0] + sum[1]) + (sum[2] + sum[3]));
+            const float dot = row_of_16_sum(static_cast<float>(sum));
             if (sl == t && t >= s) mine = dot;
         }
-        out[(2 * kChunk + 1) * C + sl * kChunk + s] = mine;
+        out[(2 * kChunk + 5) * C + sl * kChunk + s] = mine;
     }
     // the decays up to and behind every token, a channel a thread.  (Products in 64 bits, rounded once: where the decays
     // are the head's, all channels share their error, which the walk token by token spreads over the state's elements.)
     for (int c = tid; c < C; c += 256) {
         double decay = 1.0, behind = 1.0;
-        float kh[kChunk];
+        float kh[kChunk], rest[4];
 #pragma unroll
         for (int t = 0; t < kChunk; ++t) {
             decay *= f_s[t * C + c];
@@ -429,13 +442,16 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
         out[2 * kChunk * C + c] = static_cast<float>(decay);
 #pragma unroll
         for (int t = kChunk - 1; t >= 0; --t) {
-            kh[t] = static_cast<float>(k_s[t * C + c] * behind);
+            const double key = static_cast<double>(k_s[t * C + c]) * b_s[t] * behind;
+            kh[t] = static_cast<float>(key);
+            if (t >= kChunk - 4) rest[t - (kChunk - 4)] = static_cast<float>(key - kh[t]);
             behind *= f_s[t * C + c];
         }
         // (token 4u + g at place 4g + u: the u-th product of the walk then takes the tokens 4u .. 4u + 3, the oldest first)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
             *reinterpret_cast<memory_float4*>(out + kChunk * C + c * kChunk + 4 * g) = memory_float4{kh[g], kh[4 + g], kh[8 + g], kh[12 + g]};
+        *reinterpret_cast<memory_float4*>(out + (2 * kChunk + 1) * C + 4 * c) = memory_float4{rest[0], rest[1], rest[2], rest[3]};
     }
 }
 
@@ -475,15 +491,16 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
         }
     struct Operands {
         memory_float4 q[TILES], k[TILES], f[TILES];
-        float n;
+        float rest[TILES], n;
         T v[4];
     };
     const float* first = chunks + (static_cast<size_t>(q_start / kChunk + seg) * heads + h) * chunk_floats(C);
     const T* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
     // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
     const unsigned q_at = i * C + ch0 + 4 * g, k_at = kChunk * C + (ch0 + i) * kChunk + 4 * g, f_at = 2 * kChunk * C + ch0 + 4 * g;
-    const unsigned n_at = (2 * kChunk + 1) * C + i * kChunk + 4 * wave + g;
+    const unsigned rest_at = (2 * kChunk + 1) * C + (ch0 + i) * 4 + g, n_at = (2 * kChunk + 5) * C + i * kChunk + 4 * wave + g;
     const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(v_stride);
+    auto begins = [&](int c) { return min(c * kChunk, q_len - kChunk); };      // (the last chunk: the last 16 tokens)
     auto load = [&](int c) {
         Operands o;
         const float* at = first + static_cast<size_t>(c) * heads * chunk_floats(C);
@@ -492,13 +509,12 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
             o.q[j] = *reinterpret_cast<const memory_float4*>(at + q_at + 16 * j);
             o.k[j] = *reinterpret_cast<const memory_float4*>(at + k_at + 16 * kChunk * j);
             o.f[j] = *reinterpret_cast<const memory_float4*>(at + f_at + 16 * j);
+            o.rest[j] = at[rest_at + 64 * j];
         }
         o.n = at[n_at];
-        const T* v_chunk = v_first + static_cast<size_t>(c) * kChunk * v_stride;
-        const unsigned beyond = (min(kChunk, q_len - c * kChunk) - 1) * row;          // the chunk's last token
-        // (beyond it, that token's once more: what it is multiplied by is zero)
+        const T* v_chunk = v_first + static_cast<size_t>(begins(c)) * v_stride;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[min((4 * u + g) * row, beyond) + col];
+        for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[(4 * u + g) * row + col];
         return o;
     };
     const int count = (q_len + kChunk - 1) / kChunk;
@@ -506,7 +522,7 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
         memory_float4 x, read[TILES];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-            x[u] = c * kChunk + 4 * u + g < q_len ? (norm_col ? 1.f : to_float(now.v[u])) : 0.f;
+            x[u] = begins(c) + 4 * u + g >= c * kChunk ? (norm_col ? 1.f : to_float(now.v[u])) : 0.f;
         // (a sum a tile, added in the end: short chains of products, and of roundings)
 #pragma unroll
         for (int j = 0; j < TILES; ++j) read[j] = memory_float4{0.f, 0.f, 0.f, 0.f};
@@ -514,10 +530,11 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int j = 0; j < TILES; ++j) read[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][u], s[j][u], read[j], 0, 0, 0);
-        // (the chunk's own sum first, from zero, and the memory joins it with one rounding a chunk)
+        // (the chunk's own sum first, from what its newest keys lost in rounding, and the memory joins it with one rounding)
         memory_float4 own[TILES];
 #pragma unroll
-        for (int j = 0; j < TILES; ++j) own[j] = memory_float4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TILES; ++j)
+            own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.rest[j], x[3], memory_float4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -542,8 +559,8 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
         float o = parts[0];
 #pragma unroll
         for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
-        const int t = c * kChunk + 4 * g + wave;
-        if (live && t < q_len) {
+        const int t = begins(c) + 4 * g + wave;
+        if (live && t >= c * kChunk) {
             if (norm_col) nq[static_cast<size_t>(q_start + t) * heads + h] = o;
             else y[static_cast<size_t>(q_start + t) * heads * p_dim + static_cast<size_t>(h) * p_dim + p] = o;
         }

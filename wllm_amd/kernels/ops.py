@@ -1049,7 +1049,7 @@ def _memory_chunks(v: torch.Tensor, segments: int, heads: int, head_dim: int) ->
     if not places:
         return None
     c = -(-head_dim // 64) * 64
-    return torch.empty(places * heads * ((2 * SCAN_CHUNK + 1) * c + SCAN_CHUNK * SCAN_CHUNK), dtype=torch.float32, device=v.device)
+    return torch.empty(places * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK), dtype=torch.float32, device=v.device)
 
 
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
