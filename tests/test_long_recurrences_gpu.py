@@ -1,0 +1,143 @@
+"""The recurrences over long portions of a prompt (`ops.ssm_scan`, `ops.memory_scan`: 16 tokens at a time on the matrix
+cores) against the same kernels' walk token by token, which a prompt cut into portions of fewer than 64 tokens takes."""
+import pytest
+import torch
+
+from wllm_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SHORT = 40                  # a portion of so many tokens is walked token by token
+
+
+def _ints(values):
+    return torch.tensor(values, dtype=torch.int32, device=DEV)
+
+
+class StateSpace:
+    """Random operands of `ops.ssm_scan` for a sequence, and the recurrence over it in portions."""
+    parts = ("x", "B", "C", "dt")
+
+    def __init__(self, dtype, tokens, heads=4, groups=2, n_state=24, p=20, seed=1):
+        g = torch.Generator().manual_seed(seed)
+        self.heads, self.groups, self.n_state, self.p, self.tokens = heads, groups, n_state, p, tokens
+        self.inner = heads * p
+        self.xbc = (torch.randn(tokens, self.inner + 2 * groups * n_state, generator=g) * 0.7).to(dtype).to(DEV)
+        self.dt = torch.randn(tokens, heads, generator=g).to(dtype).to(DEV)
+        self.vectors = [(m + torch.randn(heads, generator=g)).to(DEV) for m in (-1.0, -0.5, 1.0)]
+        self.state0 = torch.randn(3, heads * n_state * p + 4, generator=g).to(DEV)
+
+    def put(self, part, token, value):
+        at = {"x": 7, "B": self.inner + 5, "C": self.inner + self.groups * self.n_state + 5}
+        if part == "dt":
+            self.dt[token, 1] = value
+        else:
+            self.xbc[token, at[part]] = value
+
+    def launch(self, rows, q_start, q_len, slots, state, y):
+        ops.ssm_scan(self.xbc[rows].contiguous(), self.dt[rows].contiguous(), *self.vectors, state, _ints(q_start), _ints(q_len),
+                     _ints(slots), y, heads=self.heads, groups=self.groups, state_size=self.n_state, head_dim=self.p)
+
+    def run(self, cuts):
+        state, out, at = self.state0.clone(), [], 0
+        for n in cuts:
+            y = torch.full((n, self.inner), 7.0, device=DEV)
+            self.launch(slice(at, at + n), [0], [n], [1], state, y)
+            out.append(y)
+            at += n
+        return torch.cat(out), state
+
+
+class Memory:
+    """The same of `ops.memory_scan`, for each kind of decay (`own`: steps of its own, with the normaliser)."""
+    parts = ("q", "k", "v", "decay")
+
+    def __init__(self, dtype, tokens, kind, heads=3, d=24, dv=20, seed=2):
+        g = torch.Generator().manual_seed(seed)
+        self.kind, self.heads, self.d, self.dv, self.tokens = kind, heads, d, dv, tokens
+        self.memory = heads * d * dv
+        self.qk = torch.randn(3 if kind == "rows" else 2, tokens, heads * d, generator=g).to(DEV) * d ** -0.5
+        if kind == "rows":
+            self.qk[2] = torch.rand(tokens, heads * d, generator=g).to(DEV)
+        self.v = torch.randn(tokens, heads * dv, generator=g).to(dtype).to(DEV)
+        self.decays = (1.0 - torch.logspace(0, -4, heads)).to(DEV)
+        self.steps = torch.rand(3, tokens, heads, generator=g).to(DEV)
+        self.state0 = torch.randn(3, self.memory + heads * d, generator=g).to(DEV)
+
+    def put(self, part, token, value):
+        if part == "v":
+            self.v[token, 7] = value
+        elif part != "decay":
+            self.qk[0 if part == "q" else 1, token, 9] = value
+        elif self.kind == "rows":
+            self.qk[2, token, 9] = value
+        elif self.kind == "own":
+            self.steps[0, token, 1] = value
+
+    def launch(self, rows, q_start, q_len, slots, state, y):
+        own, n = self.kind == "own", y.shape[0]
+        width = self.heads * self.dv
+        out, nq = torch.full((n, width), 7.0, device=DEV), torch.full((n, self.heads), 7.0, device=DEV)
+        ops.memory_scan(self.qk[:, rows].contiguous(), self.v[rows].contiguous(), self.steps[:, rows].contiguous() if own else None,
+                        self.decays if self.kind == "head" else None, state, _ints(q_start), _ints(q_len), _ints(slots), out,
+                        heads=self.heads, head_dim=self.d, value_dim=self.dv, nq=nq if own else None,
+                        n_offset=self.memory if own else 0, row_decays=self.kind == "rows")
+        y.copy_(torch.cat([out, nq], dim=1))
+
+    def run(self, cuts):
+        state, out, at = self.state0.clone(), [], 0
+        for n in cuts:
+            y = torch.zeros(n, self.heads * self.dv + self.heads, device=DEV)
+            self.launch(slice(at, at + n), [0], [n], [1], state, y)
+            out.append(y)
+            at += n
+        return torch.cat(out), state
+
+
+KINDS = ["space", "head", "rows", "own"]
+
+
+def _problem(kind, dtype, tokens, **sizes):
+    return StateSpace(dtype, tokens, **sizes) if kind == "space" else Memory(dtype, tokens, kind, **sizes)
+
+
+def _portions(tokens, most=SHORT):
+    return [most] * (tokens // most) + ([tokens % most] if tokens % most else [])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_value_that_is_not_finite_leaves_the_tokens_before_it_alone(dtype, kind):
+    """An infinity or NaN in any operand of a token, at either end of a chunk of 16, inside one and in a prompt's last
+    tokens: what comes before has the bits it has without it, and from there on it reaches what the walk token by token
+    says it reaches, in the results and in the state left behind."""
+    tokens = 101
+    clean = _problem(kind, dtype, tokens).run([tokens])[0]
+    parts = StateSpace.parts if kind == "space" else Memory.parts[:3] if kind == "head" else Memory.parts
+    for part in parts:
+        for at in (0, 15, 32, 40, 95, 99):
+            for value in (float("inf"), float("-inf"), float("nan")):
+                if part in ("dt", "decay") and value == float("-inf"):
+                    continue                                  # (a step size of zero; decays are not negative)
+                hit = _problem(kind, dtype, tokens)
+                hit.put(part, at, value)
+                (y, state), (ref, ref_state) = hit.run([tokens]), hit.run(_portions(tokens))
+                case = f"{part} of token {at}: {value}"
+                assert torch.equal(y[:at], clean[:at]), f"{case}: a token before it changed"
+                assert torch.equal(torch.isfinite(y), torch.isfinite(ref)), f"{case}: results"
+                assert not bool(torch.isfinite(y[at]).all()), case
+                assert torch.equal(torch.isfinite(state), torch.isfinite(ref_state)), f"{case}: the state"
+
+
+def test_a_key_that_overflows_is_infinite_and_not_nan():
+    """A key of 3e38 that its step takes out of float32: infinite in the memory, as the walk token by token leaves it."""
+    tokens = 96
+    hit = _problem("own", torch.bfloat16, tokens)
+    for t in (hit.qk, hit.v, hit.state0):
+        t.abs_()
+    hit.steps[0].clamp_(min=0.5)
+    hit.qk[1, 94, 9], hit.steps[1, 94] = 3e38, 40.0            # (one of the last four tokens of a chunk)
+    (y, state), (ref, ref_state) = hit.run([tokens]), hit.run(_portions(tokens))
+    assert not bool(torch.isnan(ref).any() or torch.isnan(ref_state).any()) and bool(torch.isinf(ref_state).any())
+    assert not bool(torch.isnan(y).any() or torch.isnan(state).any())
+    assert torch.equal(torch.isinf(state), torch.isinf(ref_state))

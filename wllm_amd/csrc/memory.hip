@@ -11,6 +11,7 @@
 // where the heads are normed (`head_norm_gate`).
 // Everything that enters the recurrence is float32: the rotated queries and keys, the gates, their
 // exponentials, the maximum, the normaliser, the state and every sum.
+#include "causal_product.h"
 #include "common.h"
 
 // ---- queries and keys as the recurrence takes them: qk[0] = q_scale * rot(q), qk[1] = k_scale * rot(k), float32.
@@ -444,7 +445,8 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
         for (int t = kChunk - 1; t >= 0; --t) {
             const double key = static_cast<double>(k_s[t * C + c]) * b_s[t] * behind;
             kh[t] = static_cast<float>(key);
-            if (t >= kChunk - 4) rest[t - (kChunk - 4)] = static_cast<float>(key - kh[t]);
+            // (a key that 32 bits do not hold is infinite, and has no remainder: inf - inf would be NaN)
+            if (t >= kChunk - 4) rest[t - (kChunk - 4)] = fabsf(kh[t]) <= 3.402823466e38f ? static_cast<float>(key - kh[t]) : 0.f;
             behind *= f_s[t * C + c];
         }
         // (token 4u + g at place 4g + u: the u-th product of the walk then takes the tokens 4u .. 4u + 3, the oldest first)
@@ -548,7 +550,7 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
         memory_float4 part = read[0];
 #pragma unroll
         for (int j = 1; j < TILES; ++j) part += read[j];
-        part = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, part, 0, 0, 0);
+        part = add_causal_product(now.n, mine, part, i, g, [&](int q) { return 4 * wave + q; });
         part_s[c % 2][wave][lane] = part;
         // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -6,6 +6,7 @@
 //   (the oldest first).
 // A fresh request's row is all zeros, which is both "S starts at zero" and "zeros before the start".
 // Everything that enters the recurrence is float32: step sizes, decays, the state, the sums.
+#include "causal_product.h"
 #include "common.h"
 #include "short_conv.h"
 
@@ -751,7 +752,7 @@ ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, con
         ssm_float4 part = read[0];
 #pragma unroll
         for (int j = 1; j < TILES; ++j) part += read[j];
-        part = __builtin_amdgcn_mfma_f32_16x16x4f32(now.n, mine, part * now.pre, 0, 0, 0);
+        part = add_causal_product(now.n, mine, part * now.pre, i, g, [&](int q) { return 4 * q + wave; });
         part_s[c % 2][wave][lane] = part;
         // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
