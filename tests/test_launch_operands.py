@@ -1,0 +1,70 @@
+"""What a launch is handed, without a GPU: every address it gets belongs to a tensor that is still held when it is made."""
+import weakref
+
+import pytest
+import torch
+
+from wllm_amd.kernels import ops
+
+
+class Launches:
+    """A backend whose launches end in a function that only looks at the arguments of the entry point."""
+
+    def __init__(self, look):
+        self.look = look
+
+    def run_registered(self, op, args, kwargs):
+        op.launch(lambda *arguments: self.look(op, arguments), 0, *args, **kwargs)
+
+
+def _ints(*values):
+    return torch.tensor(values, dtype=torch.int32)
+
+
+def _scan(kind, n, **extra):
+    heads, d = 2, 16
+    state, seg = torch.zeros(3, heads * d * d + heads * d), (_ints(0), _ints(n), _ints(1))
+    if kind == "space":
+        xbc, vectors = torch.zeros(n, heads * d + 2 * d, dtype=torch.bfloat16), [torch.zeros(heads) for _ in range(3)]
+        ops.ssm_scan(xbc, torch.zeros(n, heads, dtype=torch.bfloat16), *vectors, state, *seg, torch.zeros(n, heads * d), heads=heads,
+                     groups=1, state_size=d, head_dim=d, **extra)
+    else:
+        ops.memory_scan(torch.zeros(2, n, heads * d), torch.zeros(n, heads * d, dtype=torch.bfloat16), None, torch.zeros(heads), state,
+                        *seg, torch.zeros(n, heads * d), heads=heads, head_dim=d, value_dim=d, **extra)
+
+
+@pytest.mark.parametrize("kind", ["space", "memory"])
+def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
+    """The scratch of a recurrence walked in chunks (the third argument from the end) is a tensor that something refers to
+    when the launch is made: else its memory is the allocator's again before a kernel has run."""
+    made, empty, seen = [], torch.empty, []
+
+    def recorded(*args, **kwargs):
+        t = empty(*args, **kwargs)
+        made.append((t.data_ptr(), weakref.ref(t)))
+        return t
+
+    def look(op, arguments):
+        address = getattr(arguments[-3], "value", arguments[-3])
+        seen.append(address)
+        assert any(at == address and ref() is not None for at, ref in made), "the scratch was given back before the launch"
+        return 0
+    monkeypatch.setattr(torch, "empty", recorded)
+    with ops.use_backend(Launches(look)):
+        _scan(kind, 80)
+    assert seen and seen[0]
+
+
+@pytest.mark.parametrize("kind", ["space", "memory"])
+def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
+    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16)
+    mine = torch.zeros(size)
+    with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-3]) or 0)):
+        seen = []
+        _scan(kind, 80, chunks=mine)
+        assert seen == [mine.data_ptr()]
+        for wrong in (mine[:-1], mine.double(), torch.zeros(size, 2)[:, 0]):
+            with pytest.raises(ops.KernelShapeError):
+                _scan(kind, 80, chunks=wrong)
+        assert len(seen) == 1
+    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16)

@@ -987,10 +987,45 @@ def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, carr
              **({"single_tokens": True} if single_tokens else {}))
 
 
+# tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
+# on the matrix cores
+SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
+
+
+def _scan_places(tokens: int, segments: int) -> int:
+    """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
+    return tokens // SCAN_CHUNK + segments + 1 if tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
+
+
+def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_size: int, dtype: torch.dtype) -> int:
+    """Floats of scratch with which `ssm_scan` walks a step in chunks; 0: it does without (a decode step, so a captured graph
+    holds none)."""
+    rows = 2 * SCAN_CHUNK * (-(-state_size // 64) * 64) * dtype.itemsize // 4
+    return _scan_places(tokens, segments) * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows)
+
+
+def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int) -> int:
+    """The same for `memory_scan`."""
+    c = -(-head_dim // 64) * 64
+    return _scan_places(tokens, segments) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
+
+
+def _scan_scratch(chunks: Optional[torch.Tensor], size: int, device) -> dict:
+    """What the walk in chunks adds to a launch's operands: the scratch, the caller's or made here (an operand, so that
+    it is held until the launch has been made)."""
+    if size == 0:
+        return {}
+    if chunks is None:
+        chunks = torch.empty(size, dtype=torch.float32, device=device)
+    _dense(chunks, "chunks", torch.float32)
+    _need(chunks.numel() >= size, lambda: f"chunks: {chunks.numel()} floats of scratch, needed {size}")
+    return {"chunks": chunks}
+
+
 def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, d_skip: torch.Tensor,
              state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
              y: torch.Tensor, *, heads: int, groups: int, state_size: int, head_dim: int,
-             steps: Optional[torch.Tensor] = None) -> None:
+             steps: Optional[torch.Tensor] = None, chunks: Optional[torch.Tensor] = None) -> None:
     """The selective state-space recurrence over each segment's tokens in order, from and into the
     request's carried state.  Per head h (group h // (heads // groups)) and token:
         step = softplus(dt + dt_bias[h]);  S = exp(-exp(a_log[h]) * step) * S + step * B x^T;
@@ -998,8 +1033,8 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     xbc T [n, heads*P + 2*groups*N]: x, then B, then C; dt T [n, heads] (may be a band of a wider row);
     dt_bias, a_log, d_skip float32 [heads]; state float32 [slots, W], whose row state_slots[segment]
     begins with S as [heads, N, P]; y float32 [n, heads*P].  All of the recurrence is float32.
-    `steps`: float32 [2, n, heads] of scratch for the step sizes and decays (made here if not given; a
-    caller whose step may be captured in a graph gives its own)."""
+    `steps`: float32 [2, n, heads] of scratch for the step sizes and decays, `chunks`: float32 scratch of `ssm_chunk_size`
+    elements (made here if not given; a caller whose step may be captured in a graph gives its own)."""
     _dense(xbc, "xbc", _ACT)
     inner = heads * head_dim
     _need(heads > 0 and groups > 0 and heads % groups == 0, "heads must be a multiple of groups")
@@ -1021,35 +1056,8 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     _dense(steps, "steps", torch.float32, (2, n, heads))
     if n:
         call("ssm_scan", xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y, heads, groups,
-             state_size, head_dim, steps)
-
-
-# tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
-# on the matrix cores
-SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
-
-
-def _scan_places(tokens: int, segments: int) -> int:
-    """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
-    return tokens // SCAN_CHUNK + segments + 1 if tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
-
-
-def _ssm_chunks(xbc: torch.Tensor, segments: int, heads: int, groups: int, state_size: int) -> Optional[torch.Tensor]:
-    """The scratch of the walk in chunks, or None (a decode step has none, so a captured graph holds no address of it)."""
-    places = _scan_places(xbc.shape[0], segments)
-    if not places:
-        return None
-    rows = 2 * SCAN_CHUNK * (-(-state_size // 64) * 64) * xbc.element_size() // 4
-    return torch.empty(places * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows), dtype=torch.float32, device=xbc.device)
-
-
-def _memory_chunks(v: torch.Tensor, segments: int, heads: int, head_dim: int) -> Optional[torch.Tensor]:
-    """The same for `memory_scan`."""
-    places = _scan_places(v.shape[0], segments)
-    if not places:
-        return None
-    c = -(-head_dim // 64) * 64
-    return torch.empty(places * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK), dtype=torch.float32, device=v.device)
+             state_size, head_dim, steps,
+             **_scan_scratch(chunks, ssm_chunk_size(n, s, heads, groups, state_size, xbc.dtype), xbc.device))
 
 
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
@@ -1147,7 +1155,7 @@ def memory_gates(gates: torch.Tensor, i_bias: Optional[torch.Tensor], f_bias: Op
 def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor], decays: Optional[torch.Tensor],
                 state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
                 y: torch.Tensor, *, heads: int, head_dim: int, value_dim: int, nq: Optional[torch.Tensor] = None,
-                n_offset: int = 0, row_decays: bool = False) -> None:
+                n_offset: int = 0, row_decays: bool = False, chunks: Optional[torch.Tensor] = None) -> None:
     """The matrix memory's recurrence over each segment's tokens in order, from and into the request's
     carried state.  Per head:  S = a S + b k v^T;  y = S^T q  with (a, b) of the token from `steps` (float32
     [3, n, heads], of which the first two are read) or, with `decays` (float32 [heads]) instead, (decays[h], 1).
@@ -1156,7 +1164,8 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     keys; v T [n, heads * value_dim] (may be a band); state float32 [slots, W], whose row state_slots[segment]
     begins with S as [heads, head_dim, value_dim]; y float32 [n, heads * value_dim].  All of the recurrence is float32.
     `row_decays` (then neither `steps` nor `decays`): qk has a third plane, float32 [3, n, heads * head_dim], of decays a
-    row of S and token: S[i, :] = qk[2][i] S[i, :] + k[i] v^T."""
+    row of S and token: S[i, :] = qk[2][i] S[i, :] + k[i] v^T.  `chunks`: float32 scratch of `memory_chunk_size` elements
+    (made here if not given)."""
     if row_decays:
         _need(steps is None and decays is None, "row_decays: neither steps nor decays")
     else:
@@ -1182,7 +1191,8 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     _dense(y, "y", torch.float32, (n, heads * value_dim))
     if n:
         call("memory_scan", qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim, nq,
-             int(n_offset), **({"row_decays": True} if row_decays else {}))
+             int(n_offset), **({"row_decays": True} if row_decays else {}),
+             **_scan_scratch(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim), v.device))
 
 
 def head_norm_gate(y: torch.Tensor, gate: Optional[torch.Tensor], weight: Optional[torch.Tensor], out: torch.Tensor, *, heads: int,
@@ -1638,11 +1648,11 @@ def _register_own() -> None:
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                           c_int, c_void_p],
                 launch=lambda fn, stream, xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y,
-                heads, groups, state_size, head_dim, steps: fn(
+                heads, groups, state_size, head_dim, steps, chunks=None: fn(
                     p(xbc), p(dt), dt.stride(0), p(dt_bias), p(a_log), p(d_skip), p(state), state.stride(0), p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(steps), int(xbc.dtype == torch.bfloat16), xbc.shape[0],
                     seg_q_start.shape[0], heads, groups, state_size, head_dim,
-                    p(_ssm_chunks(xbc, seg_q_start.shape[0], heads, groups, state_size)), SCAN_CHUNK_FROM, stream))
+                    p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, stream))
     register_op("gated_group_norm", entry_point="wllm_gated_group_norm",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
                 launch=lambda fn, stream, y, z, weight, out, groups, eps: fn(
@@ -1674,11 +1684,10 @@ def _register_own() -> None:
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                           c_int, c_void_p],
                 launch=lambda fn, stream, qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads,
-                head_dim, value_dim, nq=None, n_offset=0, row_decays=False: fn(
+                head_dim, value_dim, nq=None, n_offset=0, row_decays=False, chunks=None: fn(
                     p(qk), p(v), v.stride(0), p(steps), p(decays), p(state), state.stride(0), n_offset, p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(nq), bf(v), v.shape[0], seg_q_start.shape[0], heads, head_dim,
-                    value_dim, int(row_decays), p(_memory_chunks(v, seg_q_start.shape[0], heads, head_dim)), SCAN_CHUNK_FROM,
-                    stream))
+                    value_dim, int(row_decays), p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, stream))
     register_op("head_norm_gate", entry_point="wllm_head_norm_gate",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_float, c_int,
                           c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
