@@ -57,7 +57,7 @@ def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
 def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
-    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16)
+    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, torch.bfloat16)
     mine = torch.zeros(size)
     with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-3]) or 0)):
         seen = []
@@ -67,4 +67,5 @@ def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
             with pytest.raises(ops.KernelShapeError):
                 _scan(kind, 80, chunks=wrong)
         assert len(seen) == 1
-    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16)
+    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, torch.bfloat16)
+    assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, torch.float32)

@@ -141,3 +141,14 @@ def test_a_key_that_overflows_is_infinite_and_not_nan():
     assert not bool(torch.isnan(ref).any() or torch.isnan(ref_state).any()) and bool(torch.isinf(ref_state).any())
     assert not bool(torch.isnan(y).any() or torch.isnan(state).any())
     assert torch.equal(torch.isinf(state), torch.isinf(ref_state))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_float32_has_the_same_bits_however_a_prompt_is_cut(kind):
+    """In the true 32-bit path a token's results do not depend on the portion it came in."""
+    tokens = 150
+    problem = _problem(kind, torch.float32, tokens)
+    whole, state = problem.run([tokens])
+    for cuts in ([64, 1, 85], _portions(tokens), [1] * tokens):
+        y, left = problem.run(cuts)
+        assert torch.equal(y, whole) and torch.equal(left, state), f"{cuts[:3]}"

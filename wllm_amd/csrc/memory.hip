@@ -187,7 +187,8 @@ WLLM_API int wllm_memory_gates(const void* gates, long long gates_stride, const 
 // registers.  Tokens go 16 at a time through shared memory (q, k, v, a, b), the next 16 fetched into registers
 // while these are walked; a token's sum is the slices' partial sums added in a fixed order (within the
 // wavefront, then wavefront by wavefront), so it has the same bits whether the token came alone or inside a
-// prompt.  With `steps` the column behind the last (p = P) is the normaliser: its value is 1 for every token,
+// prompt.  With values in float32 it takes every segment; in bfloat16 those of fewer than `shorter_than` tokens, the others
+// being walked in chunks further down, which add in another order.  With `steps` the column behind the last (p = P) is the normaliser: its value is 1 for every token,
 // its rows lie at `n_offset` of the request's row, and its sums go to `nq` [tokens, heads]. ----
 constexpr int kMemTokens = 16;
 constexpr int kMemWaves = 8;
@@ -334,7 +335,8 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
 // what the last four of a chunk's Kh, which weigh most, lost in being rounded to 32 bits), and
 // `memory_chunk_scan_kernel` walks a segment's chunks with v_mfma_f32_16x16x4_f32 (float32 in and out).  A chunk begins
 // every 16 tokens of a segment; the last one is its last 16 tokens, those of the chunk before it as tokens that change
-// nothing (q = k = 0, f = 1).  Chunk c of segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// nothing (q = k = 0, f = 1).  Values in bfloat16 only: in the 32-bit path a token's bits do not depend on how its prompt
+// was cut.  Chunk c of segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
 // Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 34 and
 // 156 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 19 and 127, with
 // exponential gates and the normaliser 297 against 19 and 125; 64 tokens 12.6 against 7 and 9, from where on a segment
@@ -463,9 +465,9 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
 // 4g + k), so the memory never moves between lanes.  The wavefronts' parts of y meet in shared memory (two places in
 // turn: one barrier a chunk, which the memory's own chain does not wait for).  The operands of a chunk are asked for
 // kAhead chunks before they are used.
-template <typename T, int TILES>
+template <int TILES>
 __global__ void __launch_bounds__(256)
-memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, float* __restrict__ state, long long state_stride,
+memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride, float* __restrict__ state, long long state_stride,
                          long long n_offset, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
                          const int* __restrict__ state_slots, float* __restrict__ y, float* __restrict__ nq, int heads, int d,
                          int p_dim, int from) {
@@ -494,10 +496,10 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
     struct Operands {
         memory_float4 q[TILES], k[TILES], f[TILES];
         float rest[TILES], n;
-        T v[4];
+        bf16 v[4];
     };
     const float* first = chunks + (static_cast<size_t>(q_start / kChunk + seg) * heads + h) * chunk_floats(C);
-    const T* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
+    const bf16* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
     // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
     const unsigned q_at = i * C + ch0 + 4 * g, k_at = kChunk * C + (ch0 + i) * kChunk + 4 * g, f_at = 2 * kChunk * C + ch0 + 4 * g;
     const unsigned rest_at = (2 * kChunk + 1) * C + (ch0 + i) * 4 + g, n_at = (2 * kChunk + 5) * C + i * kChunk + 4 * wave + g;
@@ -514,7 +516,7 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
             o.rest[j] = at[rest_at + 64 * j];
         }
         o.n = at[n_at];
-        const T* v_chunk = v_first + static_cast<size_t>(begins(c)) * v_stride;
+        const bf16* v_chunk = v_first + static_cast<size_t>(begins(c)) * v_stride;
 #pragma unroll
         for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[(4 * u + g) * row + col];
         return o;
@@ -596,7 +598,7 @@ memory_chunk_scan_kernel(const float* chunks, const T* v, long long v_stride, fl
 // `steps` (float32 [3, tokens, heads], of which a and b are read; then `nq` float32 [tokens, heads] takes the
 // normaliser's sums and the normaliser lies at `n_offset` of a request's row) or, if null, `decays` (float32 [heads]; b = 1),
 // or, with `row_decays`, neither: then qk has a third plane [tokens, heads * d] of decays a row and token (b = 1).
-// `from` tokens (16 at least; 0: no segment) is what a segment needs to be walked in chunks, out of the scratch `chunks`:
+// `from` tokens (16 at least; 0: no segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`:
 // tokens / 16 + segments + 1 places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
 WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride, const float* steps, const float* decays,
                               float* state, long long state_stride, long long n_offset, const int* seg_q_start,
@@ -613,26 +615,23 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
     // (a segment of `from` tokens leaves room for the others' single tokens)
     const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
     if (in_chunks) {
-        if (!chunks || from < kChunk || d > 256 || heads > 65535 || v_stride > 0x0fffffffLL ||
+        if (!is_bf16 || !chunks || from < kChunk || d > 256 || heads > 65535 || v_stride > 0x0fffffffLL ||
             reinterpret_cast<uintptr_t>(chunks) % 16)
             return -1;
         const dim3 chunk_grid(tokens / kChunk + segments + 1, heads);
-#define LAUNCH(T, R)                                                                                                   \
+#define LAUNCH(R)                                                                                                      \
     do {                                                                                                               \
         memory_chunk_kernel<R><<<chunk_grid, 256, 0, stream>>>(qk, steps, decays, seg_q_start, seg_q_len, segments, chunks, \
                                                                tokens, heads, d, row_decays, from);                    \
         if (const int err = launch_status()) return err;                                                               \
-        memory_chunk_scan_kernel<T, R><<<grid, 256, 0, stream>>>(chunks, static_cast<const T*>(v), v_stride, state,    \
-                                                                 state_stride, n_offset, seg_q_start, seg_q_len,       \
-                                                                 state_slots, y, steps ? nq : nullptr, heads, d, p_dim, from); \
+        memory_chunk_scan_kernel<R><<<grid, 256, 0, stream>>>(chunks, static_cast<const bf16*>(v), v_stride, state,    \
+                                                              state_stride, n_offset, seg_q_start, seg_q_len, state_slots, y, \
+                                                              steps ? nq : nullptr, heads, d, p_dim, from);            \
     } while (0)
-#define LAUNCH_R(T)                   \
-    if (d <= 64) LAUNCH(T, 1);        \
-    else if (d <= 128) LAUNCH(T, 2);  \
-    else if (d <= 192) LAUNCH(T, 3);  \
-    else LAUNCH(T, 4);
-        if (is_bf16) { LAUNCH_R(bf16) } else { LAUNCH_R(float) }
-#undef LAUNCH_R
+        if (d <= 64) LAUNCH(1);
+        else if (d <= 128) LAUNCH(2);
+        else if (d <= 192) LAUNCH(3);
+        else LAUNCH(4);
 #undef LAUNCH
         if (const int err = launch_status()) return err;
         if (segments == 1) return 0;

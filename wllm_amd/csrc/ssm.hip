@@ -366,7 +366,8 @@ WLLM_API int wllm_stream_conv(const float* x, const float* weight, float* state,
 // transaction) 654 / 134 / 409.  Tokens are staged 16 at a time through shared memory
 // (B, C, x, step, decay), the next 16 fetched into registers meanwhile; a token's y is the slices'
 // partial sums added in a fixed order (within the wavefront, then wavefront by wavefront), so it has
-// the same bits whether the token came alone or inside a prompt. ----
+// the same bits whether the token came alone or inside a prompt.  In float32 it takes every segment; in bfloat16 those of
+// fewer than `shorter_than` tokens, the others being walked in chunks further down, which add in another order. ----
 constexpr int kScanTokens = 16;
 constexpr int kScanWaves = 8;
 constexpr int kScanCols = 16;                       // columns of P a workgroup owns
@@ -524,6 +525,7 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
 // a head's token t, pre_t the product of a chunk's decays up to t, and suf_s that of the decays behind s,
 //   y_t = pre_t (C_t . S0) + sum over s <= t of N_ts x_s + D x_t,   S = pre_16 S0 + B^T (suf_s d_s x_s),
 //   N_ts = (C_t . B_s) (the decays s < r <= t) d_s.
+// bfloat16 inputs only: in the 32-bit path a token's bits do not depend on how its prompt was cut.
 // A product of decays is formed from the decays it is made of (never as a quotient or a difference of logarithms), so
 // the numbers are those of the walk token by token up to the order of float32 sums.  Nothing but S0 depends on the
 // tokens before, so `ssm_chunk_kernel` makes all else for every chunk at once: per (chunk, group) the rows C_t and the
@@ -542,11 +544,11 @@ constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, 
 // on the matrix cores.
 typedef float ssm_float4 __attribute__((ext_vector_type(4)));
 
-template <typename T, int TILES>        // C = 64 TILES: the rows of state, padded
+template <int TILES>        // C = 64 TILES: the rows of state, padded
 __global__ void __launch_bounds__(256)
-ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long long dt_stride, const float* __restrict__ dt_bias,
+ssm_chunk_kernel(const bf16* __restrict__ xbc, const bf16* __restrict__ dt_in, long long dt_stride, const float* __restrict__ dt_bias,
                  const float* __restrict__ a_log, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
-                 int segments, float* __restrict__ of_head, T* __restrict__ of_group, int heads, int groups, int n_state,
+                 int segments, float* __restrict__ of_head, bf16* __restrict__ of_group, int heads, int groups, int n_state,
                  int p_dim, int from) {
     constexpr int C = 64 * TILES, kRow = C + 4;
     __shared__ __align__(16) float b_s[kChunk * kRow], c_s[kChunk * kRow];
@@ -567,13 +569,13 @@ ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long lo
     const int count = min(kChunk, seg_q_len[seg] - local), token = q_start + local;
     const int inner = heads * p_dim, channels = inner + 2 * groups * n_state;
     const int b_col = inner + g * n_state, c_col = b_col + groups * n_state;
-    T* rows = of_group + (static_cast<size_t>(place) * groups + g) * 2 * kChunk * C;
+    bf16* rows = of_group + (static_cast<size_t>(place) * groups + g) * 2 * kChunk * C;
     constexpr int kEach = kChunk * C / 256;
-    T b[kEach], c[kEach];
+    bf16 b[kEach], c[kEach];
 #pragma unroll
     for (int k = 0; k < kEach; ++k) {
         const int t = (tid + 256 * k) / C, n = (tid + 256 * k) % C;
-        const T* row = xbc + static_cast<size_t>(token + min(t, count - 1)) * channels + min(n, n_state - 1);
+        const bf16* row = xbc + static_cast<size_t>(token + min(t, count - 1)) * channels + min(n, n_state - 1);
         b[k] = row[b_col];
         c[k] = row[c_col];
     }
@@ -581,7 +583,7 @@ ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long lo
     for (int k = 0; k < kEach; ++k) {
         const int t = (tid + 256 * k) / C, n = (tid + 256 * k) % C;
         const bool there = t < count && n < n_state;
-        const T bv = there ? b[k] : from_float<T>(0.f), cv = there ? c[k] : from_float<T>(0.f);
+        const bf16 bv = there ? b[k] : from_float<bf16>(0.f), cv = there ? c[k] : from_float<bf16>(0.f);
         b_s[t * kRow + n] = to_float(bv);
         c_s[t * kRow + n] = to_float(cv);
         rows[tid + 256 * k] = cv;
@@ -590,7 +592,7 @@ ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long lo
 #pragma unroll
     for (int k = 0; k < kEach; ++k) {
         const int e = tid + 256 * k;
-        rows[kChunk * C + e] = from_float<T>(b_s[e % kChunk * kRow + e / kChunk]);
+        rows[kChunk * C + e] = from_float<bf16>(b_s[e % kChunk * kRow + e / kChunk]);
     }
     const int lane = tid % kWave, wave = tid / kWave, i = lane % 16, q = lane / 16;
     {
@@ -656,11 +658,11 @@ ssm_chunk_kernel(const T* __restrict__ xbc, const T* __restrict__ dt_in, long lo
 // it takes (the k-th of four products takes the rows 4g + k), so the state never moves between lanes.  The wavefronts'
 // parts of y meet in shared memory (two places in turn: one barrier a chunk, which the state's own chain does not wait
 // for).  The operands of the next chunks are asked for kAhead chunks before they are used.
-template <typename T> struct alignas(4 * sizeof(T)) SsmFour { T v[4]; };
+struct alignas(8) SsmFour { bf16 v[4]; };
 
-template <typename T, int TILES>
+template <int TILES>
 __global__ void __launch_bounds__(256)
-ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, const float* __restrict__ d_skip,
+ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xbc, const float* __restrict__ d_skip,
                       float* __restrict__ state, long long state_stride, const int* __restrict__ seg_q_start,
                       const int* __restrict__ seg_q_len, const int* __restrict__ state_slots, float* __restrict__ y, int heads,
                       int groups, int n_state, int p_dim, int from) {
@@ -686,15 +688,15 @@ ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, con
         }
     const float skip = d_skip[h];
     struct Operands {
-        SsmFour<T> c[TILES], b[TILES];
+        SsmFour c[TILES], b[TILES];
         ssm_float4 pre, suf;
         float n, all;
-        T x[4];
+        bf16 x[4];
     };
     const size_t first = static_cast<size_t>(q_start / kChunk + seg);
     const float* head_first = of_head + (first * heads + h) * kChunkHeadFloats;
-    const T* group_first = of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C;
-    const T* x_first = xbc + static_cast<size_t>(q_start) * channels + h * p_dim;
+    const bf16* group_first = of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C;
+    const bf16* x_first = xbc + static_cast<size_t>(q_start) * channels + h * p_dim;
     float* y_first = y + static_cast<size_t>(q_start) * inner + h * p_dim;
     // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
     const unsigned c_at = i * C + n0 + 4 * g, b_at = kChunk * C + (n0 + i) * kChunk + 4 * g;
@@ -702,18 +704,18 @@ ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, con
     const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(channels);
     auto load = [&](int c) {
         Operands o;
-        const T* rows = group_first + static_cast<size_t>(c) * groups * 2 * kChunk * C;
+        const bf16* rows = group_first + static_cast<size_t>(c) * groups * 2 * kChunk * C;
         const float* of = head_first + static_cast<size_t>(c) * heads * kChunkHeadFloats;
 #pragma unroll
         for (int j = 0; j < TILES; ++j) {
-            o.c[j] = *reinterpret_cast<const SsmFour<T>*>(rows + c_at + 16 * j);
-            o.b[j] = *reinterpret_cast<const SsmFour<T>*>(rows + b_at + 16 * kChunk * j);
+            o.c[j] = *reinterpret_cast<const SsmFour*>(rows + c_at + 16 * j);
+            o.b[j] = *reinterpret_cast<const SsmFour*>(rows + b_at + 16 * kChunk * j);
         }
         o.n = of[n_at];
         o.pre = *reinterpret_cast<const ssm_float4*>(of + pre_at);
         o.suf = *reinterpret_cast<const ssm_float4*>(of + pre_at + kChunk);
         o.all = of[kChunk * kChunk + 2 * kChunk];
-        const T* x_chunk = x_first + static_cast<size_t>(c) * kChunk * channels;
+        const bf16* x_chunk = x_first + static_cast<size_t>(c) * kChunk * channels;
         const unsigned beyond = (min(kChunk, q_len - c * kChunk) - 1) * row;          // the chunk's last token
         // (beyond it, that token's once more: what it is multiplied by is zero)
 #pragma unroll
@@ -794,8 +796,8 @@ ssm_chunk_scan_kernel(const float* of_head, const T* of_group, const T* xbc, con
 }
 
 // `steps`: scratch of 2 * tokens * heads floats (the step sizes, then the decays).  `from` tokens (16 at least; 0: no
-// segment) is what a segment needs to be walked in chunks, out of the scratch `chunks`: a place for every chunk of every
-// segment (tokens / 16 + segments + 1), first [place][head] of kChunkHeadFloats floats, then [place][group] of
+// segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`: a place for every
+// chunk of every segment (tokens / 16 + segments + 1), first [place][head] of kChunkHeadFloats floats, then [place][group] of
 // 32 x (the rows of state padded to a multiple of 64) elements.
 WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stride, const float* dt_bias, const float* a_log,
                            const float* d_skip, float* state, long long state_stride, const int* seg_q_start,
@@ -810,27 +812,24 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
     // (a segment of `from` tokens leaves room for the others' single tokens)
     const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
     if (in_chunks) {
-        if (!chunks || from < kChunk || n_state > 256 || groups > 65535 || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
+        if (!is_bf16 || !chunks || from < kChunk || n_state > 256 || groups > 65535 || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
         const int places = tokens / kChunk + segments + 1;
         const dim3 chunk_grid(places, groups);
-        float* of_group = chunks + static_cast<size_t>(places) * heads * kChunkHeadFloats;
-#define LAUNCH(T, TILES)                                                                                               \
+        bf16* of_group = reinterpret_cast<bf16*>(chunks + static_cast<size_t>(places) * heads * kChunkHeadFloats);
+#define LAUNCH(TILES)                                                                                                  \
     do {                                                                                                               \
-        ssm_chunk_kernel<T, TILES><<<chunk_grid, 256, 0, stream>>>(                                                    \
-            static_cast<const T*>(xbc), static_cast<const T*>(dt_in), dt_stride, dt_bias, a_log, seg_q_start, seg_q_len, \
-            segments, chunks, reinterpret_cast<T*>(of_group), heads, groups, n_state, p_dim, from);                    \
+        ssm_chunk_kernel<TILES><<<chunk_grid, 256, 0, stream>>>(                                                       \
+            static_cast<const bf16*>(xbc), static_cast<const bf16*>(dt_in), dt_stride, dt_bias, a_log, seg_q_start, seg_q_len, \
+            segments, chunks, of_group, heads, groups, n_state, p_dim, from);                                          \
         if (const int err = launch_status()) return err;                                                               \
-        ssm_chunk_scan_kernel<T, TILES><<<grid, 256, 0, stream>>>(                                                     \
-            chunks, reinterpret_cast<const T*>(of_group), static_cast<const T*>(xbc), d_skip, state, state_stride, seg_q_start, \
-            seg_q_len, state_slots, y, heads, groups, n_state, p_dim, from);                                           \
+        ssm_chunk_scan_kernel<TILES><<<grid, 256, 0, stream>>>(                                                        \
+            chunks, of_group, static_cast<const bf16*>(xbc), d_skip, state, state_stride, seg_q_start, seg_q_len, state_slots, y, \
+            heads, groups, n_state, p_dim, from);                                                                      \
     } while (0)
-#define LAUNCH_TILES(T)                     \
-    if (n_state <= 64) LAUNCH(T, 1);        \
-    else if (n_state <= 128) LAUNCH(T, 2);  \
-    else if (n_state <= 192) LAUNCH(T, 3);  \
-    else LAUNCH(T, 4);
-        if (is_bf16) { LAUNCH_TILES(bf16) } else { LAUNCH_TILES(float) }
-#undef LAUNCH_TILES
+        if (n_state <= 64) LAUNCH(1);
+        else if (n_state <= 128) LAUNCH(2);
+        else if (n_state <= 192) LAUNCH(3);
+        else LAUNCH(4);
 #undef LAUNCH
         if (const int err = launch_status()) return err;
         if (segments == 1) return 0;

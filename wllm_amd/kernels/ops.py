@@ -987,27 +987,30 @@ def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, carr
              **({"single_tokens": True} if single_tokens else {}))
 
 
-# tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
-# on the matrix cores
+# Tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
+# on the matrix cores.  In bfloat16 only: the chunks add in another order than the walk token by token, and in the true
+# 32-bit path, which results are compared with, a token has the same bits however its prompt was cut (the products keep them
+# too).  1,500 tokens of 64 heads of 64 by 128 take 100 us in chunks and 410 token by token
+# (a float32 prompt of 1,500 tokens of the Tokuvik 2B sizes: 62.5 ms, where chunks gave 60.6).
 SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
 
 
-def _scan_places(tokens: int, segments: int) -> int:
+def _scan_places(tokens: int, segments: int, dtype: torch.dtype) -> int:
     """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
-    return tokens // SCAN_CHUNK + segments + 1 if tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
+    return tokens // SCAN_CHUNK + segments + 1 if dtype == torch.bfloat16 and tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
 
 
 def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_size: int, dtype: torch.dtype) -> int:
     """Floats of scratch with which `ssm_scan` walks a step in chunks; 0: it does without (a decode step, so a captured graph
     holds none)."""
-    rows = 2 * SCAN_CHUNK * (-(-state_size // 64) * 64) * dtype.itemsize // 4
-    return _scan_places(tokens, segments) * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows)
+    rows = SCAN_CHUNK * (-(-state_size // 64) * 64)          # (two rows a token, of bfloat16)
+    return _scan_places(tokens, segments, dtype) * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows)
 
 
-def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int) -> int:
-    """The same for `memory_scan`."""
+def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, dtype: torch.dtype) -> int:
+    """The same for `memory_scan` (`dtype`: that of the values)."""
     c = -(-head_dim // 64) * 64
-    return _scan_places(tokens, segments) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
+    return _scan_places(tokens, segments, dtype) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
 
 
 def _scan_scratch(chunks: Optional[torch.Tensor], size: int, device) -> dict:
@@ -1192,7 +1195,7 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     if n:
         call("memory_scan", qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim, nq,
              int(n_offset), **({"row_decays": True} if row_decays else {}),
-             **_scan_scratch(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim), v.device))
+             **_scan_scratch(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, v.dtype), v.device))
 
 
 def head_norm_gate(y: torch.Tensor, gate: Optional[torch.Tensor], weight: Optional[torch.Tensor], out: torch.Tensor, *, heads: int,

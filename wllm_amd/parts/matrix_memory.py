@@ -172,7 +172,7 @@ class MatrixMemoryMixer:
                              n_offset + self.qk_width, ctx.seg_q_start, ctx.seg_q_len, ctx.state_slots, steps,
                              heads=s.num_heads, cap=s.gate_cap)
         y = ctx.buffer("memory_y", (n, self.v_width), torch.float32)
-        size = ops.memory_chunk_size(n, ctx.num_segments, s.num_heads, s.head_dim)
+        size = ops.memory_chunk_size(n, ctx.num_segments, s.num_heads, s.head_dim, h.dtype)
         ops.memory_scan(qk, row[:, self.v_offset:self.v_offset + self.v_width], steps, self.decays, state,
                         ctx.seg_q_start, ctx.seg_q_len, ctx.state_slots, y, heads=s.num_heads, head_dim=s.head_dim,
                         value_dim=s.value_dim, nq=nq, n_offset=self.memory_size if self.exponential else 0,
