@@ -35,7 +35,7 @@ def _scan(kind, n, **extra):
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
 def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
-    """The scratch of a recurrence walked in chunks (the third argument from the end) is a tensor that something refers to
+    """The scratch of a recurrence walked in chunks (the fourth argument from the end) is a tensor that something refers to
     when the launch is made: else its memory is the allocator's again before a kernel has run."""
     made, empty, seen = [], torch.empty, []
 
@@ -45,7 +45,7 @@ def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
         return t
 
     def look(op, arguments):
-        address = getattr(arguments[-3], "value", arguments[-3])
+        address = getattr(arguments[-4], "value", arguments[-4])
         seen.append(address)
         assert any(at == address and ref() is not None for at, ref in made), "the scratch was given back before the launch"
         return 0
@@ -59,7 +59,7 @@ def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
 def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
     size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, torch.bfloat16)
     mine = torch.zeros(size)
-    with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-3]) or 0)):
+    with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-4]) or 0)):
         seen = []
         _scan(kind, 80, chunks=mine)
         assert seen == [mine.data_ptr()]

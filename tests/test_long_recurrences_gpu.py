@@ -152,3 +152,24 @@ def test_float32_has_the_same_bits_however_a_prompt_is_cut(kind):
     for cuts in ([64, 1, 85], _portions(tokens), [1] * tokens):
         y, left = problem.run(cuts)
         assert torch.equal(y, whole) and torch.equal(left, state), f"{cuts[:3]}"
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("length", [0, 1, 15, 40, 63, 64, 70])
+def test_one_segment_of_fewer_tokens_than_rows(kind, length):
+    """A step's only segment holds fewer tokens than the operands have rows: its tokens are walked, whether there are
+    enough for chunks or not, and the rows behind them are left alone."""
+    problem = _problem(kind, torch.bfloat16, 80)
+    state = problem.state0.clone()
+    width = problem.inner if kind == "space" else problem.heads * (problem.dv + 1)
+    y = torch.full((80, width), 7.0, device=DEV)
+    problem.launch(slice(0, 80), [0], [length], [1], state, y)
+    assert bool((y[length:] == 7.0).all())
+    if length:
+        want, left = problem.run(_portions(length))
+        scale = float(want.abs().max())
+        # float32 sums of some hundred products in two orders: some 2^-24 each, of the largest
+        assert float((y[:length] - want).abs().max()) <= 2e-6 * scale
+        assert float((state - left).abs().max()) <= 2e-6 * float(left.abs().max())
+    else:
+        assert torch.equal(state, problem.state0)

@@ -598,12 +598,14 @@ memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride,
 // `steps` (float32 [3, tokens, heads], of which a and b are read; then `nq` float32 [tokens, heads] takes the
 // normaliser's sums and the normaliser lies at `n_offset` of a request's row) or, if null, `decays` (float32 [heads]; b = 1),
 // or, with `row_decays`, neither: then qk has a third plane [tokens, heads * d] of decays a row and token (b = 1).
-// `from` tokens (16 at least; 0: no segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`:
-// tokens / 16 + segments + 1 places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
+// `from` tokens (16 at least; 0: no segment, as in float32) is what a segment needs to be walked in chunks, out of the
+// scratch `chunks`: tokens / 16 + segments + 1 places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
+// `shortest`: the caller's word that no segment has fewer tokens (0: it has none); with it at `from` or above nothing is
+// launched for shorter ones.
 WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride, const float* steps, const float* decays,
                               float* state, long long state_stride, long long n_offset, const int* seg_q_start,
                               const int* seg_q_len, const int* state_slots, float* y, float* nq, int is_bf16, int tokens,
-                              int segments, int heads, int d, int p_dim, int row_decays, float* chunks, int from,
+                              int segments, int heads, int d, int p_dim, int row_decays, float* chunks, int from, int shortest,
                               hipStream_t stream) {
     if (segments <= 0 || tokens <= 0) return 0;
     if (row_decays ? (steps || decays) : ((!steps) == (!decays) || (steps && !nq))) return -1;
@@ -634,7 +636,7 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
         else LAUNCH(4);
 #undef LAUNCH
         if (const int err = launch_status()) return err;
-        if (segments == 1) return 0;
+        if (shortest >= from) return 0;
     }
     const int shorter_than = in_chunks ? from : 0x7fffffff;
 #define LAUNCH(T, R, ROWS)                                                                                          \

@@ -798,11 +798,12 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
 // `steps`: scratch of 2 * tokens * heads floats (the step sizes, then the decays).  `from` tokens (16 at least; 0: no
 // segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`: a place for every
 // chunk of every segment (tokens / 16 + segments + 1), first [place][head] of kChunkHeadFloats floats, then [place][group] of
-// 32 x (the rows of state padded to a multiple of 64) elements.
+// 32 x (the rows of state padded to a multiple of 64) elements.  `shortest`: the caller's word that no segment has fewer
+// tokens (0: it has none); with it at `from` or above nothing is launched for shorter ones.
 WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stride, const float* dt_bias, const float* a_log,
                            const float* d_skip, float* state, long long state_stride, const int* seg_q_start,
                            const int* seg_q_len, const int* state_slots, float* y, float* steps, int is_bf16, int tokens,
-                           int segments, int heads, int groups, int n_state, int p_dim, float* chunks, int from,
+                           int segments, int heads, int groups, int n_state, int p_dim, float* chunks, int from, int shortest,
                            hipStream_t stream) {
     if (segments <= 0 || tokens <= 0) return 0;
     if (!steps) return -1;
@@ -832,7 +833,7 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
         else LAUNCH(4);
 #undef LAUNCH
         if (const int err = launch_status()) return err;
-        if (segments == 1) return 0;
+        if (shortest >= from) return 0;
     }
     const int shorter_than = in_chunks ? from : 0x7fffffff;
     const int r = (n_state + kScanSlices - 1) / kScanSlices;

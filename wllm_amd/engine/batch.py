@@ -102,6 +102,7 @@ class StepContext:
         self.host_state_slots = host_state_slots
         self.requests = requests
         self.max_q_len = int(host_q_len.max()) if num_segments else 0
+        self.min_q_len = int(host_q_len.min()) if num_segments else 0
         self.max_ctx_len = int(host_ctx_len.max()) if num_segments else 0
         self._plans: dict = {}             # key -> (plan, refresh)
         # set by a captured graph: its kernels hold the addresses of what a part makes for the step, so

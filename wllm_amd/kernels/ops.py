@@ -1013,22 +1013,22 @@ def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, dty
     return _scan_places(tokens, segments, dtype) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
 
 
-def _scan_scratch(chunks: Optional[torch.Tensor], size: int, device) -> dict:
+def _scan_extra(chunks: Optional[torch.Tensor], size: int, shortest: int, device) -> dict:
     """What the walk in chunks adds to a launch's operands: the scratch, the caller's or made here (an operand, so that
-    it is held until the launch has been made)."""
+    it is held until the launch has been made), and whether shorter segments may be beside the long ones."""
     if size == 0:
         return {}
     if chunks is None:
         chunks = torch.empty(size, dtype=torch.float32, device=device)
     _dense(chunks, "chunks", torch.float32)
     _need(chunks.numel() >= size, lambda: f"chunks: {chunks.numel()} floats of scratch, needed {size}")
-    return {"chunks": chunks}
+    return {"chunks": chunks, "shortest": int(shortest)}
 
 
 def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, d_skip: torch.Tensor,
              state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
              y: torch.Tensor, *, heads: int, groups: int, state_size: int, head_dim: int,
-             steps: Optional[torch.Tensor] = None, chunks: Optional[torch.Tensor] = None) -> None:
+             steps: Optional[torch.Tensor] = None, chunks: Optional[torch.Tensor] = None, shortest: int = 0) -> None:
     """The selective state-space recurrence over each segment's tokens in order, from and into the
     request's carried state.  Per head h (group h // (heads // groups)) and token:
         step = softplus(dt + dt_bias[h]);  S = exp(-exp(a_log[h]) * step) * S + step * B x^T;
@@ -1037,7 +1037,9 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     dt_bias, a_log, d_skip float32 [heads]; state float32 [slots, W], whose row state_slots[segment]
     begins with S as [heads, N, P]; y float32 [n, heads*P].  All of the recurrence is float32.
     `steps`: float32 [2, n, heads] of scratch for the step sizes and decays, `chunks`: float32 scratch of `ssm_chunk_size`
-    elements (made here if not given; a caller whose step may be captured in a graph gives its own)."""
+    elements (made here if not given; a caller whose step may be captured in a graph gives its own).  `shortest`: the fewest
+    tokens of a segment of the step, if the caller knows it (0: it does not): a launch for short segments is then left out
+    where there are none."""
     _dense(xbc, "xbc", _ACT)
     inner = heads * head_dim
     _need(heads > 0 and groups > 0 and heads % groups == 0, "heads must be a multiple of groups")
@@ -1060,7 +1062,7 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     if n:
         call("ssm_scan", xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y, heads, groups,
              state_size, head_dim, steps,
-             **_scan_scratch(chunks, ssm_chunk_size(n, s, heads, groups, state_size, xbc.dtype), xbc.device))
+             **_scan_extra(chunks, ssm_chunk_size(n, s, heads, groups, state_size, xbc.dtype), shortest, xbc.device))
 
 
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
@@ -1158,7 +1160,8 @@ def memory_gates(gates: torch.Tensor, i_bias: Optional[torch.Tensor], f_bias: Op
 def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor], decays: Optional[torch.Tensor],
                 state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
                 y: torch.Tensor, *, heads: int, head_dim: int, value_dim: int, nq: Optional[torch.Tensor] = None,
-                n_offset: int = 0, row_decays: bool = False, chunks: Optional[torch.Tensor] = None) -> None:
+                n_offset: int = 0, row_decays: bool = False, chunks: Optional[torch.Tensor] = None,
+                shortest: int = 0) -> None:
     """The matrix memory's recurrence over each segment's tokens in order, from and into the request's
     carried state.  Per head:  S = a S + b k v^T;  y = S^T q  with (a, b) of the token from `steps` (float32
     [3, n, heads], of which the first two are read) or, with `decays` (float32 [heads]) instead, (decays[h], 1).
@@ -1168,7 +1171,7 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     begins with S as [heads, head_dim, value_dim]; y float32 [n, heads * value_dim].  All of the recurrence is float32.
     `row_decays` (then neither `steps` nor `decays`): qk has a third plane, float32 [3, n, heads * head_dim], of decays a
     row of S and token: S[i, :] = qk[2][i] S[i, :] + k[i] v^T.  `chunks`: float32 scratch of `memory_chunk_size` elements
-    (made here if not given)."""
+    (made here if not given); `shortest`: as in `ssm_scan`."""
     if row_decays:
         _need(steps is None and decays is None, "row_decays: neither steps nor decays")
     else:
@@ -1195,7 +1198,7 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     if n:
         call("memory_scan", qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim, nq,
              int(n_offset), **({"row_decays": True} if row_decays else {}),
-             **_scan_scratch(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, v.dtype), v.device))
+             **_scan_extra(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, v.dtype), shortest, v.device))
 
 
 def head_norm_gate(y: torch.Tensor, gate: Optional[torch.Tensor], weight: Optional[torch.Tensor], out: torch.Tensor, *, heads: int,
@@ -1649,13 +1652,13 @@ def _register_own() -> None:
     register_op("ssm_scan", entry_point="wllm_ssm_scan",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
-                          c_int, c_void_p],
+                          c_int, c_int, c_void_p],
                 launch=lambda fn, stream, xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y,
-                heads, groups, state_size, head_dim, steps, chunks=None: fn(
+                heads, groups, state_size, head_dim, steps, chunks=None, shortest=0: fn(
                     p(xbc), p(dt), dt.stride(0), p(dt_bias), p(a_log), p(d_skip), p(state), state.stride(0), p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(steps), int(xbc.dtype == torch.bfloat16), xbc.shape[0],
                     seg_q_start.shape[0], heads, groups, state_size, head_dim,
-                    p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, stream))
+                    p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, shortest, stream))
     register_op("gated_group_norm", entry_point="wllm_gated_group_norm",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
                 launch=lambda fn, stream, y, z, weight, out, groups, eps: fn(
@@ -1685,12 +1688,12 @@ def _register_own() -> None:
     register_op("memory_scan", entry_point="wllm_memory_scan",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_longlong, c_longlong, c_void_p,
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
-                          c_int, c_void_p],
+                          c_int, c_int, c_void_p],
                 launch=lambda fn, stream, qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads,
-                head_dim, value_dim, nq=None, n_offset=0, row_decays=False, chunks=None: fn(
+                head_dim, value_dim, nq=None, n_offset=0, row_decays=False, chunks=None, shortest=0: fn(
                     p(qk), p(v), v.stride(0), p(steps), p(decays), p(state), state.stride(0), n_offset, p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(nq), bf(v), v.shape[0], seg_q_start.shape[0], heads, head_dim,
-                    value_dim, int(row_decays), p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, stream))
+                    value_dim, int(row_decays), p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, shortest, stream))
     register_op("head_norm_gate", entry_point="wllm_head_norm_gate",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_float, c_int,
                           c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],

@@ -101,7 +101,7 @@ class StateSpaceMixer:
                      ctx.seg_q_start, ctx.seg_q_len, ctx.state_slots, y, heads=s.num_heads, groups=s.groups,
                      state_size=s.state_size, head_dim=s.head_dim,
                      steps=ctx.buffer("ssm_steps", (2, n, s.num_heads), torch.float32),
-                     chunks=ctx.buffer("scan_chunks", (size,), torch.float32) if size else None)
+                     chunks=ctx.buffer("scan_chunks", (size,), torch.float32) if size else None, shortest=ctx.min_q_len)
         out = ctx.buffer("ssm_out", (n, self.inner), h.dtype)
         ops.gated_group_norm(y, row[:, :self.inner], self.norm_w, out, s.norm_groups, s.norm_eps)
         if product_input is not None:
