@@ -173,3 +173,28 @@ def test_one_segment_of_fewer_tokens_than_rows(kind, length):
         assert float((state - left).abs().max()) <= 2e-6 * float(left.abs().max())
     else:
         assert torch.equal(state, problem.state0)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_segments_in_any_order_of_their_rows(kind):
+    """The segments of a step need not come in the order of their rows: each has the bits that it has in that order, with
+    short ones and rows of no segment between them."""
+    places = [(0, 100), (100, 64), (167, 3), (170, 70), (245, 97), (342, 1)]           # (first row, tokens), rows left out
+    problem = _problem(kind, torch.bfloat16, 350)
+    width = problem.inner if kind == "space" else problem.heads * (problem.dv + 1)
+    problem.state0 = problem.state0.repeat(2, 1)
+
+    def run(order):
+        state, y = problem.state0.clone(), torch.full((350, width), 7.0, device=DEV)
+        problem.launch(slice(0, 350), [places[i][0] for i in order], [places[i][1] for i in order], list(order), state, y)
+        return y, state
+    want, left = run(range(6))
+    for order in ((5, 4, 3, 2, 1, 0), (1, 0, 4, 5, 3, 2), (3, 1, 2, 0, 5, 4)):
+        y, state = run(order)
+        assert torch.equal(y, want) and torch.equal(state, left), f"{order}"
+    assert bool((want[164:167] == 7.0).all()) and bool((want[240:245] == 7.0).all())
+    for i, (at, n) in enumerate(places):
+        alone = problem.state0.clone()
+        y = torch.full((n, width), 7.0, device=DEV)
+        problem.launch(slice(at, at + n), [0], [n], [i], alone, y)
+        assert torch.equal(y, want[at:at + n]) and torch.equal(alone[i], left[i]), f"segment {i}"

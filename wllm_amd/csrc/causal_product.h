@@ -2,6 +2,15 @@
 #pragma once
 #include "common.h"
 
+constexpr int kChunk = 16;           // tokens of a chunk
+
+// The place of a segment's first chunk in the scratch, for segments of `from` tokens (16 at least) and more: chunk c lies c
+// places further.  No two chunks share a place, whatever order the segments come in: a segment of n >= from tokens has at most
+// n / 16 + 1 chunks, and the first place of what begins n tokens later is at least n / 16 + 1 further.  The last place of a step
+// of t tokens is t / 16 + t / from - 1.
+__host__ __device__ __forceinline__ int first_place(int q_start, int from) { return q_start / kChunk + q_start / from; }
+__host__ __device__ __forceinline__ int chunk_places(int tokens, int from) { return tokens / kChunk + tokens / from; }
+
 typedef float causal_float4 __attribute__((ext_vector_type(4)));
 
 // part + N x on v_mfma_f32_16x16x4_f32 for the four tokens s = token_of(0 .. 3): lane (i, g) holds n = N[i][token_of(g)] and

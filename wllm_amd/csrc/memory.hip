@@ -336,14 +336,13 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
 // `memory_chunk_scan_kernel` walks a segment's chunks with v_mfma_f32_16x16x4_f32 (float32 in and out).  A chunk begins
 // every 16 tokens of a segment; the last one is its last 16 tokens, those of the chunk before it as tokens that change
 // nothing (q = k = 0, f = 1).  Values in bfloat16 only: in the 32-bit path a token's bits do not depend on how its prompt
-// was cut.  Chunk c of segment s lies at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// was cut.
 // Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 34 and
 // 156 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 19 and 127, with
 // exponential gates and the normaliser 297 against 19 and 125; 64 tokens 12.6 against 7 and 9, from where on a segment
 // gains.  Off the result in 64 bits (y; the memory left behind), here and token by token: decays a head 2.0e-7; 2.0e-7 and
 // 3.1e-7; 3.2e-7, decays a row 8.1e-8; 4.5e-8 and 9.1e-8; 4.5e-8, exponential gates 8.7e-8; 5.3e-8 and 9.9e-8; 5.7e-8.  With N
 // in 32 bits (27 us) and without the rest of Kh (138 us) decays a row are off by 9.4e-8; 4.8e-8, so both stay. ----
-constexpr int kChunk = 16;
 typedef float memory_float4 __attribute__((ext_vector_type(4)));
 
 static __host__ __device__ __forceinline__ size_t chunk_floats(int c) { return static_cast<size_t>(2 * kChunk + 5) * c + kChunk * kChunk; }
@@ -370,13 +369,13 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
     if (tid == 0) found = -1;
     __syncthreads();
     for (int s = tid; s < segments; s += 256) {
-        const int first = seg_q_start[s] / kChunk + s, len = seg_q_len[s];
+        const int first = first_place(seg_q_start[s], from), len = seg_q_len[s];
         if (len >= from && place >= first && place < first + (len + kChunk - 1) / kChunk) found = s;
     }
     __syncthreads();
     const int seg = found;
     if (seg < 0) return;
-    const int q_start = seg_q_start[seg], local = (place - q_start / kChunk - seg) * kChunk;
+    const int q_start = seg_q_start[seg], local = (place - first_place(q_start, from)) * kChunk;
     // (a segment's last chunk is its last 16 tokens, of which those that the chunk before it holds are left out)
     const int begin = min(local, seg_q_len[seg] - kChunk), out_of = local - begin, token = q_start + begin;
     float* out = chunks + (static_cast<size_t>(place) * heads + h) * chunk_floats(C);
@@ -498,7 +497,7 @@ memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride,
         float rest[TILES], n;
         bf16 v[4];
     };
-    const float* first = chunks + (static_cast<size_t>(q_start / kChunk + seg) * heads + h) * chunk_floats(C);
+    const float* first = chunks + (static_cast<size_t>(first_place(q_start, from)) * heads + h) * chunk_floats(C);
     const bf16* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
     // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
     const unsigned q_at = i * C + ch0 + 4 * g, k_at = kChunk * C + (ch0 + i) * kChunk + 4 * g, f_at = 2 * kChunk * C + ch0 + 4 * g;
@@ -599,7 +598,7 @@ memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride,
 // normaliser's sums and the normaliser lies at `n_offset` of a request's row) or, if null, `decays` (float32 [heads]; b = 1),
 // or, with `row_decays`, neither: then qk has a third plane [tokens, heads * d] of decays a row and token (b = 1).
 // `from` tokens (16 at least; 0: no segment, as in float32) is what a segment needs to be walked in chunks, out of the
-// scratch `chunks`: tokens / 16 + segments + 1 places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
+// scratch `chunks`: `chunk_places` places of heads * chunk_floats(the channels padded to a multiple of 64) floats.
 // `shortest`: the caller's word that no segment has fewer tokens (0: it has none); with it at `from` or above nothing is
 // launched for shorter ones.
 WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride, const float* steps, const float* decays,
@@ -620,7 +619,7 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
         if (!is_bf16 || !chunks || from < kChunk || d > 256 || heads > 65535 || v_stride > 0x0fffffffLL ||
             reinterpret_cast<uintptr_t>(chunks) % 16)
             return -1;
-        const dim3 chunk_grid(tokens / kChunk + segments + 1, heads);
+        const dim3 chunk_grid(chunk_places(tokens, from), heads);
 #define LAUNCH(R)                                                                                                      \
     do {                                                                                                               \
         memory_chunk_kernel<R><<<chunk_grid, 256, 0, stream>>>(qk, steps, decays, seg_q_start, seg_q_len, segments, chunks, \

@@ -531,12 +531,10 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
 // tokens before, so `ssm_chunk_kernel` makes all else for every chunk at once: per (chunk, group) the rows C_t and the
 // transposed B, per (chunk, head) N, pre, suf d and pre_16; and `ssm_chunk_scan_kernel` walks a segment's chunks with
 // v_mfma_f32_16x16x4_f32 (float32 in and out), 17 of them a wavefront and chunk.  A chunk begins every 16 tokens of a
-// segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).  Chunk c of segment s lies
-// at place q_start / 16 + s + c of the scratch (no two chunks share one).
+// segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).
 // The walk token by token is bound by its chain (0.27 us a token).  64 heads of 64 with 128 rows of state: 1,500 tokens
 // 410 us token by token, 13 and 90 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
 // 64 tokens 21 us against 7 and 9, which is where the line between the two ways lies. ----
-constexpr int kChunk = 16;
 constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, suf d, pre_16 (and padding)
 
 // The operands of a chunk and a group: 28 us at 8 heads a group with a thread an entry of N that multiplied its decays one
@@ -559,13 +557,13 @@ ssm_chunk_kernel(const bf16* __restrict__ xbc, const bf16* __restrict__ dt_in, l
     if (tid == 0) found = -1;
     __syncthreads();
     for (int s = tid; s < segments; s += 256) {
-        const int first = seg_q_start[s] / kChunk + s, len = seg_q_len[s];
+        const int first = first_place(seg_q_start[s], from), len = seg_q_len[s];
         if (len >= from && place >= first && place < first + (len + kChunk - 1) / kChunk) found = s;
     }
     __syncthreads();
     const int seg = found;
     if (seg < 0) return;
-    const int q_start = seg_q_start[seg], local = (place - q_start / kChunk - seg) * kChunk;
+    const int q_start = seg_q_start[seg], local = (place - first_place(q_start, from)) * kChunk;
     const int count = min(kChunk, seg_q_len[seg] - local), token = q_start + local;
     const int inner = heads * p_dim, channels = inner + 2 * groups * n_state;
     const int b_col = inner + g * n_state, c_col = b_col + groups * n_state;
@@ -693,7 +691,7 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
         float n, all;
         bf16 x[4];
     };
-    const size_t first = static_cast<size_t>(q_start / kChunk + seg);
+    const size_t first = static_cast<size_t>(first_place(q_start, from));
     const float* head_first = of_head + (first * heads + h) * kChunkHeadFloats;
     const bf16* group_first = of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C;
     const bf16* x_first = xbc + static_cast<size_t>(q_start) * channels + h * p_dim;
@@ -796,8 +794,8 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
 }
 
 // `steps`: scratch of 2 * tokens * heads floats (the step sizes, then the decays).  `from` tokens (16 at least; 0: no
-// segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`: a place for every
-// chunk of every segment (tokens / 16 + segments + 1), first [place][head] of kChunkHeadFloats floats, then [place][group] of
+// segment, as in float32) is what a segment needs to be walked in chunks, out of the scratch `chunks`: `chunk_places`
+// places, first [place][head] of kChunkHeadFloats floats, then [place][group] of
 // 32 x (the rows of state padded to a multiple of 64) elements.  `shortest`: the caller's word that no segment has fewer
 // tokens (0: it has none); with it at `from` or above nothing is launched for shorter ones.
 WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stride, const float* dt_bias, const float* a_log,
@@ -814,7 +812,7 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
     const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
     if (in_chunks) {
         if (!is_bf16 || !chunks || from < kChunk || n_state > 256 || groups > 65535 || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
-        const int places = tokens / kChunk + segments + 1;
+        const int places = chunk_places(tokens, from);
         const dim3 chunk_grid(places, groups);
         bf16* of_group = reinterpret_cast<bf16*>(chunks + static_cast<size_t>(places) * heads * kChunkHeadFloats);
 #define LAUNCH(TILES)                                                                                                  \

@@ -997,7 +997,9 @@ SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
 
 def _scan_places(tokens: int, segments: int, dtype: torch.dtype) -> int:
     """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
-    return tokens // SCAN_CHUNK + segments + 1 if dtype == torch.bfloat16 and tokens - (segments - 1) >= SCAN_CHUNK_FROM else 0
+    if dtype != torch.bfloat16 or tokens - (segments - 1) < SCAN_CHUNK_FROM:
+        return 0
+    return tokens // SCAN_CHUNK + tokens // SCAN_CHUNK_FROM
 
 
 def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_size: int, dtype: torch.dtype) -> int:
