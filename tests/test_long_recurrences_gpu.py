@@ -198,3 +198,13 @@ def test_segments_in_any_order_of_their_rows(kind):
         y = torch.full((n, width), 7.0, device=DEV)
         problem.launch(slice(at, at + n), [0], [n], [i], alone, y)
         assert torch.equal(y, want[at:at + n]) and torch.equal(alone[i], left[i]), f"segment {i}"
+
+
+@pytest.mark.parametrize("kind", ["space", "head"])
+def test_more_heads_than_a_grid_has_rows_are_walked_token_by_token(kind):
+    """Beyond 65,535 heads (groups) a long segment is not walked in chunks; it has the bits that its portions have."""
+    heads = 65537
+    sizes = dict(heads=heads, groups=heads, n_state=1, p=1) if kind == "space" else dict(heads=heads, d=1, dv=1)
+    problem = _problem(kind, torch.bfloat16, 70, **sizes)
+    (y, state), (want, left) = problem.run([70]), problem.run(_portions(70))
+    assert torch.equal(y, want) and torch.equal(state, left)

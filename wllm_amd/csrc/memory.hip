@@ -614,11 +614,10 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
     const int columns = p_dim + (steps ? 1 : 0);
     const dim3 grid(heads, segments, (columns + kMemCols - 1) / kMemCols);
     // (a segment of `from` tokens leaves room for the others' single tokens)
-    const bool in_chunks = from > 0 && tokens - (segments - 1) >= from;
+    // (what the chunks' kernels do not take goes token by token)
+    const bool in_chunks = from > 0 && tokens - (segments - 1) >= from && d <= 256 && heads <= 65535 && v_stride <= 0x0fffffffLL;
     if (in_chunks) {
-        if (!is_bf16 || !chunks || from < kChunk || d > 256 || heads > 65535 || v_stride > 0x0fffffffLL ||
-            reinterpret_cast<uintptr_t>(chunks) % 16)
-            return -1;
+        if (!is_bf16 || !chunks || from < kChunk || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
         const dim3 chunk_grid(chunk_places(tokens, from), heads);
 #define LAUNCH(R)                                                                                                      \
     do {                                                                                                               \
