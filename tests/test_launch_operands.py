@@ -1,4 +1,5 @@
 """What a launch is handed, without a GPU: every address it gets belongs to a tensor that is still held when it is made."""
+import ctypes
 import weakref
 
 import pytest
@@ -69,3 +70,18 @@ def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
         assert len(seen) == 1
     assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, torch.bfloat16)
     assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, torch.float32)
+
+
+@pytest.mark.parametrize("handle", [0, 0x7F0012345678])
+def test_a_registered_launch_is_handed_the_stream_as_a_pointer(handle, monkeypatch):
+    """The launch that a part registers gets the step's stream as a ctypes pointer, whatever the framework's own get."""
+    from wllm_amd.kernels import hip_backend
+    seen = []
+    monkeypatch.setattr(ops, "_REGISTERED", dict(ops._REGISTERED))
+    backend = hip_backend.HipBackend.__new__(hip_backend.HipBackend)
+    backend._registered, backend.lib = {}, type("Library", (), {"an_entry": staticmethod(lambda: 0)})()
+    monkeypatch.setattr(backend, "_stream", lambda: handle, raising=False)
+    ops.register_op("a_parts_own", entry_point="an_entry", argtypes=[], launch=lambda fn, stream: seen.append(stream) or 0)
+    with ops.use_backend(backend):
+        ops.call("a_parts_own")
+    assert isinstance(seen[0], ctypes.c_void_p) and seen[0].value == (handle or None)

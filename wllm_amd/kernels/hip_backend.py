@@ -126,7 +126,8 @@ class HipBackend:
             entry.restype = c_int
             fn = self._registered[op.name] = (op, entry)
         self._on_gpu(*[a for a in list(args) + list(kwargs.values()) if isinstance(a, torch.Tensor)])
-        self._check(op.launch(fn[1], self._stream(), *args, **kwargs), op.name)
+        stream = self._stream() if op.own else c_void_p(self._stream())
+        self._check(op.launch(fn[1], stream, *args, **kwargs), op.name)
 
     def rms_norm(self, x, weight, eps, offset, out, delta, rows, delta_bias=None):
         self._on_gpu(x, weight, out, delta, rows, delta_bias)

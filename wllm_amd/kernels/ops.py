@@ -80,6 +80,7 @@ class RegisteredOp:
     def __init__(self, name, entry_point, argtypes, launch, check, emulate, library):
         self.name, self.entry_point, self.argtypes = name, entry_point, list(argtypes)
         self.launch, self.check, self.emulate, self.library = launch, check, emulate, library
+        self.own = False            # one of the framework's own (`_register_own`), whose launch takes the stream as an integer
 
 
 _REGISTERED: dict = {}
@@ -96,7 +97,8 @@ def register_op(name: str, *, entry_point: str, argtypes, launch, check=None, em
         folder of kernels), or None for the framework's own library.
     check(*args, **kwargs): raises `KernelShapeError` unless shapes, dtypes and layouts are what the kernel
         and its grid assume; it runs on the host before every launch.
-    launch(fn, stream, *args, **kwargs) -> int: calls `fn` with raw pointers (`ops.pointer(tensor)`) and the stream.
+    launch(fn, stream, *args, **kwargs) -> int: calls `fn` with raw pointers (`ops.pointer(tensor)`) and the stream (a
+        `c_void_p`).
     emulate(*args, **kwargs): the same contract in plain torch, for the tests that run the engine's
         bookkeeping without a GPU; never used by the engine.
 
@@ -1760,4 +1762,7 @@ def _register_own() -> None:
                     p(act), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(None), p(out),
                     p(weights if weighted else None), -1, act.shape[0], w.shape[1], act.shape[1], weights.shape[1], weights.shape[0], stream))
 
+
 _register_own()
+for _op in _REGISTERED.values():
+    _op.own = True
