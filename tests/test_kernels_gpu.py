@@ -468,6 +468,22 @@ def test_float32_product_of_many_rows_has_the_same_bits_with_its_k_axis_cut(m, n
     close(out[:m], x.double() @ w.double().T, torch.float32, "product")
 
 
+def test_float32_product_of_many_rows_without_room_for_its_partial_sums(monkeypatch):
+    """Where the sums of the cut K axis find no memory the product runs uncut: the same bits."""
+    torch.manual_seed(20)
+    x, w = torch.randn(100, 4096, device=DEV), torch.randn(300, 4096, device=DEV) / 64.0
+    want, out, empty, refused = torch.empty(100, 300, device=DEV), torch.empty(100, 300, device=DEV), torch.empty, []
+    ops.linear(x, w, want)
+
+    def full(*args, **kwargs):
+        refused.append(args)
+        raise torch.OutOfMemoryError("no room")
+    monkeypatch.setattr(torch, "empty", full)
+    ops.linear(x, w, out)
+    monkeypatch.setattr(torch, "empty", empty)
+    assert len(refused) == 1 and torch.equal(out, want)
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 2048, 16384), (5, 2560, 2048), (16, 1000, 8192), (1, 777, 516), (3, 40000, 2048),
                                    (40, 2048, 4096), (64, 1000, 2048)])
 def test_float32_linear_leaves_partial_sums_to_the_caller(m, n, k):

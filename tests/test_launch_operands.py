@@ -72,6 +72,20 @@ def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
     assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, torch.float32)
 
 
+@pytest.mark.parametrize("kind", ["space", "memory"])
+def test_a_scan_without_room_for_its_scratch_is_walked_token_by_token(kind, monkeypatch):
+    seen, empty = [], torch.empty
+
+    def full(size, *args, **kwargs):
+        if isinstance(size, int):                  # (the chunks' scratch; the steps' has three axes)
+            raise torch.OutOfMemoryError("no room")
+        return empty(size, *args, **kwargs)
+    monkeypatch.setattr(torch, "empty", full)
+    with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-4:-2]) or 0)):
+        _scan(kind, 80)
+    assert seen == [(None, 0)]
+
+
 @pytest.mark.parametrize("handle", [0, 0x7F0012345678])
 def test_a_registered_launch_is_handed_the_stream_as_a_pointer(handle, monkeypatch):
     """The launch that a part registers gets the step's stream as a ctypes pointer, whatever the framework's own get."""

@@ -481,9 +481,12 @@ class HipBackend:
                 return
             self._generic(x, weight, out, segments, tiles)
             return
-        # float32, more rows: the kernel says whether it cuts the K axis over workgroups
-        segments = self.lib.wllm_gemm_f32_segments(m, weight.shape[0], k) if x.dtype == torch.float32 else 1
-        partial = torch.empty(segments * m * weight.shape[0], dtype=torch.float32, device=x.device) if segments > 1 else None
+        # float32, more rows: the kernel says whether it cuts the K axis over workgroups; without room for the segments' sums
+        # (256 MiB at most) it runs uncut, with the same bits
+        n, partial = weight.shape[0], None
+        segments = self.lib.wllm_gemm_f32_segments(m, n, k) if x.dtype == out.dtype == torch.float32 else 1
+        if segments > 1:
+            partial = ops.scratch_or_none(lambda: torch.empty(segments * m * n, dtype=torch.float32, device=x.device))
         self._generic(x, weight, out, 1, partial=partial)
 
     def _generic(self, x, weight, out, segments: int, tiles=None, partial=None) -> None:

@@ -1017,13 +1017,24 @@ def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, dty
     return _scan_places(tokens, segments, dtype) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
 
 
+def scratch_or_none(make):
+    """The scratch that `make()` gives, or None where the device has no room for it: for work that can do without."""
+    try:
+        return make()
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _scan_extra(chunks: Optional[torch.Tensor], size: int, shortest: int, device) -> dict:
     """What the walk in chunks adds to a launch's operands: the scratch, the caller's or made here (an operand, so that
-    it is held until the launch has been made), and whether shorter segments may be beside the long ones."""
+    it is held until the launch has been made), and whether shorter segments may be beside the long ones.  Nothing where
+    there is no room for the scratch: the step is then walked token by token."""
     if size == 0:
         return {}
     if chunks is None:
-        chunks = torch.empty(size, dtype=torch.float32, device=device)
+        chunks = scratch_or_none(lambda: torch.empty(size, dtype=torch.float32, device=device))
+        if chunks is None:
+            return {}
     _dense(chunks, "chunks", torch.float32)
     _need(chunks.numel() >= size, lambda: f"chunks: {chunks.numel()} floats of scratch, needed {size}")
     return {"chunks": chunks, "shortest": int(shortest)}
