@@ -133,6 +133,18 @@ def test_piece_length():
     assert ap.prefill_piece_length(span, 1, 4, 16) == 16            # the longest piece allowed: 4 a block, 8 rounds
 
 
+def test_pieces_that_give_every_compute_unit_one_and_blocks_that_stay_whole():
+    # 256 rows over 4,096 keys, 8 heads on one: 32 blocks of rows of 121 to 128 groups in 8 pieces each, 256 in all
+    _, _, _, prefill = covered([256], [4096], 8, 1, 0, 16)
+    assert prefill.shape[0] == 256
+    _, _, _, prefill = covered([240], [4096], 8, 1, 0, 16)             # a block or two less: the shortest pieces again
+    assert prefill.shape[0] > 300
+    _, reduces, _, _ = covered([384], [384], 8, 1, 0, 16)              # 12 groups and fewer
+    assert reduces.shape[0] == 0
+    _, reduces, _, _ = covered([385], [385], 8, 1, 0, 16)
+    assert reduces.shape[0] > 0
+
+
 def test_a_whole_prompt_of_many_heads_is_not_split():
     _, reduces, slots, prefill = covered([300], [300], 1, 1, 0, 16)
     assert slots == 0 and reduces.shape[0] == 0

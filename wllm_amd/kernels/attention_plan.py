@@ -37,11 +37,16 @@ ROWS_PER_TILE = 16
 ITEM_INTS = 8
 PREFILL_TABLE_PAGES = 1024      # pages one prefill item may span (the kernel's shared block table)
 # Groups of 32 keys: shorter pieces cost more in partial results than they gain, longer ones leave compute units idle where a
-# step has few blocks of rows.  Attention and its reduce kernel with pieces of at least 8, 10 and 16 groups, 8 heads of 256
-# on one key head: 104 rows over 1,000 keys 19.1 / 21.1 / 27.4 us, 448 over 896 24.2 / 24.6 / 28.0, 700 over 700 22.4 / 23.3 /
-# 26.8, 448 over 1,000 beside 20 decoded tokens 35.4 / 36.1 / 39.9, 512 over 7,000 62.0 / 58.5 / 56.7, 300 over 300 17.3 / 17.0 /
-# 16.9 (8 cuts it in two); from 1,500 keys of their own on a prompt's blocks fill the device either way.
+# step has few blocks of rows.  Attention and its reduce kernel with pieces of at least 8, 10, 13 and 16 groups, 8 heads of 256
+# on one key head: 104 rows over 1,000 keys 19.7 / 21.8 / 22.5 / 27.9 us, 448 over 896 24.9 / 25.6 / 27.9 / 29.1, 700 over 700
+# 23.4 / 24.3 / 25.8 / 28.1, 64 over 8,000 26.8 / 29.3 / 29.2 / 30.8, 448 over 3,000 beside 20 decoded tokens 48.3 / 48.3 / 47.3 /
+# 48.6; 16 heads on as many, 64 over 8,000 39.7 / 37.6 / 37.1 / 35.9.  Prompts of 2,048 and more, and portions of 512 over
+# 4,000, fill the device with longer pieces than any of these.
 PREFILL_MIN_PIECE = 10
+# Where that many groups a piece make exactly one piece for every compute unit, shorter ones make two on some of them and
+# lose: 256 rows over 4,096 keys 32.8 us in pieces of 16 groups and 33.5 in shorter ones, 128 over 8,000 33.8 and 35.4 (8 heads of 128 on
+# two 24.5 and 27.1).
+PREFILL_EVEN_PIECE = 16
 WORKGROUP_SLOTS = 512           # prefill workgroups a device runs at once unless the caller knows better (two a compute unit)
 PREFILL_ROWS = 64               # rows of a prefill item unless the kernel for the sizes at hand says otherwise
 
@@ -187,7 +192,9 @@ def prefill_piece_length(span: np.ndarray, num_kv_heads: int, workgroup_slots: i
     device at most once, twice, ... (the fewest rounds that the longest allowed piece permits): every
     further item costs a partial result that is written and read again, and items that start together
     and are about equally long end together.  Never shorter than `PREFILL_MIN_PIECE` groups, below which
-    a piece's partial result costs more than its share of the keys."""
+    a piece's partial result costs more than its share of the keys, nor than `PREFILL_EVEN_PIECE` where that gives
+    every compute unit (a half of the workgroup slots) one piece; blocks of hardly more than the least length stay
+    whole (333 rows over 333 keys 20.1 us cut, 19.2 whole)."""
     def count(length):
         return int((-(-span // length)).sum()) * num_kv_heads
     rounds = max(1, -(-count(longest) // workgroup_slots))
@@ -198,6 +205,9 @@ def prefill_piece_length(span: np.ndarray, num_kv_heads: int, workgroup_slots: i
             hi = mid
         else:
             lo = mid + 1
+    if lo < PREFILL_EVEN_PIECE and (count(PREFILL_EVEN_PIECE) == workgroup_slots // 2
+                                    or int(span.max()) <= PREFILL_MIN_PIECE + 2):
+        return min(longest, PREFILL_EVEN_PIECE)
     return min(longest, max(lo, PREFILL_MIN_PIECE))
 
 
