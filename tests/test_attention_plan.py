@@ -145,6 +145,17 @@ def test_pieces_that_give_every_compute_unit_one_and_blocks_that_stay_whole():
     assert reduces.shape[0] > 0
 
 
+@pytest.mark.parametrize("seed", range(8))
+def test_the_count_of_a_portions_tiles(seed):
+    rng = np.random.default_rng(500 + seed)
+    q_len = rng.integers(1, 200, 4)
+    ctx_len = q_len + rng.integers(0, 700, 4)
+    group, nkv, window = int(rng.choice([1, 3, 8])), int(rng.choice([1, 2])), int(rng.choice([0, 70, -90]))
+    portion = (q_len * group > ap.ROWS_PER_TILE) & (q_len != 1)
+    items = ap.build_tile_items(q_len[portion], ctx_len[portion], group, nkv, window)[0]
+    assert ap.count_tile_items(q_len, ctx_len, group, nkv, window) == items.shape[0]
+
+
 def test_a_whole_prompt_of_many_heads_is_not_split():
     _, reduces, slots, prefill = covered([300], [300], 1, 1, 0, 16)
     assert slots == 0 and reduces.shape[0] == 0

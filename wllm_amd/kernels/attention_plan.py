@@ -136,6 +136,29 @@ def lowest_keys(pos: np.ndarray, window: int) -> np.ndarray:
     return np.zeros_like(pos)
 
 
+def _tile_chunks(q_len: np.ndarray, ctx_len: np.ndarray, group: int, window: int):
+    """Segments as tiles of 16 rows: per tile its segment, its number in it, the keys `lo` <= key < `hi` its rows can need,
+    the first of their chunks of `KEY_CHUNK` keys and how many there are."""
+    rows = q_len * group
+    nt = -(-rows // ROWS_PER_TILE)
+    seg_of = np.repeat(np.arange(q_len.size), nt)
+    tile = np.arange(int(nt.sum())) - np.repeat(np.cumsum(nt) - nt, nt)
+    row0 = tile * ROWS_PER_TILE
+    first_pos = (ctx_len - q_len)[seg_of]
+    last_row = np.minimum(rows[seg_of] - 1, row0 + ROWS_PER_TILE - 1)
+    lo = lowest_keys(first_pos + row0 // group, window)
+    hi = first_pos + last_row // group + 1
+    c0 = lo // KEY_CHUNK
+    return seg_of, tile, lo, hi, c0, (hi - 1) // KEY_CHUNK - c0 + 1
+
+
+def count_tile_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_heads: int, window: int) -> int:
+    """The work items that the step's prompt portions (what is no short segment) make as tiles of 16 rows."""
+    q_len, ctx_len = np.asarray(q_len, dtype=np.int64), np.asarray(ctx_len, dtype=np.int64)
+    portion = (q_len * group > ROWS_PER_TILE) & (q_len != 1)
+    return int(_tile_chunks(q_len[portion], ctx_len[portion], group, window)[-1].sum()) * num_kv_heads
+
+
 def build_tile_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_heads: int, window: int):
     """Every segment, whatever its length, as tiles of 16 rows with their keys in chunks of `KEY_CHUNK`
     counted from key 0 (the float32 kernel takes nothing else): a tile's chunks are those its rows can
@@ -148,15 +171,8 @@ def build_tile_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
     nt = -(-rows // ROWS_PER_TILE)
     if nt.size and int(nt.max()) >= MAX_TILES:
         raise ValueError(f"a segment of {int(rows.max())} rows a key/value head: a work item numbers at most {MAX_TILES} tiles")
-    seg_of = np.repeat(np.arange(q_len.size), nt)
-    tile = np.arange(int(nt.sum())) - np.repeat(np.cumsum(nt) - nt, nt)
+    seg_of, tile, lo, hi, c0, ns = _tile_chunks(q_len, ctx_len, group, window)
     row0 = tile * ROWS_PER_TILE
-    first_pos = (ctx_len - q_len)[seg_of]
-    last_row = np.minimum(rows[seg_of] - 1, row0 + ROWS_PER_TILE - 1)
-    lo = lowest_keys(first_pos + row0 // group, window)
-    hi = first_pos + last_row // group + 1
-    c0 = lo // KEY_CHUNK
-    ns = (hi - 1) // KEY_CHUNK - c0 + 1
     n_items = int(ns.sum())
     tile_of = np.repeat(np.arange(tile.size), ns)
     j = np.arange(n_items) - np.repeat(np.cumsum(ns) - ns, ns)

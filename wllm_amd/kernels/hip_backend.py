@@ -10,7 +10,7 @@ from ctypes import c_float, c_int, c_longlong, c_void_p
 import numpy as np
 import torch
 
-from wllm_amd.kernels.attention_plan import AttentionPlan, build_work_items
+from wllm_amd.kernels.attention_plan import AttentionPlan, build_work_items, count_tile_items
 from wllm_amd.kernels import ops
 from wllm_amd.kernels.ops import gate_args
 from wllm_amd.kernels.library import load
@@ -187,6 +187,13 @@ class HipBackend:
         return (dtype in (torch.bfloat16, torch.float32) and head_dim % 32 == 0 and 32 <= head_dim <= 256
                 and page_size % 4 == 0)
 
+    # Up to how many (items of 16 rows by 128 keys) x (elements of a head) float32 prompt portions are tiles: these take a time in
+    # proportion, the blocks of 64 rows hardly less for few of them than for the 256 that give every compute unit one.
+    # Tiles against blocks, heads of 256: 309 items 27 and 67 us, 1,280 61 and 75, 1,631 73 and 77, 2,080 89 and 79, 2,304 92 and
+    # 91 (16 heads on as many) or 88 (8 on one), 2,560 104 and 112 or 105 and 104, 3,616 137 and 118; heads of 128: 2,304 items 50 and
+    # 63, 2,616 56 and 69, 3,616 70 and 78, 4,032 80 and 81, 4,776 88 and 81.
+    F32_TILE_WORK = 1 << 19
+
     def plan_paged_attention(self, host_q_len, host_ctx_len, num_heads, num_kv_heads, head_dim, page_size, window,
                              dtype, device):
         # `window`: w > 0 a sliding window, 0 none, -c < 0 chunks of c positions (the kernels' own convention)
@@ -195,10 +202,9 @@ class HipBackend:
         group, slots_of_device = num_heads // num_kv_heads, self._workgroup_slots(device)
         items, reduces, slots, prefill, prefill_rows = build_work_items(
             host_q_len, host_ctx_len, group, num_kv_heads, window, page_size, workgroup_slots=slots_of_device)
-        if dtype == torch.float32 and 0 < prefill.shape[0] < slots_of_device // 2:
-            # float32 and few blocks of 64 rows (a prompt of some hundred tokens): tiles of 16 rows fill the device
-            # better than the blocks would (512 tokens of 8 heads: 43 against 96 us).  With so few blocks the tiles
-            # are few too (at most four a block) and so are their chunks (the blocks' keys were not worth cutting).
+        if dtype == torch.float32 and prefill.shape[0] and \
+                count_tile_items(host_q_len, host_ctx_len, group, num_kv_heads, window) * head_dim < self.F32_TILE_WORK:
+            # float32 and little work: tiles of 16 rows fill the device better than the blocks of 64 rows would
             items, reduces, slots, prefill, prefill_rows = build_work_items(
                 host_q_len, host_ctx_len, group, num_kv_heads, window, page_size, workgroup_slots=slots_of_device,
                 tiles_only=True)
