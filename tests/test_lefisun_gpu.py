@@ -331,6 +331,40 @@ def test_the_router_and_the_experts(dtype, n, width, ff, count, top, groups, kee
             close(got[r], want[r], dtype, f"row {r}", scale=2.0)
 
 
+@pytest.mark.parametrize("n,count,top,width,ff", [
+    (130, 8, 2, 320, 192),              # less than a tile an expert: a column at a time, then at most three areas
+    (900, 3, 2, 1088, 640),             # some ten areas, which run at once
+    (1500, 5, 2, 1088, 1216),           # at most 21 and 14: eight at a time and some left over
+    (2600, 7, 2, 1344, 1088),           # at most 36 and 24
+    (1900, 30, 1, 2048, 512)])          # a column at a time, at most 22
+def test_every_tile_of_128_rows_is_made_however_many_there_are(n, count, top, width, ff):
+    """The products of the experts' large tiles, whose workgroups go over the tiles in areas: no tile is left out or
+    made of another's rows, whatever their number and wherever the areas reach beyond it."""
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, width, generator=g).bfloat16()
+    w_up = (torch.randn(count, 2 * ff, width, generator=g) * width ** -0.5).bfloat16()
+    w_down = (torch.randn(count, width, ff, generator=g) * ff ** -0.5).bfloat16()
+    ids = torch.stack([torch.randperm(count, generator=g)[:top] for _ in range(n)]).to(torch.int32)
+    wts = torch.rand(n, top, generator=g)
+    plan = torch.zeros(ops.moe_plan_size(n * top, count, 128), dtype=torch.int32, device=DEV)
+    ops.moe_plan(ids.to(DEV), plan, count, 128)
+    act = torch.full((n * top, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.moe_experts_up(x.to(DEV), w_up.to(DEV), plan, act, top, "silu", 128)
+    out = torch.full((top, n, width), float("nan"), dtype=torch.float32, device=DEV)
+    ops.moe_experts_down(act, w_down.to(DEV), plan, wts.to(DEV), out, 128)
+    rows, flat = x.float().repeat_interleave(top, dim=0), ids.view(-1).long()
+    want_act, want = torch.empty(n * top, ff), torch.empty(n * top, width)
+    for e in range(count):
+        of = flat == e
+        up = rows[of] @ w_up[e].float().T
+        want_act[of] = torch.nn.functional.silu(up[:, :ff]) * up[:, ff:]
+        want[of] = (act[of.to(DEV)].cpu().float() @ w_down[e].float().T) * wts.view(-1)[of, None]
+    close(act, want_act, torch.bfloat16, "first product", scale=2.0)
+    # float32 sums of bfloat16 products in two orders: some 2^-24 each of the sum of their sizes, about one
+    got = out.transpose(0, 1).reshape(n * top, width).cpu()
+    assert float((got - want).abs().max()) <= 2e-5, "second product"
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_row_of_the_experts_does_not_depend_on_the_batch(dtype):
     g = torch.Generator().manual_seed(4)

@@ -522,13 +522,39 @@ constexpr int kBigRows = 128;
 constexpr int kBigKeys = 64;
 constexpr int kBigRowBytes = kBigKeys * 2;
 constexpr int kBigStageBytes = 2 * kBigRows * kBigRowBytes;
-// The workgroups of kBlockM tiles of rows by kBlockN tiles of columns have indices that are equal modulo 8 and follow one
-// another, so they run together on one XCD and share their rows of x and of w in its L2: the sixty-four that an XCD
-// runs at once then read some 14 MB a pass over K where one column of tiles at a time made them read 39 (every tile's
-// rows of x, and nearly every expert's rows of w), which the fabric behind the L2s had to bring for all eight XCDs.
-// 9,003 rows over 16 experts of 4,096, width 2,048: the second product 276 to 252 us, the first 468 to 471 on a machine whose
-// other products ran 5% slower.
-constexpr int kBlockM = 4, kBlockN = 8;
+// An XCD's workgroups (indices equal modulo 8) take areas of kAreaRows tiles of rows by kAreaColumns tiles of columns one
+// after the other, so that they share their rows of x and of w in its L2: the sixty-four that an XCD runs at once
+// then read some 14 MB a pass over K where one column of tiles at a time made them read 39 (every tile's rows of x, and
+// nearly every expert's rows of w), which the fabric behind the L2s had to bring for all eight XCDs.  Eight areas go at a
+// time, one an XCD; those left over are shared out tile by tile, unless all areas run at once, two an XCD (700 tokens of the
+// sizes below: 14 areas, the second product 88 us, 97 shared out; but 3 areas 31 and 30).  A column of tiles at a time against that, us, 16 experts
+// of 4,096 behind a width of 2,048, three a token (first product; second): 1,000 tokens 208, 204; 93, 94; 2,048 342, 327; 185,
+// 173; 3,001 472, 454; 269, 246; 7,777 1,105, 1,079; 589, 519; four a token, 1,000 (where whole areas would give some XCDs a half
+// more: 166 in the second) 244, 240; 159, 154.
+constexpr int kAreaRows = 4, kAreaColumns = 8, kAreaTiles = kAreaRows * kAreaColumns, kAreasAtOnce = 16;
+
+// The tile of workgroup `index` among `rows` tiles of rows by any number of columns of which `across` areas (the last one
+// may reach beyond them) make a band; `across` 0: a column of tiles at a time, eight columns side by side.
+__host__ __device__ __forceinline__ void tile_of(int index, int rows, int across, int& row, int& column) {
+    const int xcd = index % 8, turn = index / 8;
+    if (across == 0) {
+        row = turn % rows;
+        column = turn / rows * 8 + xcd;
+        return;
+    }
+    const int areas = (rows + kAreaRows - 1) / kAreaRows * across;
+    const bool at_once = areas > 8 && areas <= kAreasAtOnce;
+    const int dealt = at_once ? kAreasAtOnce / 8 * kAreaTiles : areas / 8 * kAreaTiles;                // turns that deal whole areas
+    const int share = at_once ? 0 : areas % 8 * (kAreaTiles / 8), place = turn < dealt ? turn % kAreaTiles : xcd * share + turn - dealt;
+    if (turn >= dealt + share) {
+        row = rows;                                                                                      // no tile
+        column = 0;
+        return;
+    }
+    const int area = turn < dealt ? turn / kAreaTiles * 8 + xcd : areas / 8 * 8 + place / kAreaTiles;
+    row = area / across * kAreaRows + place % kAreaRows;
+    column = area % across * kAreaColumns + place % kAreaTiles / kAreaRows;
+}
 
 union MoeTFrag {
     uint4 u;
@@ -550,7 +576,7 @@ template <int GATED>
 __global__ void __launch_bounds__(256, 2)
 moe_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const int* __restrict__ plan, int max_tiles,
                 bf16* __restrict__ act, float* __restrict__ out32, const float* __restrict__ weights, int N, int K, int top,
-                int tokens) {
+                int tokens, int across) {
     // (`weights`: of the second product the factor of a row's result, 1 if null; of the first the factor of a row's
     // input, taken out of both sums, none if null)
     constexpr int kWaves = 4, kStages = 2;
@@ -561,14 +587,13 @@ moe_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const in
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = lane % 16, g = lane / 16;
     const int wm = wave / 2, wn = wave % 2;
-    // (see kBlockM, kBlockN)
     constexpr int kColumns = GATED ? kBigRows / 2 : kBigRows;
-    const int inside = blockIdx.x / 8 % (kBlockM * kBlockN);
-    const int block = blockIdx.x / 8 / (kBlockM * kBlockN) * 8 + blockIdx.x % 8;
-    const int n_blocks = ((N + kColumns - 1) / kColumns + kBlockN - 1) / kBlockN;
-    const int m_tile = block / n_blocks * kBlockM + inside % kBlockM;
-    const int n_base = (block % n_blocks * kBlockN + inside / kBlockM) * kColumns;
-    if (m_tile >= plan[0] || n_base >= N) return;
+    const int live = plan[0];
+    if (live <= 0) return;
+    int m_tile, n_tile;
+    tile_of(blockIdx.x, live, across, m_tile, n_tile);
+    const int n_base = n_tile * kColumns;
+    if (m_tile >= live || n_base >= N) return;
     const int e = plan[1 + m_tile];
     const int* rows = plan + 1 + max_tiles + m_tile * kBigRows;
     const int stages = K / kBigKeys;
@@ -682,15 +707,20 @@ WLLM_API int wllm_moe_tiles(const void* x, const void* w, const int* plan, int m
         return -1;
     const int columns = gated ? kBigRows / 2 : kBigRows;
     const int n_tiles = (N + columns - 1) / columns;
-    const long long areas = static_cast<long long>((n_tiles + kBlockN - 1) / kBlockN) * ((max_tiles + kBlockM - 1) / kBlockM);
-    const long long blocks = (areas + 7) / 8 * 8 * kBlockM * kBlockN;
+    // (the first product of steps with less than one full tile an expert, whose areas share nothing of w, takes a column at a
+    // time: 16 experts of 4,096, three a token, 256 tokens 148 us in areas, 146 so; 448 156 and 153)
+    const bool few = gated && static_cast<long long>(tokens) * top <= 64LL * max_tiles;
+    const int across = few ? 0 : (n_tiles + kAreaColumns - 1) / kAreaColumns;
+    const long long areas = static_cast<long long>(across) * ((max_tiles + kAreaRows - 1) / kAreaRows);
+    const long long blocks = few ? (static_cast<long long>(n_tiles) + 7) / 8 * 8 * max_tiles
+                                 : (areas > 8 && areas < kAreasAtOnce ? kAreasAtOnce : areas) * kAreaTiles;
     if (blocks > 0x7fffffffLL) return -1;
     const dim3 grid(static_cast<unsigned>(blocks));
     const bf16* xp = static_cast<const bf16*>(x);
     const bf16* wp = static_cast<const bf16*>(w);
 #define LAUNCH(GATED)                                                                                                 \
     moe_tile_kernel<GATED><<<grid, 256, 2 * kBigStageBytes, stream>>>(xp, wp, plan, max_tiles, static_cast<bf16*>(act), \
-                                                                      out32, weights, N, K, top, tokens)
+                                                                      out32, weights, N, K, top, tokens, across)
     if (!gated) { LAUNCH(0); }
     else { WLLM_BY_ACTIVATION(activation, LAUNCH(ACT + 1)) }
 #undef LAUNCH
