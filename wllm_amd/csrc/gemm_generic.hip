@@ -411,8 +411,8 @@ WLLM_API int wllm_tile_weight_f32(const float* w, float* tiles, int N, int K, hi
 }
 
 // Into how many partial sums [segments, M, N] a float32 product of these sizes is split (1: it is not).
-// `wllm_gemm_generic` needs `partial` to hold them (at most 64 rows; with more rows it runs unsplit without); with
-// `out` null it leaves them there for a consumer that adds them in ascending order.
+// `wllm_gemm_generic` needs `partial` to hold them (at most 64 rows; with more rows it runs unsplit without); of at most
+// 64 rows it leaves them there for a consumer that adds them in ascending order if `out` is null.
 WLLM_API int wllm_gemm_f32_segments(int M, int N, int K) {
     if (M < 1 || N < 1 || K < 4 || K % 4 != 0) return 1;
     if (M <= 64 ? !few_rows_split(N, K) : f32_cut(M, N, K, true).per_group == 0) return 1;
@@ -460,10 +460,10 @@ WLLM_API int wllm_gemm_generic(const void* x, const void* w, const void* tiles, 
 #undef FEW_ROWS
             return launch_status();
         }
+        if (!of) return -1;
         float* pf = static_cast<float*>(partial);
         const F32Cut cut = f32_cut(M, N, K, pf != nullptr);
         const int segments = (K + kF32Segment - 1) / kF32Segment;
-        if (!of && !cut.per_group) return -1;
         const dim3 grid((N + 32 * cut.wn - 1) / (32 * cut.wn), (M + 32 * cut.wm - 1) / (32 * cut.wm),
                         cut.per_group ? (segments + cut.per_group - 1) / cut.per_group : 1);
         if (grid.y > 65535) return -1;
@@ -478,7 +478,7 @@ WLLM_API int wllm_gemm_generic(const void* x, const void* w, const void* tiles, 
         else TILES(2, 2);
 #undef TILES
         if (const int err = launch_status()) return err;
-        return cut.per_group && of ? sum_segments(pf, of, static_cast<long long>(M) * N, segments, stream) : 0;
+        return cut.per_group ? sum_segments(pf, of, static_cast<long long>(M) * N, segments, stream) : 0;
     }
     const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
     if (grid.y > 65535) return -1;

@@ -316,29 +316,35 @@ gemm_skinny_joined_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w
     }
 }
 
-// out = x w^T of at most 64 rows, the K axis in `splits` (at most 16) pieces of whole steps of 32 keys, whole.  Returns 0,
+// out = x w^T of at most 64 rows, the K axis in `splits` (at most 16, of more than 32 rows 8) pieces of whole steps of 32 keys, whole.  Returns 0,
 // a HIP error code, or -1 for sizes this kernel does not take.
 WLLM_API int wllm_gemm_skinny_joined(const void* x, const void* w, int tiled, void* out, int out_bf16, int M, int N, int K,
                                      int splits, hipStream_t stream) {
     if (M < 1 || M > 64 || N < 1 || splits < 1 || splits > 16 || K % 32 != 0 || K % splits != 0 || (K / splits) % 32 != 0 || !out)
         return -1;
     const int mt = (M + 15) / 16, blocks = (N + 15) / 16;
+    if (mt > 2 && splits > 8) return -1;
     const size_t smem = static_cast<size_t>(splits) * mt * kWave * sizeof(float4_t);
 #define LAUNCH_T(MT, TO, T, THREADS)                                                                                    \
     gemm_skinny_joined_kernel<MT, TO, T, THREADS><<<blocks, 64 * splits, smem, stream>>>(                               \
         static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<TO*>(out), M, N, K, K / splits)
+#define LAUNCH_8(MT, TO) do { if (tiled) LAUNCH_T(MT, TO, true, 512); else LAUNCH_T(MT, TO, false, 512); } while (0)
 #define LAUNCH(MT, TO)                                                                                        \
-    if (splits <= 8) { if (tiled) LAUNCH_T(MT, TO, true, 512); else LAUNCH_T(MT, TO, false, 512); }            \
-    else { if (tiled) LAUNCH_T(MT, TO, true, 1024); else LAUNCH_T(MT, TO, false, 1024); }
+    do {                                                                                                      \
+        if (splits <= 8) LAUNCH_8(MT, TO);                                                                    \
+        else if (tiled) LAUNCH_T(MT, TO, true, 1024);                                                         \
+        else LAUNCH_T(MT, TO, false, 1024);                                                                   \
+    } while (0)
 #define BY_MT(TO)                         \
     switch (mt) {                         \
         case 1: LAUNCH(1, TO); break;     \
         case 2: LAUNCH(2, TO); break;     \
-        case 3: LAUNCH(3, TO); break;     \
-        default: LAUNCH(4, TO); break;    \
+        case 3: LAUNCH_8(3, TO); break;   \
+        default: LAUNCH_8(4, TO); break;  \
     }
     if (out_bf16) { BY_MT(bf16) } else { BY_MT(float) }
 #undef BY_MT
+#undef LAUNCH_8
 #undef LAUNCH
 #undef LAUNCH_T
     return launch_status();
