@@ -43,6 +43,11 @@ def close(got, ref, dtype, what="", scale=1.0):
     assert err <= 1.0, f"{what}: worst error {err:.2f} x tolerance, max abs diff {(got - ref).abs().max().item():.3e}"
 
 
+def near(got, ref, what):
+    far = (got.double().cpu() - ref.double().cpu()).abs().max().item() / ref.abs().max().item()
+    assert far <= 2e-6, f"{what}: off by {far:.2e} of the largest"
+
+
 @pytest.fixture(scope="module")
 def folders(tmp_path_factory):
     root = tmp_path_factory.mktemp("tokuvik_gpu")
@@ -280,10 +285,11 @@ def test_the_recurrence_over_long_segments(dtype, heads, groups, n_state, p, len
             s64[:, :inner].view(-1, heads, p), s64[:, inner:inner + groups * n_state].view(-1, groups, n_state),
             s64[:, inner + groups * n_state:].view(-1, groups, n_state),
             plain.softplus(dt[at:at + length, 1:1 + heads].double() + dt_bias.double()), a_log.double(), d_skip.double(), first)
-        # float32 sums of up to 256 products a token and of every token before: a few units of 2^-24 of the largest
-        close(y[at:at + length], want.reshape(-1, inner), torch.float32, f"segment {i}", scale=float(want.abs().max()))
+        # float32 sums of up to 256 products a token and of every token before: measured up to some 5 units of 2^-24 of the
+        # largest, the bound is 2e-6 of it
+        near(y[at:at + length], want.reshape(-1, inner), f"segment {i}")
         kept = state[int(slots[i]), :heads * n_state * p].view(heads, n_state, p)
-        close(kept, last, torch.float32, f"the state segment {i} leaves", scale=float(last.abs().max()))
+        near(kept, last, f"the state segment {i} leaves")
     assert torch.equal(state[:, heads * n_state * p:].cpu(), state0[:, heads * n_state * p:]), "what lies behind the states"
     others = [i for i in range(slots_total) if i not in slots.tolist()]
     assert torch.equal(state[others].cpu(), state0[others]), "a state of another request changed"
