@@ -450,6 +450,20 @@ def test_split_products_wanted_whole_have_the_bits_of_their_partial_sums(n, k):
     close(want, x.double() @ w.double().T, torch.float32, "product")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_split_products_into_a_result_at_any_address(dtype):
+    """The result may begin at any element: what begins at no multiple of four is written element by element."""
+    torch.manual_seed(22)
+    x, w = torch.randn(9, 2048, device=DEV).bfloat16(), (torch.randn(260, 2048, device=DEV) / 45.0).bfloat16()
+    want = torch.empty(9, 260, device=DEV, dtype=dtype)
+    ops.linear(x, w, want)
+    for offset in (1, 2, 3, 4):
+        flat = torch.full((9 * 260 + 8,), 7.0, device=DEV, dtype=dtype)
+        ops.linear(x, w, flat[offset:offset + 9 * 260].view(9, 260))
+        assert torch.equal(flat[offset:offset + 9 * 260].view(9, 260), want)
+        assert bool((flat[:offset] == 7.0).all()) and bool((flat[offset + 9 * 260:] == 7.0).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 2048, 16384), (129, 2048, 2064), (333, 2560, 2048), (200, 30, 4100), (128, 513, 520),
                                    (300, 70, 500), (520, 4096, 1536)])
 def test_float32_product_of_many_rows_has_the_same_bits_with_its_k_axis_cut(m, n, k):

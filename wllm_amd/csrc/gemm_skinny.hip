@@ -306,7 +306,7 @@ gemm_skinny_joined_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w
         const int m = 16 * t + i, n = n0 + 4 * g;
         if (m >= M || n >= N) continue;
         TO* o = out + static_cast<size_t>(m) * N + n;
-        if (n + 3 < N && (N % 4 == 0)) {
+        if (n + 3 < N && N % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(TO)) == 0) {
             store4<TO>(o, sum);
         } else {
 #pragma unroll
