@@ -533,7 +533,7 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
 // v_mfma_f32_16x16x4_f32 (float32 in and out), 17 of them a wavefront and chunk.  A chunk begins every 16 tokens of a
 // segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).
 // The walk token by token is bound by its chain (0.27 us a token).  64 heads of 64 with 128 rows of state: 1,500 tokens
-// 410 us token by token, 13 and 90 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
+// 410 us token by token, 13 and 86 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
 // 64 tokens 21 us against 7 and 9, which is where the line between the two ways lies. ----
 constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, suf d, pre_16 (and padding)
 
