@@ -134,15 +134,24 @@ def test_piece_length():
 
 
 def test_pieces_that_give_every_compute_unit_one_and_blocks_that_stay_whole():
-    # 256 rows over 4,096 keys, 8 heads on one: 32 blocks of rows of 121 to 128 groups in 8 pieces each, 256 in all
-    _, _, _, prefill = covered([256], [4096], 8, 1, 0, 16)
-    assert prefill.shape[0] == 256
-    _, _, _, prefill = covered([240], [4096], 8, 1, 0, 16)             # a block or two less: the shortest pieces again
+    # rows far behind their first key, 8 heads on one: blocks of about equal spans, cut so that no compute unit of 256 has two items
+    for rows, keys, pieces in ((256, 4096, 256), (240, 4096, 240), (256, 3000, 256), (128, 6000, 256), (200, 4000, 250)):
+        _, _, _, prefill = covered([rows], [keys], 8, 1, 0, 16)
+        assert prefill.shape[0] == pieces, (rows, keys)
+    _, _, _, prefill = covered([1100], [1100], 8, 1, 0, 16)            # spans of 1 to 35 groups: the shortest pieces
     assert prefill.shape[0] > 300
     _, reduces, _, _ = covered([384], [384], 8, 1, 0, 16)              # 12 groups and fewer
     assert reduces.shape[0] == 0
     _, reduces, _, _ = covered([385], [385], 8, 1, 0, 16)
     assert reduces.shape[0] > 0
+
+
+def test_pieces_over_many_keys_and_of_more_than_one_round_are_long():
+    # 16 heads on as many, 448 rows: seven blocks a head, of 2,000 keys (32,000 in all) in 4 pieces each, of 1,500 (24,000) shorter
+    assert covered([448], [2000], 1, 16, 0, 16)[3].shape[0] == 16 * 7 * 4
+    assert covered([448], [1500], 1, 16, 0, 16)[3].shape[0] > 16 * 7 * 4
+    assert covered([256, 256], [1024, 1024], 1, 16, 0, 16)[3].shape[0] == 16 * 2 * 4 * 2
+    assert covered([1100], [1100], 4, 8, 0, 16)[3].shape[0] == 888
 
 
 @pytest.mark.parametrize("seed", range(8))

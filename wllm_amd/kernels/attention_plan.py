@@ -43,10 +43,13 @@ PREFILL_TABLE_PAGES = 1024      # pages one prefill item may span (the kernel's 
 # 48.6; 16 heads on as many, 64 over 8,000 39.7 / 37.6 / 37.1 / 35.9.  Prompts of 2,048 and more, and portions of 512 over
 # 4,000, fill the device with longer pieces than any of these.
 PREFILL_MIN_PIECE = 10
-# Where that many groups a piece make exactly one piece for every compute unit, shorter ones make two on some of them and
-# lose: 256 rows over 4,096 keys 32.8 us in pieces of 16 groups and 33.5 in shorter ones, 128 over 8,000 33.8 and 35.4 (8 heads of 128 on
-# two 24.5 and 27.1).
-PREFILL_EVEN_PIECE = 16
+# Groups of a piece above which nothing is gained by shorter ones for their own sake (see `prefill_piece_length`).
+PREFILL_LONG_PIECE = 16
+# Keys of all segments and key/value heads above which a step's blocks keep long pieces: the keys and values (of heads of
+# 256 some 30 MB) then come past the L2s, and so do the partial results.
+# Pieces of 16 groups against the shortest, us, 16 heads of 256 on as many: 448 rows over 2,000 keys 38.8 and 44.3, 256 over 3,000 39.0 and
+# 43.3, 128 over 6,000 42.5 and 44.7, two of 256 over 1,024 32.8 and 33.8, but 512 over 1,500 36.3 and 35.7, 700 over 1,000 36.4 and 33.0.
+PREFILL_MANY_KEYS = 30000
 WORKGROUP_SLOTS = 512           # prefill workgroups a device runs at once unless the caller knows better (two a compute unit)
 PREFILL_ROWS = 64               # rows of a prefill item unless the kernel for the sizes at hand says otherwise
 
@@ -202,29 +205,43 @@ def build_tile_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
     return it.reshape(-1, ITEM_INTS), rs.reshape(-1, ITEM_INTS), per_head * num_kv_heads
 
 
-def prefill_piece_length(span: np.ndarray, num_kv_heads: int, workgroup_slots: int, longest: int) -> int:
+def prefill_piece_length(span: np.ndarray, num_kv_heads: int, workgroup_slots: int, longest: int, first=(0,)) -> int:
     """The most groups of 32 keys a prefill item gets, for blocks of rows that span `span` groups each
     (per key/value head).  The shortest length with which the items fill the workgroup slots of the
     device at most once, twice, ... (the fewest rounds that the longest allowed piece permits): every
     further item costs a partial result that is written and read again, and items that start together
     and are about equally long end together.  Never shorter than `PREFILL_MIN_PIECE` groups, below which
-    a piece's partial result costs more than its share of the keys, nor than `PREFILL_EVEN_PIECE` where that gives
-    every compute unit (a half of the workgroup slots) one piece; blocks of hardly more than the least length stay
-    whole (333 rows over 333 keys 20.1 us cut, 19.2 whole)."""
+    a piece's partial result costs more than its share of the keys.  Of lengths up to `PREFILL_LONG_PIECE`:
+    blocks of hardly more than the least length stay whole (333 rows over 333 keys 20.1 us cut, 19.2 whole);
+    blocks of about equal spans take the least with which every compute unit (half of the workgroup slots) has one
+    item and none has two, which take as long as one that is seven groups longer (8 heads of 256 on one, the least
+    length, this one and `PREFILL_LONG_PIECE`: 256 rows over 3,000 keys 31.0 / 27.1 / 30.2 us, 128 over 6,000 30.4 / 27.2 / 30.3; of
+    unequal spans the long items run alone in the end: 1,100 over 1,100 29.6 / 31.1 / 31.9); else a step of more than one
+    round (1,100 over 1,100 of 32 heads of 128 on eight: 36.9 us, in shorter pieces 37.9) or over more than
+    `PREFILL_MANY_KEYS` keys takes the longest.  `first`: the first block of every segment."""
+    most = int(span.max())
+    if most <= PREFILL_MIN_PIECE + 2:
+        return min(longest, PREFILL_LONG_PIECE)
+
     def count(length):
         return int((-(-span // length)).sum()) * num_kv_heads
     rounds = max(1, -(-count(longest) // workgroup_slots))
-    lo, hi = 1, longest                      # the least length whose count fits
+    lo, hi = 1, min(longest, most)           # the least length whose count fits
     while lo < hi:
         mid = (lo + hi) // 2
         if count(mid) <= rounds * workgroup_slots:
             hi = mid
         else:
             lo = mid + 1
-    if lo < PREFILL_EVEN_PIECE and (count(PREFILL_EVEN_PIECE) == workgroup_slots // 2
-                                    or int(span.max()) <= PREFILL_MIN_PIECE + 2):
-        return min(longest, PREFILL_EVEN_PIECE)
-    return min(longest, max(lo, PREFILL_MIN_PIECE))
+    lo = max(lo, PREFILL_MIN_PIECE)
+    if lo < PREFILL_LONG_PIECE:
+        units = workgroup_slots // 2
+        if 8 * int(span.min()) >= 7 * most and count(PREFILL_LONG_PIECE) <= units:
+            while count(lo) > units:
+                lo += 1
+        elif rounds > 1 or 32 * num_kv_heads * int(np.maximum.reduceat(span, first).sum()) > PREFILL_MANY_KEYS:
+            lo = PREFILL_LONG_PIECE
+    return min(longest, lo)
 
 
 def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_heads: int, window: int,
@@ -304,7 +321,8 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
         # the blocks of rows of all long segments, one after the other
         n_blocks = -(-rows[long_idx] // prefill_rows)
         seg_of = np.repeat(long_idx, n_blocks)
-        rb = (np.arange(int(n_blocks.sum())) - np.repeat(np.cumsum(n_blocks) - n_blocks, n_blocks)) * prefill_rows
+        first = np.cumsum(n_blocks) - n_blocks
+        rb = (np.arange(int(n_blocks.sum())) - np.repeat(first, n_blocks)) * prefill_rows
         first_pos = (ctx_len - q_len)[seg_of]
         hi = first_pos + np.minimum(rows[seg_of] - 1, rb + prefill_rows - 1) // group + 1
         lo = lowest_keys(first_pos + rb // group, window)
@@ -314,7 +332,7 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
         span = -(-(hi - lo32) // 32)                                                  # in groups of 32 keys
         # a piece that starts inside a page touches up to two pages more than its keys fill
         longest = max(KEY_CHUNK, (PREFILL_TABLE_PAGES - 2) * page_size // KEY_CHUNK * KEY_CHUNK) // 32
-        ns = -(-span // prefill_piece_length(span, num_kv_heads, workgroup_slots, longest))
+        ns = -(-span // prefill_piece_length(span, num_kv_heads, workgroup_slots, longest, first))
         piece = -(-span // ns)
         ns = -(-span // piece)
         tiles = prefill_rows // ROWS_PER_TILE
