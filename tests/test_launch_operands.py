@@ -99,3 +99,11 @@ def test_a_registered_launch_is_handed_the_stream_as_a_pointer(handle, monkeypat
     with ops.use_backend(backend):
         ops.call("a_parts_own")
     assert isinstance(seen[0], ctypes.c_void_p) and seen[0].value == (handle or None)
+
+
+def test_where_pieces_of_few_rows_products_are_joined():
+    """By rows and keys: every band of columns reads the rows for itself."""
+    from wllm_amd.kernels.hip_backend import HipBackend
+    takes = HipBackend.joined_takes
+    assert takes(16, 2048, 16, 6144) and not takes(17, 2048, 16, 6144) and takes(12, 2048, 16, 8192) and not takes(1, 2048, 16, 8224)
+    assert takes(24, 2048, 16, 4096) and not takes(25, 2048, 16, 4096) and takes(64, 2048, 2, 768) and not takes(64, 2048, 2, 2048)

@@ -402,12 +402,16 @@ class HipBackend:
                     "tile_weight")
 
     @staticmethod
-    def joined_takes(rows: int, n: int, splits: int) -> bool:
+    def joined_takes(rows: int, n: int, splits: int, k: int) -> bool:
         """Where a split product whose sum the caller wants itself runs as one launch, the pieces of the K axis meeting
         inside a workgroup (a wavefront each, at most 16).  There every band of 16 columns reads x for itself, so with
         more rows and more columns the two launches that stage x once win: 2,048 keys to 2,568 columns 9.1 against 5.0 us
         at 8 rows, 10.3 against 7.2 at 24, but to 2,048 columns 10.9 against 12.2 at 64; to 10,304 columns 13.9
-        against 11.1 at 8 and 15.8 against 16.3 at 24; in two pieces (768 keys to 2,048 columns) 9.9 against 6.7 at 64."""
+        against 11.1 at 8 and 15.8 against 16.3 at 24; in two pieces (768 keys to 2,048 columns) 9.9 against 6.7 at 64.
+        And with more keys, to 2,048 columns: at 8 rows of 8,192 keys 13.1 against 11.3, of 12,288 14.7 against 16.5; at 16 of
+        6,144 12.3 against 11.5, of 8,192 13.4 against 14.0; at 24 of 4,096 12.0 against 11.3, of 6,144 12.8 against 15.3."""
+        if k > 8192 or rows * k > 98304:
+            return False
         return 1 < splits <= 16 and (rows <= 16 or n <= 8192 and (rows <= 32 or rows <= 64 and splits == 2))
 
     def _skinny(self, x, weight, out, tiles=None) -> None:
@@ -420,7 +424,7 @@ class HipBackend:
             self._check(self.lib.wllm_gemm_skinny(_ptr(x), _ptr(w), tiled, c_void_p(0), 0, _ptr(out), m, n, k, splits,
                                                   chunk, self._stream()), "linear (few rows, partial sums)")
             return
-        if self.joined_takes(m, n, splits):
+        if self.joined_takes(m, n, splits, k):
             self._check(self.lib.wllm_gemm_skinny_joined(_ptr(x), _ptr(w), tiled, _ptr(out), int(out.dtype == torch.bfloat16),
                                                          m, n, k, splits, self._stream()), "linear (few rows, pieces of K joined)")
             return
