@@ -168,10 +168,11 @@ def test_the_convolution_whole_and_cut_with_its_carried_inputs(dtype, channels, 
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("channels,extra,lengths", [(40, 8, [1, 70, 3, 2]), (1028, 4, [64]), (42, 2, [66, 1]), (64, 3, [9, 8, 7, 6, 5, 33]), (2048, 0, [63, 1, 1]),
-                                                    (64, 8, [7, 2, 14, 3, 40]), (1028, 4, [6, 2, 7, 1, 6, 1, 1, 42])])
+                                                    (64, 8, [7, 2, 14, 3, 40]), (1028, 4, [6, 2, 7, 1, 6, 1, 1, 42]),
+                                                    (6144, 0, [64]), (6140, 8, [64]), (32768, 8, [7, 2, 14, 3, 40]), (32772, 4, [6, 2, 7, 1, 6, 1, 1, 42])])
 def test_convolutions_of_many_tokens_have_the_bits_of_few(dtype, channels, extra, lengths):
-    """From 64 tokens on a thread walks tokens with the last inputs in registers (4 taps; channels and strides in fours, else
-    the kernel for any): the bits of the same segments in steps of fewer tokens, in both convolutions, from carried rows,
+    """From 64 tokens and some 400,000 elements on a thread walks tokens with the last inputs in registers (4 taps; channels and
+    strides in fours, else the kernel for any): the bits of the same segments in steps of fewer tokens, in both convolutions, from carried rows,
     with segments that begin inside a thread's run of tokens or whose first tokens lie on either side of its end."""
     g = torch.Generator().manual_seed(channels + len(lengths))
     n, slots_total = sum(lengths), len(lengths) + 2

@@ -37,7 +37,14 @@ causal_conv_kernel(const T* __restrict__ in, long long in_stride, const float* _
 // The same sums for the many tokens of a prompt's portion and convolutions of kSlideTaps taps: a thread takes four
 // consecutive channels and walks kSlideTokens tokens with the last inputs in registers, so a row is read once and not
 // once a tap, in 8-byte (float32: 16-byte) pieces (6,144 channels of 1,500 tokens: 62 to 17 us).
+// Fewer elements than `many_elements` are bound by a launch's chain, which is longer here (the kernel a token and the one for the
+// carried rows behind it, against this one, us: 256 channels of 200 tokens 5.1 and 5.5, 2,048 of 64 5.4 and 6.0, of 200 6.6 and 6.1, 6,144 of
+// 64 6.4 and 6.2), and tokens that each begin a segment are a chain of their own (6,144 channels of 96 segments of one token 9.2 and
+// 10.1, 2,048 of 200 segments of two 12.5 and 8.2).
 constexpr int kSlideTaps = 4, kSlideTokens = 8, kSlideFrom = 64;
+static bool slides(int tokens, int segments, int channels, long long many_elements) {
+    return tokens >= kSlideFrom && tokens >= 2LL * segments && static_cast<long long>(tokens) * channels >= many_elements;
+}
 template <typename T> struct alignas(4 * sizeof(T)) ConvFour { T v[4]; };
 
 template <typename T>
@@ -52,7 +59,7 @@ __device__ __forceinline__ float4 conv_four(const T* p) {
 // first: a tile that begins at a segment's second or third token leaves them to the tile before it, which walks up to
 // kSlideOver tokens more.  So the thread that has read a request's carried rows is the only one that will, and writes
 // the new ones (the segment's last inputs) without a launch behind this one.  2,048 channels of 3,001 float32 tokens: 9.3
-// us and 3.0 in a launch behind it, now 10.0; 96 segments of one token, 6,144 channels: 8.0 and 6.4, now 10.6.
+// us and 3.0 in a launch behind it, now 10.0.
 constexpr int kSlideOver = kSlideTaps - 2;
 template <typename T, typename MAKE>
 __device__ __forceinline__ void slide(const T* in, long long in_stride, float* state, long long state_stride,
@@ -161,7 +168,7 @@ WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* 
                                                                 state_stride, carried_offset, token_segment, seg_q_start, \
                                                                 seg_q_len, state_slots, static_cast<T*>(out), tokens, \
                                                                 channels)
-    const bool many = taps == kSlideTaps && tokens >= kSlideFrom;          // (these keep the carried rows themselves)
+    const bool many = taps == kSlideTaps && slides(tokens, segments, channels, 3LL << 17);   // (these keep the carried rows themselves)
     if (many && is_bf16 && in_fours<bf16>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
         return SLIDE(bf16), launch_status();
     if (many && !is_bf16 && in_fours<float>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
@@ -311,7 +318,9 @@ WLLM_API int wllm_stream_conv(const float* x, const float* weight, float* state,
     if (four) {
         const dim3 grid4(tokens, (channels / 4 + 255) / 256);
         const dim3 slide_grid((tokens + kSlideTokens - 1) / kSlideTokens, (channels / 4 + 255) / 256);
-        if (taps == kSlideTaps && tokens >= kSlideFrom) {
+        // (the kernel that it replaces reads in fours too, and its chain is no shorter: beside many single tokens only, 2,048
+        // channels of 60 and a segment of 448, 6.2 us and here 6.8, 6,144 channels of them 14.6 and 11.2)
+        if (taps == kSlideTaps && slides(tokens, segments, channels, tokens >= 16LL * segments ? 0 : 1 << 21)) {
             if (out_bf16)
                 stream_conv_slide_kernel<bf16><<<slide_grid, 256, 0, stream>>>(x, weight, state, state_stride, carried_offset,
                                                                                token_segment, seg_q_start, seg_q_len, state_slots,
