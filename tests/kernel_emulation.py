@@ -355,7 +355,7 @@ class EmulatedKernels:
                 carried.copy_(seq[ql:ql + taps - 1].float())
 
     def ssm_scan(self, xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y, heads, groups,
-                 state_size, head_dim, steps=None, chunks=None, shortest=0):
+                 state_size, head_dim, steps=None, chunks=None, begin=0, shortest=0):
         self._count("ssm_scan")
         inner, n_s = heads * head_dim, state_size
         per = heads // groups
@@ -441,7 +441,7 @@ class EmulatedKernels:
             state[slot, m_offset:m_offset + heads] = m.float()
 
     def memory_scan(self, qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim,
-                    nq=None, n_offset=0, row_decays=False, chunks=None, shortest=0):
+                    nq=None, n_offset=0, row_decays=False, chunks=None, begin=0, shortest=0):
         self._count("memory_scan")
         acc = self.acc
         size, width = heads * head_dim * value_dim, heads * head_dim

@@ -8,6 +8,12 @@ import torch
 from wllm_amd.kernels import ops
 
 
+@pytest.fixture
+def chunks_from_64(monkeypatch):
+    monkeypatch.setattr(ops, "ssm_chunk_from", lambda heads, groups: 64)
+    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim: 64)
+
+
 class Launches:
     """A backend whose launches end in a function that only looks at the arguments of the entry point."""
 
@@ -35,7 +41,7 @@ def _scan(kind, n, **extra):
 
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
-def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
+def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch, chunks_from_64):
     """The scratch of a recurrence walked in chunks (the fourth argument from the end) is a tensor that something refers to
     when the launch is made: else its memory is the allocator's again before a kernel has run."""
     made, empty, seen = [], torch.empty, []
@@ -57,8 +63,8 @@ def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch):
 
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
-def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
-    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, torch.bfloat16)
+def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind, chunks_from_64):
+    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, 16, torch.bfloat16)
     mine = torch.zeros(size)
     with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-4]) or 0)):
         seen = []
@@ -68,12 +74,12 @@ def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind):
             with pytest.raises(ops.KernelShapeError):
                 _scan(kind, 80, chunks=wrong)
         assert len(seen) == 1
-    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, torch.bfloat16)
-    assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, torch.float32)
+    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, 16, torch.bfloat16)
+    assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, 16, torch.float32)
 
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
-def test_a_scan_without_room_for_its_scratch_is_walked_token_by_token(kind, monkeypatch):
+def test_a_scan_without_room_for_its_scratch_is_walked_token_by_token(kind, monkeypatch, chunks_from_64):
     seen, empty = [], torch.empty
 
     def full(size, *args, **kwargs):
@@ -99,6 +105,19 @@ def test_a_registered_launch_is_handed_the_stream_as_a_pointer(handle, monkeypat
     with ops.use_backend(backend):
         ops.call("a_parts_own")
     assert isinstance(seen[0], ctypes.c_void_p) and seen[0].value == (handle or None)
+
+
+@pytest.mark.parametrize("kind,first", [("space", 64), ("memory", 128)])
+def test_a_scan_is_walked_in_chunks_from_where_they_pay(kind, first):
+    """The tokens from which a segment takes chunks go to the launch, and a step without such a segment has none of it."""
+    with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-4:-1]) or 0)):
+        seen = []
+        for n, extra in ((first - 1, {}), (first, {}), (first, {"longest": first - 1}), (first + 40, {"longest": first, "shortest": 5})):
+            _scan(kind, n, **extra)
+    assert [begin for _, begin, _ in seen] == [0, first, 0, first] and [bool(chunks) for chunks, _, _ in seen] == [False, True, False, True]
+    assert seen[-1][2] == 5
+    assert [ops.ssm_chunk_from(h, g) for h, g in ((16, 1), (17, 1), (64, 1), (65, 1), (64, 8))] == [64, 128, 128, 130, 64]
+    assert [ops.memory_chunk_from(h, v) for h, v in ((4, 512), (8, 64), (8, 65), (16, 128), (1, 511))] == [96, 128, 192, 192, 128]
 
 
 def test_where_pieces_of_few_rows_products_are_joined():

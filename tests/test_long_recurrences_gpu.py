@@ -10,6 +10,13 @@ DEV = "cuda"
 SHORT = 40                  # a portion of so many tokens is walked token by token
 
 
+@pytest.fixture(autouse=True)
+def _chunks_from_64_tokens(monkeypatch):
+    """Whatever the sizes: where the chunks pay is not what is tested."""
+    monkeypatch.setattr(ops, "ssm_chunk_from", lambda heads, groups: 64)
+    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim: 64)
+
+
 def _ints(values):
     return torch.tensor(values, dtype=torch.int32, device=DEV)
 

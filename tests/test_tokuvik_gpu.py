@@ -264,10 +264,11 @@ def test_the_recurrence_whole_and_token_by_token(dtype, heads, groups, n_state, 
 @pytest.mark.parametrize("heads,groups,n_state,p,lengths", [
     (4, 2, 16, 16, [64, 3, 80]), (3, 1, 7, 10, [63, 64, 65]), (2, 2, 130, 72, [79, 1]), (20, 1, 64, 20, [97]), (6, 3, 200, 33, [1, 300, 1, 70]),
     (1, 1, 256, 4, [128]), (64, 8, 128, 64, [333, 40])])
-def test_the_recurrence_over_long_segments(dtype, heads, groups, n_state, p, lengths):
+def test_the_recurrence_over_long_segments(dtype, heads, groups, n_state, p, lengths, monkeypatch):
     """Segments of 64 tokens and more go over the matrix cores in chunks of 16, the ones beside them token by token: on
     either side of that line, whole chunks and one token more or less, rows of state and columns that fill no tile, more
     heads a group than a pass of the operands' kernel, from states that are not zero."""
+    monkeypatch.setattr(ops, "ssm_chunk_from", lambda heads, groups: 64)      # (of every group's heads)
     g = torch.Generator().manual_seed(n_state + p + len(lengths))
     inner, slots_total = heads * p, len(lengths) + 2
     width, n = inner + 2 * groups * n_state, sum(lengths)

@@ -339,8 +339,8 @@ memory_scan_kernel(const float* __restrict__ qk, const T* __restrict__ v, long l
 // was cut.
 // Three segments of 500, 1,000 and 1,501 tokens, 16 heads of 128 by 128 with decays a row: 301 us token by token, 34 and
 // 156 for the two kernels here; 2,048 tokens of 8 heads of 128 by 256 with a decay a head 305 against 19 and 127, with
-// exponential gates and the normaliser 297 against 19 and 125; 64 tokens 12.6 against 7 and 9, from where on a segment
-// gains.  Off the result in 64 bits (y; the memory left behind), here and token by token: decays a head 2.0e-7; 2.0e-7 and
+// exponential gates and the normaliser 297 against 19 and 125; 64 tokens 12.6 against 7 and 9 (where a segment
+// gains is the caller's rule, `from`).  Off the result in 64 bits (y; the memory left behind), here and token by token: decays a head 2.0e-7; 2.0e-7 and
 // 3.1e-7; 3.2e-7, decays a row 8.1e-8; 4.5e-8 and 9.1e-8; 4.5e-8, exponential gates 8.7e-8; 5.3e-8 and 9.9e-8; 5.7e-8.  With N
 // in 32 bits (27 us) and without the rest of Kh (138 us) decays a row are off by 9.4e-8; 4.8e-8, so both stay. ----
 typedef float memory_float4 __attribute__((ext_vector_type(4)));

@@ -543,7 +543,7 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
 // segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).
 // The walk token by token is bound by its chain (0.27 us a token).  64 heads of 64 with 128 rows of state: 1,500 tokens
 // 410 us token by token, 13 and 86 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
-// 64 tokens 21 us against 7 and 9, which is where the line between the two ways lies. ----
+// 64 tokens 21 us against 7 and 9, one line between the two ways; of more heads a group it lies further on. ----
 constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, suf d, pre_16 (and padding)
 
 // The operands of a chunk and a group: 28 us at 8 heads a group with a thread an entry of N that multiplied its decays one

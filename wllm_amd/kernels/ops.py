@@ -989,32 +989,54 @@ def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, carr
              **({"single_tokens": True} if single_tokens else {}))
 
 
-# Tokens of a request in a step from which the recurrences with a carried state are walked in chunks of 16 tokens
+# The recurrences with a carried state over a request's many tokens are walked in chunks of 16 tokens
 # on the matrix cores.  In bfloat16 only: the chunks add in another order than the walk token by token, and in the true
 # 32-bit path, which results are compared with, a token has the same bits however its prompt was cut (the products keep them
-# too).  1,500 tokens of 64 heads of 64 by 128 take 100 us in chunks and 410 token by token
+# too).  1,500 tokens of 64 heads of 64 by 128 take 98 us in chunks and 410 token by token
 # (a float32 prompt of 1,500 tokens of the Tokuvik 2B sizes: 62.5 ms, where chunks gave 60.6).
-SCAN_CHUNK, SCAN_CHUNK_FROM = 16, 64
+SCAN_CHUNK = 16
 
 
-def _scan_places(tokens: int, segments: int, dtype: torch.dtype) -> int:
-    """Places for the chunks of every segment of a step, 0 if no segment of it can be long enough for chunks."""
-    if dtype != torch.bfloat16 or tokens - (segments - 1) < SCAN_CHUNK_FROM:
+def ssm_chunk_from(heads: int, groups: int) -> int:
+    """Tokens of a request in a step from which `ssm_scan` walks them in chunks.  Their first kernel walks the heads of a
+    group sixteen at a time, 5 us each, whatever the tokens.  Token by token against chunks, us: 64 heads of 64 by 128 in 8
+    groups, 64 tokens 22.7 and 16.3; 32 of 64 by 16 in one, 64 tokens 17.7 and 22.1, 128 29.5 and 24.6; 128 of 64 by 128 in one, 128
+    tokens 47.7 and 66.3, 200 69.8 and 72.2, 300 99 and 79."""
+    per_group = heads // groups
+    return 64 if per_group <= 16 else max(128, 2 * per_group)
+
+
+def memory_chunk_from(heads: int, value_dim: int) -> int:
+    """The same for `memory_scan`, whose first kernel's work goes by the keys and the walk's by keys and values: it comes back
+    later the narrower the values are, and where requests side by side fill the device it is work and not a chain that
+    counts.  Token by token against chunks, us: 16 heads of 128 by 128, one request of 128 tokens 21.9 and 21.5, eight 60 and 66, eight of
+    200 92 and 89; 8 of 128 by 256, eight of 128 62 and 65, of 200 93 and 84; 4 of 256 by 512, four of 64 34 and 35, one of 96
+    28 and 26; 4 of 64 by 64 (few workgroups, a chain alone), 20 of 100 20 and 21, one of 128 18.3 and 14.9."""
+    return 96 if value_dim >= 512 else 128 if heads * value_dim <= 512 else 192
+
+
+def _scan_places(tokens: int, segments: int, dtype: torch.dtype, begin: int, longest: int) -> int:
+    """Places for the chunks of every segment of a step, 0 if no segment of it is long enough for chunks (`longest`: the
+    most tokens of one, 0: not known, then what the others' single tokens leave)."""
+    if dtype != torch.bfloat16 or (longest or tokens - (segments - 1)) < begin:
         return 0
-    return tokens // SCAN_CHUNK + tokens // SCAN_CHUNK_FROM
+    return tokens // SCAN_CHUNK + tokens // begin
 
 
-def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_size: int, dtype: torch.dtype) -> int:
+def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_size: int, dtype: torch.dtype, longest: int = 0) -> int:
     """Floats of scratch with which `ssm_scan` walks a step in chunks; 0: it does without (a decode step, so a captured graph
     holds none)."""
     rows = SCAN_CHUNK * (-(-state_size // 64) * 64)          # (two rows a token, of bfloat16)
-    return _scan_places(tokens, segments, dtype) * (heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows)
+    return _scan_places(tokens, segments, dtype, ssm_chunk_from(heads, groups), longest) * (
+        heads * (SCAN_CHUNK + 3) * SCAN_CHUNK + groups * rows)
 
 
-def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, dtype: torch.dtype) -> int:
+def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, value_dim: int, dtype: torch.dtype,
+                      longest: int = 0) -> int:
     """The same for `memory_scan` (`dtype`: that of the values)."""
     c = -(-head_dim // 64) * 64
-    return _scan_places(tokens, segments, dtype) * heads * ((2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
+    return _scan_places(tokens, segments, dtype, memory_chunk_from(heads, value_dim), longest) * heads * (
+        (2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
 
 
 def scratch_or_none(make):
@@ -1025,9 +1047,9 @@ def scratch_or_none(make):
         return None
 
 
-def _scan_extra(chunks: Optional[torch.Tensor], size: int, shortest: int, device) -> dict:
+def _scan_extra(chunks: Optional[torch.Tensor], size: int, begin: int, shortest: int, device) -> dict:
     """What the walk in chunks adds to a launch's operands: the scratch, the caller's or made here (an operand, so that
-    it is held until the launch has been made), and whether shorter segments may be beside the long ones.  Nothing where
+    it is held until the launch has been made), the tokens from which a segment takes it, and whether shorter ones may be beside.  Nothing where
     there is no room for the scratch: the step is then walked token by token."""
     if size == 0:
         return {}
@@ -1037,13 +1059,14 @@ def _scan_extra(chunks: Optional[torch.Tensor], size: int, shortest: int, device
             return {}
     _dense(chunks, "chunks", torch.float32)
     _need(chunks.numel() >= size, lambda: f"chunks: {chunks.numel()} floats of scratch, needed {size}")
-    return {"chunks": chunks, "shortest": int(shortest)}
+    return {"chunks": chunks, "begin": begin, "shortest": int(shortest)}
 
 
 def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, d_skip: torch.Tensor,
              state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
              y: torch.Tensor, *, heads: int, groups: int, state_size: int, head_dim: int,
-             steps: Optional[torch.Tensor] = None, chunks: Optional[torch.Tensor] = None, shortest: int = 0) -> None:
+             steps: Optional[torch.Tensor] = None, chunks: Optional[torch.Tensor] = None, shortest: int = 0,
+             longest: int = 0) -> None:
     """The selective state-space recurrence over each segment's tokens in order, from and into the
     request's carried state.  Per head h (group h // (heads // groups)) and token:
         step = softplus(dt + dt_bias[h]);  S = exp(-exp(a_log[h]) * step) * S + step * B x^T;
@@ -1053,8 +1076,8 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     begins with S as [heads, N, P]; y float32 [n, heads*P].  All of the recurrence is float32.
     `steps`: float32 [2, n, heads] of scratch for the step sizes and decays, `chunks`: float32 scratch of `ssm_chunk_size`
     elements (made here if not given; a caller whose step may be captured in a graph gives its own).  `shortest`: the fewest
-    tokens of a segment of the step, if the caller knows it (0: it does not): a launch for short segments is then left out
-    where there are none."""
+    tokens of a segment of the step, if the caller knows it (0: it does not), `longest` the most: the launches for short or
+    for long segments are then left out where there are none."""
     _dense(xbc, "xbc", _ACT)
     inner = heads * head_dim
     _need(heads > 0 and groups > 0 and heads % groups == 0, "heads must be a multiple of groups")
@@ -1077,7 +1100,8 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: 
     if n:
         call("ssm_scan", xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y, heads, groups,
              state_size, head_dim, steps,
-             **_scan_extra(chunks, ssm_chunk_size(n, s, heads, groups, state_size, xbc.dtype), shortest, xbc.device))
+             **_scan_extra(chunks, ssm_chunk_size(n, s, heads, groups, state_size, xbc.dtype, longest), ssm_chunk_from(heads, groups),
+                           shortest, xbc.device))
 
 
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, groups: int,
@@ -1176,7 +1200,7 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
                 state: torch.Tensor, seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, state_slots: torch.Tensor,
                 y: torch.Tensor, *, heads: int, head_dim: int, value_dim: int, nq: Optional[torch.Tensor] = None,
                 n_offset: int = 0, row_decays: bool = False, chunks: Optional[torch.Tensor] = None,
-                shortest: int = 0) -> None:
+                shortest: int = 0, longest: int = 0) -> None:
     """The matrix memory's recurrence over each segment's tokens in order, from and into the request's
     carried state.  Per head:  S = a S + b k v^T;  y = S^T q  with (a, b) of the token from `steps` (float32
     [3, n, heads], of which the first two are read) or, with `decays` (float32 [heads]) instead, (decays[h], 1).
@@ -1186,7 +1210,7 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     begins with S as [heads, head_dim, value_dim]; y float32 [n, heads * value_dim].  All of the recurrence is float32.
     `row_decays` (then neither `steps` nor `decays`): qk has a third plane, float32 [3, n, heads * head_dim], of decays a
     row of S and token: S[i, :] = qk[2][i] S[i, :] + k[i] v^T.  `chunks`: float32 scratch of `memory_chunk_size` elements
-    (made here if not given); `shortest`: as in `ssm_scan`."""
+    (made here if not given); `shortest`, `longest`: as in `ssm_scan`."""
     if row_decays:
         _need(steps is None and decays is None, "row_decays: neither steps nor decays")
     else:
@@ -1213,7 +1237,8 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     if n:
         call("memory_scan", qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim, nq,
              int(n_offset), **({"row_decays": True} if row_decays else {}),
-             **_scan_extra(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, v.dtype), shortest, v.device))
+             **_scan_extra(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, value_dim, v.dtype, longest),
+                           memory_chunk_from(heads, value_dim), shortest, v.device))
 
 
 def head_norm_gate(y: torch.Tensor, gate: Optional[torch.Tensor], weight: Optional[torch.Tensor], out: torch.Tensor, *, heads: int,
@@ -1669,11 +1694,11 @@ def _register_own() -> None:
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                           c_int, c_int, c_void_p],
                 launch=lambda fn, stream, xbc, dt, dt_bias, a_log, d_skip, state, seg_q_start, seg_q_len, state_slots, y,
-                heads, groups, state_size, head_dim, steps, chunks=None, shortest=0: fn(
+                heads, groups, state_size, head_dim, steps, chunks=None, begin=0, shortest=0: fn(
                     p(xbc), p(dt), dt.stride(0), p(dt_bias), p(a_log), p(d_skip), p(state), state.stride(0), p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(steps), int(xbc.dtype == torch.bfloat16), xbc.shape[0],
                     seg_q_start.shape[0], heads, groups, state_size, head_dim,
-                    p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, shortest, stream))
+                    p(chunks), begin, shortest, stream))
     register_op("gated_group_norm", entry_point="wllm_gated_group_norm",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
                 launch=lambda fn, stream, y, z, weight, out, groups, eps: fn(
@@ -1705,10 +1730,10 @@ def _register_own() -> None:
                           c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                           c_int, c_int, c_void_p],
                 launch=lambda fn, stream, qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads,
-                head_dim, value_dim, nq=None, n_offset=0, row_decays=False, chunks=None, shortest=0: fn(
+                head_dim, value_dim, nq=None, n_offset=0, row_decays=False, chunks=None, begin=0, shortest=0: fn(
                     p(qk), p(v), v.stride(0), p(steps), p(decays), p(state), state.stride(0), n_offset, p(seg_q_start),
                     p(seg_q_len), p(state_slots), p(y), p(nq), bf(v), v.shape[0], seg_q_start.shape[0], heads, head_dim,
-                    value_dim, int(row_decays), p(chunks), SCAN_CHUNK_FROM if chunks is not None else 0, shortest, stream))
+                    value_dim, int(row_decays), p(chunks), begin, shortest, stream))
     register_op("head_norm_gate", entry_point="wllm_head_norm_gate",
                 argtypes=[c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_float, c_int,
                           c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],

@@ -96,13 +96,13 @@ class StateSpaceMixer:
         ops.causal_conv(row[:, self.inner:self.inner + self.channels], self.conv_w, self.conv_b, state, self.recurrent_size,
                         ctx.token_segment, ctx.seg_q_start, ctx.seg_q_len, ctx.state_slots, xbc)
         y = ctx.buffer("ssm_y", (n, self.inner), torch.float32)
-        size = ops.ssm_chunk_size(n, ctx.num_segments, s.num_heads, s.groups, s.state_size, h.dtype)
+        size = ops.ssm_chunk_size(n, ctx.num_segments, s.num_heads, s.groups, s.state_size, h.dtype, ctx.max_q_len)
         chunks = ops.scratch_or_none(lambda: ctx.buffer("scan_chunks", (size,), torch.float32)) if size else None
         ops.ssm_scan(xbc, row[:, self.inner + self.channels:], self.dt_bias, self.a_log, self.d_skip, state,
                      ctx.seg_q_start, ctx.seg_q_len, ctx.state_slots, y, heads=s.num_heads, groups=s.groups,
                      state_size=s.state_size, head_dim=s.head_dim,
                      steps=ctx.buffer("ssm_steps", (2, n, s.num_heads), torch.float32),
-                     chunks=chunks, shortest=ctx.min_q_len)
+                     chunks=chunks, shortest=ctx.min_q_len, longest=ctx.max_q_len)
         out = ctx.buffer("ssm_out", (n, self.inner), h.dtype)
         ops.gated_group_norm(y, row[:, :self.inner], self.norm_w, out, s.norm_groups, s.norm_eps)
         if product_input is not None:
