@@ -11,7 +11,7 @@ from wllm_amd.kernels import ops
 @pytest.fixture
 def chunks_from_64(monkeypatch):
     monkeypatch.setattr(ops, "ssm_chunk_from", lambda heads, groups: 64)
-    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim: 64)
+    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim, row_decays: 64)
 
 
 class Launches:
@@ -64,7 +64,7 @@ def test_scratch_that_a_scan_makes_is_held_until_its_launch(kind, monkeypatch, c
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
 def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind, chunks_from_64):
-    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, 16, torch.bfloat16)
+    size = ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.bfloat16) if kind == "space" else ops.memory_chunk_size(80, 1, 2, 16, 16, torch.bfloat16, False)
     mine = torch.zeros(size)
     with ops.use_backend(Launches(lambda op, arguments: seen.append(arguments[-4]) or 0)):
         seen = []
@@ -74,8 +74,8 @@ def test_a_scan_uses_the_callers_scratch_and_refuses_less_than_it_needs(kind, ch
             with pytest.raises(ops.KernelShapeError):
                 _scan(kind, 80, chunks=wrong)
         assert len(seen) == 1
-    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, 16, torch.bfloat16)
-    assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, 16, torch.float32)
+    assert ops.ssm_chunk_size(63, 1, 2, 1, 16, torch.bfloat16) == 0 == ops.memory_chunk_size(96, 96, 2, 16, 16, torch.bfloat16, False)
+    assert ops.ssm_chunk_size(80, 1, 2, 1, 16, torch.float32) == 0 == ops.memory_chunk_size(80, 1, 2, 16, 16, torch.float32, False)
 
 
 @pytest.mark.parametrize("kind", ["space", "memory"])
@@ -117,7 +117,9 @@ def test_a_scan_is_walked_in_chunks_from_where_they_pay(kind, first):
     assert [begin for _, begin, _ in seen] == [0, first, 0, first] and [bool(chunks) for chunks, _, _ in seen] == [False, True, False, True]
     assert seen[-1][2] == 5
     assert [ops.ssm_chunk_from(h, g) for h, g in ((16, 1), (17, 1), (64, 1), (65, 1), (64, 8))] == [64, 128, 128, 130, 64]
-    assert [ops.memory_chunk_from(h, v) for h, v in ((4, 512), (8, 64), (8, 65), (16, 128), (1, 511))] == [96, 128, 192, 192, 128]
+    sizes = ((4, 512), (8, 64), (8, 65), (16, 128), (8, 256), (1, 511))
+    assert [ops.memory_chunk_from(h, v, True) for h, v in sizes] == [96, 128, 192, 192, 192, 128]
+    assert [ops.memory_chunk_from(h, v, False) for h, v in sizes] == [160, 128, 256, 256, 192, 128]
 
 
 def test_where_pieces_of_few_rows_products_are_joined():

@@ -230,7 +230,7 @@ def test_the_memory_over_long_segments(dtype, kind, heads, d, dv, lengths, monke
     """Segments of 64 tokens and more go over the matrix cores in chunks of 16, the ones beside them token by token, for
     each kind of decay: on either side of that line, whole chunks and one token more or less, channels and columns that
     fill no tile, a normaliser's column that begins a tile or ends one, from memories that are not zero."""
-    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim: 64)      # (whatever the sizes)
+    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim, row_decays: 64)      # (whatever the sizes)
     g = torch.Generator().manual_seed(d + dv + len(lengths))
     n, slots_total, memory = sum(lengths), len(lengths) + 2, heads * d * dv
     qk = torch.randn(3 if kind == "rows" else 2, n, heads * d, generator=g) * d ** -0.5

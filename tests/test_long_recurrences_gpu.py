@@ -14,7 +14,7 @@ SHORT = 40                  # a portion of so many tokens is walked token by tok
 def _chunks_from_64_tokens(monkeypatch):
     """Whatever the sizes: where the chunks pay is not what is tested."""
     monkeypatch.setattr(ops, "ssm_chunk_from", lambda heads, groups: 64)
-    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim: 64)
+    monkeypatch.setattr(ops, "memory_chunk_from", lambda heads, value_dim, row_decays: 64)
 
 
 def _ints(values):

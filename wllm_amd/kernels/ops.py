@@ -1006,13 +1006,19 @@ def ssm_chunk_from(heads: int, groups: int) -> int:
     return 64 if per_group <= 16 else max(128, 2 * per_group)
 
 
-def memory_chunk_from(heads: int, value_dim: int) -> int:
+def memory_chunk_from(heads: int, value_dim: int, row_decays: bool) -> int:
     """The same for `memory_scan`, whose first kernel's work goes by the keys and the walk's by keys and values: it comes back
     later the narrower the values are, and where requests side by side fill the device it is work and not a chain that
-    counts.  Token by token against chunks, us: 16 heads of 128 by 128, one request of 128 tokens 21.9 and 21.5, eight 60 and 66, eight of
+    counts.  Token by token against chunks, us, with decays a row: 16 heads of 128 by 128, one request of 128 tokens 21.9 and 21.5, eight 60 and 66, eight of
     200 92 and 89; 8 of 128 by 256, eight of 128 62 and 65, of 200 93 and 84; 4 of 256 by 512, four of 64 34 and 35, one of 96
-    28 and 26; 4 of 64 by 64 (few workgroups, a chain alone), 20 of 100 20 and 21, one of 128 18.3 and 14.9."""
-    return 96 if value_dim >= 512 else 128 if heads * value_dim <= 512 else 192
+    28 and 26; 4 of 64 by 64 (few workgroups, a chain alone), 20 of 100 20 and 21, one of 128 18.3 and 14.9.  With a decay a head
+    the walk reads less: 16 of 128 by 128, eight of 200 80 and 89, four of 300 66 and 65, one of 200 32 and 27; 8 of 128 by 256, four of 160
+    38 and 40, of 200 47 and 47; 4 of 256 by 512, twenty of 100 158 and 170, four of 160 55 and 54."""
+    if heads * value_dim <= 512:
+        return 128
+    if value_dim >= 512:
+        return 96 if row_decays else 160
+    return 192 if row_decays or value_dim >= 256 else 256
 
 
 def _scan_places(tokens: int, segments: int, dtype: torch.dtype, begin: int, longest: int) -> int:
@@ -1032,10 +1038,10 @@ def ssm_chunk_size(tokens: int, segments: int, heads: int, groups: int, state_si
 
 
 def memory_chunk_size(tokens: int, segments: int, heads: int, head_dim: int, value_dim: int, dtype: torch.dtype,
-                      longest: int = 0) -> int:
+                      row_decays: bool, longest: int = 0) -> int:
     """The same for `memory_scan` (`dtype`: that of the values)."""
     c = -(-head_dim // 64) * 64
-    return _scan_places(tokens, segments, dtype, memory_chunk_from(heads, value_dim), longest) * heads * (
+    return _scan_places(tokens, segments, dtype, memory_chunk_from(heads, value_dim, row_decays), longest) * heads * (
         (2 * SCAN_CHUNK + 5) * c + SCAN_CHUNK * SCAN_CHUNK)
 
 
@@ -1237,8 +1243,8 @@ def memory_scan(qk: torch.Tensor, v: torch.Tensor, steps: Optional[torch.Tensor]
     if n:
         call("memory_scan", qk, v, steps, decays, state, seg_q_start, seg_q_len, state_slots, y, heads, head_dim, value_dim, nq,
              int(n_offset), **({"row_decays": True} if row_decays else {}),
-             **_scan_extra(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, value_dim, v.dtype, longest),
-                           memory_chunk_from(heads, value_dim), shortest, v.device))
+             **_scan_extra(chunks, memory_chunk_size(n, seg_q_start.shape[0], heads, head_dim, value_dim, v.dtype, row_decays,
+                                                         longest), memory_chunk_from(heads, value_dim, row_decays), shortest, v.device))
 
 
 def head_norm_gate(y: torch.Tensor, gate: Optional[torch.Tensor], weight: Optional[torch.Tensor], out: torch.Tensor, *, heads: int,
