@@ -200,6 +200,26 @@ __device__ __forceinline__ float gate_product(float gate, float up, GateShape sh
     return g / (1.f + expf(-shape.slope * g)) * (u + shape.shift);
 }
 
+// z / (1 + 2^(-t)): the sigmoid's product by the hardware's exponential and reciprocal (an infinite power gives 0).
+__device__ __forceinline__ float sigmoid_product_fast(float z, float t) {
+    return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-t));
+}
+
+// The same for kernels that make both streams in float32 and write bfloat16: with the hardware's exponential and
+// reciprocal (an ulp each) in the place of tanh and a division.  0.5 z (1 + tanh(u)) is z / (1 + e^(-2u)), without the
+// difference of nearly equal numbers where u is far below zero.
+template <int GATE>
+__device__ __forceinline__ float gate_product_fast(float gate, float up, GateShape shape) {
+    static_assert(GATE >= 0 && GATE < kGates, "unknown gate");
+    constexpr float kLog2e = 1.4426950408889634f;
+    if (GATE == kActGeluTanh)
+        return sigmoid_product_fast(gate, gate * (2.f * 0.7978845608028654f * kLog2e) * (1.f + 0.044715f * gate * gate)) * up;
+    if (GATE == kActSilu) return sigmoid_product_fast(gate, gate * kLog2e) * up;
+    const float g = gate > shape.limit ? shape.limit : gate;
+    const float u = up > shape.limit ? shape.limit : (up < -shape.limit ? -shape.limit : up);
+    return sigmoid_product_fast(g, shape.slope * g * kLog2e) * (u + shape.shift);
+}
+
 // Runs `statement` with the compile-time constant GATE set to the gate's number.
 #define WLLM_BY_GATE(gate, statement)                                                       \
     switch (gate) {                                                                          \

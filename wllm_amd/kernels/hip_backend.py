@@ -61,6 +61,8 @@ _SIGNATURES = {
                                      c_int, c_float, c_int, c_void_p, c_void_p],
     "wllm_gemm_tile": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float,
                        c_void_p],
+    "wllm_gemm_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
+                       c_float, c_void_p],
     "wllm_split_sum": [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
     "wllm_gemm_generic": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p],
     "wllm_tile_weight_f32": [c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -346,7 +348,7 @@ class HipBackend:
         return dtype == torch.bfloat16 and rows <= 64 and in_features % 32 == 0
 
     # The tiled matrix-core product (`gemm_tile.hip`) for the rows of a mixed step or a large decode
-    # batch.  Measured against the library's product it is ahead where the output has few columns and
+    # batch, where the tiles of 256 further down do not take the product.  Measured against the library's product it is ahead where the output has few columns and
     # the K axis is long, so that the library's tiles leave compute units idle and a split of the K axis
     # fills them (the down projection: 1.3 to 1.6 times as fast at 128 to 1,024 rows), and for the gated
     # product, which it writes once, up to 256 rows (at 512 rows it takes 84 us in a mixed step where
@@ -383,9 +385,67 @@ class HipBackend:
                 and in_features % 64 == 0 and self.tile_splits(out_features, in_features, rows) > 1
                 and max(rows, out_features) * in_features * 2 < 2 ** 32)
 
+    # The product in tiles of 256 x 256 (`gemm_wide.hip`), a workgroup a compute unit, against the library's product and
+    # the tiles of 128 x 128, with the pass that follows each (the activation kernel; the norm that adds the pieces).
+    # It is ahead wherever its tiles fill the rounds of 256 compute units: the gated product of 2,048 keys to 2 x 16,384
+    # columns at 384 / 768 / 1,500 / 2,048 / 7,777 rows 56 / 101 / 157 / 211 / 753 us against 58 / 106 / 183 / 234 / 880, to 2 x 4,096
+    # columns at 1,500 / 2,048 / 3,001 rows 43 / 49 / 88 against 50 / 61 / 93; where a round is less than 0.7 full the others are
+    # (to 2 x 16,384 at 257 / 640 rows 55 / 98 against 51 / 95, to 2 x 4,096 at 512 / 1,024 rows 36 / 39 against 26 / 38).  At most 256
+    # rows are bound by the weights: there the tile's whole height keeps these from being read twice, which pays beyond 128
+    # rows where the columns give half the compute units a tile (to 2 x 24,576 at 129 / 256 rows 72 / 82 us against 107 / 134 in
+    # tiles of 128; to 2 x 16,384 at 224 rows 46 against 48; at 128 rows 44 against 39).
+    WIDE_TILE = 256
+    COMPUTE_UNITS = 256
+    WIDE_FULL = 0.7
+
+    @classmethod
+    def wide_gated_takes(cls, rows: int, columns: int, k: int) -> bool:
+        """Whether the gated product of `columns` output columns goes in tiles of 256 rows (of x, and of both streams' weights)."""
+        if rows <= 128 or k % 64 != 0 or max(rows, 2 * columns) * k * 2 >= 2 ** 32:
+            return False
+        tiles = -(-rows // cls.WIDE_TILE) * -(-columns // (cls.WIDE_TILE // 2))
+        if rows <= cls.WIDE_TILE:
+            return tiles >= cls.COMPUTE_UNITS // 2
+        rounds = -(-tiles // cls.COMPUTE_UNITS)
+        return rows * columns * 2 >= cls.WIDE_FULL * rounds * cls.COMPUTE_UNITS * cls.WIDE_TILE ** 2
+
+    @classmethod
+    def wide_takes(cls, rows: int, n: int, k: int) -> bool:
+        """Whether a product rounded to bfloat16 goes in tiles of 256 x 256 instead of to the library.  The library is ahead where
+        the columns fill its tiles (2,048 keys to 8,192 columns at 1,500 / 2,048 rows: 44 / 52 us against 46 / 53); where they are no
+        multiple of 128 it falls back (to 10,304 columns at 1,024 / 1,500 / 4,096 rows 51 / 62 / 180 against 45 / 52 / 144; to 5,160
+        at 3,001 rows 64 against 52), unless the rounds of tiles are less than 0.6 full (to 10,304 at 768 rows 38 against 44)."""
+        if rows <= 128 or n % 128 == 0 or k % 64 != 0 or max(rows, n) * k * 2 >= 2 ** 32:
+            return False
+        rounds = -(-(-(-rows // cls.WIDE_TILE) * -(-n // cls.WIDE_TILE)) // cls.COMPUTE_UNITS)
+        return rows * n >= 0.6 * rounds * cls.COMPUTE_UNITS * cls.WIDE_TILE ** 2
+
+    @classmethod
+    def wide_splits(cls, n: int, k: int, rows: int) -> int:
+        """Over how many workgroups the product in tiles of 256 splits a long K axis (1: another kernel is better): as many
+        pieces as make one round of workgroups, at least 512 keys each and 16 at most.  Product and norm, 16,384 keys to 2,048
+        columns at 512 / 1,024 / 1,500 / 2,048 / 3,001 / 4,096 rows 50 / 73 / 102 / 124 / 193 / 221 us against 55 / 91 in tiles of 128
+        (up to 1,024 rows) and 66 / 104 / 120 / 153 / 199 / 239 with the library's; 24,576 to 3,072 at 160 / 512 / 1,024 / 2,048 rows
+        52 / 84 / 136 / 268 against 63 / 128 / 239 and 151 / 275 / 282 / 421.  More tiles than half a round leave one piece, and the
+        library is mostly ahead (5,000 rows: 280 against 329); fewer than 168 workgroups leave too much of the machine idle (256
+        rows to 2,048 columns: 40 against 33 in tiles of 128), and a K axis of 4,096 is too short for what its pieces cost (2,048
+        rows: 54 against 48)."""
+        if rows <= 128 or k < cls.TILE_LONG_K or k % 64 != 0 or max(rows, n) * k * 2 >= 2 ** 32:
+            return 1
+        tiles = -(-rows // cls.WIDE_TILE) * -(-n // cls.WIDE_TILE)
+        splits = min(16, cls.COMPUTE_UNITS // tiles, k // 512)
+        return splits if splits > 1 and tiles * splits >= 168 else 1
+
+    @staticmethod
+    def _wide_operand(t: torch.Tensor) -> torch.Tensor:
+        # the kernel's loads are of 16 bytes; a view that begins elsewhere is copied
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+
     def linear_splits(self, rows, out_features, in_features, dtype) -> int:
         if self.skinny_takes(dtype, rows, in_features):
             return self.skinny_split(out_features, in_features)
+        if dtype == torch.bfloat16 and self.wide_splits(out_features, in_features, rows) > 1:
+            return self.wide_splits(out_features, in_features, rows)
         if self.tile_takes(dtype, rows, out_features, in_features):
             return self.tile_splits(out_features, in_features, rows)
         if dtype == torch.float32 and rows <= self.F32_FEW_ROWS:
@@ -440,13 +500,21 @@ class HipBackend:
             if self.skinny_takes(x.dtype, m, k):
                 self._skinny(x, weight, out, tiles)
                 return
-            if self.tile_takes(x.dtype, m, weight.shape[0], k):
-                # some hundred rows and a long K axis: the tiled product, its K axis in pieces whose
-                # sums the caller adds, or a kernel here in their order
-                n, splits = weight.shape[0], self.tile_splits(weight.shape[0], k, m)
-                stack = out if out.dim() == 3 else torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
-                self._check(self.lib.wllm_gemm_tile(_ptr(x), _ptr(weight), None, _ptr(stack), m, n, k, splits, 0, 0.0, 0.0, 0.0,
-                                                    self._stream()), "linear (tiles, partial sums)")
+            n, wide = weight.shape[0], self.wide_splits(weight.shape[0], k, m)
+            splits = wide if wide > 1 else self.tile_splits(n, k, m) if self.tile_takes(x.dtype, m, n, k) else 1
+            # many rows and a long K axis: a tiled product, its K axis in pieces whose sums the caller adds, or a kernel
+            # here in their order (without room for them the kernels below make the product)
+            stack = out if out.dim() == 3 else None
+            if splits > 1 and stack is None:
+                stack = ops.scratch_or_none(lambda: torch.empty((splits, m, n), dtype=torch.float32, device=x.device))
+            if stack is not None:
+                if wide > 1:
+                    x, weight = self._wide_operand(x), self._wide_operand(weight)
+                    self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), None, _ptr(stack), m, n, k, n, splits, 0, 0.0, 0.0,
+                                                        0.0, self._stream()), "linear (tiles of 256, partial sums)")
+                else:
+                    self._check(self.lib.wllm_gemm_tile(_ptr(x), _ptr(weight), None, _ptr(stack), m, n, k, splits, 0, 0.0, 0.0,
+                                                        0.0, self._stream()), "linear (tiles, partial sums)")
                 if out.dim() == 2:
                     self._check(self.lib.wllm_split_sum(_ptr(stack), _ptr(out), int(out.dtype == torch.bfloat16), m * n, splits,
                                                         self._stream()), "linear (sum of partial sums)")
@@ -459,6 +527,11 @@ class HipBackend:
             if k % 32 == 0 and out.dtype == torch.float32:
                 for r in range(0, m, 64):
                     self._skinny(x[r:r + 64], weight, out[r:r + 64], tiles)
+                return
+            if out.dtype == torch.bfloat16 and self.wide_takes(m, n, k):
+                x, weight = self._wide_operand(x), self._wide_operand(weight)
+                self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, n, 1, 0, 0.0, 0.0, 0.0,
+                                                    self._stream()), "linear (tiles of 256)")
                 return
             if out.dtype == torch.bfloat16 and m > 64:
                 # many rows: the library's matrix-core product (float32 accumulation)
@@ -526,6 +599,12 @@ class HipBackend:
                 "gated_linear (few rows, matrix cores)")
             return
         n = out.shape[1]
+        if x.dtype == torch.bfloat16 and self.wide_gated_takes(m, n, k):
+            number, *shape = gate_args(activation)
+            x, weight = self._wide_operand(x), self._wide_operand(weight)
+            self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, out.stride(0), 1, 1 + number,
+                                                *shape, self._stream()), "gated_linear (tiles of 256)")
+            return
         if (x.dtype == torch.bfloat16 and 64 < m <= self.TILE_GATED_MAX_ROWS and k % 64 == 0
                 and max(m, 2 * n) * k * 2 < 2 ** 32):
             # some hundred rows: the tiled product with the activation in its registers
@@ -552,6 +631,11 @@ class HipBackend:
                 self._check(self.lib.wllm_gemm_skinny_gated(
                     _ptr(x), _ptr(w), tiled, _ptr(out), m, half, k, number, 0.0, 0.0, 0.0, self.GATED_CHUNK[-(-m // 16)], n,
                     self._stream()), "activated_linear (few rows, matrix cores)")
+                return
+            if self.wide_gated_takes(m, half, k):
+                x, weight = self._wide_operand(x), self._wide_operand(weight)
+                self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, half, k, n, 1, 1 + number, 0.0, 0.0,
+                                                    0.0, self._stream()), "activated_linear (tiles of 256)")
                 return
             if 64 < m <= self.TILE_GATED_MAX_ROWS and k % 64 == 0 and max(m, n) * k * 2 < 2 ** 32:
                 self._check(self.lib.wllm_gemm_tile(_ptr(x), _ptr(weight), _ptr(out), None, m, half, k, 1, 1 + number, 0.0, 0.0,

@@ -17,9 +17,11 @@ def project(ctx, name: str, x: torch.Tensor, weight: torch.Tensor, out: Optional
     n, width = x.shape[0], weight.shape[0]
     splits = ops.linear_splits(n, width, x.shape[1], x.dtype)
     if splits > 1:
-        stack = ctx.buffer(name + "_parts", (splits, n, width), torch.float32)
-        ops.linear(x, weight, stack, tiles)
-        return stack
+        # (without room for the stack the kernels make the whole sum)
+        stack = ops.scratch_or_none(lambda: ctx.buffer(name + "_parts", (splits, n, width), torch.float32))
+        if stack is not None:
+            ops.linear(x, weight, stack, tiles)
+            return stack
     if out is None:
         out = ctx.buffer(name, (n, width), x.dtype)
     ops.linear(x, weight, out, tiles)
