@@ -52,6 +52,13 @@ PREFILL_LONG_PIECE = 16
 PREFILL_MANY_KEYS = 30000
 WORKGROUP_SLOTS = 512           # prefill workgroups a device runs at once unless the caller knows better (two a compute unit)
 PREFILL_ROWS = 64               # rows of a prefill item unless the kernel for the sizes at hand says otherwise
+PROMPT_ROWS = 128               # rows of a prefill item of the kernel for long prompts, one workgroup a compute unit
+# Groups of 32 keys that a step's blocks of 128 rows must span, in all and the longest, for the kernel for long prompts:
+# it does a group faster (8 heads of 256 on one, us, blocks of 64 and of 128 rows: 7,777 rows over 7,777 keys 362 / 261, 4,096 over 4,096
+# 148 / 112, 2,048 over 2,048 46 / 43, 2,048 over 8,192 208 / 131, 512 over 8,192 70 / 51; 16 heads on as many: 4,096 rows 222 / 140, 1,500 52 /
+# 47), but a workgroup begins and ends slower and there are half as many (8 heads on one: 1,500 rows, 2,270 groups, 35 / 36; 500, 1,000 and
+# 1,501 rows, 3,300 groups, 41 / 46; four times 1,000 rows, 4,150 groups, the longest of 32, 47 / 47; 448 rows over 448 20 / 22).
+PROMPT_GROUPS, PROMPT_LONGEST = 3500, 44
 
 
 @dataclass
@@ -244,12 +251,38 @@ def prefill_piece_length(span: np.ndarray, num_kv_heads: int, workgroup_slots: i
     return min(longest, lo)
 
 
+def _row_blocks(q_len, ctx_len, group, window, prefill_rows, long_idx):
+    """The blocks of rows of the long segments, one segment after the other: (segment, its first block's number, first row, the
+    first key seen rounded down to a multiple of 32, the end of the keys, the span in groups of 32 keys), by block but for
+    the second, which is by segment."""
+    n_blocks = -(-(q_len[long_idx] * group) // prefill_rows)
+    seg_of = np.repeat(long_idx, n_blocks)
+    first = np.cumsum(n_blocks) - n_blocks
+    rb = (np.arange(int(n_blocks.sum())) - np.repeat(first, n_blocks)) * prefill_rows
+    first_pos = (ctx_len - q_len)[seg_of]
+    hi = first_pos + np.minimum(q_len[seg_of] * group - 1, rb + prefill_rows - 1) // group + 1
+    lo = lowest_keys(first_pos + rb // group, window)
+    lo32 = lo // 32 * 32
+    return seg_of, first, rb, lo32, hi, -(-(hi - lo32) // 32)
+
+
+def prompt_kernel_pays(q_len, ctx_len, group: int, num_kv_heads: int, window: int) -> bool:
+    """Whether a step's long segments are work enough for the kernel for long prompts (`PROMPT_GROUPS`)."""
+    q_len, ctx_len = np.asarray(q_len, dtype=np.int64), np.asarray(ctx_len, dtype=np.int64)
+    long_idx = np.nonzero((q_len * group > ROWS_PER_TILE) & (q_len != 1))[0]
+    # (the keys of all rows in blocks of 128 bound the groups from above: most steps end here)
+    if not long_idx.size or int((-(-q_len[long_idx] * group // PROMPT_ROWS) * (ctx_len[long_idx] + 63)).sum()) * num_kv_heads < 32 * PROMPT_GROUPS:
+        return False
+    span = _row_blocks(q_len, ctx_len, group, window, PROMPT_ROWS, long_idx)[-1]
+    return int(span.max()) >= PROMPT_LONGEST and int(span.sum()) * num_kv_heads >= PROMPT_GROUPS
+
+
 def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_heads: int, window: int,
                      page_size: int = 16, prefill_rows: int = PREFILL_ROWS, workgroup_slots: int = WORKGROUP_SLOTS,
-                     tiles_only: bool = False):
+                     tiles_only: bool = False, slots_a_unit: int = 2):
     """Returns (items [n, 8], reduce_items [m, 8], partial slots, prefill items [p, 8], rows per
     prefill item) as int32 arrays.  `tiles_only`: no prefill items; long segments too are cut into
-    tiles of 16 rows (`build_tile_items`)."""
+    tiles of 16 rows (`build_tile_items`).  `slots_a_unit`: how many of the workgroup slots are one compute unit's."""
     if tiles_only:
         if group * num_kv_heads >= MAX_HEADS:
             raise ValueError(f"{group * num_kv_heads} query heads: a work item has 16 bits for a head")
@@ -318,18 +351,9 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
     prefill = np.zeros((0, ITEM_INTS), np.int32)
     long_idx = np.nonzero(~short)[0]
     if long_idx.size:
-        # the blocks of rows of all long segments, one after the other
-        n_blocks = -(-rows[long_idx] // prefill_rows)
-        seg_of = np.repeat(long_idx, n_blocks)
-        first = np.cumsum(n_blocks) - n_blocks
-        rb = (np.arange(int(n_blocks.sum())) - np.repeat(first, n_blocks)) * prefill_rows
-        first_pos = (ctx_len - q_len)[seg_of]
-        hi = first_pos + np.minimum(rows[seg_of] - 1, rb + prefill_rows - 1) // group + 1
-        lo = lowest_keys(first_pos + rb // group, window)
         # a block's keys are cut into equal pieces whose boundaries are multiples of 32 counted from the block's
         # first group of 32
-        lo32 = lo // 32 * 32
-        span = -(-(hi - lo32) // 32)                                                  # in groups of 32 keys
+        seg_of, first, rb, lo32, hi, span = _row_blocks(q_len, ctx_len, group, window, prefill_rows, long_idx)
         # a piece that starts inside a page touches up to two pages more than its keys fill
         longest = max(KEY_CHUNK, (PREFILL_TABLE_PAGES - 2) * page_size // KEY_CHUNK * KEY_CHUNK) // 32
         ns = -(-span // prefill_piece_length(span, num_kv_heads, workgroup_slots, longest, first))
@@ -355,11 +379,12 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
         it = it.reshape(-1, ITEM_INTS)
         # The workgroups start in the order of the items, the first ones one on each compute unit, the next ones
         # beside them: the longest pieces come first, and each further run of `workgroup_slots / 2` turns round,
-        # so that a long piece gets a short one for its neighbour and the last to start are the shortest.
+        # so that a long piece gets a short one for its neighbour and the last to start are the shortest (one to a compute unit
+        # has no neighbours: longest first throughout).
         length = np.minimum(it[:, 4], hi[block_of][None, :].repeat(num_kv_heads, 0).reshape(-1)) - it[:, 3]
         order = np.argsort(-length, kind="stable")
         run = max(1, workgroup_slots // 2)
-        turned = (np.arange(order.size) // run) % 2 == 1
+        turned = ((np.arange(order.size) // run) % 2 == 1) & (slots_a_unit > 1)
         place = np.arange(order.size)
         run_first = place // run * run
         run_last = np.minimum(run_first + run, order.size) - 1

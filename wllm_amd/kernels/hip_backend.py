@@ -10,7 +10,7 @@ from ctypes import c_float, c_int, c_longlong, c_void_p
 import numpy as np
 import torch
 
-from wllm_amd.kernels.attention_plan import AttentionPlan, build_work_items, count_tile_items
+from wllm_amd.kernels.attention_plan import PROMPT_ROWS, AttentionPlan, build_work_items, count_tile_items, prompt_kernel_pays
 from wllm_amd.kernels import ops
 from wllm_amd.kernels.ops import gate_args
 from wllm_amd.kernels.library import load
@@ -59,6 +59,9 @@ _SIGNATURES = {
     "wllm_paged_attention_prefill": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p,
                                      c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                      c_int, c_float, c_int, c_void_p, c_void_p],
+    "wllm_paged_attention_prompt": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                    c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                                    c_int, c_float, c_int, c_void_p, c_void_p],
     "wllm_gemm_tile": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float,
                        c_void_p],
     "wllm_gemm_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
@@ -202,8 +205,13 @@ class HipBackend:
         if not self.mfma_attention_takes(dtype, head_dim, page_size):
             return None
         group, slots_of_device = num_heads // num_kv_heads, self._workgroup_slots(device)
-        items, reduces, slots, prefill, prefill_rows = build_work_items(
-            host_q_len, host_ctx_len, group, num_kv_heads, window, page_size, workgroup_slots=slots_of_device)
+        if (dtype == torch.bfloat16 and head_dim == 256 and page_size >= 16 and page_size & (page_size - 1) == 0
+                and prompt_kernel_pays(host_q_len, host_ctx_len, group, num_kv_heads, window)):
+            items, reduces, slots, prefill, prefill_rows = build_work_items(
+                host_q_len, host_ctx_len, group, num_kv_heads, window, page_size, PROMPT_ROWS, slots_of_device // 2, slots_a_unit=1)
+        else:
+            items, reduces, slots, prefill, prefill_rows = build_work_items(
+                host_q_len, host_ctx_len, group, num_kv_heads, window, page_size, workgroup_slots=slots_of_device)
         if dtype == torch.float32 and prefill.shape[0] and \
                 count_tile_items(host_q_len, host_ctx_len, group, num_kv_heads, window) * head_dim < self.F32_TILE_WORK:
             # float32 and little work: tiles of 16 rows fill the device better than the blocks of 64 rows would
@@ -276,7 +284,8 @@ class HipBackend:
                     "paged_attention (matrix cores, float32)")
                 return
             if plan.num_prefill:
-                self._check(self.lib.wllm_paged_attention_prefill(
+                prefill = self.lib.wllm_paged_attention_prompt if plan.prefill_rows == PROMPT_ROWS else self.lib.wllm_paged_attention_prefill
+                self._check(prefill(
                     _ptr(qkv), _ptr(cache), _ptr(block_tables), _ptr(plan.prefill_items), plan.num_prefill,
                     plan.prefill_rows,
                     _ptr(seg_q_start), _ptr(seg_q_len), _ptr(seg_ctx_len), _ptr(out), _ptr(plan.partial_o),
