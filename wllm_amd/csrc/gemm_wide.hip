@@ -2,27 +2,8 @@
 // form out[M, I] = act(x . Wg^T) * (x . Wu^T) with w = [Wg; Wu], whose activation and product are made in
 // the registers the sums are in, so that only [M, I] is written.
 //
-// A workgroup of eight wavefronts makes a tile of 256 rows of x by 256 rows of w (gated: 128 gate rows and
-// the 128 up rows that belong to them).  The tile is two halves of 128 rows of x by two halves of 128 rows
-// of w; wavefront (wm, wn) of the 2 x 4 makes, of each of the four quarters, the 64 x 32 at (64 wm, 32 wn),
-// as products v_mfma_f32_16x16x32_bf16 (w is the A operand, x the B operand: lane (i, g) ends with four
-// consecutive columns of one output row).  In the gated form a lane so holds a column's gate and up sums.
-//
-// The K axis is walked in stages of 64 keys, two stages of 64 KB in shared memory.  A stage's halves (16 KB
-// each) go there straight from memory (global_load_lds_dwordx4, 8 rows of 8 chunks of 16 bytes a load;
-// chunk c of row r lies at place c ^ (r % 8) of its row, so that the reads of a fragment meet no bank
-// twice).  The two wavefronts of a vector unit (wave and wave + 4) work half a step apart: while one reads
-// fragments and sends loads, the other has the matrix cores for 32 products.  The step of one stage:
-//   A  read both w halves and the first x half; send the second x half of the next stage
-//   B  32 products (first x half)
-//   C  read the second x half; send the first x half and both w halves of the stage after the next
-//   D  32 products (second x half)
-// with a barrier after each; the second group of wavefronts is one barrier behind the first.  Why the
-// buffers are safe: a half is sent over only after a barrier that follows the last read of it by either group
-// (each waits for its reads before the barrier that ends A and C), and it is read only after a barrier that
-// follows both groups' wait for their loads of it: in front of a read at most 8 newer loads a lane may be
-// on their way (vmcnt counts in order), which is what the order of sending leaves.  A load has about
-// a stage and a half to arrive.
+// A workgroup of eight wavefronts makes tiles of 256 rows of x by 256 rows of w (gated: 128 gate rows and the 128 up rows that
+// belong to them, so that a lane holds a column's gate and up sums), as `wide_tile.h` says.
 //
 // A launch has at most a workgroup a compute unit; each takes items (tile, piece of the K axis) one after
 // the other, and sends the first stages of its next item before it writes the results of the last.  The items
@@ -39,44 +20,11 @@
 //
 // `splits` > 1 leaves float32 partial sums [splits, M, N], for the consumer to add in order.  Every output element
 // is summed over k in ascending order within a piece; pieces depend on K and `splits` alone.
-#include "common.h"
+#include "wide_tile.h"
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
-constexpr int kWideRows = 256;                       // rows of x, and rows of w, a tile
-constexpr int kWideHalf = kWideRows / 2;
-constexpr int kWideKeys = 64;                        // keys a stage
-constexpr int kHalfBytes = kWideHalf * kWideKeys * 2;
-constexpr int kWideStage = 4 * kHalfBytes;           // x halves, w halves
-constexpr int kWideShared = 2 * kWideStage;
-
-union WFrag {
-    uint4 u;
-    bf16x8_t v;
+struct WideItem {
+    int m_base, n_base, piece;
 };
-
-// 16 bytes a lane from base + offset into shared memory at `lds_address` + 16 * lane.  M0 is put back as it
-// was: naming it as clobbered instead makes the compiler wait for every load in flight before the
-// next read of shared memory.  The compiler does not see these loads; the kernel waits for them itself.
-static __device__ __forceinline__ void load_to_shared(const void* base, uint32_t offset, uint32_t lds_address) {
-    uint32_t saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0) : "v"(offset), "s"(base), "s"(lds_address) : "memory");
-}
-
-// Until at most N of this lane's loads into shared memory are on their way.
-template <int N>
-static __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
-static __device__ __forceinline__ void wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-// A barrier that nothing is moved across (the products before it stay before it, and the reads behind it behind).
-static __device__ __forceinline__ void meet() {
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-}
 
 // GATED: 0 plain, 1 + the gate's number for the gated product.  N is the number of rows of w (plain) or of gate rows
 // (gated); `stride` elements from a row of `out` to the next.  `vectors`: rows of `out` begin at multiples of 16 bytes.
@@ -86,168 +34,59 @@ gemm_wide_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* _
                  int M, int N, int K, int stride, bool vectors, int m_tiles, int n_tiles, int splits, GateShape shape) {
     constexpr int kColumns = GATED ? kWideHalf : kWideRows;         // output columns a tile
     constexpr bool kPair = GATED == kGatePairSquaredRelu + 1;
-    extern __shared__ __align__(16) unsigned char tiles_s[];        // [2 stages][x half, x half, w half, w half]
+    extern __shared__ __align__(16) unsigned char tiles_s[];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = lane % 16, g = lane / 16;
-    const int wm = wave / 4, wn = wave % 4;                          // wm is also the group: waves of one vector unit are 4 apart
+    const int wm = wave / 4, wn = wave % 4;
 
     const int tiles = m_tiles * n_tiles, items = tiles * splits, all_stages = K / kWideKeys;
     const int xcd = blockIdx.x % 8, per_xcd = items / 8, left = items % 8;
     const int first = xcd * per_xcd + min(xcd, left), end = first + per_xcd + (xcd < left ? 1 : 0);
-    const int step = gridDim.x / 8;
-    int item = first + blockIdx.x / 8;
-    if (item >= end) return;
+    if (first + static_cast<int>(blockIdx.x) / 8 >= end) return;
 
-    const int chunk = (lane % 8) ^ (lane / 8);
-    const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
-        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)tiles_s)));
-    uint32_t offset[4][2];      // what this lane brings of each half: rows 8 (wave + 8 u) + lane / 8
-    int m_base, n_base, piece, stages;
-    const unsigned char *x_bytes, *w_bytes;
-    auto place_item = [&](int it) {
-        piece = it / tiles;
-        const int t = it - piece * tiles;
+    auto place = [&](int it, WideSource& from) {
+        WideItem at;
+        at.piece = it / tiles;
+        const int t = it - at.piece * tiles;
         const int band = t / (8 * n_tiles), in_band = t - band * 8 * n_tiles;
         const int band_rows = min(8, m_tiles - 8 * band);
         const int n_tile = in_band / band_rows;
-        m_base = (8 * band + in_band - n_tile * band_rows) * kWideRows;
-        n_base = n_tile * kColumns;
-        const int begin = static_cast<int>(static_cast<long long>(piece) * all_stages / splits);
-        stages = static_cast<int>(static_cast<long long>(piece + 1) * all_stages / splits) - begin;
-        x_bytes = reinterpret_cast<const unsigned char*>(x) + static_cast<size_t>(begin) * (kWideKeys * 2);
-        w_bytes = reinterpret_cast<const unsigned char*>(w) + static_cast<size_t>(begin) * (kWideKeys * 2);
+        at.m_base = (8 * band + in_band - n_tile * band_rows) * kWideRows;
+        at.n_base = n_tile * kColumns;
+        const int begin = static_cast<int>(static_cast<long long>(at.piece) * all_stages / splits);
+        from.stages = static_cast<int>(static_cast<long long>(at.piece + 1) * all_stages / splits) - begin;
+        from.two = true;
+        from.x_bytes = reinterpret_cast<const unsigned char*>(x) + static_cast<size_t>(begin) * (kWideKeys * 2);
+        from.w_bytes = reinterpret_cast<const unsigned char*>(w) + static_cast<size_t>(begin) * (kWideKeys * 2);
 #pragma unroll
         for (int h = 0; h < 4; ++h)
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                const int r = 8 * (wave + 8 * u) + lane / 8;
+                const int r = wide_row(u);
                 size_t row;
-                if (h < 2) row = min(m_base + kWideHalf * h + r, M - 1);
-                else if (GATED) row = static_cast<size_t>(min(n_base + r, N - 1)) + (h == 3 ? N : 0);
-                else row = min(n_base + kWideHalf * (h - 2) + r, N - 1);
-                offset[h][u] = static_cast<uint32_t>((row * K + chunk * 8) * 2);
+                if (h < 2) row = min(at.m_base + kWideHalf * h + r, M - 1);
+                else if (GATED) row = static_cast<size_t>(min(at.n_base + r, N - 1)) + (h == 3 ? N : 0);
+                else row = min(at.n_base + kWideHalf * (h - 2) + r, N - 1);
+                from.offset[h][u] = static_cast<uint32_t>((row * K + wide_chunk() * 8) * 2);
             }
+        return at;
     };
-    auto send = [&](int h, int s) {
-        const unsigned char* base = (h < 2 ? x_bytes : w_bytes) + static_cast<size_t>(s) * (kWideKeys * 2);
-        const uint32_t to = lds_base + (s & 1) * kWideStage + h * kHalfBytes + wave * 1024;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) load_to_shared(base, offset[h][u], to + u * 8192);
-    };
-    auto send_first = [&] {
-        send(0, 0);
-        send(2, 0);
-        send(3, 0);
-        send(1, 0);
-        if (stages > 1) {
-            send(0, 1);
-            send(2, 1);
-            send(3, 1);
-        }
-    };
-
-    WFrag fx[4][2], fw[2][2][2];         // [16 rows of the x half][32 keys], [w half][16 rows][32 keys]
-    const int place0 = (g ^ (i % 8)) * 16, place1 = ((4 + g) ^ (i % 8)) * 16;
-    auto read_x = [&](int s, int h) {
-        const unsigned char* p = tiles_s + (s & 1) * kWideStage + h * kHalfBytes + (wm * 64 + i) * 128;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            fx[b][0].u = *reinterpret_cast<const uint4*>(p + b * 2048 + place0);
-            fx[b][1].u = *reinterpret_cast<const uint4*>(p + b * 2048 + place1);
-        }
-    };
-    auto read_w = [&](int s, int h) {
-        const unsigned char* p = tiles_s + (s & 1) * kWideStage + (2 + h) * kHalfBytes + (wn * 32 + i) * 128;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            fw[h][a][0].u = *reinterpret_cast<const uint4*>(p + a * 2048 + place0);
-            fw[h][a][1].u = *reinterpret_cast<const uint4*>(p + a * 2048 + place1);
-        }
-    };
-
-    place_item(item);
-    send_first();
-    for (;;) {
-        float4_t acc[2][2][2][4];        // [x half][w half][16 rows of w][16 rows of x]
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int c = 0; c < 2; ++c)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) acc[a][b][c][d] = float4_t{0.f, 0.f, 0.f, 0.f};
-        auto products = [&](int xh) {
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int wh = 0; wh < 2; ++wh)
-#pragma unroll
-                for (int k = 0; k < 2; ++k)
-#pragma unroll
-                    for (int a = 0; a < 2; ++a)
-#pragma unroll
-                        for (int b = 0; b < 4; ++b)
-                            acc[xh][wh][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[wh][a][k].v, fx[b][k].v,
-                                                                                        acc[xh][wh][a][b], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
-        };
-        const int n_stages = stages;
-        if (n_stages > 1) wait_loads<8>();         // stage 0's first x half and w halves, 3 of the 7 halves sent, and more
-        else wait_loads<0>();
-        meet();
-        if (wm == 1) meet();
-        for (int s = 0; s < n_stages; ++s) {
-            read_w(s, 0);
-            read_x(s, 0);
-            read_w(s, 1);
-            if (s + 1 < n_stages) {
-                send(1, s + 1);
-                wait_loads<8>();                   // behind x's second half of this stage: the next stage's four halves
-            } else {
-                wait_loads<0>();
-            }
-            wait_reads();
-            meet();
-            products(0);
-            meet();
-            read_x(s, 1);
-            if (s + 2 < n_stages) {
-                send(0, s + 2);
-                send(2, s + 2);
-                send(3, s + 2);
-                wait_loads<8>();                   // behind the next stage's first three halves: its fourth, and these three
-            } else {
-                wait_loads<0>();
-            }
-            wait_reads();
-            meet();
-            products(1);
-            meet();
-        }
-        if (wm == 0) meet();                       // every wavefront is done with the shared memory
-
-        const int m_now = m_base, n_now = n_base, piece_now = piece;
-        item += step;
-        const bool again = item < end;
-        if (again) {
-            place_item(item);
-            send_first();
-        }
-        // ---- lane (i, g) holds, of quarter (xh, wh) and tile (a, b), output row 16 b + i and columns 4g .. 4g + 3 ----
+    // lane (i, g) holds, of quarter (xh, wh) and tile (a, b), output row 16 b + i and columns 4g .. 4g + 3
+    auto finish = [&](const WideItem& at, const WideSums& acc) {
 #pragma unroll
         for (int xh = 0; xh < 2; ++xh)
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                const int m = m_now + xh * kWideHalf + wm * 64 + 16 * b + i;
+                const int m = at.m_base + xh * kWideHalf + wm * 64 + 16 * b + i;
                 if (m >= M) continue;
                 if (!GATED && partial != nullptr) {
-                    float* row = partial + (static_cast<size_t>(piece_now) * M + m) * N;
+                    float* row = partial + (static_cast<size_t>(at.piece) * M + m) * N;
 #pragma unroll
                     for (int wh = 0; wh < 2; ++wh)
 #pragma unroll
                         for (int a = 0; a < 2; ++a) {
-                            const int n = n_now + wh * kWideHalf + wn * 32 + 16 * a + 4 * g;
+                            const int n = at.n_base + wh * kWideHalf + wn * 32 + 16 * a + 4 * g;
                             if (n + 3 < N && N % 4 == 0) {
                                 *reinterpret_cast<float4_t*>(row + n) = acc[xh][wh][a][b];
                             } else {
@@ -275,16 +114,12 @@ gemm_wide_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* _
                         q[a][0] = pack2_bf16(r[0], r[1]);
                         q[a][1] = pack2_bf16(r[2], r[3]);
                     }
-                    // the lanes g and g + 1 (g even) exchange, so that each holds eight neighbouring columns: of the 32, the
-                    // even lane 8 (g / 2) .. + 7, the odd one those 16 further on
-                    typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
-                    const uint2_t lo = __builtin_amdgcn_permlane16_swap(q[0][0], q[1][0], false, false);
-                    const uint2_t hi = __builtin_amdgcn_permlane16_swap(q[0][1], q[1][1], false, false);
-                    const int n = n_now + (GATED ? 0 : wh * kWideHalf) + wn * 32 + 16 * (g & 1) + 8 * (g >> 1);
+                    const uint4 columns = wide_eight_columns(q);
+                    const int n = at.n_base + (GATED ? 0 : wh * kWideHalf) + wn * 32 + 16 * (g & 1) + 8 * (g >> 1);
                     bf16* to = row + (kPair && wh == 1 ? N : 0) + n;
-                    const uint32_t words[4] = {lo.x, hi.x, lo.y, hi.y};
+                    const uint32_t words[4] = {columns.x, columns.y, columns.z, columns.w};
                     if (vectors && n + 7 < N) {
-                        *reinterpret_cast<uint4*>(to) = make_uint4(words[0], words[1], words[2], words[3]);
+                        *reinterpret_cast<uint4*>(to) = columns;
                     } else {
 #pragma unroll
                         for (int v = 0; v < 8; ++v)
@@ -292,8 +127,8 @@ gemm_wide_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* _
                     }
                 }
             }
-        if (!again) break;
-    }
+    };
+    wide_products<false>(tiles_s, first + blockIdx.x / 8, end, gridDim.x / 8, place, finish);
 }
 
 // out[M, N] = x . w^T (gated 0, w [N, K]), or the gated product (gated = 1 + the gate's number, with limit, slope and

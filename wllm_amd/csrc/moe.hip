@@ -509,220 +509,3 @@ WLLM_API int wllm_moe_down(const void* act, const void* w, const void* tiles, co
 #undef LAUNCH_MT
     return launch_status();
 }
-
-// ---- many rows an expert: the two products in tiles of 128 rows of one expert by 128 rows of its weights,
-// through shared memory, as the framework's tiled product does it (four wavefronts of 64 x 64, stages of 64 keys
-// that go from memory straight into shared memory in an XOR-swizzled order, two stages in turn, two workgroups a
-// compute unit).  What differs: a tile's rows of x are gathered (row r of tile t is the assignment the plan names:
-// the token's row of x for the first product, the assignment's row of act for the second), the weights are the
-// tile's expert's, and a row's result goes where its assignment belongs.  A row's sums run over k in ascending
-// stages whatever tile it lies in.
-// bfloat16; K a multiple of 64. ----
-constexpr int kBigRows = 128;
-constexpr int kBigKeys = 64;
-constexpr int kBigRowBytes = kBigKeys * 2;
-constexpr int kBigStageBytes = 2 * kBigRows * kBigRowBytes;
-// An XCD's workgroups (indices equal modulo 8) take areas of kAreaRows tiles of rows by kAreaColumns tiles of columns one
-// after the other, so that they share their rows of x and of w in its L2: the sixty-four that an XCD runs at once
-// then read some 14 MB a pass over K where one column of tiles at a time made them read 39 (every tile's rows of x, and
-// nearly every expert's rows of w), which the fabric behind the L2s had to bring for all eight XCDs.  Eight areas go at a
-// time, one an XCD; those left over are shared out tile by tile, unless all areas run at once, two an XCD (700 tokens of the
-// sizes below: 14 areas, the second product 88 us, 97 shared out; but 3 areas 31 and 30).  A column of tiles at a time against that, us, 16 experts
-// of 4,096 behind a width of 2,048, three a token (first product; second): 1,000 tokens 208, 204; 93, 94; 2,048 342, 327; 185,
-// 173; 3,001 472, 454; 269, 246; 7,777 1,105, 1,079; 589, 519; four a token, 1,000 (where whole areas would give some XCDs a half
-// more: 166 in the second) 244, 240; 159, 154.
-constexpr int kAreaRows = 4, kAreaColumns = 8, kAreaTiles = kAreaRows * kAreaColumns, kAreasAtOnce = 16;
-
-// The tile of workgroup `index` among `rows` tiles of rows by any number of columns of which `across` areas (the last one
-// may reach beyond them) make a band; `across` 0: a column of tiles at a time, eight columns side by side.
-__host__ __device__ __forceinline__ void tile_of(int index, int rows, int across, int& row, int& column) {
-    const int xcd = index % 8, turn = index / 8;
-    if (across == 0) {
-        row = turn % rows;
-        column = turn / rows * 8 + xcd;
-        return;
-    }
-    const int areas = (rows + kAreaRows - 1) / kAreaRows * across;
-    const bool at_once = areas > 8 && areas <= kAreasAtOnce;
-    const int dealt = at_once ? kAreasAtOnce / 8 * kAreaTiles : areas / 8 * kAreaTiles;                // turns that deal whole areas
-    const int share = at_once ? 0 : areas % 8 * (kAreaTiles / 8), place = turn < dealt ? turn % kAreaTiles : xcd * share + turn - dealt;
-    if (turn >= dealt + share) {
-        row = rows;                                                                                      // no tile
-        column = 0;
-        return;
-    }
-    const int area = turn < dealt ? turn / kAreaTiles * 8 + xcd : areas / 8 * 8 + place / kAreaTiles;
-    row = area / across * kAreaRows + place % kAreaRows;
-    column = area % across * kAreaColumns + place % kAreaTiles / kAreaRows;
-}
-
-union MoeTFrag {
-    uint4 u;
-    bf16x8_t v;
-};
-
-// 16 bytes a lane from base + offset into shared memory at dst + 16 * lane (M0 is put back as it was).
-static __device__ __forceinline__ void moe_load_to_shared(const void* base, uint32_t offset, void* dst) {
-    const uint32_t lds_address = __builtin_amdgcn_readfirstlane(
-        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)dst)));
-    uint32_t saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0) : "v"(offset), "s"(base), "s"(lds_address) : "memory");
-}
-
-// GATED: 0 the second product (out32[a % top][a / top][n] = weight[a] * sum), 1 + the activation's number the
-// first (act[a][n] = activation(gate) * up; w holds an expert's N gate rows, then its N up rows).
-template <int GATED>
-__global__ void __launch_bounds__(256, 2)
-moe_tile_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const int* __restrict__ plan, int max_tiles,
-                bf16* __restrict__ act, float* __restrict__ out32, const float* __restrict__ weights, int N, int K, int top,
-                int tokens, int across) {
-    // (`weights`: of the second product the factor of a row's result, 1 if null; of the first the factor of a row's
-    // input, taken out of both sums, none if null)
-    constexpr int kWaves = 4, kStages = 2;
-    constexpr int kWBytes = kBigRows * kBigRowBytes;
-    constexpr int kLoads = 2 * kBigRows / 8 / kWaves;
-    extern __shared__ __align__(16) unsigned char tiles_s[];
-    const int lane = threadIdx.x % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int i = lane % 16, g = lane / 16;
-    const int wm = wave / 2, wn = wave % 2;
-    constexpr int kColumns = GATED ? kBigRows / 2 : kBigRows;
-    const int live = plan[0];
-    if (live <= 0) return;
-    int m_tile, n_tile;
-    tile_of(blockIdx.x, live, across, m_tile, n_tile);
-    const int n_base = n_tile * kColumns;
-    if (m_tile >= live || n_base >= N) return;
-    const int e = plan[1 + m_tile];
-    const int* rows = plan + 1 + max_tiles + m_tile * kBigRows;
-    const int stages = K / kBigKeys;
-    const bf16* we = w + static_cast<size_t>(e) * (GATED ? 2 : 1) * N * K;
-
-    const int chunk = (lane % 8) ^ (lane / 8);
-    uint32_t offset[kLoads];
-#pragma unroll
-    for (int u = 0; u < kLoads; ++u) {
-        const int r = 8 * (wave + kWaves * u) + lane / 8;
-        size_t row;
-        if (r < kBigRows) {
-            if (GATED) row = r < 64 ? min(n_base + r, N - 1) : N + min(n_base + r - 64, N - 1);
-            else row = min(n_base + r, N - 1);
-        } else {
-            const int a = rows[r - kBigRows];
-            row = a < 0 ? 0 : (GATED ? a / top : a);
-        }
-        offset[u] = static_cast<uint32_t>((row * K + chunk * 8) * 2);
-    }
-    const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(we);
-    const unsigned char* x_bytes = reinterpret_cast<const unsigned char*>(x);
-    auto issue = [&](int stage, int s) {
-        const unsigned char* wb = w_bytes + static_cast<size_t>(s) * kBigRowBytes;
-        const unsigned char* xb = x_bytes + static_cast<size_t>(s) * kBigRowBytes;
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int q = wave + kWaves * u;
-            moe_load_to_shared(q < kBigRows / 8 ? wb : xb, offset[u], tiles_s + stage * kBigStageBytes + q * 1024);
-        }
-    };
-
-    float4_t acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
-    int w_row_s[4], x_row_s[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        w_row_s[a] = GATED ? (a < 2 ? wn * 32 + 16 * a + i : 64 + wn * 32 + 16 * (a - 2) + i) : wn * 64 + 16 * a + i;
-        x_row_s[a] = wm * 64 + 16 * a + i;
-    }
-    issue(0, 0);
-    for (int s = 0; s < stages; ++s) {
-        const int stage = s % kStages;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (s + 1 < stages) issue((s + 1) % kStages, s + 1);
-        const unsigned char* ws = tiles_s + stage * kBigStageBytes;
-        const unsigned char* xs = ws + kWBytes;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int place = ((ks * 4 + g) ^ (i % 8)) * 16;
-            MoeTFrag fw[4], fx[4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                fw[a].u = *reinterpret_cast<const uint4*>(ws + w_row_s[a] * 128 + place);
-                fx[a].u = *reinterpret_cast<const uint4*>(xs + x_row_s[a] * 128 + place);
-            }
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[a].v, fx[b].v, acc[a][b], 0, 0, 0);
-        }
-    }
-
-    // lane (i, g) holds, of tile (a, b), the tile's row 16 b + i and columns 4g .. 4g + 3 of the tile's 16
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int asg = rows[wm * 64 + 16 * b + i];
-        if (asg < 0) continue;
-        if (GATED) {
-            bf16* o_row = act + static_cast<size_t>(asg) * N;
-            const float scale = weights ? weights[asg] : 1.f;
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                const int n = n_base + wn * 32 + 16 * a + 4 * g;
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (n + v < N)
-                        o_row[n + v] = from_float<bf16>(activate<(GATED > 0 ? GATED - 1 : 0)>(acc[a][b][v] * scale) *
-                                                        (acc[a + 2][b][v] * scale));
-            }
-        } else {
-            const float weight = weights ? weights[asg] : 1.f;
-            float* o_row = out32 + (static_cast<size_t>(asg % top) * tokens + asg / top) * N;
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const int n = n_base + wn * 64 + 16 * a + 4 * g;
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (n + v < N) o_row[n + v] = weight * acc[a][b][v];
-            }
-        }
-    }
-}
-
-// The first product (activation >= 0: `act` [assignments, N] from x [tokens, K] and w [experts, 2N, K]) or the second
-// (activation < 0: out32 [top, tokens, N] from x = act [assignments, K] and w [experts, N, K]) over a plan of tiles of
-// 128 rows.  Returns -1 for sizes it does not take (K no multiple of 64, operands of 4 GiB).
-WLLM_API int wllm_moe_tiles(const void* x, const void* w, const int* plan, int max_tiles, void* act, float* out32,
-                            const float* weights, int activation, int x_rows, int N, int K, int top, int tokens,
-                            hipStream_t stream) {
-    if (max_tiles <= 0 || x_rows <= 0) return 0;
-    if (N <= 0 || K < kBigKeys || K % kBigKeys || top <= 0 || tokens <= 0 || activation >= kActivations) return -1;
-    const bool gated = activation >= 0;
-    if ((gated && !act) || (!gated && !out32)) return -1;
-    if (static_cast<size_t>(gated ? 2 : 1) * N * K * 2 >= (size_t(1) << 32) || static_cast<size_t>(x_rows) * K * 2 >= (size_t(1) << 32))
-        return -1;
-    const int columns = gated ? kBigRows / 2 : kBigRows;
-    const int n_tiles = (N + columns - 1) / columns;
-    // (the first product of steps with less than one full tile an expert, whose areas share nothing of w, takes a column at a
-    // time: 16 experts of 4,096, three a token, 256 tokens 148 us in areas, 146 so; 448 156 and 153)
-    const bool few = gated && static_cast<long long>(tokens) * top <= 64LL * max_tiles;
-    const int across = few ? 0 : (n_tiles + kAreaColumns - 1) / kAreaColumns;
-    const long long areas = static_cast<long long>(across) * ((max_tiles + kAreaRows - 1) / kAreaRows);
-    const long long blocks = few ? (static_cast<long long>(n_tiles) + 7) / 8 * 8 * max_tiles
-                                 : (areas > 8 && areas < kAreasAtOnce ? kAreasAtOnce : areas) * kAreaTiles;
-    if (blocks > 0x7fffffffLL) return -1;
-    const dim3 grid(static_cast<unsigned>(blocks));
-    const bf16* xp = static_cast<const bf16*>(x);
-    const bf16* wp = static_cast<const bf16*>(w);
-#define LAUNCH(GATED)                                                                                                 \
-    moe_tile_kernel<GATED><<<grid, 256, 2 * kBigStageBytes, stream>>>(xp, wp, plan, max_tiles, static_cast<bf16*>(act), \
-                                                                      out32, weights, N, K, top, tokens, across)
-    if (!gated) { LAUNCH(0); }
-    else { WLLM_BY_ACTIVATION(activation, LAUNCH(ACT + 1)) }
-#undef LAUNCH
-    return launch_status();
-}

@@ -1406,7 +1406,7 @@ def delta_chunk_scan(qk: torch.Tensor, f: torch.Tensor, beta: torch.Tensor, v: t
 # ---- a mixture of experts ------------------------------------------------------------------------------
 MOE_TILE_ROWS = 16           # rows of a tile of the kernels that stream an expert's weights past a few rows: 16, 32 or 64
 MOE_STREAM_TILE_ROWS = (16, 32, 64)
-MOE_BIG_TILE_ROWS = 128      # rows of a tile of the kernel that tiles many rows an expert through shared memory
+MOE_BIG_TILE_ROWS = 128      # rows of a tile of the plan of the kernel that tiles many rows an expert through shared memory
 MOE_MAX_EXPERTS = 256
 
 
@@ -1795,14 +1795,20 @@ def _register_own() -> None:
                     p(weights if weighted else None), p(out), bf(act), weights.shape[0], act.shape[1], w.shape[1], weights.shape[1], stream))
     tiles = [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
              c_void_p]
-    register_op("moe_experts_up_tiled", entry_point="wllm_moe_tiles", argtypes=tiles,
-                launch=lambda fn, stream, x, w, plan, act, top, activation, in_weights=None: fn(
-                    p(x), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(act), p(None), p(in_weights),
-                    ACTIVATIONS[activation], x.shape[0], act.shape[1], x.shape[1], top, x.shape[0], stream))
-    register_op("moe_experts_down_tiled", entry_point="wllm_moe_tiles", argtypes=tiles,
-                launch=lambda fn, stream, act, w, plan, weights, out, weighted=True: fn(
-                    p(act), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(None), p(out),
-                    p(weights if weighted else None), -1, act.shape[0], w.shape[1], act.shape[1], weights.shape[1], weights.shape[0], stream))
+    def aligned(t):                 # the tiled kernel's loads are of 16 bytes; a view that begins elsewhere is copied
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+
+    def up_tiled(fn, stream, x, w, plan, act, top, activation, in_weights=None):
+        x, w = aligned(x), aligned(w)
+        return fn(p(x), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(act), p(None), p(in_weights),
+                  ACTIVATIONS[activation], x.shape[0], act.shape[1], x.shape[1], top, x.shape[0], stream)
+
+    def down_tiled(fn, stream, act, w, plan, weights, out, weighted=True):
+        act, w = aligned(act), aligned(w)
+        return fn(p(act), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(None), p(out),
+                  p(weights if weighted else None), -1, act.shape[0], w.shape[1], act.shape[1], weights.shape[1], weights.shape[0], stream)
+    register_op("moe_experts_up_tiled", entry_point="wllm_moe_wide", argtypes=tiles, launch=up_tiled)
+    register_op("moe_experts_down_tiled", entry_point="wllm_moe_wide", argtypes=tiles, launch=down_tiled)
 
 
 _register_own()
