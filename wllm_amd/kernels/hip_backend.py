@@ -66,6 +66,8 @@ _SIGNATURES = {
                        c_void_p],
     "wllm_gemm_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                        c_float, c_void_p],
+    "wllm_gemm_stream": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
+                         c_float, c_void_p],
     "wllm_split_sum": [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
     "wllm_gemm_generic": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p],
     "wllm_tile_weight_f32": [c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -483,13 +485,30 @@ class HipBackend:
             return False
         return 1 < splits <= 16 and (rows <= 16 or n <= 8192 and (rows <= 32 or rows <= 64 and splits == 2))
 
+    # The kernel of at most 64 rows that brings everything through shared memory (`gemm_stream.hip`, which has the figures): split
+    # sums that the caller adds or a second launch, and gated products of more rows than two tiles of 16.  Its loads are of 16 bytes.
+    @staticmethod
+    def stream_takes(x_address: int, w_address: int, rows: int, w_rows: int, k: int, splits: int) -> bool:
+        return (x_address | w_address) % 16 == 0 and k % (64 * splits) == 0 and rows <= 64 and w_rows * k < 1 << 31
+
     def _skinny(self, x, weight, out, tiles=None) -> None:
         m, k = x.shape
         n = weight.shape[0]
         splits = self.skinny_split(n, k)
-        chunk = self.SKINNY_CHUNK[min(4, -(-m // 16))]
         w, tiled = (tiles, 1) if tiles is not None else (weight, 0)
-        if out.dim() == 3:      # the caller adds the partial sums later
+        whole = out.dim() == 2
+        if splits > 1 and not (whole and self.joined_takes(m, n, splits, k)):
+            px, pw = x.data_ptr(), w.data_ptr()
+            if self.stream_takes(px, pw, m, n, k, splits):
+                sums = self._gemm_partial(splits * m * n, x.device) if whole else out
+                self._check(self.lib.wllm_gemm_stream(px, pw, tiled, None, sums.data_ptr(), m, n, k, n, splits, 0, 0.0, 0.0, 0.0,
+                                                      self._stream()), "linear (at most 64 rows, partial sums)")
+                if whole:
+                    self._check(self.lib.wllm_split_sum(_ptr(sums), _ptr(out), int(out.dtype == torch.bfloat16), m * n, splits,
+                                                        self._stream()), "linear (sum of partial sums)")
+                return
+        chunk = self.SKINNY_CHUNK[min(4, -(-m // 16))]
+        if not whole:           # the caller adds the partial sums later
             self._check(self.lib.wllm_gemm_skinny(_ptr(x), _ptr(w), tiled, c_void_p(0), 0, _ptr(out), m, n, k, splits,
                                                   chunk, self._stream()), "linear (few rows, partial sums)")
             return
@@ -601,6 +620,13 @@ class HipBackend:
         self._on_gpu(x, weight, out, scratch, tiles)
         m, k = x.shape
         w, tiled = (tiles, 1) if tiles is not None else (weight, 0)
+        if 32 < m <= 64 and x.dtype == torch.bfloat16:
+            px, pw, n = x.data_ptr(), w.data_ptr(), out.shape[1]
+            if self.stream_takes(px, pw, m, 2 * n, k, 2):
+                number, *shape = gate_args(activation)
+                self._check(self.lib.wllm_gemm_stream(px, pw, tiled, out.data_ptr(), None, m, n, k, out.stride(0), 1, 1 + number, *shape,
+                                                      self._stream()), "gated_linear (at most 64 rows)")
+                return
         if self.skinny_takes(x.dtype, m, k) and k % 64 == 0:
             self._check(self.lib.wllm_gemm_skinny_gated(
                 _ptr(x), _ptr(w), tiled, _ptr(out), m, out.shape[1], k, *gate_args(activation),
@@ -635,8 +661,12 @@ class HipBackend:
         # the kernels that make a gated product's two streams make the two halves of these columns
         if name == "squared_relu" and n % 2 == 0 and x.dtype == torch.bfloat16:
             number = len(ops.ACTIVATIONS) + 1
+            w, tiled = (paired_tiles, 1) if paired_tiles is not None else (weight, 0)
+            if 32 < m and self.stream_takes(x.data_ptr(), w.data_ptr(), m, n, k, 2):
+                self._check(self.lib.wllm_gemm_stream(_ptr(x), _ptr(w), tiled, _ptr(out), None, m, half, k, n, 1, 1 + number, 0.0, 0.0,
+                                                      0.0, self._stream()), "activated_linear (at most 64 rows)")
+                return
             if self.skinny_takes(x.dtype, m, k) and k % 64 == 0 and out.data_ptr() % 8 == 0:
-                w, tiled = (paired_tiles, 1) if paired_tiles is not None else (weight, 0)
                 self._check(self.lib.wllm_gemm_skinny_gated(
                     _ptr(x), _ptr(w), tiled, _ptr(out), m, half, k, number, 0.0, 0.0, 0.0, self.GATED_CHUNK[-(-m // 16)], n,
                     self._stream()), "activated_linear (few rows, matrix cores)")

@@ -17,9 +17,11 @@ def project(ctx, name: str, x: torch.Tensor, weight: torch.Tensor, out: Optional
     n, width = x.shape[0], weight.shape[0]
     splits = ops.linear_splits(n, width, x.shape[1], x.dtype)
     if splits > 1:
-        # (without room for the stack the kernels make the whole sum)
-        stack = ops.scratch_or_none(lambda: ctx.buffer(name + "_parts", (splits, n, width), torch.float32))
-        if stack is not None:
+        try:
+            stack = ctx.buffer(name + "_parts", (splits, n, width), torch.float32)
+        except torch.OutOfMemoryError:
+            pass        # without room for the stack the kernels make the whole sum
+        else:
             ops.linear(x, weight, stack, tiles)
             return stack
     if out is None:
