@@ -11,9 +11,10 @@
 // columns 16.3 us against 13.9 at 64 rows, to 2 x 24,576 of 3,072 keys 56.9 against 54.0.
 //
 // Measured, us, the few-row kernels and this one: gated, 2,048 keys to 2 x 16,384 columns, 40 / 64 rows 28.3 / 33.2 and 25.8 / 26.0 (5.2 TB/s);
-// 3,072 keys to 2 x 24,576 63.3 / 74.1 and 51.3 / 54.0; 16,384 keys to 2,048 columns in 16 pieces at 1 / 24 / 64 rows 13.0 / 15.1 / 18.3 and
-// 11.7 / 12.5 / 13.9; 24,576 to 3,072 at 17 / 64 rows 29.0 / 37.5 and 24.4 / 29.1.  At 32 rows and below the gated few-row kernel is as fast (24 rows 25.8 and
+// 3,072 keys to 2 x 24,576 63.3 / 74.1 and 51.3 / 54.0; plain, 3,072 keys to 12,288 columns in two pieces at 8 / 24 / 64 rows 15.2 / 17.4 / 21.7 and
+// 14.7 / 15.1 / 17.2; 1,024 to 16,384 8.9 / 9.5 / 11.8 and 8.3 / 8.8 / 10.0.  At 32 rows and below the gated few-row kernel is as fast (24 rows 25.8 and
 // 25.5; 8 rows 24.8 and 26.3), and so many columns that no K axis is cut belong to the unsplit one (256,000 columns, 64 rows: 199 and 214).
+// Fewer columns belong to the kernel that leaves fewer pieces (`gemm_pieces.hip`).
 //
 // A wavefront brings and reads its own two bands, so only x is waited for together: one barrier a stage, behind which
 // the buffer of the stage before is free as well.  w is read from its tile-major copy (`wllm_tile_weight`: a band's 16 rows by 32

@@ -73,6 +73,7 @@ _SIGNATURES = {
     "wllm_tile_weight_f32": [c_void_p, c_void_p, c_int, c_int, c_void_p],
     "wllm_gemm_f32_segments": [c_int, c_int, c_int],
     "wllm_argmax_rows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
+    "wllm_gemm_pieces": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "wllm_gemm_skinny": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int,
                          c_void_p],
     "wllm_sample_rows": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -339,6 +340,28 @@ class HipBackend:
             splits *= 2
         return splits
 
+    # The kernel whose wavefronts meet (`gemm_pieces.hip`, which has the figures).  Where a split product goes to a consumer as a
+    # stack of partial sums: (pieces of the K axis, bands of 16 columns a workgroup), or (0, 0).  A workgroup a compute unit at
+    # most: its time goes by its bytes of w, at about 26 KB a us, and by x, which several workgroups read (half its bytes, at 24 rows);
+    # every piece costs the consumer 0.6 us a launch (a norm of 8 to 64 rows after a product 2.4 us with 2 pieces, 3.2 with 4, 4.3 with
+    # 8, 6.6 with 16).  A function of the weight's shape only, so that a row's sum does not depend on the rows beside it.
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def piece_split(n: int, k: int) -> tuple:
+        best, least = (0, 0), None
+        if HipBackend.skinny_split(n, k) == 1 or (n + 15) * k >= 1 << 31 or k >= 1 << 24:
+            return best
+        for bands in (1, 2, 3):
+            groups, pieces = -(-n // (16 * bands)), 2
+            while groups * pieces <= HipBackend.COMPUTE_UNITS and k % (64 * pieces) == 0 and k // pieces >= 256 and pieces <= 16:
+                cost = (16 * bands + 12) * 2 * (k // pieces) / 26000 + 0.6 * pieces
+                if least is None or cost < least:
+                    best, least = (pieces, bands), cost
+                pieces *= 2
+        if least is None and n <= 48 * HipBackend.COMPUTE_UNITS and k <= 2048 and k % 128 == 0 and k >= 512:
+            best = (2, 3)       # two workgroups a compute unit: 2,048 keys to 10,304 columns 10.1 / 13.9 to 8.9 / 15.0 us, with the norm 22.4 / 29.4 to 20.7 / 28.6
+        return best
+
     # splits * N stays below 3072 * 16 by the rule of `skinny_split`; 64 rows of float32 of that
     GEMM_PARTIAL_FLOATS = 3072 * 16 * 64
 
@@ -454,7 +477,7 @@ class HipBackend:
 
     def linear_splits(self, rows, out_features, in_features, dtype) -> int:
         if self.skinny_takes(dtype, rows, in_features):
-            return self.skinny_split(out_features, in_features)
+            return self.piece_split(out_features, in_features)[0] or self.skinny_split(out_features, in_features)
         if dtype == torch.bfloat16 and self.wide_splits(out_features, in_features, rows) > 1:
             return self.wide_splits(out_features, in_features, rows)
         if self.tile_takes(dtype, rows, out_features, in_features):
@@ -480,13 +503,14 @@ class HipBackend:
         at 8 rows, 10.3 against 7.2 at 24, but to 2,048 columns 10.9 against 12.2 at 64; to 10,304 columns 13.9
         against 11.1 at 8 and 15.8 against 16.3 at 24; in two pieces (768 keys to 2,048 columns) 9.9 against 6.7 at 64.
         And with more keys, to 2,048 columns: at 8 rows of 8,192 keys 13.1 against 11.3, of 12,288 14.7 against 16.5; at 16 of
-        6,144 12.3 against 11.5, of 8,192 13.4 against 14.0; at 24 of 4,096 12.0 against 11.3, of 6,144 12.8 against 15.3."""
+        6,144 12.3 against 11.5, of 8,192 13.4 against 14.0; at 24 of 4,096 12.0 against 11.3, of 6,144 12.8 against 15.3.  (What
+        `piece_split` takes comes here only with operands at odd addresses, in its pieces.)"""
         if k > 8192 or rows * k > 98304:
             return False
         return 1 < splits <= 16 and (rows <= 16 or n <= 8192 and (rows <= 32 or rows <= 64 and splits == 2))
 
     # The kernel of at most 64 rows that brings everything through shared memory (`gemm_stream.hip`, which has the figures): split
-    # sums that the caller adds or a second launch, and gated products of more rows than two tiles of 16.  Its loads are of 16 bytes.
+    # sums of more columns than `piece_split` takes, and gated products of more rows than two tiles of 16.  Its loads are of 16 bytes.
     @staticmethod
     def stream_takes(x_address: int, w_address: int, rows: int, w_rows: int, k: int, splits: int) -> bool:
         return (x_address | w_address) % 16 == 0 and k % (64 * splits) == 0 and rows <= 64 and w_rows * k < 1 << 31
@@ -494,12 +518,29 @@ class HipBackend:
     def _skinny(self, x, weight, out, tiles=None) -> None:
         m, k = x.shape
         n = weight.shape[0]
-        splits = self.skinny_split(n, k)
+        pieces, bands = self.piece_split(n, k)
+        splits = pieces or self.skinny_split(n, k)
         w, tiled = (tiles, 1) if tiles is not None else (weight, 0)
         whole = out.dim() == 2
-        if splits > 1 and not (whole and self.joined_takes(m, n, splits, k)):
+        if splits > 1:
             px, pw = x.data_ptr(), w.data_ptr()
-            if self.stream_takes(px, pw, m, n, k, splits):
+            if pieces and (px | pw) % 16 == 0:
+                # A whole sum meets inside the workgroups, as many bands each as leave a compute unit one, or, of a long K axis, in a
+                # second launch.  us, inside and in two: 2,048 keys to 2,568 columns at 8 / 64 rows 5.1 / 7.8 and 6.7 / 8.9; 4,096 to 2,048
+                # 7.9 / 12.2 and 7.8 / 10.3; 5,632 to 2,048 at 8 / 24 rows 10.4 / 11.9 and 8.5 / 9.2.  (The kernels below: 4.9 / 11.1, 6.9 / 14.8 and 9.7 / 15.4.)
+                inside = whole and k < 4096
+                if inside:
+                    bands = min(3, -(-n // (16 * self.COMPUTE_UNITS)))
+                sums = self._gemm_partial(pieces * m * n, x.device) if whole and not inside else out
+                rounded = inside and out.dtype == torch.bfloat16
+                self._check(self.lib.wllm_gemm_pieces(px, pw, tiled, None if rounded else sums.data_ptr(),
+                                                      out.data_ptr() if rounded else None, m, n, k, pieces, inside, bands, self._stream()),
+                            "linear (at most 64 rows, wavefronts' sums joined)")
+                if whole and not inside:
+                    self._check(self.lib.wllm_split_sum(_ptr(sums), _ptr(out), int(out.dtype == torch.bfloat16), m * n, pieces,
+                                                        self._stream()), "linear (sum of partial sums)")
+                return
+            if not (whole and self.joined_takes(m, n, splits, k)) and self.stream_takes(px, pw, m, n, k, splits):
                 sums = self._gemm_partial(splits * m * n, x.device) if whole else out
                 self._check(self.lib.wllm_gemm_stream(px, pw, tiled, None, sums.data_ptr(), m, n, k, n, splits, 0, 0.0, 0.0, 0.0,
                                                       self._stream()), "linear (at most 64 rows, partial sums)")
