@@ -12,7 +12,7 @@
 //
 // Measured, us, the kernels before (registers, or four wavefronts on one stage of eight bands) and this one, product and norm together, 8 / 24 / 64 rows:
 // 2,048 keys to 2,048 columns 8.8 / 9.5 / 11.1 and 6.2 / 6.7 / 8.1; to 2,560 9.1 / 10.2 / 12.4 and 7.1 / 7.7 / 9.4; 4,096 to 2,048
-// 11.7 / 12.6 / 15.3 and 7.8 / 8.4 / 10.5; 5,632 to 2,048 13.5 / 14.3 / 18.2 and 8.8 / 9.4 / 11.9; 16,384 to 2,048 18.3 / 19.1 / 22.4 and
+// 11.7 / 12.6 / 15.3 and 7.8 / 8.5 / 10.3; 5,632 to 2,048 13.5 / 14.3 / 18.2 and 8.8 / 9.4 / 11.9; 16,384 to 2,048 18.3 / 19.1 / 22.4 and
 // 15.0 / 16.1 / 20.5 (the product alone 11.9 / 12.3 / 14.0 and 12.0 / 12.8 / 16.7); 24,576 to 3,072 30.5 / 31.4 / 35.6 and 27.8 / 28.7 / 35.8.
 // Row by row instead of the tile-major copy: 2,048 to 2,048 3.7 us alone against 4.3, but 16,384 to 2,048 16.2 against 12.4.
 //
