@@ -162,13 +162,17 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, offset: float, o
     read, x is left alone and out[i] belongs to row rows[i].
     """
     _dense(x, "x", torch.float32)
-    _need(x.dim() == 2, "x: expected [tokens, hidden]")
-    n, h = x.shape
+    shape = x.shape
+    if len(shape) != 2:
+        raise KernelShapeError("x: expected [tokens, hidden]")
+    n, h = shape
     _dense(weight, "weight", torch.float32, (h,))
     if delta is not None:
-        if delta.dim() == 3:
-            _dense(delta, "delta", torch.float32, (delta.shape[0], n, h))
-            _need(delta.shape[0] >= 1, "delta: an empty stack")
+        stack = delta.shape
+        if len(stack) == 3:
+            _dense(delta, "delta", torch.float32, (stack[0], n, h))
+            if stack[0] < 1:
+                raise KernelShapeError("delta: an empty stack")
         else:
             _dense(delta, "delta", _ACT, (n, h))
     m = n
@@ -566,8 +570,9 @@ def tile_weight(weight: torch.Tensor, halves: int = 1) -> Optional[torch.Tensor]
 def _check_tiles(tiles, weight, halves: int) -> None:
     if tiles is None:
         return
-    if weight.dtype is torch.bfloat16 and tiles.dtype is torch.bfloat16 and weight.shape[1] % 32 == 0 and tiles.dim() == 1 \
-            and tiles.is_contiguous() and tiles.shape[0] == halves * (-(-(weight.shape[0] // halves) // 16) * 16 * weight.shape[1]):
+    rows, k = weight.shape
+    if weight.dtype is torch.bfloat16 and tiles.dtype is torch.bfloat16 and k % 32 == 0 and tiles.dim() == 1 \
+            and tiles.is_contiguous() and tiles.shape[0] == halves * (-(-(rows // halves) // 16) * 16 * k):
         return
     if weight.dtype == torch.float32:
         _need(weight.shape[1] % 4 == 0, "tiles: float32 weights have them only with in_features % 4 == 0")
@@ -585,18 +590,24 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, tiles: Opti
     `tiles` is `tile_weight(weight)`, the same numbers in the order the few-row kernels read
     fastest; with it they read that copy instead."""
     _dense(x, "x", _ACT)
-    _need(x.dim() == 2, "x: expected [rows, in]")
-    _dense(weight, "weight", x.dtype)
-    if weight.dim() != 2 or weight.shape[1] != x.shape[1]:
-        raise KernelShapeError(f"weight: shape {tuple(weight.shape)}, expected [out, {x.shape[1]}]")
+    dtype, rows = x.dtype, x.shape      # (asked for once: a tensor makes a new shape for every question)
+    if len(rows) != 2:
+        raise KernelShapeError("x: expected [rows, in]")
+    _dense(weight, "weight", dtype)
+    wanted = weight.shape
+    if len(wanted) != 2 or wanted[1] != rows[1]:
+        raise KernelShapeError(f"weight: shape {tuple(wanted)}, expected [out, {rows[1]}]")
     _check_tiles(tiles, weight, 1)
+    m, k = rows
+    n = wanted[0]
     if out.dim() == 3:
-        s = linear_splits(x.shape[0], weight.shape[0], x.shape[1], x.dtype)
-        _dense(out, "out", torch.float32, (s, x.shape[0], weight.shape[0]))
-        _need(s > 1, "out: a stack of partial sums where the product is not split")
+        s = linear_splits(m, n, k, dtype)
+        _dense(out, "out", torch.float32, (s, m, n))
+        if s <= 1:
+            raise KernelShapeError("out: a stack of partial sums where the product is not split")
     else:
-        _dense(out, "out", (x.dtype, torch.float32), (x.shape[0], weight.shape[0]))
-    if x.shape[0]:
+        _dense(out, "out", (dtype, torch.float32), (m, n))
+    if m:
         backend().linear(x, weight, out, tiles)
 
 
