@@ -187,7 +187,10 @@ gemm_f32_few_rows_kernel(const float* __restrict__ x, const float* __restrict__ 
 // 4,096 x 4,096 x 4,096 ran at 109 TFLOP/s, every chunk a trip to memory).
 // SPLIT: a workgroup (blockIdx.z) takes `per_group` segments of the K axis and leaves each one's sum in
 // out[segment]; the kernel below adds them in the order in which the unsplit walk does.
-template <int WM, int WN, bool SPLIT>
+// PART: the last tile's blocks of 16 rows that lie beyond the rows are left out, a branch in front of each block's products.  A wavefront
+// has every second block, so that both halves of the workgroup get less to do (333 rows of 2,048 keys to 32,768 columns 423 to 400 us, 260 rows 421
+// to 352, 140 rows 231 to 192; 16,384 keys to 2,048 columns, 333 rows, 241 to 227).
+template <int WM, int WN, bool SPLIT, bool PART>
 __global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
                      int per_group) {
@@ -199,7 +202,9 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int i = lane % 16, g = lane / 16;
     const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const int wm0 = (wave / 2) * (TM / 2), wn0 = (wave % 2) * (TN / 2);
+    // a wavefront has every second block of 16 rows, so that the rows that the last tile has not are left out by both halves
+    const int wm0 = wave / 2 * 16, wn0 = (wave % 2) * (TN / 2);
+    const int live = __builtin_amdgcn_readfirstlane(min(WM, (M - m0 - wm0 + 31) / 32));       // of its blocks, those with rows
     // a thread's pieces: row tid / 4 (+ 64 per further piece), keys 4 (tid % 4) ..
     const int p_row = tid / 4, p_k = (tid % 4) * 4;
     const float* xsrc[XP];
@@ -239,7 +244,7 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
     auto put = [&](float* to, const f32x4 (&value)[WM][WN]) {
 #pragma unroll
         for (int jm = 0; jm < WM; ++jm) {
-            const int m = m0 + wm0 + 16 * jm + i;
+            const int m = m0 + wm0 + 32 * jm + i;
             if (m >= M) continue;
 #pragma unroll
             for (int jn = 0; jn < WN; ++jn) {
@@ -267,14 +272,26 @@ gemm_f32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w, f
 #pragma unroll
         for (int jn = 0; jn < WN; ++jn) a[jn] = *reinterpret_cast<const f32x4*>(&ws[buf][(wn0 + 16 * jn + i) * kStride + 4 * g]);
 #pragma unroll
-        for (int jm = 0; jm < WM; ++jm) b[jm] = *reinterpret_cast<const f32x4*>(&xs[buf][(wm0 + 16 * jm + i) * kStride + 4 * g]);
+        for (int jm = 0; jm < WM; ++jm) b[jm] = *reinterpret_cast<const f32x4*>(&xs[buf][(wm0 + 32 * jm + i) * kStride + 4 * g]);
+        if (PART) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+            for (int jm = 0; jm < WM; ++jm) {
+                if (jm >= live) break;
 #pragma unroll
-            for (int jm = 0; jm < WM; ++jm)
+                for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int jn = 0; jn < WN; ++jn)
-                    acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[jn][t], b[jm][t], acc[jm][jn], 0, 0, 0);
+                    for (int jn = 0; jn < WN; ++jn)
+                        acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[jn][t], b[jm][t], acc[jm][jn], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int jm = 0; jm < WM; ++jm)
+#pragma unroll
+                    for (int jn = 0; jn < WN; ++jn)
+                        acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[jn][t], b[jm][t], acc[jm][jn], 0, 0, 0);
+        }
         if ((q + 1) % kChunksPerSegment == 0 || q + 1 == chunks) {
             // a segment ends: its sum joins the sums of the segments before it, or goes to its own place
             const bool alone = q < kChunksPerSegment;
@@ -350,14 +367,16 @@ int sum_segments(const float* partial, float* out, long long count, int segments
 // 2,048: 596 to 94.
 struct F32Cut {
     int wm, wn, per_group;
+    bool part;                   // the last tile's blocks without rows are left out
 };
 constexpr long long kMostPartials = 64LL << 20;       // floats of partial sums a product may leave (256 MiB)
 
 F32Cut f32_cut(int M, int N, int K, bool may_split) {
-    constexpr struct { int wm, wn; float shared, alone; } kTiles[] = {{4, 4, 32.6f, 38.f}, {4, 2, 18.4f, 22.7f}, {2, 4, 18.4f, 22.7f}, {2, 2, 9.7f, 14.3f}};
+    constexpr struct { int wm, wn; float shared, alone, part; } kTiles[] = {
+        {4, 4, 32.6f, 38.f, 1.02f}, {4, 2, 18.4f, 22.7f, 0.95f}, {2, 4, 18.4f, 22.7f, 0.95f}, {2, 2, 9.7f, 14.3f, 0.97f}};
     constexpr int kUnits = 256;
     const int segments = (K + kF32Segment - 1) / kF32Segment;
-    F32Cut best{4, 4, 0};
+    F32Cut best{4, 4, 0, false};
     float least = 3.4e38f;
     for (const auto& t : kTiles) {
         const long long tiles = static_cast<long long>((M + 32 * t.wm - 1) / (32 * t.wm)) * ((N + 32 * t.wn - 1) / (32 * t.wn));
@@ -367,10 +386,16 @@ F32Cut f32_cut(int M, int N, int K, bool may_split) {
             if (split && (!may_split || groups > 65535 || static_cast<long long>(segments) * M * N > kMostPartials)) break;
             const long long on_a_unit = (tiles * groups + kUnits - 1) / kUnits;
             float us = per_group * ((on_a_unit & ~1LL) * t.shared + (on_a_unit & 1) * t.alone);
+            // The last tile costs 0.3 and 0.7 of what it has rows for, and the branches make the others slower or faster (measured, `part`).  Tiles of 64 x 64
+            // gain only where four and more share a compute unit (260 rows of 2,048 keys to 2,560 columns 50 to 45 us; to 2,048 39 to 40).
+            const int in_last = (M - 1) % (32 * t.wm) / 32 + 1;
+            const float shorter = t.part * (1.f - 0.7f * (t.wm - in_last) / t.wm / ((M + 32 * t.wm - 1) / (32 * t.wm)));
+            const bool part = in_last < t.wm && shorter < 1.f && (t.wm + t.wn > 4 || on_a_unit > 3);
+            if (part) us *= shorter;
             if (split) us += 4.f + 2e-6f * segments * M * N;
             if (us < least) {
                 least = us;
-                best = F32Cut{t.wm, t.wn, split ? per_group : 0};
+                best = F32Cut{t.wm, t.wn, split ? per_group : 0, part};
             }
         }
     }
@@ -467,16 +492,22 @@ WLLM_API int wllm_gemm_generic(const void* x, const void* w, const void* tiles, 
         const dim3 grid((N + 32 * cut.wn - 1) / (32 * cut.wn), (M + 32 * cut.wm - 1) / (32 * cut.wm),
                         cut.per_group ? (segments + cut.per_group - 1) / cut.per_group : 1);
         if (grid.y > 65535) return -1;
-#define TILES(WM, WN)                                                                                                   \
-    do {                                                                                                                \
-        if (cut.per_group) gemm_f32_tile_kernel<WM, WN, true><<<grid, 256, 0, stream>>>(xf, wf, pf, M, N, K, cut.per_group); \
-        else gemm_f32_tile_kernel<WM, WN, false><<<grid, 256, 0, stream>>>(xf, wf, of, M, N, K, 0);                     \
+#define TILES_P(WM, WN, PART)                                                                                                  \
+    do {                                                                                                                        \
+        if (cut.per_group) gemm_f32_tile_kernel<WM, WN, true, PART><<<grid, 256, 0, stream>>>(xf, wf, pf, M, N, K, cut.per_group); \
+        else gemm_f32_tile_kernel<WM, WN, false, PART><<<grid, 256, 0, stream>>>(xf, wf, of, M, N, K, 0);                       \
+    } while (0)
+#define TILES(WM, WN)                           \
+    do {                                        \
+        if (cut.part) TILES_P(WM, WN, true);    \
+        else TILES_P(WM, WN, false);            \
     } while (0)
         if (cut.wm == 4 && cut.wn == 4) TILES(4, 4);
         else if (cut.wm == 4) TILES(4, 2);
         else if (cut.wn == 4) TILES(2, 4);
         else TILES(2, 2);
 #undef TILES
+#undef TILES_P
         if (const int err = launch_status()) return err;
         return cut.per_group ? sum_segments(pf, of, static_cast<long long>(M) * N, segments, stream) : 0;
     }
