@@ -463,6 +463,57 @@ struct NormOnLoad {
     float eps, offset;
 };
 
+// The second half of the K axis hands its sums to the first through shared memory, which makes the results and writes them.
+template <int MT, int GATE, int TPW>
+__device__ __forceinline__ void gated_finish(float* shared, int tile, int half, int lane, int n0, const float4_t (&accg)[MT],
+                                             const float4_t (&accu)[MT], bf16* __restrict__ out, int M, int inter, int out_stride,
+                                             GateShape shape) {
+    const int i = lane % 16, g = lane / 16;
+    __syncthreads();
+    float* red = shared + (tile * kWave + lane) * (MT * 8);
+    if (half == 1) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                red[t * 8 + v] = accg[t][v];
+                red[t * 8 + 4 + v] = accu[t][v];
+            }
+    }
+    __syncthreads();
+    if (half == 1 || n0 >= inter) return;
+    const int n = n0 + 4 * g;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int m = t * 16 + i;
+        if (m >= M) continue;
+        constexpr bool kPair = GATE == kGatePairSquaredRelu;
+        float4_t r, r2;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float gate = accg[t][v] + red[t * 8 + v], upv = accu[t][v] + red[t * 8 + 4 + v];
+            if (kPair) {
+                r[v] = squared_relu(gate);
+                r2[v] = squared_relu(upv);
+            } else {
+                r[v] = gate_product<(kPair ? 0 : GATE)>(gate, upv, shape);
+            }
+        }
+        bf16* o = out + static_cast<size_t>(m) * out_stride + n;     // out may be a band of columns of a wider buffer
+        if (n + 3 < inter && (inter % 4 == 0) && (out_stride % 4 == 0)) {
+            store4<bf16>(o, r);
+            if (kPair) store4<bf16>(o + inter, r2);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < inter) {
+                    o[v] = from_float<bf16>(r[v]);
+                    if (kPair) o[inter + v] = from_float<bf16>(r2[v]);
+                }
+        }
+    }
+}
+
 template <int MT, int GATE, bool TILED, int TPW, bool NORM, int XR>
 __global__ void __launch_bounds__(TPW * 128, MT == 1 ? (NORM && XR > 2 ? 3 : 4) : (MT == 2 ? 3 : 2))
 gemm_skinny_gated_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16* __restrict__ w, bf16* __restrict__ out,
@@ -615,50 +666,135 @@ gemm_skinny_gated_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16
             step += kBatch;
         }
     }
-    // the second half hands its sums to the first through shared memory
-    __syncthreads();
-    float* red = reinterpret_cast<float*>(xs) + (tile * kWave + lane) * (MT * 8);
-    if (half == 1) {
+    gated_finish<MT, GATE, TPW>(reinterpret_cast<float*>(xs), tile, half, lane, n0, accg, accu, out, M, inter, out_stride, shape);
+}
+
+// The same with all of x in shared memory before the first product, for an x that leaves a compute unit room for three workgroups: no
+// barrier stands between the first load of weights and the last.  x is asked for before the weights, because loads come back in
+// the order they went out: behind them its first use would wait for all of theirs.  Tiles, halves of the K axis and the order of the
+// sums are those of the kernel above: the same bits.
+//
+// Bound by reading w: 134 MB of gate and up (2,048 keys to 2 x 16,384 columns) in 24.7 / 25.2 us with the norm at 1 / 8 rows and 23.5 / 23.9 without, where a
+// kernel that only reads them takes 21.8 to 22.2 (the kernel above, with two barriers for every 256 keys of a half, 26.4 / 26.2 and 24.4 / 24.6); 34 MB (to 2 x 4,096)
+// 10.6 / 11.3 and 9.4 / 9.5 (12.2 / 12.3 and 10.8 / 10.7).  More loads on their way and two workgroups a compute unit are no better (16 steps a
+// wavefront 24.5 / 25.3; of 3,072 keys to 2 x 24,576 columns 53 / 56 against 51 / 52), nor is one workgroup of twice the tiles, for an x of more than
+// half the shared memory (24 rows 27.6 against the kernel above's 25.4).
+template <int MT, int GATE, bool TILED, bool NORM>
+__global__ void __launch_bounds__(256, 3)
+gemm_gated_rows_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16* __restrict__ w, bf16* __restrict__ out, int M, int inter,
+                       int K, int out_stride, GateShape shape) {
+    extern __shared__ uint4 xs[];                 // [M][K / 8 + 1]
+    __shared__ float inv_s[16];                   // NORM: a row's rsqrt(mean square + eps)
+    constexpr int TPW = 2, kThreads = TPW * 128, kBatch = 8, kRows = 8;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int i = lane % 16, g = lane / 16;
+    const int tile = wave % TPW, half = wave / TPW;
+    const int n0 = (blockIdx.x * TPW + tile) * 16;
+    const int pieces = K / 8, stride = pieces + 1, half_k = K / 2, steps = half_k / 32;
+    const bool live = n0 < inter;
+    constexpr int kStep = TILED ? 512 : 32;
+    const int nrow = min(n0 + i, inter - 1);
+    const int bands = (inter + 15) / 16, band = min(n0 / 16, bands - 1);
+    const bf16* gp = TILED ? w + (static_cast<size_t>(band) * (K / 32) + half * steps) * 512 + lane * 8
+                           : w + static_cast<size_t>(nrow) * K + half * half_k + 8 * g;
+    const bf16* up = TILED ? w + (static_cast<size_t>(bands + band) * (K / 32) + half * steps) * 512 + lane * 8
+                           : w + static_cast<size_t>(inter + nrow) * K + half * half_k + 8 * g;
+    Frag curg[kBatch], curu[kBatch];
+    auto load_step = [&](int u, int at) {
+        if (!live || at >= steps) return;
+        curg[u].u = load_streamed(gp + static_cast<size_t>(at) * kStep);
+        curu[u].u = load_streamed(up + static_cast<size_t>(at) * kStep);
+    };
+    // a thread's 8 keys `c` of the rows r0 .. r0 + 7
+    float4 raw[NORM ? kRows : 1][2], wn[2];
+    uint4 given[NORM ? 1 : kRows];
+    auto ask_x = [&](int c, int r0) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                red[t * 8 + v] = accg[t][v];
-                red[t * 8 + 4 + v] = accu[t][v];
+        for (int r = 0; r < kRows; ++r) {
+            if (r0 + r >= M) break;
+            if (NORM) {
+                const float* src = norm.residual + static_cast<size_t>(r0 + r) * K + c * 8;
+                raw[NORM ? r : 0][0] = *reinterpret_cast<const float4*>(src);
+                raw[NORM ? r : 0][1] = *reinterpret_cast<const float4*>(src + 4);
+            } else {
+                given[NORM ? 0 : r] = *reinterpret_cast<const uint4*>(x + static_cast<size_t>(r0 + r) * K + c * 8);
             }
+        }
+    };
+    auto put_x = [&](int c, int r0) {
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            if (r0 + r >= M) break;
+            uint4 v = given[NORM ? 0 : r];
+            if (NORM) {
+                const float inv = inv_s[r0 + r];
+                const float4 a = raw[NORM ? r : 0][0], b = raw[NORM ? r : 0][1];
+                v.x = pack2_bf16(a.x * inv * (norm.offset + wn[0].x), a.y * inv * (norm.offset + wn[0].y));
+                v.y = pack2_bf16(a.z * inv * (norm.offset + wn[0].z), a.w * inv * (norm.offset + wn[0].w));
+                v.z = pack2_bf16(b.x * inv * (norm.offset + wn[1].x), b.y * inv * (norm.offset + wn[1].y));
+                v.w = pack2_bf16(b.z * inv * (norm.offset + wn[1].z), b.w * inv * (norm.offset + wn[1].w));
+            }
+            xs[(r0 + r) * stride + c] = v;
+        }
+    };
+    auto ask_weight = [&](int c) {
+        if (!NORM) return;
+        wn[0] = *reinterpret_cast<const float4*>(norm.weight + c * 8);
+        wn[1] = *reinterpret_cast<const float4*>(norm.weight + c * 8 + 4);
+    };
+    const int tid = threadIdx.x;
+    // 16 threads a row add the row of `sumsq` in a fixed order
+    float total = 0.f;
+    if (NORM && tid / 16 < M)
+        for (int b = tid % 16; b < norm.sumsq_cols; b += 16) total += norm.sumsq[static_cast<size_t>(tid / 16) * norm.sumsq_cols + b];
+    if (tid < pieces) {
+        ask_weight(tid);
+        ask_x(tid, 0);
     }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) load_step(u, u);
+    if (NORM) {
+        total += __shfl_xor(total, 8, kWave);
+        total += __shfl_xor(total, 4, kWave);
+        total += __shfl_xor(total, 2, kWave);
+        total += __shfl_xor(total, 1, kWave);
+        if (tid % 16 == 0) inv_s[tid / 16] = rsqrtf(total / static_cast<float>(K) + norm.eps);
+        __syncthreads();
+    }
+    for (int c = tid; c < pieces; c += kThreads)
+        for (int r0 = 0; r0 < M; r0 += kRows) {
+            if (c != tid || r0 > 0) {
+                if (r0 == 0) ask_weight(c);
+                ask_x(c, r0);
+            }
+            put_x(c, r0);
+        }
     __syncthreads();
-    if (half == 1 || n0 >= inter) return;
-    const int n = n0 + 4 * g;
+    float4_t accg[MT], accu[MT];
+    const uint4* xp[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const int m = t * 16 + i;
-        if (m >= M) continue;
-        constexpr bool kPair = GATE == kGatePairSquaredRelu;
-        float4_t r, r2;
+        accg[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        accu[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        // (rows that are not there read some row that is: they only feed results that are not written)
+        xp[t] = xs + min(16 * t + i, M - 1) * stride + half * (half_k / 8) + g;
+    }
+    for (int s = 0; s < steps; s += kBatch) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const float gate = accg[t][v] + red[t * 8 + v], upv = accu[t][v] + red[t * 8 + 4 + v];
-            if (kPair) {
-                r[v] = squared_relu(gate);
-                r2[v] = squared_relu(upv);
-            } else {
-                r[v] = gate_product<(kPair ? 0 : GATE)>(gate, upv, shape);
+        for (int u = 0; u < kBatch; ++u) {
+            if (s + u < steps) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    Frag b;
+                    b.u = xp[t][(s + u) * 4];
+                    accg[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(curg[u].v, b.v, accg[t], 0, 0, 0);
+                    accu[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(curu[u].v, b.v, accu[t], 0, 0, 0);
+                }
+                load_step(u, s + u + kBatch);
             }
         }
-        bf16* o = out + static_cast<size_t>(m) * out_stride + n;     // out may be a band of columns of a wider buffer
-        if (n + 3 < inter && (inter % 4 == 0) && (out_stride % 4 == 0)) {
-            store4<bf16>(o, r);
-            if (kPair) store4<bf16>(o + inter, r2);
-        } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if (n + v < inter) {
-                    o[v] = from_float<bf16>(r[v]);
-                    if (kPair) o[inter + v] = from_float<bf16>(r2[v]);
-                }
-        }
     }
+    gated_finish<MT, GATE, TPW>(reinterpret_cast<float*>(xs), tile, half, lane, n0, accg, accu, out, M, inter, out_stride, shape);
 }
 
 static int gated_launch(const void* x, NormOnLoad norm, bool with_norm, const void* w, int tiled, void* out, int M,
@@ -669,6 +805,30 @@ static int gated_launch(const void* x, NormOnLoad norm, bool with_norm, const vo
     if (chunk > K / 2) chunk = K / 2;
     // the norm on load: at most 16 rows, whole chunks of 256 keys
     if (with_norm && (mt != 1 || chunk != 256 || (K / 2) % 256 != 0)) return -1;
+    // x whole in shared memory, where three workgroups of it share a compute unit (of 2,048 keys 13 rows, of 3,072 8): at 16 rows of 2,048 keys two would,
+    // and are no faster (26.6 us with the norm against 26.9; to 2 x 24,576 columns 38.6 against 36.4)
+    const size_t whole = static_cast<size_t>(M) * (K / 8 + 1) * sizeof(uint4), sums = static_cast<size_t>(2) * kWave * mt * 8 * sizeof(float);
+    if (mt <= 2 && whole <= 53 * 1024) {
+        const dim3 grid((inter + 31) / 32);
+#define ROWS_T(MT, A, T, NORM)                                                                                        \
+    gemm_gated_rows_kernel<MT, A, T, NORM><<<grid, 256, whole > sums ? whole : sums, stream>>>(                       \
+        static_cast<const bf16*>(x), norm, static_cast<const bf16*>(w), static_cast<bf16*>(out), M, inter, K, out_stride, shape)
+#define ROWS(MT, A, NORM)                       \
+    do {                                        \
+        if (tiled) ROWS_T(MT, A, true, NORM);   \
+        else ROWS_T(MT, A, false, NORM);        \
+    } while (0)
+        if (with_norm) {
+            WLLM_BY_GATE(gate, ROWS(1, GATE, true))
+        } else if (mt == 1) {
+            WLLM_BY_PAIRED_GATE(gate, ROWS(1, GATE, false))
+        } else {
+            WLLM_BY_PAIRED_GATE(gate, ROWS(2, GATE, false))
+        }
+#undef ROWS
+#undef ROWS_T
+        return launch_status();
+    }
     const int tpw = 2;                               // tiles of 16 gate rows per workgroup
     size_t smem = static_cast<size_t>(2) * mt * 16 * (chunk / 8 + 1) * sizeof(uint4);
     const size_t red = static_cast<size_t>(tpw) * kWave * mt * 8 * sizeof(float);
