@@ -6,6 +6,7 @@ from __future__ import annotations
 import ctypes
 import functools
 from ctypes import c_float, c_int, c_longlong, c_void_p
+from types import SimpleNamespace
 
 import numpy as np
 import torch
@@ -13,7 +14,7 @@ import torch
 from wllm_amd.kernels.attention_plan import PROMPT_ROWS, AttentionPlan, build_work_items, count_tile_items, prompt_kernel_pays
 from wllm_amd.kernels import ops
 from wllm_amd.kernels.ops import gate_args
-from wllm_amd.kernels.library import load
+from wllm_amd.kernels.library import door, load
 from wllm_amd.kernels.staging import pack_int32
 
 
@@ -25,9 +26,7 @@ class KernelError(RuntimeError):
 _raw_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _ptr(t):
-    # (an address as an integer: the entry points' signatures make a pointer of it)
-    return t.data_ptr() if t is not None else None
+_ptr = ops._address
 
 
 _SIGNATURES = {
@@ -88,7 +87,9 @@ class HipBackend:
     def __init__(self):
         if not torch.cuda.is_available():
             raise KernelError("no GPU is visible; the kernels run on gfx950 only and there is no other path")
-        self.lib = load()
+        self._door = door()
+        self._on_gpu = self._door.make_on_gpu(KernelError)
+        raw = load()
         self._device_index = torch.cuda.current_device()
         self._partial_o = None
         self._slots_of = {}                # device -> workgroups of the prompt kernel it runs at once
@@ -99,16 +100,26 @@ class HipBackend:
         self._generic_partial_o = None
         self._registered: dict = {}
         self.library_events = None      # a list: every library product is bracketed by a pair of timing events
+        self.lib = SimpleNamespace(raw=raw)        # the entry points by name, and the library itself
         for name, argtypes in _SIGNATURES.items():
-            fn = getattr(self.lib, name)
-            fn.argtypes = argtypes
-            fn.restype = c_int
+            setattr(self.lib, name, self._entry(getattr(raw, name), argtypes))
 
     @staticmethod
-    def _on_gpu(*tensors) -> None:
+    def _on_gpu(*tensors) -> None:      # (a backend with a library has the native one)
         for t in tensors:
             if t is not None and not t.is_cuda:
                 raise KernelError("a kernel operand is not on the GPU")
+
+    _CODES = {c_void_p: "p", c_int: "i", c_longlong: "l", c_float: "f"}
+
+    def _entry(self, fn, argtypes):
+        """What calls the library's function `fn` with arguments of these types: an entry of the native module, or, for
+        other types or a function that is not a library's, `fn` itself."""
+        fn.argtypes, fn.restype = argtypes, c_int
+        codes = [self._CODES.get(a) for a in argtypes]
+        if None in codes or len(codes) > 48 or codes.count("f") > 8 or len(codes) - codes.count("f") > 40:
+            return fn
+        return self._door.Entry(ctypes.cast(fn, c_void_p).value, "".join(codes))
 
     def _stream(self) -> int:
         # the raw handle of torch's current stream on this process's GPU, asked for at every launch
@@ -125,15 +136,21 @@ class HipBackend:
 
     def run_registered(self, op, args, kwargs) -> None:
         """An operation that a part registered (`ops.register_op`): its entry point is looked up once in
-        its library, given its signature, and launched on the current stream."""
+        its library, given its signature, and launched on the current stream (a part's own through ctypes: its launch may hand it
+        whatever ctypes takes)."""
         fn = self._registered.get(op.name)
         if fn is None or fn[0] is not op:
-            lib = op.library() if op.library is not None else self.lib
+            lib = op.library() if op.library is not None else getattr(self.lib, "raw", self.lib)
             entry = getattr(lib, op.entry_point)
-            entry.argtypes = op.argtypes
-            entry.restype = c_int
+            if op.own:
+                entry = self._entry(entry, op.argtypes)
+            else:
+                entry.argtypes = op.argtypes
+                entry.restype = c_int
             fn = self._registered[op.name] = (op, entry)
-        self._on_gpu(*[a for a in list(args) + list(kwargs.values()) if isinstance(a, torch.Tensor)])
+        self._on_gpu(*[a for a in args if isinstance(a, torch.Tensor)])
+        if kwargs:
+            self._on_gpu(*[a for a in kwargs.values() if isinstance(a, torch.Tensor)])
         stream = self._stream() if op.own else c_void_p(self._stream())
         self._check(op.launch(fn[1], stream, *args, **kwargs), op.name)
 

@@ -2,8 +2,10 @@
 
 The kernels under `wllm_amd/csrc` are compiled with hipcc for gfx950 into one
 shared library, `wllm_amd/libwllm_kernels.so`, whose `extern "C"` entry points
-are called through ctypes with raw device pointers and a stream.  Nothing of
-torch is compiled against, so a build takes about a minute from nothing.
+are called with raw device pointers and a stream.  The kernels are compiled against nothing of
+torch; beside them `csrc/launch_door.cpp`, host code alone, becomes a CPython module
+(`door()`) through which the framework's own calls go, since ctypes would take half
+as long for each as the launch itself.  A build takes about a minute from nothing.
 
 `load()` loads the library if it is built from the present sources and builds it
 first if not (a line is printed per compiled file, so that a first call in a
@@ -25,6 +27,7 @@ from concurrent.futures import ThreadPoolExecutor
 PACKAGE_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE_DIR = os.path.join(PACKAGE_DIR, "csrc")
 LIBRARY_NAME = "libwllm_kernels.so"
+DOOR_SOURCE, DOOR_NAME = "launch_door.cpp", "launch_door.so"
 ARCH = "gfx950"
 # packed float32 instructions are switched off for all device code
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
@@ -47,7 +50,7 @@ def _fingerprint(source_dir: str = SOURCE_DIR) -> str:
     folders = [source_dir] if os.path.samefile(source_dir, SOURCE_DIR) else [source_dir, SOURCE_DIR]
     for folder in folders:
         for name in sorted(os.listdir(folder)):
-            if name.endswith(".h") or (folder == source_dir and name.endswith(".hip")):
+            if name.endswith(".h") or (folder == source_dir and name.endswith((".hip", ".cpp"))):
                 h.update(name.encode())
                 with open(os.path.join(folder, name), "rb") as f:
                     h.update(f.read())
@@ -91,6 +94,19 @@ def _is_current(lib_path: str, fingerprint: str) -> bool:
         return f.read().strip() == fingerprint
 
 
+def _door_command(hipcc: str, target: str) -> list:
+    """Compiles the module of `DOOR_SOURCE`: host code, against the interpreter's and torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    include = [a for folder in [sysconfig.get_paths()["include"]] + include_paths() for a in ("-isystem", folder)]
+    return [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + include + [
+            os.path.join(SOURCE_DIR, DOOR_SOURCE), "-o", target] + [f"-L{p}" for p in library_paths()] + [
+            "-ltorch_python", "-ltorch_cpu", "-lc10"]         # (found where `import torch` has loaded them)
+
+
 def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR, library_name: str = LIBRARY_NAME) -> str:
     """Compiles every source of the folder for gfx950 and links the library; returns its path.
     The framework's headers are on the include path of any folder."""
@@ -123,12 +139,21 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
         return name, obj, r
 
     objects = []
+    door_path = door_tmp = None
+    if os.path.samefile(source_dir, SOURCE_DIR):
+        door_path = os.path.join(os.path.dirname(lib_path), DOOR_NAME)
+        door_tmp = door_path + f".tmp{os.getpid()}"
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(names)))) as pool:
+        door_run = pool.submit(subprocess.run, _door_command(hipcc, door_tmp), capture_output=True, text=True, env=env) if door_path else None
         for name, obj, r in pool.map(compile_one, names):
             if r.returncode != 0:
                 raise KernelLibraryMissing(f"hipcc failed on {name}:\n{r.stderr[-4000:]}")
             say(f"compiled {name} ({time.time() - t0:.0f} s)")
             objects.append(obj)
+        if door_run is not None:
+            if door_run.result().returncode != 0:
+                raise KernelLibraryMissing(f"hipcc failed on {DOOR_SOURCE}:\n{door_run.result().stderr[-4000:]}")
+            os.replace(door_tmp, door_path)
     tmp = lib_path + f".tmp{os.getpid()}"
     r = subprocess.run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objects,
                        capture_output=True, text=True, env=env)
@@ -142,6 +167,37 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
 
 
 _loaded: dict = {}
+
+
+def built_door():
+    """The module of `launch_door.cpp` if it is built from the present sources, else None: nothing is built for it."""
+    if DOOR_NAME not in _loaded:
+        from importlib import util
+        fingerprint = _fingerprint()
+        for lib_path, _ in _locations(fingerprint):
+            path = os.path.join(os.path.dirname(lib_path), DOOR_NAME)
+            if _is_current(lib_path, fingerprint) and os.path.isfile(path):
+                import torch  # noqa: F401  (the module's symbols of torch)
+                spec = util.spec_from_file_location("launch_door", path)
+                try:
+                    module = util.module_from_spec(spec)
+                    spec.loader.exec_module(module)
+                except ImportError as e:
+                    raise KernelLibraryMissing(f"{path} cannot be loaded: {e}") from e
+                _loaded[DOOR_NAME] = module
+                break
+    return _loaded.get(DOOR_NAME)
+
+
+def door():
+    """The module of `launch_door.cpp`; built first, with the kernels, when no build of the present sources exists."""
+    module = built_door()
+    if module is None:
+        build()
+        module = built_door()
+    if module is None:
+        raise KernelLibraryMissing(f"{DOOR_NAME} is missing beside the kernel library")
+    return module
 
 
 def load(verbose: bool = True, source_dir: str = SOURCE_DIR, library_name: str = LIBRARY_NAME) -> ctypes.CDLL:

@@ -20,6 +20,8 @@ from typing import Optional
 
 import torch
 
+from wllm_amd.kernels.library import built_door
+
 _ACT = (torch.float32, torch.bfloat16)
 HEAD_DIM_STEP, MAX_HEAD_DIM = 4, 256      # what `paged_attention` takes: multiples of 4 up to 256
 _backend = None
@@ -70,6 +72,18 @@ def _dense(t: torch.Tensor, name: str, dtype, shape=None) -> None:
         raise KernelShapeError(f"{name}: must be contiguous")
     if shape is not None and tuple(t.shape) != tuple(shape):
         raise KernelShapeError(f"{name}: shape {tuple(t.shape)}, expected {tuple(shape)}")
+
+
+def _address(t):
+    # (an address as an integer: the entry points' signatures make a pointer of it)
+    return t.data_ptr() if t is not None else None
+
+
+# The same two as native code, where it is built: they run some forty times a layer.  (What is not plainly in order comes back to the
+# functions above; without the build these do.)
+_native = built_door()
+if _native is not None:
+    _dense, _address = _native.make_dense(_dense), _native.address
 
 
 # ---- operations that parts bring with them ------------------------------------------------------
@@ -1577,8 +1591,7 @@ def moe_experts_down(act: torch.Tensor, w: torch.Tensor, plan: torch.Tensor, wei
 # ---- the framework's own operations that go through the same door as a part's ------------------
 def _register_own() -> None:
     from ctypes import c_float, c_int, c_longlong, c_void_p
-    def p(t):                       # an address as an integer, which the signatures make a pointer of
-        return t.data_ptr() if t is not None else None
+    p = _address
 
     register_op("embed_lookup", entry_point="wllm_embed_lookup",
                 argtypes=[c_void_p, c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
