@@ -67,6 +67,7 @@ _SIGNATURES = {
                        c_float, c_void_p],
     "wllm_gemm_stream": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                          c_float, c_void_p],
+    "wllm_gemm_block": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "wllm_split_sum": [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
     "wllm_gemm_generic": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p],
     "wllm_tile_weight_f32": [c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -419,9 +420,8 @@ class HipBackend:
     # fills them (the down projection: 1.3 to 1.6 times as fast at 128 to 1,024 rows), and for the gated
     # product, which it writes once, up to 256 rows (at 512 rows it takes 84 us in a mixed step where
     # the library's product and the activation kernel take 69).  With these two the decode step of 256
-    # requests is 5% and the stress workload 2% faster.  The projections of the attention block are
-    # twice as fast alone (K axis of 2,048 in four pieces at 128 to 512 rows), but the rotation and the
-    # norm that then add the pieces lose more than that: left to the library.
+    # requests is 5% and the stress workload 2% faster.  The projections of the attention block are not cut:
+    # the rotation and the norm that then add the pieces lose more than the product gains (`block_tile` has them).
     TILE_MAX_ROWS = 1024
     F32_FEW_ROWS = 64         # rows up to which the float32 product streams its weights a band a wavefront
     TILE_LONG_K = 8192
@@ -485,6 +485,31 @@ class HipBackend:
             return False
         rounds = -(-(-(-rows // cls.WIDE_TILE) * -(-n // cls.WIDE_TILE)) // cls.COMPUTE_UNITS)
         return rows * n >= 0.6 * rounds * cls.COMPUTE_UNITS * cls.WIDE_TILE ** 2
+
+    # Tiles of the products of some hundred to two thousand rows (`gemm_block.hip`, which has the figures): rows of x, rows of w, and the time of a
+    # launch that fills at most one round of workgroups, us and us a stage of 64 keys.
+    BLOCK_TILES = ((64, 64, 2.9, 0.27), (128, 64, 3.2, 0.37), (192, 64, 3.6, 0.42), (128, 128, 4.0, 0.51), (192, 128, 4.6, 0.58))
+
+    @classmethod
+    @functools.lru_cache(maxsize=4096)
+    def block_tile(cls, rows: int, n: int, k: int):
+        """The tile in which a product rounded to bfloat16 goes instead of to the library, or None: the quickest of which one round of a
+        workgroup a compute unit is enough.  A K axis of more than 3,072 keys has to fill nine tenths of the round, as the library cuts it where
+        its tiles are few (4,096 keys to 2,048 columns at 128 / 256 / 508 / 1,024 rows 12.9 / 16.2 / 22.0 / 30.6 us there, 20.3 / 20.0 / 21.3 / 28.1
+        here).  Few columns are as quick there (2,048 keys to 64 columns 8.2 and 10.0), which only shows where the step does not wait for the host:
+        at more than 512 rows they are the library's.  A launch at one side of a line or the other differs by some per cent (768 rows to 2,048
+        columns 14.6 and 15.2, to 6,144 26.6 and 27.4); none of 100 sizes within the rule lost more than 5%, most gained 5 to 15, some 30."""
+        if rows <= 64 or n < 1 or k < 64 or k % 64 != 0 or k > 4096 or (n < 1024 and rows > 512) or max(rows, n) * k * 2 >= 2 ** 32:
+            return None
+        best = None
+        for tm, tn, launch, stage in cls.BLOCK_TILES:
+            tiles = -(-rows // tm) * -(-n // tn)
+            time = launch + stage * (k // 64)
+            if tiles <= cls.COMPUTE_UNITS and (best is None or time < best[0]):
+                best = (time, tm, tn, tiles)
+        if best is None or (k > 3072 and best[3] < 0.9 * cls.COMPUTE_UNITS):
+            return None
+        return best[1], best[2]
 
     @classmethod
     def wide_splits(cls, n: int, k: int, rows: int) -> int:
@@ -634,6 +659,11 @@ class HipBackend:
             if k % 32 == 0 and out.dtype == torch.float32:
                 for r in range(0, m, 64):
                     self._skinny(x[r:r + 64], weight, out[r:r + 64], tiles)
+                return
+            block = self.block_tile(m, n, k) if out.dtype == torch.bfloat16 else None
+            if block is not None and not self._odd(x, weight):
+                self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), _ptr(out), m, n, k, n, *block, self._stream()),
+                            "linear (tiles in one round)")
                 return
             if out.dtype == torch.bfloat16 and self.wide_takes(m, n, k):
                 self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, n, 1, 0, 0.0, 0.0, 0.0,
