@@ -87,3 +87,88 @@ def test_results_at_any_address_and_captured():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def odd_copy(t):
+    return torch.empty(t.numel() + 1, device=DEV, dtype=t.dtype)[1:].view(t.shape).copy_(t)
+
+
+def test_the_rules_of_gated_products_and_stacks():
+    gated, stack = HipBackend.block_gated_tile, HipBackend.block_split_tile
+    assert gated(64, 16384, 2048) is None and gated(128, 16384, 2048) == (128, 128) and gated(129, 16384, 2048) == (192, 128)
+    assert gated(256, 16384, 2048) == (256, 128) and gated(257, 16384, 2048) is None and gated(100, 16385, 2048) is None
+    assert gated(65, 4096, 2048) == (64, 64) and gated(512, 4096, 2048) == (128, 128) and gated(1500, 4096, 2048) is None
+    assert gated(100, 4096, 4160) is None and gated(100, 4096, 2080) is None and gated(100, 0, 2048) is None
+    assert stack(65, 2048, 16384, 8) == (128, 64) and stack(164, 2048, 16384, 8) == (192, 64) and stack(256, 2048, 16384, 8) == (128, 128)
+    assert stack(257, 2048, 16384, 16) is None and stack(200, 3072, 24576, 16) is None and stack(100, 2048, 192, 4) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu", ops.ClampedSwish(1.5, 1.702, 1.0)], ids=["gelu_tanh", "silu", "clamped"])
+@pytest.mark.parametrize("inter,k", [(16384, 2048), (4096, 1984), (250, 64), (777, 192), (33, 320)])
+def test_gated_products_have_the_bits_of_other_tiles(act, inter, k):
+    """Operands at odd addresses go in tiles of 256 x 256, whose gate up to 256 rows is as exact and whose sums go in the same order."""
+    torch.manual_seed(62)
+    w = (torch.randn(2 * inter, k, device=DEV) / math.sqrt(k)).bfloat16()
+    for m in (65, 100, 128, 129, 191, 192, 193, 256):
+        assert HipBackend.block_gated_tile(m, inter, k) is not None
+        x = torch.randn(m, k, device=DEV).bfloat16()
+        scratch = torch.empty(m, 2 * inter, device=DEV, dtype=torch.bfloat16)
+        want, out = (torch.full((m + 1, inter), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        ops.gated_linear(odd_copy(x), w, want[:m], act, scratch)
+        ops.gated_linear(x, w, out[:m], act, scratch)
+        assert torch.equal(out, want), f"{m} rows"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("m,inter,k", [(257, 4096, 2048), (385, 1000, 192), (512, 4096, 2048), (600, 250, 64), (1030, 778, 128)])
+def test_gated_products_of_more_rows(act, m, inter, k):
+    assert HipBackend.block_gated_tile(m, inter, k) is not None
+    torch.manual_seed(63)
+    x, w = torch.randn(m, k, device=DEV).bfloat16(), (torch.randn(2 * inter, k, device=DEV) / math.sqrt(k)).bfloat16()
+    wide = torch.full((m, inter + 16), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops.gated_linear(x, w, wide[:, 8:8 + inter], act, torch.empty(m, 2 * inter, device=DEV, dtype=torch.bfloat16))
+    gate, up = (x.double() @ w.double().T).split(inter, 1)
+    f = torch.nn.functional
+    exact = (f.gelu(gate, approximate="tanh") if act == "gelu_tanh" else f.silu(gate)) * up
+    # sums of deviation one, each off by at most k roundings of half a unit of numbers below 8: both factors (slope of the gate below 1.2), the gate's
+    # own arithmetic (a few units of 2^-24), and one rounding to bfloat16
+    off = k * 2.0 ** -24 * 8
+    bound = 1.2 * off * (up.abs() + gate.abs() + off) + 2.0 ** -20 * exact.abs() + 2.0 ** -8 * exact.abs() + 1e-6
+    assert bool(((wide[:, 8:8 + inter].double() - exact).abs() <= bound).all())
+    assert bool((wide[:, :8] == 7.0).all()) and bool((wide[:, 8 + inter:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("half,k", [(300, 128), (4096, 2048)])
+def test_squared_relu_of_two_halves(half, k):
+    torch.manual_seed(64)
+    w = (torch.randn(2 * half, k, device=DEV) / math.sqrt(k)).bfloat16()
+    for m in (65, 192, 256):
+        x = torch.randn(m, k, device=DEV).bfloat16()
+        want, out = (torch.empty(m, 2 * half, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        ops.activated_linear(odd_copy(x), w, want, "squared_relu")
+        ops.activated_linear(x, w, out, "squared_relu")
+        assert torch.equal(out, want), f"{m} rows"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(2048, 16384), (2047, 8192), (1030, 8192), (64, 8192)])
+def test_stacks_have_the_bits_of_other_tiles(n, k):
+    torch.manual_seed(65)
+    w, taken = (torch.randn(n, k, device=DEV) / math.sqrt(k)).bfloat16(), 0
+    for m in (65, 128, 129, 192, 193, 256):
+        s = ops.linear_splits(m, n, k, torch.bfloat16)
+        if s == 1 or HipBackend.wide_splits(n, k, m) > 1 or HipBackend.block_split_tile(m, n, k, s) is None:
+            continue
+        taken += 1
+        x = torch.randn(m, k, device=DEV).bfloat16()
+        want, out = (torch.full((s + 1, m, n), 7.0, device=DEV) for _ in range(2))
+        ops.linear(odd_copy(x), w, want[:s])
+        ops.linear(x, w, out[:s])
+        assert torch.equal(out, want), f"{m} rows in {s} pieces"
+        flat = torch.full((s * m * n + 5,), 7.0, device=DEV)
+        ops.linear(x, w, flat[3:3 + s * m * n].view(s, m, n))
+        assert torch.equal(flat[3:3 + s * m * n].view(s, m, n), want[:s]) and bool((flat[:3] == 7.0).all()) and bool((flat[-2:] == 7.0).all())
+    assert taken

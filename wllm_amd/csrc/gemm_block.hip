@@ -1,5 +1,8 @@
 // out[M, N] = x[M, K] . w[N, K]^T for bfloat16 with some hundred to two thousand rows and few columns (a prompt's projections), on the matrix
 // cores, in tiles of 64 to 192 rows of x by 64 or 128 rows of w: as many as make one round of a workgroup a compute unit.
+// And, where one round is enough, the stack of the sums of a long K axis in pieces, and the gated form out[M, I] = act(x . Wg^T) * (x . Wu^T) with
+// w = [Wg; Wu], whose activation and product are made in the registers the sums are in: a tile's rows of w are then half gate rows, half
+// the up rows that belong to them, and a wavefront has 16 of each.
 //
 // A workgroup of eight wavefronts walks the K axis in stages of 64 keys, a ring of them in shared memory.  A stage goes there straight from
 // memory (global_load_lds_dwordx4: a wavefront's load is 8 rows of 8 chunks of 16 bytes; chunk c of row r lies at place c ^ (r % 8) of its
@@ -19,8 +22,11 @@
 // 6.3 / 9.2.  Tiles of a second round find the machine half empty, and more rows are the library's (4,096 rows to 2,048 columns 34 and 41).  A
 // call of the library costs the host 19 us where a launch costs 6, and a step of a few hundred rows waits for the host.
 //
+// Gated, 2,048 keys to 2 x 16,384 columns at 100 / 164 / 256 rows 35.3 / 37.4 / 42.1, in tiles of 128 37.0 / 44.3 / 48.7; to 2 x 4,096 13.2 / 16.1 / 17.6 and
+// 24.1 / 23.7 / 24.6.  16,384 keys to 2,048 columns in 8 pieces at 65 / 164 rows 20.9 / 24.7 and 26.2 / 26.5.
+//
 // Tried: four wavefronts of 64 x 64 (25.4 for 19.8: nothing is left to multiply while one sends), loads by wavefronts of their own (as fast), rings of more
-// than four stages (slower but for 64 x 64).  Every element is summed over k in ascending order, whatever the tile.
+// than four stages (slower but for 64 x 64).  Every element is summed over k in ascending order (of a piece), whatever the tile.
 #include "lds_load.h"
 
 constexpr int kBlockKeys = 64;                       // keys a stage
@@ -30,16 +36,20 @@ struct BlockShape {
     static constexpr int kWavesN = TN / 32, kWavesM = 8 / kWavesN;
     static constexpr int kXBlocks = TM / 16 / kWavesM;                          // blocks of 16 rows of x a wavefront has
     static constexpr int kStage = (TM + TN) * kBlockKeys * 2;                   // bytes
-    static constexpr int kRing = TM + TN <= 128 ? 6 : 4;
+    static constexpr int kRing = TM + TN <= 128 ? 6 : (160 * 1024 / kStage < 4 ? 160 * 1024 / kStage : 4);
     static constexpr int kLoadsX = TM / 64, kLoadsW = TN / 64, kLoads = kLoadsX + kLoadsW;        // a wavefront and stage
-    static_assert(TM % 64 == 0 && TN % 64 == 0 && kXBlocks >= 1 && kRing * kStage <= 160 * 1024, "whole loads, and room for the ring");
+    static_assert(TM % 64 == 0 && TN % 64 == 0 && kXBlocks >= 1 && kRing >= 3 && kRing * kStage <= 160 * 1024, "whole loads, and room for the ring");
 };
 
-template <int TM, int TN>
+// GATED: 0 plain, 1 + the gate's number for the gated product.  N is the number of rows of w (plain) or of gate rows (gated); `vectors`: a lane's
+// neighbouring results (16 bytes, gated 8) lie at multiples of their size.
+template <int TM, int TN, int GATED>
 __global__ void __launch_bounds__(512, 2)
-gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* __restrict__ out, int M, int N, int K, int stride,
-                  bool vectors, int m_tiles, int n_tiles) {
+gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* __restrict__ out, float* __restrict__ partial, int M, int N,
+                  int K, int stride, bool vectors, int m_tiles, int n_tiles, int splits, GateShape shape) {
     using S = BlockShape<TM, TN>;
+    constexpr int kColumns = GATED ? TN / 2 : TN;                    // output columns a tile
+    constexpr bool kPair = GATED == kGatePairSquaredRelu + 1;
     constexpr int XB = S::kXBlocks, D = S::kRing, L = S::kLoads;
     extern __shared__ __align__(16) unsigned char ring_s[];
     const int lane = threadIdx.x % kWave;
@@ -49,7 +59,7 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
     const uint32_t lds_base = shared_address(ring_s);
 
     // The items go to the XCDs in equal runs of an order in which 8 tiles of x rows share a tile of w rows.
-    const int items = m_tiles * n_tiles, stages = K / kBlockKeys;
+    const int tiles = m_tiles * n_tiles, items = tiles * splits, all_stages = K / kBlockKeys;
     const int xcd = blockIdx.x % 8, per_xcd = items / 8, left = items % 8;
     int item = xcd * per_xcd + min(xcd, left) + blockIdx.x / 8;
     const int end = xcd * per_xcd + min(xcd, left) + per_xcd + (xcd < left ? 1 : 0);
@@ -57,23 +67,30 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
 
     // what this lane brings of a stage: rows 8 (wave + 8 u) + lane / 8 of the tiles, in bytes from the stage's first key
     uint32_t offset_x[S::kLoadsX], offset_w[S::kLoadsW];
-    int m_base, n_base;
-    auto place = [&](int t) {
+    int m_base, n_base, piece, begin, stages;
+    auto place = [&](int it) {
+        piece = it / tiles;
+        const int t = it - piece * tiles;
+        begin = static_cast<int>(static_cast<long long>(piece) * all_stages / splits);
+        stages = static_cast<int>(static_cast<long long>(piece + 1) * all_stages / splits) - begin;
         const int band = t / (8 * n_tiles), in_band = t - band * 8 * n_tiles;
         const int band_rows = min(8, m_tiles - 8 * band);
         const int n_tile = in_band / band_rows;
         m_base = (8 * band + in_band - n_tile * band_rows) * TM;
-        n_base = n_tile * TN;
+        n_base = n_tile * kColumns;
         const int r = 8 * wave + lane / 8, c = (lane % 8) ^ (lane / 8);
 #pragma unroll
         for (int u = 0; u < S::kLoadsX; ++u)
             offset_x[u] = (static_cast<uint32_t>(min(m_base + r + 64 * u, M - 1)) * K + c * 8) * 2;
 #pragma unroll
-        for (int u = 0; u < S::kLoadsW; ++u)
-            offset_w[u] = (static_cast<uint32_t>(min(n_base + r + 64 * u, N - 1)) * K + c * 8) * 2;
+        for (int u = 0; u < S::kLoadsW; ++u) {
+            const int at = r + 64 * u;               // gated: the gate rows, then the up rows that belong to them
+            const int row = !GATED || at < TN / 2 ? min(n_base + at, N - 1) : N + min(n_base + at - TN / 2, N - 1);
+            offset_w[u] = (static_cast<uint32_t>(row) * K + c * 8) * 2;
+        }
     };
     auto send_one = [&](int s, int slot, int u) {
-        const size_t at = static_cast<size_t>(s) * (kBlockKeys * 2);
+        const size_t at = static_cast<size_t>(begin + s) * (kBlockKeys * 2);
         const uint32_t to = lds_base + slot * S::kStage + wave * 1024;
         if (u < S::kLoadsX) load_to_shared(reinterpret_cast<const unsigned char*>(x) + at, offset_x[u < S::kLoadsX ? u : 0], to + u * 8192);
         else load_to_shared(reinterpret_cast<const unsigned char*>(w) + at, offset_w[u < S::kLoadsX ? 0 : u - S::kLoadsX],
@@ -103,7 +120,7 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
             constexpr int F = decltype(set)::value ? 1 : 0;
             const int k = r / (2 + XB), f = r % (2 + XB);
             const unsigned char* from = ring_s + slot * S::kStage + (k ? place1 : place0);
-            if (f < 2) fw[F][k][f].u = *reinterpret_cast<const uint4*>(from + TM * 128 + (wn * 32 + f * 16 + i) * 128);
+            if (f < 2) fw[F][k][f].u = *reinterpret_cast<const uint4*>(from + TM * 128 + ((GATED ? f * (TN / 2) + wn * 16 : wn * 32 + f * 16) + i) * 128);
             else fx[F][k][f - 2].u = *reinterpret_cast<const uint4*>(from + ((wm * XB + f - 2) * 16 + i) * 128);
         };
         // stage s is in the registers `set`
@@ -145,7 +162,7 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
         }
         wait_reads();
         meet();                                          // every wavefront is done with the shared memory
-        const int m0 = m_base, n0 = n_base;
+        const int m0 = m_base, n0 = n_base, of_piece = piece;
         item += gridDim.x / 8;
         const bool again = item < end;
         if (again) {
@@ -156,6 +173,44 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
         for (int b = 0; b < XB; ++b) {
             const int m = m0 + (wm * XB + b) * 16 + i;
             if (m >= M) continue;
+            if (GATED) {
+                // a lane has four columns' gate and up sums
+                const int n = n0 + wn * 16 + 4 * g;
+                bf16* to = out + static_cast<size_t>(m) * stride + n;
+#pragma unroll
+                for (int h = 0; h < (kPair ? 2 : 1); ++h) {
+                    float r[4];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        r[v] = kPair ? squared_relu(acc[h][b][v])
+                                     : gate_product<(GATED > 0 && !kPair ? GATED - 1 : 0)>(acc[0][b][v], acc[1][b][v], shape);
+                    const uint32_t words[2] = {pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3])};
+                    bf16* here = to + h * N;
+                    if (vectors && n + 3 < N) {
+                        *reinterpret_cast<uint2*>(here) = make_uint2(words[0], words[1]);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (n + v < N) here[v] = bf16{static_cast<uint16_t>(words[v / 2] >> (16 * (v % 2)))};
+                    }
+                }
+                continue;
+            }
+            if (partial != nullptr) {
+                float* row = partial + (static_cast<size_t>(of_piece) * M + m) * N;
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    const int n = n0 + wn * 32 + 16 * a + 4 * g;
+                    if (vectors && n + 3 < N) {
+                        *reinterpret_cast<float4_t*>(row + n) = acc[a][b];
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (n + v < N) row[n + v] = acc[a][b][v];
+                    }
+                }
+                continue;
+            }
             uint32_t q[2][2];
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
@@ -181,36 +236,56 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
     }
 }
 
-// out = x w^T, rounded to bfloat16, in tiles of tile_m rows of x by tile_n rows of w (64, 128 or 192 by 64, 128 or 192 by 128); `stride` elements from a
-// row of out to the next.  K is a multiple of 64, x and w begin at multiples of 16 bytes and are smaller than 4 GiB.  Returns 0, a HIP error
-// code, or -1 for what it does not take.
-WLLM_API int wllm_gemm_block(const void* x, const void* w, void* out, int M, int N, int K, int stride, int tile_m, int tile_n,
-                             hipStream_t stream) {
-    if (M < 1 || N < 1 || K < kBlockKeys || K % kBlockKeys != 0 || stride < N || tile_m < 64 || tile_n < 64) return -1;
-    if (static_cast<size_t>(N) * K * 2 >= (size_t(1) << 32) || static_cast<size_t>(M) * K * 2 >= (size_t(1) << 32)) return -1;
+// out = x w^T, rounded to bfloat16, in tiles of tile_m rows of x by tile_n rows of w (64, 128, 192 by 64, 128 and 192 by 128; gated 256 by 128 too); `stride` elements from a
+// row of out to the next.  `splits` > 1: `out` is null and `partial` float32 [splits, M, N] takes the sums of the K axis's pieces.  `gated` = 1 + the
+// gate's number (with limit, slope and shift for the clamped swish): the gated product, w [2N, K], gate rows first; with the paired squared
+// relu out [M, 2N] = relu(x . w^T)^2.  K is a multiple of 64 and at least 64 * splits, x and w begin at multiples of 16 bytes and are smaller
+// than 4 GiB.  Returns 0, a HIP error code, or -1 for what it does not take.
+WLLM_API int wllm_gemm_block(const void* x, const void* w, void* out, float* partial, int M, int N, int K, int stride, int splits, int gated,
+                             float limit, float slope, float shift, int tile_m, int tile_n, hipStream_t stream) {
+    if (M < 1 || N < 1 || K < kBlockKeys || K % kBlockKeys != 0 || splits < 1 || splits > K / kBlockKeys || gated < 0 || gated > kPairedGates ||
+        tile_m < 64 || tile_n < 64)
+        return -1;
+    if ((splits > 1) != (partial != nullptr) || (splits > 1) != (out == nullptr) || (splits > 1 && gated != 0)) return -1;
+    const bool pair = gated == kGatePairSquaredRelu + 1;
+    if (out != nullptr && stride < (pair ? 2LL * N : N)) return -1;
+    if (static_cast<size_t>(gated ? 2 : 1) * N * K * 2 >= (size_t(1) << 32) || static_cast<size_t>(M) * K * 2 >= (size_t(1) << 32)) return -1;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 != 0) return -1;
-    const bool vectors = reinterpret_cast<uintptr_t>(out) % 16 == 0 && stride % 8 == 0;
-    const int m_tiles = (M - 1) / tile_m + 1, n_tiles = (N - 1) / tile_n + 1;
-    const long long items = static_cast<long long>(m_tiles) * n_tiles;
+    const bool vectors = partial ? reinterpret_cast<uintptr_t>(partial) % 16 == 0 && N % 4 == 0
+                         : gated ? reinterpret_cast<uintptr_t>(out) % 8 == 0 && stride % 4 == 0 && (!pair || N % 4 == 0)
+                                 : reinterpret_cast<uintptr_t>(out) % 16 == 0 && stride % 8 == 0;
+    const int columns = gated ? tile_n / 2 : tile_n;
+    const int m_tiles = (M - 1) / tile_m + 1, n_tiles = (N - 1) / columns + 1;
+    const long long items = static_cast<long long>(m_tiles) * n_tiles * splits;
     if (items > 0x3fffffffLL) return -1;
     // a multiple of 8, so that a workgroup's items stay in its XCD's run
     const int grid = items < 256 ? static_cast<int>((items + 7) / 8 * 8) : 256;
-#define LAUNCH(TM, TN)                                                                                                            \
+    const int longest = (K / kBlockKeys + splits - 1) / splits;          // stages of an item
+    const GateShape shape{limit, slope, shift};
+#define LAUNCH(TM, TN, GATED)                                                                                                     \
     if (tile_m == TM && tile_n == TN) {                                                                                            \
         using S = BlockShape<TM, TN>;                                                                                              \
         static bool roomy = false;     /* more than 64 KiB of shared memory must be asked for once */                             \
         if (!roomy) {                                                                                                              \
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_block_kernel<TM, TN>),                                     \
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_block_kernel<TM, TN, GATED>),                              \
                                     hipFuncAttributeMaxDynamicSharedMemorySize, S::kRing * S::kStage) != hipSuccess)               \
                 return launch_status();                                                                                            \
             roomy = true;                                                                                                          \
         }                                                                                                                          \
-        const int slots = K / kBlockKeys < S::kRing ? K / kBlockKeys : S::kRing;                                                   \
-        gemm_block_kernel<TM, TN><<<grid, 512, slots * S::kStage, stream>>>(static_cast<const bf16*>(x), static_cast<const bf16*>(w), \
-                                                                            static_cast<bf16*>(out), M, N, K, stride, vectors, m_tiles, n_tiles); \
+        gemm_block_kernel<TM, TN, GATED><<<grid, 512, (longest < S::kRing ? longest : S::kRing) * S::kStage, stream>>>(            \
+            static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(out), partial, M, N, K, stride, vectors,  \
+            m_tiles, n_tiles, splits, shape);                                                                                      \
         return launch_status();                                                                                                    \
     }
-    LAUNCH(64, 64) LAUNCH(128, 64) LAUNCH(192, 64) LAUNCH(128, 128) LAUNCH(192, 128)
+#define TILES(GATED)                                                                                    \
+    do {                                                                                                \
+        LAUNCH(64, 64, GATED) LAUNCH(128, 64, GATED) LAUNCH(192, 64, GATED)                             \
+        LAUNCH(128, 128, GATED) LAUNCH(192, 128, GATED)                                                 \
+        if (GATED) { LAUNCH(256, 128, (GATED ? GATED : 1)) }                                            \
+    } while (0)
+    if (gated == 0) { TILES(0); }
+    else { WLLM_BY_PAIRED_GATE(gated - 1, TILES(GATE + 1)) }
+#undef TILES
 #undef LAUNCH
     return -1;
 }

@@ -67,7 +67,8 @@ _SIGNATURES = {
                        c_float, c_void_p],
     "wllm_gemm_stream": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                          c_float, c_void_p],
-    "wllm_gemm_block": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "wllm_gemm_block": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int,
+                        c_int, c_void_p],
     "wllm_split_sum": [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
     "wllm_gemm_generic": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p],
     "wllm_tile_weight_f32": [c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -487,11 +488,42 @@ class HipBackend:
         return rows * n >= 0.6 * rounds * cls.COMPUTE_UNITS * cls.WIDE_TILE ** 2
 
     # Tiles of the products of some hundred to two thousand rows (`gemm_block.hip`, which has the figures): rows of x, rows of w, and the time of a
-    # launch that fills at most one round of workgroups, us and us a stage of 64 keys.
-    BLOCK_TILES = ((64, 64, 2.9, 0.27), (128, 64, 3.2, 0.37), (192, 64, 3.6, 0.42), (128, 128, 4.0, 0.51), (192, 128, 4.6, 0.58))
+    # launch that fills at most one round of workgroups, us and us a stage of 64 keys.  (256 rows: only the gated product has them.)
+    BLOCK_TILES = ((64, 64, 2.9, 0.27), (128, 64, 3.2, 0.37), (192, 64, 3.6, 0.42), (128, 128, 4.0, 0.51), (192, 128, 4.6, 0.58), (256, 128, 4.6, 0.75))
 
     @classmethod
     @functools.lru_cache(maxsize=4096)
+    def _one_round(cls, rows: int, n: int, k: int, pieces: int = 1, gated: bool = False):
+        """The quickest tile of which one round of a workgroup a compute unit is enough, and how many make it; None if none is."""
+        if rows <= 64 or n < 1 or k < 64 * pieces or k % 64 != 0 or max(rows, 2 * n if gated else n) * k * 2 >= 2 ** 32:
+            return None
+        best = None
+        for tm, tn, launch, stage in cls.BLOCK_TILES:
+            tiles = -(-rows // tm) * -(-n // (tn // 2 if gated else tn)) * pieces
+            time = launch + stage * -(-k // (64 * pieces))
+            if tiles <= cls.COMPUTE_UNITS and (gated or tm <= 192) and (best is None or time < best[0]):
+                best = (time, tm, tn, tiles)
+        return best[1:] if best is not None else None
+
+    @classmethod
+    def block_gated_tile(cls, rows: int, columns: int, k: int):
+        """The tile of a gated product of `columns` output columns, or None: where one round is enough, up to 256 rows, and beyond where the tiles of
+        256 x 256 do not take it.  us, tiles of 128 and here, 2,048 keys to 2 x 16,384 columns at 100 / 164 / 256 rows 37.0 / 44.3 / 48.7 and 35.3 / 37.4 /
+        42.1; to 2 x 4,096 24.1 / 23.7 / 24.6 and 13.2 / 16.1 / 17.6, at 300 / 512 rows the library's product with the activation's pass 27.6 / 29.2 and
+        19.7 / 23.9.  One and a half rounds lose (to 2 x 24,576 at 164 rows 57 and 64).  Up to 256 rows all have the same bits."""
+        if k > 4096 or (rows > cls.WIDE_TILE and cls.wide_gated_takes(rows, columns, k)):
+            return None
+        found = cls._one_round(rows, columns, k, gated=True)
+        return found[:2] if found is not None else None
+
+    @classmethod
+    def block_split_tile(cls, rows: int, n: int, k: int, pieces: int):
+        """The tile of a stack of `pieces` partial sums, or None: where one round is enough, up to 256 rows (16,384 keys to 2,048 columns in 8 pieces at 65 /
+        128 / 164 / 256 rows 20.9 / 21.9 / 24.7 / 28.0 us, in tiles of 128, two a compute unit, 26.2 / 26.6 / 26.5 / 28.7).  The same bits."""
+        found = cls._one_round(rows, n, k, pieces) if rows <= 256 else None
+        return found[:2] if found is not None else None
+
+    @classmethod
     def block_tile(cls, rows: int, n: int, k: int):
         """The tile in which a product rounded to bfloat16 goes instead of to the library, or None: the quickest of which one round of a
         workgroup a compute unit is enough.  A K axis of more than 3,072 keys has to fill nine tenths of the round, as the library cuts it where
@@ -499,17 +531,10 @@ class HipBackend:
         here).  Few columns are as quick there (2,048 keys to 64 columns 8.2 and 10.0), which only shows where the step does not wait for the host:
         at more than 512 rows they are the library's.  A launch at one side of a line or the other differs by some per cent (768 rows to 2,048
         columns 14.6 and 15.2, to 6,144 26.6 and 27.4); none of 100 sizes within the rule lost more than 5%, most gained 5 to 15, some 30."""
-        if rows <= 64 or n < 1 or k < 64 or k % 64 != 0 or k > 4096 or (n < 1024 and rows > 512) or max(rows, n) * k * 2 >= 2 ** 32:
+        if k > 4096 or (n < 1024 and rows > 512):
             return None
-        best = None
-        for tm, tn, launch, stage in cls.BLOCK_TILES:
-            tiles = -(-rows // tm) * -(-n // tn)
-            time = launch + stage * (k // 64)
-            if tiles <= cls.COMPUTE_UNITS and (best is None or time < best[0]):
-                best = (time, tm, tn, tiles)
-        if best is None or (k > 3072 and best[3] < 0.9 * cls.COMPUTE_UNITS):
-            return None
-        return best[1], best[2]
+        found = cls._one_round(rows, n, k)
+        return found[:2] if found is not None and (k <= 3072 or found[2] >= 0.9 * cls.COMPUTE_UNITS) else None
 
     @classmethod
     def wide_splits(cls, n: int, k: int, rows: int) -> int:
@@ -641,7 +666,12 @@ class HipBackend:
             if splits > 1 and stack is None:
                 stack = ops.scratch_or_none(lambda: torch.empty((splits, m, n), dtype=torch.float32, device=x.device))
             if stack is not None:
-                if wide > 1 or self._odd(x, weight):
+                odd = self._odd(x, weight)
+                block = self.block_split_tile(m, n, k, splits) if wide == 1 and not odd else None
+                if block is not None:
+                    self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), None, _ptr(stack), m, n, k, n, splits, 0, 0.0, 0.0, 0.0,
+                                                         *block, self._stream()), "linear (tiles in one round, partial sums)")
+                elif wide > 1 or odd:
                     self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), None, _ptr(stack), m, n, k, n, splits, 0, 0.0, 0.0,
                                                         0.0, self._stream()), "linear (tiles of 256, partial sums)")
                 else:
@@ -662,8 +692,8 @@ class HipBackend:
                 return
             block = self.block_tile(m, n, k) if out.dtype == torch.bfloat16 else None
             if block is not None and not self._odd(x, weight):
-                self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), _ptr(out), m, n, k, n, *block, self._stream()),
-                            "linear (tiles in one round)")
+                self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, n, 1, 0, 0.0, 0.0, 0.0, *block,
+                                                     self._stream()), "linear (tiles in one round)")
                 return
             if out.dtype == torch.bfloat16 and self.wide_takes(m, n, k):
                 self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, n, 1, 0, 0.0, 0.0, 0.0,
@@ -744,6 +774,12 @@ class HipBackend:
         n = out.shape[1]
         tiles_of_128 = (x.dtype == torch.bfloat16 and 64 < m <= self.TILE_GATED_MAX_ROWS and k % 64 == 0
                         and max(m, 2 * n) * k * 2 < 2 ** 32)
+        block = self.block_gated_tile(m, n, k) if x.dtype == torch.bfloat16 else None
+        if block is not None and not self._odd(x, weight):
+            number, *shape = gate_args(activation)
+            self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, out.stride(0), 1, 1 + number, *shape, *block,
+                                                 self._stream()), "gated_linear (tiles in one round)")
+            return
         if x.dtype == torch.bfloat16 and self.wide_gated_takes(m, n, k) or tiles_of_128 and self._odd(x, weight):
             number, *shape = gate_args(activation)
             self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, n, k, out.stride(0), 1, 1 + number,
@@ -780,6 +816,11 @@ class HipBackend:
                     self._stream()), "activated_linear (few rows, matrix cores)")
                 return
             tiles_of_128 = 64 < m <= self.TILE_GATED_MAX_ROWS and k % 64 == 0 and max(m, n) * k * 2 < 2 ** 32
+            block = self.block_gated_tile(m, half, k)
+            if block is not None and not self._odd(x, weight):
+                self._check(self.lib.wllm_gemm_block(_ptr(x), _ptr(weight), _ptr(out), None, m, half, k, n, 1, 1 + number, 0.0, 0.0, 0.0, *block,
+                                                     self._stream()), "activated_linear (tiles in one round)")
+                return
             if self.wide_gated_takes(m, half, k) or tiles_of_128 and self._odd(x, weight):
                 self._check(self.lib.wllm_gemm_wide(_ptr(x), _ptr(weight), _ptr(out), None, m, half, k, n, 1, 1 + number, 0.0, 0.0,
                                                     0.0, self._stream()), "activated_linear (tiles of 256)")
