@@ -35,7 +35,7 @@
 // and become fragments in the wavefront's part of shared memory: a fragment load straight from the
 // cache asks for 64-byte pieces of 16 rows, a pattern the memory system serves more slowly.
 // Scores, maxima, sums and accumulators are float32.
-#include "common.h"
+#include "attention_portion.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
@@ -54,43 +54,50 @@ union Pack16 {
 
 __device__ __forceinline__ uint16_t bf16_bits(float f) { return from_float<bf16>(f).bits; }
 
-// Three workgroups a compute unit (168 registers a lane) where the kernel fits them without spilling;
-// two for the head sizes and page sizes whose staging needs more.
+// Shared memory, a part for each wavefront, used four times: three workgroups share a compute
+// unit's 160 KB.  The wavefront turns its block of keys, which it reads from the cache row by row
+// (whole key rows: contiguous runs the memory system streams much faster than the 64-byte pieces
+// a fragment load straight from the cache would ask for), into fragments, the 16 keys of the
+// first score tile and then the 16 of the second: [16 keys][HD + 8] bfloat16, rows padded so that
+// the fragment reads spread over the banks.  Then it leaves its sums there for the merge, one
+// half of the head after the other: [16 rows][HD / 2 + 4] floats.
+template <int HD>
+struct FewRowsShared {
+    static constexpr int kKeyStride = HD + 8;                                      // elements
+    static constexpr int kPartBytes = 16 * kKeyStride * 2;
+    static constexpr int kMergeStride = HD / 2 + 4;                                // floats
+    static_assert(kRowsPerTile * kMergeStride * 4 <= kPartBytes, "half of the sums fits a wavefront's part");
+    alignas(16) unsigned char raw[4 * kPartBytes];
+    float row_max[4][kRowsPerTile], row_sum[4][kRowsPerTile];
+};
+
+// One work item, by the whole workgroup of 256 threads.
 // SPLIT: the weights of the second product keep 16 bits (rounded weight and remainder, two products).
 template <int HD, bool V16, bool SPLIT>
-__global__ void __launch_bounds__(256, (HD <= 160 || (HD == 256 && V16)) ? 3 : 2)
-paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
-                            const int* __restrict__ block_tables, const int* __restrict__ items,
-                            const int* __restrict__ live_items, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
-                            const int* __restrict__ seg_ctx_len, bf16* __restrict__ out,
-                            float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
-                            int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window,
-                            int q_stride, float cap_scale, float softcap, const float* __restrict__ sinks) {
+__device__ __forceinline__ void
+few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
+              const int* __restrict__ block_tables, const int* __restrict__ items, const int* __restrict__ live_items,
+              const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len, const int* __restrict__ seg_ctx_len,
+              bf16* __restrict__ out, float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
+              int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window, int q_stride, float cap_scale,
+              float softcap, const float* __restrict__ sinks) {
     constexpr int DC = HD / 32;   // 32-wide chunks of the head for the score product
     constexpr int DT = HD / 16;   // 16-row tiles of out^T
-    // Shared memory, a part for each wavefront, used four times: three workgroups share a compute
-    // unit's 160 KB.  The wavefront turns its block of keys, which it reads from the cache row by row
-    // (whole key rows: contiguous runs the memory system streams much faster than the 64-byte pieces
-    // a fragment load straight from the cache would ask for), into fragments, the 16 keys of the
-    // first score tile and then the 16 of the second: [16 keys][HD + 8] bfloat16, rows padded so that
-    // the fragment reads spread over the banks.  Then it leaves its sums there for the merge, one
-    // half of the head after the other: [16 rows][HD / 2 + 4] floats.
-    constexpr int kKeyStride = HD + 8;                                      // elements
-    constexpr int kPartBytes = 16 * kKeyStride * 2;
-    constexpr int kMergeStride = HD / 2 + 4;                                // floats
-    static_assert(kRowsPerTile * kMergeStride * 4 <= kPartBytes, "half of the sums fits a wavefront's part");
-    __shared__ __align__(16) unsigned char shared_raw[4 * kPartBytes];
-    __shared__ float row_max_s[4][kRowsPerTile], row_sum_s[4][kRowsPerTile];
+    constexpr int kKeyStride = FewRowsShared<HD>::kKeyStride, kPartBytes = FewRowsShared<HD>::kPartBytes;
+    constexpr int kMergeStride = FewRowsShared<HD>::kMergeStride;
+    unsigned char* const shared_raw = shared.raw;
+    auto& row_max_s = shared.row_max;
+    auto& row_sum_s = shared.row_sum;
 
     // A captured graph launches as many workgroups as its plan has room for items; the live ones come
     // first.  The item is asked for together with their number, not after it (there is an item, live
     // or stale, for every workgroup of the launch), and brings the segment's lengths with it: one trip
     // to memory for all of them.
-    const int* item = items + static_cast<size_t>(blockIdx.x) * kItemInts;
+    const int* item = items + static_cast<size_t>(index) * kItemInts;
     const int seg = item[0], kvh = item[1] & 0xffff, q_len = item[2], q_start = item[3];
     const int key_begin = item[4], key_end = item[5], partial_slot = item[6], ctx = item[7];
     const int live = live_items != nullptr ? live_items[0] : 0x7fffffff;
-    if (static_cast<int>(blockIdx.x) >= live) return;
+    if (static_cast<int>(index) >= live) return;
     const int row_begin = (item[1] >> 16) * kRowsPerTile;      // the tile's first row: 0 unless a token has more than 16 heads a group
     if (seg < 0) return;    // padding item
     const int lane = threadIdx.x % kWave;
@@ -338,6 +345,70 @@ paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
     }
 }
 
+// Three workgroups a compute unit (168 registers a lane) where the kernel fits them without spilling;
+// two for the head sizes and page sizes whose staging needs more.
+template <int HD, bool V16, bool SPLIT>
+__global__ void __launch_bounds__(256, (HD <= 160 || (HD == 256 && V16)) ? 3 : 2)
+paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
+                            const int* __restrict__ block_tables, const int* __restrict__ items,
+                            const int* __restrict__ live_items, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                            const int* __restrict__ seg_ctx_len, bf16* __restrict__ out,
+                            float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
+                            int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window,
+                            int q_stride, float cap_scale, float softcap, const float* __restrict__ sinks) {
+    __shared__ FewRowsShared<HD> shared;
+    few_rows_item<HD, V16, SPLIT>(shared, blockIdx.x, qkv, cache, block_tables, items, live_items, seg_q_start, seg_q_len,
+                                  seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads, page_size, max_pages,
+                                  scale_log2e, window, q_stride, cap_scale, softcap, sinks);
+}
+
+// A step that carries both prompt portions and decoded tokens: the items of both kernels in one launch, each with the bits it
+// has in its own.  A portion's items are few (at most two a compute unit) and a chain of blocks each, which waits for memory's
+// latency and leaves its bandwidth idle; the decoded tokens' are many and bound by that bandwidth.  One after the other they took
+// the sum of both (8 heads of 256 on one, a portion of 448 tokens over 448 to 1,000 keys beside 60 tokens over 1,500 each: 19.7 + 17.1 us), in one
+// launch 23.5 us.  A compute unit holds two of its workgroups (shared memory and registers of the portions), where it held
+// three of the decoded tokens' kernel; two are enough beside the portions.
+// The kinds alternate in runs of kRoleRun workgroups, eight an XCD, portions first: with all portions in front (runs of 512), 30 tokens
+// over 1,250 keys beside 448 over 896 (16 heads of 128 on four; with the sum of the pieces) took 30.4 us, in runs of 256 / 64
+// 30.2 / 29.8, in runs of 8, one an XCD, 32.2; with few items all are the same.
+constexpr int kRoleRun = 64;
+
+template <int HD, bool SPLIT>
+__global__ void __launch_bounds__(kPrefillThreads, 2)
+paged_attention_both_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
+                            const int* __restrict__ block_tables, const int* __restrict__ portion_items, int num_portions,
+                            const int* __restrict__ items, int num_items,
+                            const int* __restrict__ live_items, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                            const int* __restrict__ seg_ctx_len, bf16* __restrict__ out,
+                            float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
+                            int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window,
+                            int q_stride, float cap_scale, float softcap, const float* __restrict__ sinks) {
+    __shared__ union Either {
+        PortionShared<HD> portion;
+        FewRowsShared<HD> few;
+    } shared;
+    // runs of either kind in turn, then what is left of both lists
+    const int b = blockIdx.x, shorter = min(num_portions, num_items) / kRoleRun * kRoleRun;
+    bool portion;
+    int index;
+    if (b < 2 * shorter) {
+        portion = b / kRoleRun % 2 == 0;
+        index = b / (2 * kRoleRun) * kRoleRun + b % kRoleRun;
+    } else {
+        index = b - shorter;
+        portion = index < num_portions;
+        if (!portion) index = b - num_portions;
+    }
+    if (portion)
+        portion_item<HD, SPLIT>(shared.portion, index, qkv, cache, block_tables, portion_items, seg_q_start, seg_q_len,
+                                seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads, page_size, max_pages,
+                                scale_log2e, window, q_stride, cap_scale, softcap, sinks);
+    else
+        few_rows_item<HD, true, SPLIT>(shared.few, index, qkv, cache, block_tables, items, live_items, seg_q_start,
+                                       seg_q_len, seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads,
+                                       page_size, max_pages, scale_log2e, window, q_stride, cap_scale, softcap, sinks);
+}
+
 // Combines the partial results of a (segment, key/value head) whose keys were split over workgroups.
 // reduce items: seg, kvh, first partial slot, number of splits, first row, slots between splits, 2 unused.
 template <int HD>
@@ -461,6 +532,8 @@ struct AttentionArguments {
     const bf16* qkv;
     const bf16* cache;
     const int* block_tables;
+    const int* portion_items;      // null: the step has none, or they have been launched by themselves
+    int num_portions;
     const int* items;
     const int* live_items;
     int num_items;
@@ -491,9 +564,25 @@ int launch_items(const AttentionArguments& a) {
     return 0;
 }
 
+template <int HD, bool SPLIT>
+int launch_both(const AttentionArguments& a) {
+    paged_attention_both_kernel<HD, SPLIT><<<a.num_portions + a.num_items, kPrefillThreads, 0, a.stream>>>(
+        a.qkv, a.cache, a.block_tables, a.portion_items, a.num_portions, a.items, a.num_items, a.live_items, a.seg_q_start,
+        a.seg_q_len, a.seg_ctx_len, a.out, a.partial_o, a.partial_ml, a.num_heads, a.num_kv_heads, a.page_size, a.max_pages,
+        a.scale_log2e, a.window, a.q_stride, a.cap_scale, a.softcap, a.sinks);
+    return 0;
+}
+
 template <int HD>
 int launch_all(const AttentionArguments& a) {
-    if (a.num_items > 0) {
+    if (a.num_portions > 0) {
+        if constexpr (HD == 64 || HD == 128 || HD == 256) {
+            const int status = a.split_weights ? launch_both<HD, true>(a) : launch_both<HD, false>(a);
+            if (status != 0) return status;
+        } else {
+            return -1;
+        }
+    } else if (a.num_items > 0) {
         const int status = a.page_size % 8 == 0
             ? (a.split_weights ? launch_items<HD, true, true>(a) : launch_items<HD, true, false>(a))
             : (a.split_weights ? launch_items<HD, false, true>(a) : launch_items<HD, false, false>(a));
@@ -515,7 +604,10 @@ int launch_all(const AttentionArguments& a) {
 
 // Returns 0, a HIP error code, or -1 for sizes these kernels do not take.  `live_items`: null, or a
 // device int that says how many of the `num_items` items count (a captured graph's plan).
-WLLM_API int wllm_paged_attention_mfma(const void* qkv, const void* cache, const int* block_tables, const int* items,
+// `portion_items`: null, or the items of the prompt portions of the same step, which then run in the same launch: pages of a power
+// of two from 8, heads of 64, 128 and 256.
+WLLM_API int wllm_paged_attention_mfma(const void* qkv, const void* cache, const int* block_tables,
+                                       const int* portion_items, int num_portions, const int* items,
                                        const int* live_items, int num_items, const int* reduce_items,
                                        int num_reduce_items, const int* seg_q_start, const int* seg_q_len,
                                        const int* seg_ctx_len, void* out, float* partial_o, float* partial_ml,
@@ -526,11 +618,14 @@ WLLM_API int wllm_paged_attention_mfma(const void* qkv, const void* cache, const
         num_heads >= (1 << 16))       // an item holds a key/value head and a tile's first row in 16 bits each
         return -1;
     if (q_stride < num_heads * head_dim || q_stride % 8 != 0 || softcap < 0.f) return -1;
+    if (num_portions < 0 || (num_portions > 0 && (portion_items == nullptr || num_items <= 0 || page_size < 8 ||
+                                                  (page_size & (page_size - 1)) != 0)))
+        return -1;
     // with a cap the kernel scales and bends the score itself; the softmax then works on final scores
     const float in_exponent = softcap > 0.f ? 1.f : scale;
     const float cap_scale = softcap > 0.f ? scale / softcap : 0.f;
-    const AttentionArguments a = {static_cast<const bf16*>(qkv), static_cast<const bf16*>(cache), block_tables, items,
-                                  live_items, num_items, reduce_items, num_reduce_items, seg_q_start, seg_q_len,
+    const AttentionArguments a = {static_cast<const bf16*>(qkv), static_cast<const bf16*>(cache), block_tables,
+                                  portion_items, num_portions, items, live_items, num_items, reduce_items, num_reduce_items, seg_q_start, seg_q_len,
                                   seg_ctx_len, static_cast<bf16*>(out), partial_o, partial_ml, num_heads, num_kv_heads,
                                   page_size, max_pages, in_exponent * 1.4426950408889634f, window, q_stride, cap_scale,
                                   softcap, split_weights, sinks, stream};

@@ -46,7 +46,7 @@ _SIGNATURES = {
                                      c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                      c_float, c_int, c_int, c_float, c_void_p, c_void_p],
     "wllm_paged_attention_generic_chunk_keys": [],
-    "wllm_paged_attention_mfma": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
+    "wllm_paged_attention_mfma": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float,
                                   c_int, c_int, c_float, c_int, c_void_p, c_void_p],
     "wllm_paged_attention_mfma_f32": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
@@ -214,6 +214,12 @@ class HipBackend:
         return (dtype in (torch.bfloat16, torch.float32) and head_dim % 32 == 0 and 32 <= head_dim <= 256
                 and page_size % 4 == 0)
 
+    @staticmethod
+    def portions_beside(head_dim: int, page_size: int) -> bool:
+        """Whether a step's prompt portions run in one launch with its decoded tokens: the sizes of the portions' kernel that loads
+        into shared memory (`attention_portion.h`).  The blocks of 128 rows of long prompts fill the device by themselves."""
+        return head_dim in (64, 128, 256) and page_size >= 8 and page_size & (page_size - 1) == 0
+
     # Up to how many (items of 16 rows by 128 keys) x (elements of a head) float32 prompt portions are tiles: these take a time in
     # proportion, the blocks of 64 rows hardly less for few of them than for the 256 that give every compute unit one.
     # Tiles against blocks, heads of 256: 309 items 27 and 67 us, 1,280 61 and 75, 1,631 73 and 77, 2,080 89 and 79, 2,304 92 and
@@ -305,7 +311,9 @@ class HipBackend:
                     block_tables.shape[1], scale, window, q_stride, softcap, _ptr(sinks), self._stream()),
                     "paged_attention (matrix cores, float32)")
                 return
-            if plan.num_prefill:
+            together = (plan.num_prefill and plan.num_items and plan.prefill_rows != PROMPT_ROWS
+                        and self.portions_beside(head_dim, page_size))
+            if plan.num_prefill and not together:
                 prefill = self.lib.wllm_paged_attention_prompt if plan.prefill_rows == PROMPT_ROWS else self.lib.wllm_paged_attention_prefill
                 self._check(prefill(
                     _ptr(qkv), _ptr(cache), _ptr(block_tables), _ptr(plan.prefill_items), plan.num_prefill,
@@ -317,8 +325,8 @@ class HipBackend:
             if plan.num_items == 0 and plan.num_reduce == 0:
                 return
             self._check(self.lib.wllm_paged_attention_mfma(
-                _ptr(qkv), _ptr(cache), _ptr(block_tables), _ptr(plan.items),
-                _ptr(plan.live_items), plan.num_items, _ptr(plan.reduce_items),
+                _ptr(qkv), _ptr(cache), _ptr(block_tables), _ptr(plan.prefill_items) if together else None,
+                plan.num_prefill if together else 0, _ptr(plan.items), _ptr(plan.live_items), plan.num_items, _ptr(plan.reduce_items),
                 plan.num_reduce, _ptr(seg_q_start), _ptr(seg_q_len), _ptr(seg_ctx_len), _ptr(out),
                 _ptr(plan.partial_o), _ptr(plan.partial_ml), num_heads, num_kv_heads, head_dim, page_size,
                 block_tables.shape[1], scale, window, q_stride, softcap, int(exact_weights), _ptr(sinks), self._stream()),
