@@ -392,6 +392,15 @@ __global__ void rope_cache_vec_kernel(T* __restrict__ qkv, const int* __restrict
     }
 }
 
+// (`head_prepare.hip`)
+WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const float* parts, int splits,
+                               long long split_stride, const float* bias, int bias_width, const int* positions,
+                               const float* inv_freq, const int* slots, void* cache, long long num_pages, int n,
+                               int num_heads, int num_kv_heads, int head_dim, int rotary_dim, int interleaved,
+                               float norm_eps, int norm_dim, int values_are_keys, int page_size, const float* pre_q,
+                               const float* pre_k, float pre_eps, float rot_scale, float temp_coef, int temp_every,
+                               hipStream_t stream);
+
 WLLM_API int wllm_rope_cache_write(void* qkv, int is_bf16, const float* parts, int splits, long long split_stride,
                                    const float* bias, const int* positions, const float* inv_freq, const int* slots,
                                    void* cache, long long num_pages, int n, int num_heads, int num_kv_heads,
@@ -413,6 +422,17 @@ WLLM_API int wllm_rope_cache_write(void* qkv, int is_bf16, const float* parts, i
                 num_kv_heads, head_dim, rotary_dim, page_size, num_pages);
         return launch_status();
     }
+    const int width = (num_heads + 2 * num_kv_heads) * head_dim;
+    // Few tokens with a bias or a stack of partial sums: the kernel above is a workgroup a token that goes to memory once for the
+    // positions, once for each round of heads and once for the values; that of `head_prepare.hip` has a workgroup for every four
+    // heads, which ask for all they need at once (the same numbers in the same order, so the same bits).  64 tokens of 8 heads of 256 on one
+    // in a captured step: 5.5 to 5.2 us traced, the step 2,183 to 2,166; 64 of 40 heads of 64 on 40 9.1 to 7.0.  From some 200 tokens on the
+    // workgroups are more than run at once and each makes the sines again (200 / 256 tokens 4.7 / 4.8 and 5.2 / 5.3).
+    if (n <= 128 && inv_freq && head_dim <= 256 && head_dim % 4 == 0 && rotary_dim % 8 == 0 && rotary_dim <= head_dim &&
+        page_size > 0 && num_heads + 2 * num_kv_heads <= 4096)
+        return wllm_head_prepare(qkv, is_bf16, width, parts, splits, split_stride, bias, bias ? width : 0, positions, inv_freq,
+                                 slots, cache, num_pages, n, num_heads, num_kv_heads, head_dim, rotary_dim, 0, -1.f, head_dim,
+                                 0, page_size, nullptr, nullptr, -1.f, 1.f, 0.f, 0, stream);
     const int threads = pairs >= 1024 ? 1024 : (pairs >= 512 ? 512 : 256);
     if (is_bf16)
         rope_cache_kernel<bf16><<<n, threads, 0, stream>>>(static_cast<bf16*>(qkv), parts, splits,
