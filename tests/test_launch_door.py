@@ -119,3 +119,54 @@ def test_operands_of_the_wrong_kind_are_named():
                           ((t, "x", torch.float32, (4, 9)), r"x: shape \(4, 8\), expected \(4, 9\)"), ((None, "x", torch.float32), "x: expected a tensor")):
         with pytest.raises(ops.KernelShapeError, match=message):
             ops._dense(*args)
+
+
+# ---- which build of the module is loaded, and how it is built -----------------------------------------------------------------------
+
+@pytest.fixture
+def elsewhere(tmp_path, monkeypatch):
+    """A package folder and a temporary folder that hold no build, in a process that has loaded none."""
+    (tmp_path / "package").mkdir()
+    monkeypatch.setattr(library, "PACKAGE_DIR", str(tmp_path / "package"))
+    monkeypatch.setattr(library.tempfile, "tempdir", str(tmp_path))
+    monkeypatch.setattr(library, "_loaded", {})
+    return tmp_path / "package"
+
+
+def a_build_that_fails(monkeypatch):
+    monkeypatch.setattr(library, "_door_command", lambda hipcc, target: ["/bin/sh", "-c", "echo no headers >&2; exit 1"])
+
+
+@pytest.mark.parametrize("of", ["torch", "abi", "interpreter", "source"])
+def test_a_build_for_something_else_is_not_loaded(of, elsewhere, monkeypatch):
+    """The module is compiled against headers of torch and of the interpreter: one for others would look for a tensor's fields in the wrong
+    places, so it is none."""
+    here = library._door_places()[0]
+    with open(here, "w") as f:
+        f.write("a build that would be taken")
+    if of == "torch":
+        monkeypatch.setattr(torch, "__version__", "9.9.9")
+    elif of == "abi":
+        monkeypatch.setattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", not torch._C._GLIBCXX_USE_CXX11_ABI)
+    elif of == "interpreter":
+        monkeypatch.setattr(library.sysconfig, "get_config_var", lambda name: "cpython-399")
+    else:
+        (elsewhere / "launch_door.cpp").write_text("// another")
+        monkeypatch.setattr(library, "SOURCE_DIR", str(elsewhere))
+    assert here not in library._door_places()
+    a_build_that_fails(monkeypatch)
+    assert library.built_door() is None
+    with pytest.raises(library.KernelLibraryMissing, match="no headers"):
+        library.door()
+
+
+def test_a_module_that_cannot_be_loaded_is_built_again(elsewhere):
+    """And importing the operations needs none that can be loaded."""
+    here = library._door_places()[0]
+    for name in (here, here.replace(".so", "0.so").rsplit(".", 2)[0] + ".0123456789ab.so"):
+        with open(name, "w") as f:
+            f.write("no module")
+    assert library.built_door() is None
+    door = library.door()
+    assert door is not None and door.address(None) is None
+    assert [p.name for p in elsewhere.iterdir()] == [here.rsplit("/", 1)[1]]         # what older sources left is gone

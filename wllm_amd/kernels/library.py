@@ -5,7 +5,8 @@ shared library, `wllm_amd/libwllm_kernels.so`, whose `extern "C"` entry points
 are called with raw device pointers and a stream.  The kernels are compiled against nothing of
 torch; beside them `csrc/launch_door.cpp`, host code alone, becomes a CPython module
 (`door()`) through which the framework's own calls go, since ctypes would take half
-as long for each as the launch itself.  A build takes about a minute from nothing.
+as long for each as the launch itself.  The module is compiled against the interpreter's and torch's
+headers, so its file's name says for which of them it is.  A build takes about a minute from nothing.
 
 `load()` loads the library if it is built from the present sources and builds it
 first if not (a line is printed per compiled file, so that a first call in a
@@ -14,20 +15,23 @@ written to, the build goes to a folder under the system's temporary directory.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import hashlib
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
+from importlib import util
 
 PACKAGE_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE_DIR = os.path.join(PACKAGE_DIR, "csrc")
 LIBRARY_NAME = "libwllm_kernels.so"
-DOOR_SOURCE, DOOR_NAME = "launch_door.cpp", "launch_door.so"
+DOOR_SOURCE, DOOR_NAME = "launch_door.cpp", "launch_door"
 ARCH = "gfx950"
 # packed float32 instructions are switched off for all device code
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
@@ -50,7 +54,7 @@ def _fingerprint(source_dir: str = SOURCE_DIR) -> str:
     folders = [source_dir] if os.path.samefile(source_dir, SOURCE_DIR) else [source_dir, SOURCE_DIR]
     for folder in folders:
         for name in sorted(os.listdir(folder)):
-            if name.endswith(".h") or (folder == source_dir and name.endswith((".hip", ".cpp"))):
+            if name.endswith(".h") or (folder == source_dir and name.endswith(".hip")):
                 h.update(name.encode())
                 with open(os.path.join(folder, name), "rb") as f:
                     h.update(f.read())
@@ -96,8 +100,6 @@ def _is_current(lib_path: str, fingerprint: str) -> bool:
 
 def _door_command(hipcc: str, target: str) -> list:
     """Compiles the module of `DOOR_SOURCE`: host code, against the interpreter's and torch's headers."""
-    import sysconfig
-
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
     include = [a for folder in [sysconfig.get_paths()["include"]] + include_paths() for a in ("-isystem", folder)]
@@ -105,6 +107,40 @@ def _door_command(hipcc: str, target: str) -> list:
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + include + [
             os.path.join(SOURCE_DIR, DOOR_SOURCE), "-o", target] + [f"-L{p}" for p in library_paths()] + [
             "-ltorch_python", "-ltorch_cpu", "-lc10"]         # (found where `import torch` has loaded them)
+
+
+def _door_places() -> list:
+    """Where the module lies, beside the kernel library first.  Its name holds a hash of what it is compiled against (the interpreter, and
+    torch, whose inline accessors know how a tensor is laid out) and one of its source: a file of that name can be loaded, and a build for
+    another torch or interpreter is left alone."""
+    import torch
+    host = "\n".join([sys.version, str(sysconfig.get_config_var("SOABI")), torch.__version__, str(getattr(torch.version, "git_version", "")),
+                      str(torch._C._GLIBCXX_USE_CXX11_ABI)])
+    with open(os.path.join(SOURCE_DIR, DOOR_SOURCE), "rb") as f:
+        source = f.read()
+    name = ".".join([DOOR_NAME, hashlib.sha256(host.encode()).hexdigest()[:12], hashlib.sha256(source).hexdigest()[:12], "so"])
+    return [os.path.join(PACKAGE_DIR, name), os.path.join(tempfile.gettempdir(), f"wllm_amd_build_{os.getuid()}_door", name)]
+
+
+def build_door(verbose: bool = True) -> str:
+    """Compiles the module and returns its path."""
+    path = next((p for p in _door_places() if _writable(os.path.dirname(p))), None)
+    if path is None:
+        raise KernelLibraryMissing(f"no writable place for {DOOR_NAME}")
+    t0, tmp = time.time(), f"{path}.tmp{os.getpid()}"
+    r = subprocess.run(_door_command(_hipcc(), tmp), capture_output=True, text=True)
+    if r.returncode != 0:
+        raise KernelLibraryMissing(f"hipcc failed on {DOOR_SOURCE}:\n{r.stderr[-4000:]}")
+    os.replace(tmp, path)
+    # (builds of older sources for the same interpreter and torch; a process that has one loaded keeps it)
+    of_host = os.path.basename(path).rsplit(".", 2)[0] + "."
+    for name in os.listdir(os.path.dirname(path)):
+        if name.startswith(of_host) and name.endswith(".so") and name != os.path.basename(path):
+            with contextlib.suppress(FileNotFoundError):
+                os.remove(os.path.join(os.path.dirname(path), name))
+    if verbose:
+        print(f"[wllm_amd build] built {path} in {time.time() - t0:.0f} s", file=sys.stderr, flush=True)
+    return path
 
 
 def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR, library_name: str = LIBRARY_NAME) -> str:
@@ -139,21 +175,15 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
         return name, obj, r
 
     objects = []
-    door_path = door_tmp = None
-    if os.path.samefile(source_dir, SOURCE_DIR):
-        door_path = os.path.join(os.path.dirname(lib_path), DOOR_NAME)
-        door_tmp = door_path + f".tmp{os.getpid()}"
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(names)))) as pool:
-        door_run = pool.submit(subprocess.run, _door_command(hipcc, door_tmp), capture_output=True, text=True, env=env) if door_path else None
+        door_run = pool.submit(build_door, verbose) if os.path.samefile(source_dir, SOURCE_DIR) else None
         for name, obj, r in pool.map(compile_one, names):
             if r.returncode != 0:
                 raise KernelLibraryMissing(f"hipcc failed on {name}:\n{r.stderr[-4000:]}")
             say(f"compiled {name} ({time.time() - t0:.0f} s)")
             objects.append(obj)
         if door_run is not None:
-            if door_run.result().returncode != 0:
-                raise KernelLibraryMissing(f"hipcc failed on {DOOR_SOURCE}:\n{door_run.result().stderr[-4000:]}")
-            os.replace(door_tmp, door_path)
+            door_run.result()
     tmp = lib_path + f".tmp{os.getpid()}"
     r = subprocess.run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objects,
                        capture_output=True, text=True, env=env)
@@ -170,33 +200,32 @@ _loaded: dict = {}
 
 
 def built_door():
-    """The module of `launch_door.cpp` if it is built from the present sources, else None: nothing is built for it."""
+    """The module of `launch_door.cpp` if it is built from the present source for this interpreter and this torch and can be loaded, else
+    None: nothing is built for it."""
     if DOOR_NAME not in _loaded:
-        from importlib import util
-        fingerprint = _fingerprint()
-        for lib_path, _ in _locations(fingerprint):
-            path = os.path.join(os.path.dirname(lib_path), DOOR_NAME)
-            if _is_current(lib_path, fingerprint) and os.path.isfile(path):
-                import torch  # noqa: F401  (the module's symbols of torch)
-                spec = util.spec_from_file_location("launch_door", path)
-                try:
-                    module = util.module_from_spec(spec)
-                    spec.loader.exec_module(module)
-                except ImportError as e:
-                    raise KernelLibraryMissing(f"{path} cannot be loaded: {e}") from e
-                _loaded[DOOR_NAME] = module
-                break
+        import torch  # noqa: F401  (the module's symbols of torch)
+        for path in _door_places():
+            if not os.path.isfile(path):
+                continue
+            spec = util.spec_from_file_location(DOOR_NAME, path)
+            try:
+                module = util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+            except ImportError:
+                continue
+            _loaded[DOOR_NAME] = module
+            break
     return _loaded.get(DOOR_NAME)
 
 
 def door():
-    """The module of `launch_door.cpp`; built first, with the kernels, when no build of the present sources exists."""
+    """The module of `launch_door.cpp`, built first when there is none that can be loaded."""
     module = built_door()
     if module is None:
-        build()
+        path = build_door()
         module = built_door()
-    if module is None:
-        raise KernelLibraryMissing(f"{DOOR_NAME} is missing beside the kernel library")
+        if module is None:
+            raise KernelLibraryMissing(f"{path} cannot be loaded")
     return module
 
 
