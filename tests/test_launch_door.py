@@ -121,7 +121,7 @@ def test_operands_of_the_wrong_kind_are_named():
             ops._dense(*args)
 
 
-# ---- which build of the module is loaded, and how it is built -----------------------------------------------------------------------
+# ---- which build of the module is loaded, and what happens without one --------------------------------------------------------------
 
 @pytest.fixture
 def elsewhere(tmp_path, monkeypatch):
@@ -155,9 +155,7 @@ def test_a_build_for_something_else_is_not_loaded(of, elsewhere, monkeypatch):
         monkeypatch.setattr(library, "SOURCE_DIR", str(elsewhere))
     assert here not in library._door_places()
     a_build_that_fails(monkeypatch)
-    assert library.built_door() is None
-    with pytest.raises(library.KernelLibraryMissing, match="no headers"):
-        library.door()
+    assert library.built_door() is None and library.door() is None
 
 
 def test_a_module_that_cannot_be_loaded_is_built_again(elsewhere):
@@ -170,3 +168,34 @@ def test_a_module_that_cannot_be_loaded_is_built_again(elsewhere):
     door = library.door()
     assert door is not None and door.address(None) is None
     assert [p.name for p in elsewhere.iterdir()] == [here.rsplit("/", 1)[1]]         # what older sources left is gone
+
+
+def test_the_kernels_are_built_without_the_module(elsewhere, monkeypatch, capsys):
+    """Where the module cannot be compiled (no headers, another processor) the kernels are, as if there were none."""
+    (elsewhere / "one.hip").write_text('extern "C" __attribute__((visibility("default"))) int one() { return 1; }\n')
+    (elsewhere / "launch_door.cpp").write_text("#error no")
+    monkeypatch.setattr(library, "SOURCE_DIR", str(elsewhere))
+    a_build_that_fails(monkeypatch)
+    path = library.build(source_dir=str(elsewhere))
+    assert ctypes.CDLL(path).one() == 1 and library.door() is None
+    assert "calls go through ctypes: no headers" in capsys.readouterr().err
+
+
+@pytest.fixture
+def a_backend(monkeypatch):
+    """Makes one as it would be made on a GPU."""
+    from wllm_amd.kernels import hip_backend
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    return hip_backend.HipBackend
+
+
+def test_a_backend_without_the_module_calls_through_ctypes(a_backend, monkeypatch):
+    from wllm_amd.kernels import hip_backend
+    monkeypatch.setattr(hip_backend, "door", lambda: None)
+    backend = a_backend()
+    assert isinstance(backend.lib.wllm_split_sum, ctypes._CFuncPtr) and backend.lib.wllm_split_sum.argtypes[-1] is ctypes.c_void_p
+    with pytest.raises(hip_backend.KernelError, match="not on the GPU"):
+        backend._on_gpu(None, torch.zeros(2))
+    op = next(o for o in ops._REGISTERED.values() if o.own)
+    assert backend._entry(getattr(backend.lib.raw, op.entry_point), op.argtypes) is getattr(backend.lib.raw, op.entry_point)

@@ -89,9 +89,10 @@ class HipBackend:
     def __init__(self):
         if not torch.cuda.is_available():
             raise KernelError("no GPU is visible; the kernels run on gfx950 only and there is no other path")
-        self._door = door()
-        self._on_gpu = self._door.make_on_gpu(KernelError)
         raw = load()
+        self._door = door()
+        if self._door is not None:
+            self._on_gpu = self._door.make_on_gpu(KernelError)
         self._device_index = torch.cuda.current_device()
         self._partial_o = None
         self._slots_of = {}                # device -> workgroups of the prompt kernel it runs at once
@@ -107,7 +108,7 @@ class HipBackend:
             setattr(self.lib, name, self._entry(getattr(raw, name), argtypes))
 
     @staticmethod
-    def _on_gpu(*tensors) -> None:      # (a backend with a library has the native one)
+    def _on_gpu(*tensors) -> None:      # (a backend with the native module has its)
         for t in tensors:
             if t is not None and not t.is_cuda:
                 raise KernelError("a kernel operand is not on the GPU")
@@ -115,11 +116,11 @@ class HipBackend:
     _CODES = {c_void_p: "p", c_int: "i", c_longlong: "l", c_float: "f"}
 
     def _entry(self, fn, argtypes):
-        """What calls the library's function `fn` with arguments of these types: an entry of the native module, or, for
-        other types or a function that is not a library's, `fn` itself."""
+        """What calls the function `fn`, a ctypes library's, with arguments of these types: an entry of the native module, or,
+        without the module and for types or numbers of arguments that it has no room for, `fn` itself."""
         fn.argtypes, fn.restype = argtypes, c_int
         codes = [self._CODES.get(a) for a in argtypes]
-        if None in codes or len(codes) > 48 or codes.count("f") > 8 or len(codes) - codes.count("f") > 40:
+        if self._door is None or None in codes or len(codes) > 48 or codes.count("f") > 8 or len(codes) - codes.count("f") > 40:
             return fn
         return self._door.Entry(ctypes.cast(fn, c_void_p).value, "".join(codes))
 

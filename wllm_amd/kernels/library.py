@@ -6,7 +6,8 @@ are called with raw device pointers and a stream.  The kernels are compiled agai
 torch; beside them `csrc/launch_door.cpp`, host code alone, becomes a CPython module
 (`door()`) through which the framework's own calls go, since ctypes would take half
 as long for each as the launch itself.  The module is compiled against the interpreter's and torch's
-headers, so its file's name says for which of them it is.  A build takes about a minute from nothing.
+headers, so its file's name says for which of them it is; where it cannot be built, ctypes does its
+work.  A build takes about a minute from nothing.
 
 `load()` loads the library if it is built from the present sources and builds it
 first if not (a line is printed per compiled file, so that a first call in a
@@ -27,6 +28,7 @@ import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
 from importlib import util
+from typing import Optional
 
 PACKAGE_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE_DIR = os.path.join(PACKAGE_DIR, "csrc")
@@ -122,15 +124,28 @@ def _door_places() -> list:
     return [os.path.join(PACKAGE_DIR, name), os.path.join(tempfile.gettempdir(), f"wllm_amd_build_{os.getuid()}_door", name)]
 
 
-def build_door(verbose: bool = True) -> str:
-    """Compiles the module and returns its path."""
+def build_door(verbose: bool = True) -> Optional[str]:
+    """Compiles the module and returns its path; None, with a line that says why, where that is not possible here (no compiler, no headers
+    of the interpreter or of torch, another processor): the kernels don't need it."""
+    def say(msg: str) -> None:
+        if verbose:
+            print(f"[wllm_amd build] {msg}", file=sys.stderr, flush=True)
+
     path = next((p for p in _door_places() if _writable(os.path.dirname(p))), None)
     if path is None:
-        raise KernelLibraryMissing(f"no writable place for {DOOR_NAME}")
+        say(f"no writable place for {DOOR_NAME}: calls go through ctypes")
+        return None
     t0, tmp = time.time(), f"{path}.tmp{os.getpid()}"
-    r = subprocess.run(_door_command(_hipcc(), tmp), capture_output=True, text=True)
-    if r.returncode != 0:
-        raise KernelLibraryMissing(f"hipcc failed on {DOOR_SOURCE}:\n{r.stderr[-4000:]}")
+    try:
+        r = subprocess.run(_door_command(_hipcc(), tmp), capture_output=True, text=True)
+        failure = r.stderr[-4000:] if r.returncode != 0 else ""
+    except (KernelLibraryMissing, OSError, ImportError) as e:
+        failure = str(e)
+    if failure or not os.path.isfile(tmp):
+        say(f"{DOOR_SOURCE} cannot be built here, calls go through ctypes: {failure or 'no module came out'}")
+        if os.path.isfile(tmp):
+            os.remove(tmp)
+        return None
     os.replace(tmp, path)
     # (builds of older sources for the same interpreter and torch; a process that has one loaded keeps it)
     of_host = os.path.basename(path).rsplit(".", 2)[0] + "."
@@ -138,8 +153,7 @@ def build_door(verbose: bool = True) -> str:
         if name.startswith(of_host) and name.endswith(".so") and name != os.path.basename(path):
             with contextlib.suppress(FileNotFoundError):
                 os.remove(os.path.join(os.path.dirname(path), name))
-    if verbose:
-        print(f"[wllm_amd build] built {path} in {time.time() - t0:.0f} s", file=sys.stderr, flush=True)
+    say(f"built {path} in {time.time() - t0:.0f} s")
     return path
 
 
@@ -176,14 +190,13 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
 
     objects = []
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(names)))) as pool:
-        door_run = pool.submit(build_door, verbose) if os.path.samefile(source_dir, SOURCE_DIR) else None
+        if os.path.samefile(source_dir, SOURCE_DIR):
+            pool.submit(build_door, verbose)
         for name, obj, r in pool.map(compile_one, names):
             if r.returncode != 0:
                 raise KernelLibraryMissing(f"hipcc failed on {name}:\n{r.stderr[-4000:]}")
             say(f"compiled {name} ({time.time() - t0:.0f} s)")
             objects.append(obj)
-        if door_run is not None:
-            door_run.result()
     tmp = lib_path + f".tmp{os.getpid()}"
     r = subprocess.run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objects,
                        capture_output=True, text=True, env=env)
@@ -219,13 +232,12 @@ def built_door():
 
 
 def door():
-    """The module of `launch_door.cpp`, built first when there is none that can be loaded."""
+    """The module of `launch_door.cpp`, built first when there is none that can be loaded; None where it cannot be built."""
     module = built_door()
-    if module is None:
-        path = build_door()
+    if module is None and (path := build_door()) is not None:
         module = built_door()
         if module is None:
-            raise KernelLibraryMissing(f"{path} cannot be loaded")
+            print(f"[wllm_amd build] {path} cannot be loaded, calls go through ctypes", file=sys.stderr, flush=True)
     return module
 
 
