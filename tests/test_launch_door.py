@@ -159,7 +159,7 @@ def test_a_build_for_something_else_is_not_loaded(of, elsewhere, monkeypatch):
 
 
 def test_a_module_that_cannot_be_loaded_is_built_again(elsewhere):
-    """And importing the operations needs none that can be loaded."""
+    """And importing the operations needs none."""
     here = library._door_places()[0]
     for name in (here, here.replace(".so", "0.so").rsplit(".", 2)[0] + ".0123456789ab.so"):
         with open(name, "w") as f:
@@ -183,11 +183,32 @@ def test_the_kernels_are_built_without_the_module(elsewhere, monkeypatch, capsys
 
 @pytest.fixture
 def a_backend(monkeypatch):
-    """Makes one as it would be made on a GPU."""
+    """Makes one as it would be made on a GPU, and undoes at the end of the test what it changes."""
     from wllm_amd.kernels import hip_backend
     monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
-    return hip_backend.HipBackend
+    before = ops._address
+    for module, name, plain in ((ops, "_dense", ops._plain_dense), (ops, "_address", plain_address), (hip_backend, "_ptr", plain_address)):
+        monkeypatch.setattr(module, name, plain)
+    ops._use_address(plain_address)
+    yield hip_backend.HipBackend
+    ops._use_address(before)
+
+
+def plain_address(t):
+    return t.data_ptr() if t is not None else None
+
+
+def test_a_backend_brings_the_native_look_at_operands(door, a_backend, monkeypatch):
+    """Also in a process that imported the operations before there was a build."""
+    from wllm_amd.kernels import hip_backend
+    backend = a_backend()
+    assert type(backend.lib.wllm_split_sum) is door.Entry and type(backend._on_gpu).__name__ == "Bound"
+    assert type(ops._dense).__name__ == "Bound" and ops._address is hip_backend._ptr is door.address
+    seen = []
+    monkeypatch.setattr(ops, "_use_address", seen.append)
+    ops.use_native(door)
+    assert seen == [door.address]
 
 
 def test_a_backend_without_the_module_calls_through_ctypes(a_backend, monkeypatch):
@@ -195,7 +216,17 @@ def test_a_backend_without_the_module_calls_through_ctypes(a_backend, monkeypatc
     monkeypatch.setattr(hip_backend, "door", lambda: None)
     backend = a_backend()
     assert isinstance(backend.lib.wllm_split_sum, ctypes._CFuncPtr) and backend.lib.wllm_split_sum.argtypes[-1] is ctypes.c_void_p
+    assert ops._dense is ops._plain_dense and hip_backend._ptr is plain_address
     with pytest.raises(hip_backend.KernelError, match="not on the GPU"):
         backend._on_gpu(None, torch.zeros(2))
     op = next(o for o in ops._REGISTERED.values() if o.own)
     assert backend._entry(getattr(backend.lib.raw, op.entry_point), op.argtypes) is getattr(backend.lib.raw, op.entry_point)
+
+
+def test_registered_launches_take_the_address_that_is_in_use():
+    t, seen = torch.zeros(3, 4, dtype=torch.bfloat16), []
+    try:
+        ops._use_address(lambda x: seen.append(x) or 7)
+        assert ops._REGISTERED["activation"].launch(lambda *args: args, 0, t, t, "silu")[:2] == (7, 7) and len(seen) == 2
+    finally:
+        ops._use_address(ops._address)

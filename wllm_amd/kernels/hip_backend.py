@@ -92,6 +92,9 @@ class HipBackend:
         raw = load()
         self._door = door()
         if self._door is not None:
+            global _ptr
+            ops.use_native(self._door)
+            _ptr = ops._address
             self._on_gpu = self._door.make_on_gpu(KernelError)
         self._device_index = torch.cuda.current_device()
         self._partial_o = None

@@ -20,8 +20,6 @@ from typing import Optional
 
 import torch
 
-from wllm_amd.kernels.library import built_door
-
 _ACT = (torch.float32, torch.bfloat16)
 HEAD_DIM_STEP, MAX_HEAD_DIM = 4, 256      # what `paged_attention` takes: multiples of 4 up to 256
 _backend = None
@@ -79,11 +77,15 @@ def _address(t):
     return t.data_ptr() if t is not None else None
 
 
-# The same two as native code, where it is built: they run some forty times a layer.  (What is not plainly in order comes back to the
-# functions above; without the build these do.)
-_native = built_door()
-if _native is not None:
-    _dense, _address = _native.make_dense(_dense), _native.address
+_plain_dense = _dense
+
+
+def use_native(door) -> None:
+    """The two above as native code, for this process: they run some forty times a layer.  (What is not plainly in order comes back to the
+    plain look at an operand.)"""
+    global _dense, _address
+    _dense, _address = door.make_dense(_plain_dense), door.address
+    _use_address(_address)
 
 
 # ---- operations that parts bring with them ------------------------------------------------------
@@ -1589,9 +1591,14 @@ def moe_experts_down(act: torch.Tensor, w: torch.Tensor, plan: torch.Tensor, wei
 
 
 # ---- the framework's own operations that go through the same door as a part's ------------------
-def _register_own() -> None:
+def _register_own():
+    """Registers them, and returns what gives their launches another function for an operand's address."""
     from ctypes import c_float, c_int, c_longlong, c_void_p
     p = _address
+
+    def use_address(address) -> None:
+        nonlocal p
+        p = address
 
     register_op("embed_lookup", entry_point="wllm_embed_lookup",
                 argtypes=[c_void_p, c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
@@ -1827,8 +1834,9 @@ def _register_own() -> None:
                 launch=lambda fn, stream, act, w, plan, weights, out, weighted=True: fn(
                     p(act), p(w), p(plan), moe_max_tiles(act.shape[0], w.shape[0], MOE_BIG_TILE_ROWS), p(None), p(out),
                     p(weights if weighted else None), -1, act.shape[0], w.shape[1], act.shape[1], weights.shape[1], weights.shape[0], stream))
+    return use_address
 
 
-_register_own()
+_use_address = _register_own()
 for _op in _REGISTERED.values():
     _op.own = True
