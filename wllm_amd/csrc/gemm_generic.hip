@@ -378,24 +378,37 @@ F32Cut f32_cut(int M, int N, int K, bool may_split) {
     const int segments = (K + kF32Segment - 1) / kF32Segment;
     F32Cut best{4, 4, 0, false};
     float least = 3.4e38f;
-    for (const auto& t : kTiles) {
-        const long long tiles = static_cast<long long>((M + 32 * t.wm - 1) / (32 * t.wm)) * ((N + 32 * t.wn - 1) / (32 * t.wn));
-        for (int per_group = segments; per_group >= 1; per_group = per_group == 1 ? 0 : (per_group + 1) / 2) {
-            const int groups = (segments + per_group - 1) / per_group;
-            const bool split = groups > 1;
-            if (split && (!may_split || groups > 65535 || static_cast<long long>(segments) * M * N > kMostPartials)) break;
-            const long long on_a_unit = (tiles * groups + kUnits - 1) / kUnits;
-            float us = per_group * ((on_a_unit & ~1LL) * t.shared + (on_a_unit & 1) * t.alone);
-            // The last tile costs 0.3 and 0.7 of what it has rows for, and the branches make the others slower or faster (measured, `part`).  Tiles of 64 x 64
-            // gain only where four and more share a compute unit (260 rows of 2,048 keys to 2,560 columns 50 to 45 us; to 2,048 39 to 40).
+    // With all blocks first.  Then with the blocks left out that the last tiles have no rows for: these tiles cost 0.3 and 0.7 of what they have rows
+    // for, and the branches make the others slower or faster (measured, `part`).  A launch is shorter for it only where the compute units get about the
+    // same share of such tiles: where all are, two to a unit and more; where each unit has five and more; or two, one with all rows and one without (as
+    // many columns of tiles as units: 140 rows of 2,048 keys to 32,768 columns 237 to 195 us).  Else it ends with the units that have none (2,048 keys,
+    // two to a unit, 333 rows to 2,048 and 2,560 columns 38.7 and 46.6 to 47.7 and 49.1, 192 to 8,192 74 to 102; four to a unit, 400 rows of 16,384
+    // keys to 2,048 294 to 322).  3% are left for what the estimate does not see (600 rows to 32,768 columns 689 to 716), 6% where other tiles in pieces
+    // would take the place of the best without (192 rows of 16,384 keys to 2,560 173 to 197).  Tiles of 64 x 64 gain only where four and more share a unit.
+    for (const bool part : {false, true}) {
+        const F32Cut whole = best;
+        for (const auto& t : kTiles) {
+            const int row_tiles = (M + 32 * t.wm - 1) / (32 * t.wm), column_tiles = (N + 32 * t.wn - 1) / (32 * t.wn);
             const int in_last = (M - 1) % (32 * t.wm) / 32 + 1;
-            const float shorter = t.part * (1.f - 0.7f * (t.wm - in_last) / t.wm / ((M + 32 * t.wm - 1) / (32 * t.wm)));
-            const bool part = in_last < t.wm && shorter < 1.f && (t.wm + t.wn > 4 || on_a_unit > 3);
-            if (part) us *= shorter;
-            if (split) us += 4.f + 2e-6f * segments * M * N;
-            if (us < least) {
-                least = us;
-                best = F32Cut{t.wm, t.wn, split ? per_group : 0, part};
+            if (part && in_last == t.wm) continue;
+            const float shorter = t.part * (1.f - 0.7f * (t.wm - in_last) / t.wm / row_tiles);
+            for (int per_group = segments; per_group >= 1; per_group = per_group == 1 ? 0 : (per_group + 1) / 2) {
+                const int groups = (segments + per_group - 1) / per_group;
+                const bool split = groups > 1;
+                if (split && (!may_split || groups > 65535 || static_cast<long long>(segments) * M * N > kMostPartials)) break;
+                const long long on_a_unit = (static_cast<long long>(row_tiles) * column_tiles * groups + kUnits - 1) / kUnits;
+                float us = per_group * ((on_a_unit & ~1LL) * t.shared + (on_a_unit & 1) * t.alone);
+                if (part) {
+                    const bool evenly = row_tiles == 1 ? on_a_unit > 1 : on_a_unit > 4 || (on_a_unit == 2 && !split && column_tiles >= kUnits);
+                    if (!evenly || (t.wm + t.wn == 4 && on_a_unit < 4)) continue;
+                    const bool other = t.wm != whole.wm || t.wn != whole.wn || (split ? per_group : 0) != whole.per_group;
+                    us *= shorter * (row_tiles == 1 ? 1.f : other && split ? 1.06f : 1.03f);
+                }
+                if (split) us += 4.f + 2e-6f * segments * M * N;
+                if (us < least) {
+                    least = us;
+                    best = F32Cut{t.wm, t.wn, split ? per_group : 0, part};
+                }
             }
         }
     }
@@ -442,6 +455,11 @@ WLLM_API int wllm_gemm_f32_segments(int M, int N, int K) {
     if (M < 1 || N < 1 || K < 4 || K % 4 != 0) return 1;
     if (M <= 64 ? !few_rows_split(N, K) : f32_cut(M, N, K, true).per_group == 0) return 1;
     return (K + kF32Segment - 1) / kF32Segment;
+}
+
+// Whether the product of these sizes, of more than 64 rows, leaves out the blocks of 16 rows that its last tiles have no rows for.
+WLLM_API int wllm_gemm_f32_leaves_out(int M, int N, int K) {
+    return M > 64 && N > 0 && K >= 4 && K % 4 == 0 && f32_cut(M, N, K, true).part;
 }
 
 // `tiles`: null, or the tile-major copy of a float32 w (`wllm_tile_weight_f32`), which the few-row kernel
