@@ -20,3 +20,11 @@ def lib():
     (128, 32768, 2048, 0), (256, 2048, 16384, 0), (64, 32768, 2048, 0)])                                            # full tiles, few rows
 def test_float32_tiles_leave_out_rows_where_the_launch_gets_shorter(lib, m, n, k, out):
     assert lib.wllm_gemm_f32_leaves_out(m, n, k) == out
+
+
+@pytest.mark.parametrize("m,k,norm,takes", [
+    (1, 256, 0, 1), (8, 256, 0, 1), (9, 256, 0, 0), (16, 512, 0, 0), (16, 960, 0, 0), (16, 1024, 0, 1), (17, 1024, 0, 0), (32, 512, 0, 0), (25, 768, 0, 0),
+    (13, 2048, 0, 1), (14, 2048, 0, 0), (8, 3072, 0, 1), (9, 3072, 0, 0),
+    (8, 512, 1, 1), (9, 512, 1, 0), (16, 1024, 1, 0), (9, 1536, 1, 0), (13, 2048, 1, 1), (14, 2048, 1, 0)])
+def test_gated_products_keep_x_whole_where_that_pays(lib, m, k, norm, takes):
+    assert lib.wllm_gated_rows_take(m, k, norm) == takes

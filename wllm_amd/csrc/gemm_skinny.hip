@@ -679,13 +679,13 @@ gemm_skinny_gated_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16
 // 10.6 / 11.3 and 9.4 / 9.5 (12.2 / 12.3 and 10.8 / 10.7).  More loads on their way and two workgroups a compute unit are no better (16 steps a
 // wavefront 24.5 / 25.3; of 3,072 keys to 2 x 24,576 columns 53 / 56 against 51 / 52), nor is one workgroup of twice the tiles, for an x of more than
 // half the shared memory (24 rows 27.6 against the kernel above's 25.4).
-template <int MT, int GATE, bool TILED, bool NORM>
+template <int GATE, bool TILED, bool NORM>
 __global__ void __launch_bounds__(256, 3)
 gemm_gated_rows_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16* __restrict__ w, bf16* __restrict__ out, int M, int inter,
                        int K, int out_stride, GateShape shape) {
     extern __shared__ uint4 xs[];                 // [M][K / 8 + 1]
     __shared__ float inv_s[16];                   // NORM: a row's rsqrt(mean square + eps)
-    constexpr int TPW = 2, kThreads = TPW * 128, kBatch = 8, kRows = 8;
+    constexpr int MT = 1, TPW = 2, kThreads = TPW * 128, kBatch = 8, kRows = 8;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int i = lane % 16, g = lane / 16;
     const int tile = wave % TPW, half = wave / TPW;
@@ -797,6 +797,17 @@ gemm_gated_rows_kernel(const bf16* __restrict__ x, NormOnLoad norm, const bf16* 
     gated_finish<MT, GATE, TPW>(reinterpret_cast<float*>(xs), tile, half, lane, n0, accg, accu, out, M, inter, out_stride, shape);
 }
 
+static size_t gated_rows_bytes(int M, int K) { return static_cast<size_t>(M) * (K / 8 + 1) * sizeof(uint4); }
+// x goes whole in shared memory, where three workgroups of it share a compute unit (of 2,048 keys 13 rows, of 3,072 8): at 16 rows of 2,048 keys two would,
+// and are no faster (26.6 us with the norm against 26.9; to 2 x 24,576 columns 38.6 against 36.4).  More than 8 rows are asked for in two turns, a
+// trip to memory more before the first product, which few keys don't win back: 16 rows to 2 x 4,096 columns, here and below, of 256 / 512 / 1,024 keys
+// 4.4 / 5.3 / 7.0 and 3.9 / 5.1 / 7.3 us, with the norm of 512 / 1,024 6.6 / 8.5 and 5.8 / 8.2, 12 of 2,048 11.7 and 12.7.  So more than 8 rows take this
+// way from 1,024 keys on, with the norm from 2,048, more than 16 nowhere (32 rows of 512 keys 7.2 and 6.4).
+static bool gated_rows_take(int M, int K, bool with_norm) {
+    return gated_rows_bytes(M, K) <= 53 * 1024 && (M <= 8 || (M <= 16 && K >= (with_norm ? 2048 : 1024)));
+}
+WLLM_API int wllm_gated_rows_take(int M, int K, int with_norm) { return M >= 1 && K >= 64 && gated_rows_take(M, K, with_norm != 0); }
+
 static int gated_launch(const void* x, NormOnLoad norm, bool with_norm, const void* w, int tiled, void* out, int M,
                         int inter, int K, int gate, GateShape shape, int chunk, int out_stride, hipStream_t stream) {
     if (out_stride < (gate == kGatePairSquaredRelu ? 2 * inter : inter)) return -1;
@@ -805,25 +816,21 @@ static int gated_launch(const void* x, NormOnLoad norm, bool with_norm, const vo
     if (chunk > K / 2) chunk = K / 2;
     // the norm on load: at most 16 rows, whole chunks of 256 keys
     if (with_norm && (mt != 1 || chunk != 256 || (K / 2) % 256 != 0)) return -1;
-    // x whole in shared memory, where three workgroups of it share a compute unit (of 2,048 keys 13 rows, of 3,072 8): at 16 rows of 2,048 keys two would,
-    // and are no faster (26.6 us with the norm against 26.9; to 2 x 24,576 columns 38.6 against 36.4)
-    const size_t whole = static_cast<size_t>(M) * (K / 8 + 1) * sizeof(uint4), sums = static_cast<size_t>(2) * kWave * mt * 8 * sizeof(float);
-    if (mt <= 2 && whole <= 53 * 1024) {
+    if (gated_rows_take(M, K, with_norm)) {
+        const size_t whole = gated_rows_bytes(M, K), sums = static_cast<size_t>(2) * kWave * 8 * sizeof(float);
         const dim3 grid((inter + 31) / 32);
-#define ROWS_T(MT, A, T, NORM)                                                                                        \
-    gemm_gated_rows_kernel<MT, A, T, NORM><<<grid, 256, whole > sums ? whole : sums, stream>>>(                       \
+#define ROWS_T(A, T, NORM)                                                                                            \
+    gemm_gated_rows_kernel<A, T, NORM><<<grid, 256, whole > sums ? whole : sums, stream>>>(                           \
         static_cast<const bf16*>(x), norm, static_cast<const bf16*>(w), static_cast<bf16*>(out), M, inter, K, out_stride, shape)
-#define ROWS(MT, A, NORM)                       \
-    do {                                        \
-        if (tiled) ROWS_T(MT, A, true, NORM);   \
-        else ROWS_T(MT, A, false, NORM);        \
+#define ROWS(A, NORM)                       \
+    do {                                    \
+        if (tiled) ROWS_T(A, true, NORM);   \
+        else ROWS_T(A, false, NORM);        \
     } while (0)
         if (with_norm) {
-            WLLM_BY_GATE(gate, ROWS(1, GATE, true))
-        } else if (mt == 1) {
-            WLLM_BY_PAIRED_GATE(gate, ROWS(1, GATE, false))
+            WLLM_BY_GATE(gate, ROWS(GATE, true))
         } else {
-            WLLM_BY_PAIRED_GATE(gate, ROWS(2, GATE, false))
+            WLLM_BY_PAIRED_GATE(gate, ROWS(GATE, false))
         }
 #undef ROWS
 #undef ROWS_T
