@@ -28,3 +28,12 @@ def test_float32_tiles_leave_out_rows_where_the_launch_gets_shorter(lib, m, n, k
     (8, 512, 1, 1), (9, 512, 1, 0), (16, 1024, 1, 0), (9, 1536, 1, 0), (13, 2048, 1, 1), (14, 2048, 1, 0)])
 def test_gated_products_keep_x_whole_where_that_pays(lib, m, k, norm, takes):
     assert lib.wllm_gated_rows_take(m, k, norm) == takes
+
+
+@pytest.mark.parametrize("n,nh,nkv,d,rot,by_heads", [
+    (1, 1, 1, 32, 32, 0), (64, 14, 2, 64, 64, 0), (1, 14, 2, 64, 64, 0),                              # at most one round of pairs
+    (1, 8, 1, 256, 256, 1), (64, 8, 1, 256, 256, 1), (65, 8, 1, 256, 256, 0), (42, 16, 4, 128, 128, 1), (43, 16, 4, 128, 128, 0),
+    (64, 32, 8, 128, 128, 1), (64, 16, 16, 256, 256, 1), (64, 40, 40, 64, 64, 1), (65, 40, 40, 64, 64, 0), (128, 64, 64, 64, 64, 0),
+    (16, 16, 16, 256, 36, 0), (16, 2100, 1000, 4, 8, 0), (16, 16, 16, 260, 256, 0)])                  # sizes that the other kernel does not take
+def test_the_rotation_goes_by_heads_where_that_pays(lib, n, nh, nkv, d, rot, by_heads):
+    assert lib.wllm_rope_by_heads(n, nh, nkv, d, rot, 16) == by_heads

@@ -401,6 +401,25 @@ WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const flo
                                const float* pre_k, float pre_eps, float rot_scale, float temp_coef, int temp_every,
                                hipStream_t stream);
 
+// Few tokens with a bias or a stack of partial sums: `rope_cache_kernel` is a workgroup a token that goes to memory once for the
+// positions, once for each round of heads and once for the values; that of `head_prepare.hip` has a workgroup for every four
+// heads, which ask for all they need at once (the same numbers in the same order, so the same bits).  It is ahead where a token's pairs are more
+// than one round of the other's threads, and behind by its second kernel's arguments and sines where they are not (us, 32 tokens, two partial
+// sums, there and here: 14 heads of 64 on two 3.8 and 4.3, 8 of 256 on one 4.6 and 4.4, 32 of 128 on eight 6.8 and 5.1, 16 of 256 on as many 11.5
+// and 5.9); and as long as the workgroups, each of which makes the sines again, are not more than run at once: with fewer than two rounds 256 (8 of
+// 256 on one, eight sums, 64 / 96 tokens 5.0 / 5.1 and 4.7 / 5.1; 16 of 128 on four 33 / 64 tokens 5.0 / 5.1 and 5.1 / 5.5), else up to 64 tokens
+// (40 of 64 on 40, four sums, 64 / 96 tokens 9.0 / 9.7 and 7.7 / 11.1).
+static bool rope_by_heads(int n, int num_heads, int num_kv_heads, int head_dim, int rotary_dim, int page_size) {
+    if (head_dim > 256 || head_dim % 4 != 0 || rotary_dim % 8 != 0 || rotary_dim > head_dim || page_size < 1 || num_heads + 2 * num_kv_heads > 4096)
+        return false;
+    const int pairs = (num_heads + num_kv_heads) * (rotary_dim / 2);                                            // a token's
+    const int workgroups = (num_heads + num_kv_heads + 3) / 4 + (num_kv_heads * head_dim + 1023) / 1024;
+    return n <= 64 && pairs >= 1024 && (pairs >= 2048 || n * workgroups <= 256);
+}
+WLLM_API int wllm_rope_by_heads(int n, int num_heads, int num_kv_heads, int head_dim, int rotary_dim, int page_size) {
+    return rope_by_heads(n, num_heads, num_kv_heads, head_dim, rotary_dim, page_size);
+}
+
 WLLM_API int wllm_rope_cache_write(void* qkv, int is_bf16, const float* parts, int splits, long long split_stride,
                                    const float* bias, const int* positions, const float* inv_freq, const int* slots,
                                    void* cache, long long num_pages, int n, int num_heads, int num_kv_heads,
@@ -423,13 +442,7 @@ WLLM_API int wllm_rope_cache_write(void* qkv, int is_bf16, const float* parts, i
         return launch_status();
     }
     const int width = (num_heads + 2 * num_kv_heads) * head_dim;
-    // Few tokens with a bias or a stack of partial sums: the kernel above is a workgroup a token that goes to memory once for the
-    // positions, once for each round of heads and once for the values; that of `head_prepare.hip` has a workgroup for every four
-    // heads, which ask for all they need at once (the same numbers in the same order, so the same bits).  64 tokens of 8 heads of 256 on one
-    // in a captured step: 5.5 to 5.2 us traced, the step 2,183 to 2,166; 64 of 40 heads of 64 on 40 9.1 to 7.0.  From some 200 tokens on the
-    // workgroups are more than run at once and each makes the sines again (200 / 256 tokens 4.7 / 4.8 and 5.2 / 5.3).
-    if (n <= 128 && inv_freq && head_dim <= 256 && head_dim % 4 == 0 && rotary_dim % 8 == 0 && rotary_dim <= head_dim &&
-        page_size > 0 && num_heads + 2 * num_kv_heads <= 4096)
+    if (inv_freq && rope_by_heads(n, num_heads, num_kv_heads, head_dim, rotary_dim, page_size))
         return wllm_head_prepare(qkv, is_bf16, width, parts, splits, split_stride, bias, bias ? width : 0, positions, inv_freq,
                                  slots, cache, num_pages, n, num_heads, num_kv_heads, head_dim, rotary_dim, 0, -1.f, head_dim,
                                  0, page_size, nullptr, nullptr, -1.f, 1.f, 0.f, 0, stream);
