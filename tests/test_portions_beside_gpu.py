@@ -24,6 +24,7 @@ def test_the_rule():
     (4, 4, 64, 8, [(400, 410)] + [(1, 200)] * 3),                                   # the other way round
     (8, 4, 128, 32, [(130, 700), (1, 300), (33, 65)] + [(1, 500 + i) for i in range(40)]),      # runs of both, some of each left
     (64, 64, 64, 16, [(64, 64), (1, 100)]),                                         # 64 items of either kind
+    (64, 64, 64, 16, [(270, 270)] + [(1, 100 + i) for i in range(5)]),              # 320 of either, heads of 64: a run of 256 each, and some left
 ])
 def test_together_as_apart(nh, nkv, d, ps, segs, option, monkeypatch):
     window = {"window": 100, "chunk": -70}.get(option, 0)

@@ -368,10 +368,13 @@ paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
 // the sum of both (8 heads of 256 on one, a portion of 448 tokens over 448 to 1,000 keys beside 60 tokens over 1,500 each: 19.7 + 17.1 us), in one
 // launch 23.5 us.  A compute unit holds two of its workgroups (shared memory and registers of the portions), where it held
 // three of the decoded tokens' kernel; two are enough beside the portions.
-// The kinds alternate in runs of kRoleRun workgroups, eight an XCD, portions first: with all portions in front (runs of 512), 30 tokens
+// The kinds alternate in runs of workgroups, eight an XCD, portions first: with all portions in front (runs of 512), 30 tokens
 // over 1,250 keys beside 448 over 896 (16 heads of 128 on four; with the sum of the pieces) took 30.4 us, in runs of 256 / 64
 // 30.2 / 29.8, in runs of 8, one an XCD, 32.2; with few items all are the same.
-constexpr int kRoleRun = 64;
+// With heads of 64 a compute unit holds four workgroups, and a run of eight an XCD, whose 32 units take them in turn, would bring the same
+// unit the same kind every time: four portions here, none there (448 tokens over 3,000 keys beside 24 over 800, 64 heads of 64 on eight: 97.7 us, in
+// runs of one workgroup a unit 71.3, in two launches 78).
+template <int HD> constexpr int kRoleRun = HD == 64 ? 256 : 64;
 
 template <int HD, bool SPLIT>
 __global__ void __launch_bounds__(kPrefillThreads, 2)
@@ -388,12 +391,12 @@ paged_attention_both_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
         FewRowsShared<HD> few;
     } shared;
     // runs of either kind in turn, then what is left of both lists
-    const int b = blockIdx.x, shorter = min(num_portions, num_items) / kRoleRun * kRoleRun;
+    const int b = blockIdx.x, shorter = min(num_portions, num_items) / kRoleRun<HD> * kRoleRun<HD>;
     bool portion;
     int index;
     if (b < 2 * shorter) {
-        portion = b / kRoleRun % 2 == 0;
-        index = b / (2 * kRoleRun) * kRoleRun + b % kRoleRun;
+        portion = b / kRoleRun<HD> % 2 == 0;
+        index = b / (2 * kRoleRun<HD>) * kRoleRun<HD> + b % kRoleRun<HD>;
     } else {
         index = b - shorter;
         portion = index < num_portions;
