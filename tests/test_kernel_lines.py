@@ -1,8 +1,9 @@
 """Where one kernel hands over to another, as the library's own rules say it (host code of the built library, no GPU).  Each case lies in
 a range that was measured slower on the other side of its line."""
+import numpy as np
 import pytest
 
-from wllm_amd.kernels import library
+from wllm_amd.kernels import attention_plan, hip_backend, library
 
 
 @pytest.fixture(scope="module")
@@ -37,3 +38,14 @@ def test_gated_products_keep_x_whole_where_that_pays(lib, m, k, norm, takes):
     (16, 16, 16, 256, 36, 0), (16, 2100, 1000, 4, 8, 0), (16, 16, 16, 260, 256, 0)])                  # sizes that the other kernel does not take
 def test_the_rotation_goes_by_heads_where_that_pays(lib, n, nh, nkv, d, rot, by_heads):
     assert lib.wllm_rope_by_heads(n, nh, nkv, d, rot, 16) == by_heads
+
+
+@pytest.mark.parametrize("nh,nkv,portion,decoded,pays", [
+    (8, 1, (448, 896), (60, 1500), True), (16, 16, (448, 896), (32, 1500), True), (64, 8, (448, 3000), (8, 2048), True),
+    (16, 16, (448, 896), (256, 300), False), (32, 8, (64, 64), (128, 4000), False), (40, 40, (448, 896), (60, 4000), False),
+    (64, 8, (448, 3000), (128, 1500), True), (64, 8, (448, 3000), (256, 1500), True), (40, 40, (448, 3000), (40, 1500), True)])
+def test_portions_run_beside_decoded_tokens_where_that_pays(nh, nkv, portion, decoded, pays):
+    count, keys = decoded
+    q_len, ctx_len = np.array([portion[0]] + [1] * count), np.array([portion[1]] + [keys] * count)
+    items, _, _, prefill, rows = attention_plan.build_work_items(q_len, ctx_len, nh // nkv, nkv, 0)
+    assert hip_backend.HipBackend.portions_pay_beside(prefill, rows, items.shape[0]) is pays

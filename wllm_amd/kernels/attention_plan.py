@@ -74,6 +74,7 @@ class AttentionPlan:
     num_prefill: int = 0
     prefill_rows: int = 64
     live_items: Optional[torch.Tensor] = None     # int32 [1] on the device: how many of `items` count (None: all)
+    together: bool = False              # the prefill items run in the launch of the others, where there is a kernel for that
 
 
 class StaticAttentionPlan(AttentionPlan):

@@ -224,6 +224,22 @@ class HipBackend:
         into shared memory (`attention_portion.h`).  The blocks of 128 rows of long prompts fill the device by themselves."""
         return head_dim in (64, 128, 256) and page_size >= 8 and page_size & (page_size - 1) == 0
 
+    # Decoded tokens' items (of 16 rows by 128 keys) from which on a step's portions run by themselves, unless they are as much work.  Together
+    # a compute unit runs two of the decoded tokens' workgroups instead of three: as long as they are some rounds that is less than the portions' own
+    # launch, of many rounds it is up to a tenth.  us, apart and together, a portion of 448 tokens over 896 keys: 8 heads of 256 on one beside 128 of
+    # 1,500 keys (1,189 items) 62.7 / 49.4, 16 on as many beside 8 of 2,048 and 256 of 300 (1,584 and 9,392) 70 / 64 and 211 / 224, 32 of 128 on eight
+    # beside 60 of 1,500 and 128 of 4,000 (4,464 and 24,512) 81 / 80 and 332 / 347, 40 of 64 on as many beside 8 of 2,048 and 60 of 4,000 (3,960 and
+    # 57,440) 50 / 43 and 337 / 366; one of 448 over 3,000 beside 128 of 1,500 (64 of 64 on eight, 9,512) 133 / 111.
+    MANY_DECODED_ITEMS = 8192
+
+    @classmethod
+    def portions_pay_beside(cls, prefill, prefill_rows: int, num_items: int) -> bool:
+        """Whether a step's portions gain by running in its decoded tokens' launch (see above): `prefill` are their items, whose tiles of 16
+        rows by their keys are compared with the decoded tokens' of 128 keys."""
+        if num_items < cls.MANY_DECODED_ITEMS:
+            return True
+        return int((prefill[:, 4] - prefill[:, 3]).sum()) * (prefill_rows // 16) >= 128 * num_items
+
     # Up to how many (items of 16 rows by 128 keys) x (elements of a head) float32 prompt portions are tiles: these take a time in
     # proportion, the blocks of 64 rows hardly less for few of them than for the 256 that give every compute unit one.
     # Tiles against blocks, heads of 256: 309 items 27 and 67 us, 1,280 61 and 75, 1,631 73 and 77, 2,080 89 and 79, 2,304 92 and
@@ -257,7 +273,7 @@ class HipBackend:
         a, b = n_i * 8, (n_i + n_r) * 8
         return AttentionPlan(dev[:a].view(n_i, 8), dev[a:b].view(n_r, 8) if n_r else None, n_i, n_r, slots,
                              self._partial_o, self._partial_ml, dev[b:].view(n_p, 8) if n_p else None, n_p,
-                             prefill_rows)
+                             prefill_rows, together=bool(n_p and n_i) and self.portions_pay_beside(prefill, prefill_rows, n_i))
 
     def _workgroup_slots(self, device) -> int:
         """Workgroups of the kernel for prompt portions that the device runs at once: two a compute unit."""
@@ -315,8 +331,7 @@ class HipBackend:
                     block_tables.shape[1], scale, window, q_stride, softcap, _ptr(sinks), self._stream()),
                     "paged_attention (matrix cores, float32)")
                 return
-            together = (plan.num_prefill and plan.num_items and plan.prefill_rows != PROMPT_ROWS
-                        and self.portions_beside(head_dim, page_size))
+            together = plan.together and plan.prefill_rows != PROMPT_ROWS and self.portions_beside(head_dim, page_size)
             if plan.num_prefill and not together:
                 prefill = self.lib.wllm_paged_attention_prompt if plan.prefill_rows == PROMPT_ROWS else self.lib.wllm_paged_attention_prefill
                 self._check(prefill(
