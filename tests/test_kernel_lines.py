@@ -49,3 +49,12 @@ def test_portions_run_beside_decoded_tokens_where_that_pays(nh, nkv, portion, de
     q_len, ctx_len = np.array([portion[0]] + [1] * count), np.array([portion[1]] + [keys] * count)
     items, _, _, prefill, rows = attention_plan.build_work_items(q_len, ctx_len, nh // nkv, nkv, 0)
     assert hip_backend.HipBackend.portions_pay_beside(prefill, rows, items.shape[0]) is pays
+
+
+@pytest.mark.parametrize("rows,columns,k,tile", [
+    (300, 250, 3072, None), (2048, 64, 3072, None), (1024, 128, 3072, None), (2049, 64, 3072, (64, 64)), (300, 512, 3072, (64, 64)),
+    (512, 512, 4096, None), (1024, 250, 4096, None), (2048, 128, 4096, None), (640, 512, 4096, (64, 64)),
+    (256, 64, 4096, (64, 64)), (257, 64, 2048, (64, 64))])
+def test_gated_products_of_few_tiles_and_many_keys_are_the_librarys(rows, columns, k, tile):
+    """Beyond 256 rows; up to there the tiles of 128 take twice as long."""
+    assert hip_backend.HipBackend.block_gated_tile(rows, columns, k) == tile

@@ -541,7 +541,9 @@ class HipBackend:
         if k > 4096 or (rows > cls.WIDE_TILE and cls.wide_gated_takes(rows, columns, k)):
             return None
         found = cls._one_round(rows, columns, k, gated=True)
-        return found[:2] if found is not None else None
+        if found is None or (rows > cls.WIDE_TILE and k > 2048 and found[2] <= (64 if k <= 3072 else 128)):
+            return None
+        return found[:2]
 
     @classmethod
     def block_split_tile(cls, rows: int, n: int, k: int, pieces: int):
