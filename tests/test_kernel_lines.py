@@ -58,3 +58,13 @@ def test_portions_run_beside_decoded_tokens_where_that_pays(nh, nkv, portion, de
 def test_gated_products_of_few_tiles_and_many_keys_are_the_librarys(rows, columns, k, tile):
     """Beyond 256 rows; up to there the tiles of 128 take twice as long."""
     assert hip_backend.HipBackend.block_gated_tile(rows, columns, k) == tile
+
+
+def test_products_of_one_round_refuse_more(lib):
+    """257 tiles of 64 by 64; 256 pieces times two tiles."""
+    fn = lib.wllm_gemm_block
+    fn.argtypes = hip_backend._SIGNATURES["wllm_gemm_block"]
+    sizes = [(64 * 257, 64, 64, 64, 1), (64, 64 * 256 + 1, 64, 64 * 257, 1), (65, 64, 64 * 256, 64, 256)]
+    for m, n, k, stride, splits in sizes:
+        out, partial = (None, 4096) if splits > 1 else (4096, None)
+        assert fn(4096, 4096, out, partial, m, n, k, stride, splits, 0, 0.0, 0.0, 0.0, 64, 64, None) == -1

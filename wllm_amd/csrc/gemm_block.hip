@@ -58,37 +58,30 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
     const int wm = wave / S::kWavesN, wn = wave % S::kWavesN;
     const uint32_t lds_base = shared_address(ring_s);
 
-    // The items go to the XCDs in equal runs of an order in which 8 tiles of x rows share a tile of w rows.
+    // The items, at most one a workgroup, go to the XCDs in equal runs of an order in which 8 tiles of x rows share a tile of w rows.
     const int tiles = m_tiles * n_tiles, items = tiles * splits, all_stages = K / kBlockKeys;
-    const int xcd = blockIdx.x % 8, per_xcd = items / 8, left = items % 8;
-    int item = xcd * per_xcd + min(xcd, left) + blockIdx.x / 8;
-    const int end = xcd * per_xcd + min(xcd, left) + per_xcd + (xcd < left ? 1 : 0);
-    if (item >= end) return;
+    const int xcd = blockIdx.x % 8, per_xcd = items / 8, left = items % 8, in_run = blockIdx.x / 8;
+    if (in_run >= per_xcd + (xcd < left ? 1 : 0)) return;
+    const int item = xcd * per_xcd + min(xcd, left) + in_run;
+    const int piece = item / tiles, tile = item - piece * tiles;
+    const int begin = static_cast<int>(static_cast<long long>(piece) * all_stages / splits);
+    const int stages = static_cast<int>(static_cast<long long>(piece + 1) * all_stages / splits) - begin;
+    const int band = tile / (8 * n_tiles), in_band = tile - band * 8 * n_tiles;
+    const int band_rows = min(8, m_tiles - 8 * band);
+    const int n_tile = in_band / band_rows;
+    const int m0 = (8 * band + in_band - n_tile * band_rows) * TM, n0 = n_tile * kColumns;
 
     // what this lane brings of a stage: rows 8 (wave + 8 u) + lane / 8 of the tiles, in bytes from the stage's first key
     uint32_t offset_x[S::kLoadsX], offset_w[S::kLoadsW];
-    int m_base, n_base, piece, begin, stages;
-    auto place = [&](int it) {
-        piece = it / tiles;
-        const int t = it - piece * tiles;
-        begin = static_cast<int>(static_cast<long long>(piece) * all_stages / splits);
-        stages = static_cast<int>(static_cast<long long>(piece + 1) * all_stages / splits) - begin;
-        const int band = t / (8 * n_tiles), in_band = t - band * 8 * n_tiles;
-        const int band_rows = min(8, m_tiles - 8 * band);
-        const int n_tile = in_band / band_rows;
-        m_base = (8 * band + in_band - n_tile * band_rows) * TM;
-        n_base = n_tile * kColumns;
-        const int r = 8 * wave + lane / 8, c = (lane % 8) ^ (lane / 8);
+    const int r0 = 8 * wave + lane / 8, c0 = (lane % 8) ^ (lane / 8);
 #pragma unroll
-        for (int u = 0; u < S::kLoadsX; ++u)
-            offset_x[u] = (static_cast<uint32_t>(min(m_base + r + 64 * u, M - 1)) * K + c * 8) * 2;
+    for (int u = 0; u < S::kLoadsX; ++u) offset_x[u] = (static_cast<uint32_t>(min(m0 + r0 + 64 * u, M - 1)) * K + c0 * 8) * 2;
 #pragma unroll
-        for (int u = 0; u < S::kLoadsW; ++u) {
-            const int at = r + 64 * u;               // gated: the gate rows, then the up rows that belong to them
-            const int row = !GATED || at < TN / 2 ? min(n_base + at, N - 1) : N + min(n_base + at - TN / 2, N - 1);
-            offset_w[u] = (static_cast<uint32_t>(row) * K + c * 8) * 2;
-        }
-    };
+    for (int u = 0; u < S::kLoadsW; ++u) {
+        const int at = r0 + 64 * u;               // gated: the gate rows, then the up rows that belong to them
+        const int row = !GATED || at < TN / 2 ? min(n0 + at, N - 1) : N + min(n0 + at - TN / 2, N - 1);
+        offset_w[u] = (static_cast<uint32_t>(row) * K + c0 * 8) * 2;
+    }
     auto send_one = [&](int s, int slot, int u) {
         const size_t at = static_cast<size_t>(begin + s) * (kBlockKeys * 2);
         const uint32_t to = lds_base + slot * S::kStage + wave * 1024;
@@ -96,143 +89,127 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
         else load_to_shared(reinterpret_cast<const unsigned char*>(w) + at, offset_w[u < S::kLoadsX ? 0 : u - S::kLoadsX],
                             to + TM * 128 + (u - S::kLoadsX) * 8192);
     };
-    auto send_first = [&] {
 #pragma unroll
-        for (int s = 0; s < D; ++s)
-            if (s < stages)
+    for (int s = 0; s < D; ++s)
+        if (s < stages)
 #pragma unroll
-                for (int u = 0; u < L; ++u) send_one(s, s, u);
-    };
+            for (int u = 0; u < L; ++u) send_one(s, s, u);
     const int place0 = (g ^ (i % 8)) * 16, place1 = ((4 + g) ^ (i % 8)) * 16;
 
-    place(item);
-    send_first();
-    for (;;) {
-        float4_t acc[2][XB];
+    float4_t acc[2][XB];
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int b = 0; b < XB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
-        Fragment fx[2][2][XB], fw[2][2][2];              // [set][32 keys][block]
-        constexpr int kReads = 2 * (2 + XB), kProducts = 4 * XB;
-        // fragment number r of a stage: w's and x's of its first 32 keys, then of the others
-        auto read_one = [&](auto set, int slot, int r) {
-            constexpr int F = decltype(set)::value ? 1 : 0;
-            const int k = r / (2 + XB), f = r % (2 + XB);
-            const unsigned char* from = ring_s + slot * S::kStage + (k ? place1 : place0);
-            if (f < 2) fw[F][k][f].u = *reinterpret_cast<const uint4*>(from + TM * 128 + ((GATED ? f * (TN / 2) + wn * 16 : wn * 32 + f * 16) + i) * 128);
-            else fx[F][k][f - 2].u = *reinterpret_cast<const uint4*>(from + ((wm * XB + f - 2) * 16 + i) * 128);
-        };
-        // stage s is in the registers `set`
-        auto step = [&](auto set, auto other, int s, int slot, int next) {
-            constexpr int F = decltype(set)::value ? 1 : 0;
-            if (s + D - 1 < stages) wait_loads<(D - 2) * L>();
-            else wait_loads<0>();
-            // (through the builtin, so that the compiler knows that this stage's reads are done and does not wait for the next one's)
-            __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
-            meet();
-            const bool more = s + D < stages;
-            int r = 0, u = 0;
-#pragma unroll
-            for (int p = 0; p < kProducts; ++p) {
-                const int k = p / (2 * XB), b = p / 2 % XB, a = p % 2;
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[F][k][a].v, fx[F][k][b].v, acc[a][b], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (; r * kProducts < (p + 1) * kReads; ++r) read_one(other, next, r);
-#pragma unroll
-                for (; u * kProducts < (p + 1) * L; ++u)
-                    if (more) send_one(s + D, slot, u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        if (stages >= D) wait_loads<(D - 1) * L>();
+        for (int b = 0; b < XB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    Fragment fx[2][2][XB], fw[2][2][2];              // [set][32 keys][block]
+    constexpr int kReads = 2 * (2 + XB), kProducts = 4 * XB;
+    // fragment number r of a stage: w's and x's of its first 32 keys, then of the others
+    auto read_one = [&](auto set, int slot, int r) {
+        constexpr int F = decltype(set)::value ? 1 : 0;
+        const int k = r / (2 + XB), f = r % (2 + XB);
+        const unsigned char* from = ring_s + slot * S::kStage + (k ? place1 : place0);
+        if (f < 2) fw[F][k][f].u = *reinterpret_cast<const uint4*>(from + TM * 128 + ((GATED ? f * (TN / 2) + wn * 16 : wn * 32 + f * 16) + i) * 128);
+        else fx[F][k][f - 2].u = *reinterpret_cast<const uint4*>(from + ((wm * XB + f - 2) * 16 + i) * 128);
+    };
+    // stage s is in the registers `set`
+    auto step = [&](auto set, auto other, int s, int slot, int next) {
+        constexpr int F = decltype(set)::value ? 1 : 0;
+        if (s + D - 1 < stages) wait_loads<(D - 2) * L>();
         else wait_loads<0>();
+        // (through the builtin, so that the compiler knows that this stage's reads are done and does not wait for the next one's)
+        __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
         meet();
+        const bool more = s + D < stages;
+        int r = 0, u = 0;
 #pragma unroll
-        for (int r = 0; r < kReads; ++r) read_one(Flag<false>(), 0, r);
-        int slot = 0;
-        auto after = [](int q) { return q + 1 == D ? 0 : q + 1; };
-        for (int s = 0; s < stages; s += 2) {
-            // (behind the last stage a step reads its own once more, and nothing uses it)
-            const int second = s + 1 < stages ? after(slot) : slot, third = s + 2 < stages ? after(second) : second;
-            step(Flag<false>(), Flag<true>(), s, slot, second);
-            if (s + 1 < stages) step(Flag<true>(), Flag<false>(), s + 1, second, third);
-            slot = third;
+        for (int p = 0; p < kProducts; ++p) {
+            const int k = p / (2 * XB), b = p / 2 % XB, a = p % 2;
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[F][k][a].v, fx[F][k][b].v, acc[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (; r * kProducts < (p + 1) * kReads; ++r) read_one(other, next, r);
+#pragma unroll
+            for (; u * kProducts < (p + 1) * L; ++u)
+                if (more) send_one(s + D, slot, u);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        wait_reads();
-        meet();                                          // every wavefront is done with the shared memory
-        const int m0 = m_base, n0 = n_base, of_piece = piece;
-        item += gridDim.x / 8;
-        const bool again = item < end;
-        if (again) {
-            place(item);
-            send_first();
-        }
+    };
+    if (stages >= D) wait_loads<(D - 1) * L>();
+    else wait_loads<0>();
+    meet();
 #pragma unroll
-        for (int b = 0; b < XB; ++b) {
-            const int m = m0 + (wm * XB + b) * 16 + i;
-            if (m >= M) continue;
-            if (GATED) {
-                // a lane has four columns' gate and up sums
-                const int n = n0 + wn * 16 + 4 * g;
-                bf16* to = out + static_cast<size_t>(m) * stride + n;
+    for (int r = 0; r < kReads; ++r) read_one(Flag<false>(), 0, r);
+    int slot = 0;
+    auto after = [](int q) { return q + 1 == D ? 0 : q + 1; };
+    for (int s = 0; s < stages; s += 2) {
+        // (behind the last stage a step reads its own once more, and nothing uses it)
+        const int second = s + 1 < stages ? after(slot) : slot, third = s + 2 < stages ? after(second) : second;
+        step(Flag<false>(), Flag<true>(), s, slot, second);
+        if (s + 1 < stages) step(Flag<true>(), Flag<false>(), s + 1, second, third);
+        slot = third;
+    }
 #pragma unroll
-                for (int h = 0; h < (kPair ? 2 : 1); ++h) {
-                    float r[4];
+    for (int b = 0; b < XB; ++b) {
+        const int m = m0 + (wm * XB + b) * 16 + i;
+        if (m >= M) continue;
+        if (GATED) {
+            // a lane has four columns' gate and up sums
+            const int n = n0 + wn * 16 + 4 * g;
+            bf16* to = out + static_cast<size_t>(m) * stride + n;
+#pragma unroll
+            for (int h = 0; h < (kPair ? 2 : 1); ++h) {
+                float r[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    r[v] = kPair ? squared_relu(acc[h][b][v])
+                                 : gate_product<(GATED > 0 && !kPair ? GATED - 1 : 0)>(acc[0][b][v], acc[1][b][v], shape);
+                const uint32_t words[2] = {pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3])};
+                bf16* here = to + h * N;
+                if (vectors && n + 3 < N) {
+                    *reinterpret_cast<uint2*>(here) = make_uint2(words[0], words[1]);
+                } else {
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        r[v] = kPair ? squared_relu(acc[h][b][v])
-                                     : gate_product<(GATED > 0 && !kPair ? GATED - 1 : 0)>(acc[0][b][v], acc[1][b][v], shape);
-                    const uint32_t words[2] = {pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3])};
-                    bf16* here = to + h * N;
-                    if (vectors && n + 3 < N) {
-                        *reinterpret_cast<uint2*>(here) = make_uint2(words[0], words[1]);
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                            if (n + v < N) here[v] = bf16{static_cast<uint16_t>(words[v / 2] >> (16 * (v % 2)))};
-                    }
+                        if (n + v < N) here[v] = bf16{static_cast<uint16_t>(words[v / 2] >> (16 * (v % 2)))};
                 }
-                continue;
             }
-            if (partial != nullptr) {
-                float* row = partial + (static_cast<size_t>(of_piece) * M + m) * N;
-#pragma unroll
-                for (int a = 0; a < 2; ++a) {
-                    const int n = n0 + wn * 32 + 16 * a + 4 * g;
-                    if (vectors && n + 3 < N) {
-                        *reinterpret_cast<float4_t*>(row + n) = acc[a][b];
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                            if (n + v < N) row[n + v] = acc[a][b][v];
-                    }
-                }
-                continue;
-            }
-            uint32_t q[2][2];
+            continue;
+        }
+        if (partial != nullptr) {
+            float* row = partial + (static_cast<size_t>(piece) * M + m) * N;
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
-                q[a][0] = pack2_bf16(acc[a][b][0], acc[a][b][1]);
-                q[a][1] = pack2_bf16(acc[a][b][2], acc[a][b][3]);
-            }
-            // lanes g and g + 1 (g even) exchange halves, so that each has eight neighbouring columns of the 32
-            typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
-            const uint2_t lo = __builtin_amdgcn_permlane16_swap(q[0][0], q[1][0], false, false);
-            const uint2_t hi = __builtin_amdgcn_permlane16_swap(q[0][1], q[1][1], false, false);
-            const uint32_t words[4] = {lo.x, hi.x, lo.y, hi.y};
-            const int n = n0 + wn * 32 + 16 * (g & 1) + 8 * (g >> 1);
-            bf16* to = out + static_cast<size_t>(m) * stride + n;
-            if (vectors && n + 7 < N) {
-                *reinterpret_cast<uint4*>(to) = make_uint4(words[0], words[1], words[2], words[3]);
-            } else {
+                const int n = n0 + wn * 32 + 16 * a + 4 * g;
+                if (vectors && n + 3 < N) {
+                    *reinterpret_cast<float4_t*>(row + n) = acc[a][b];
+                } else {
 #pragma unroll
-                for (int v = 0; v < 8; ++v)
-                    if (n + v < N) to[v] = bf16{static_cast<uint16_t>(words[v / 2] >> (16 * (v % 2)))};
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < N) row[n + v] = acc[a][b][v];
+                }
             }
+            continue;
         }
-        if (!again) break;
+        uint32_t q[2][2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            q[a][0] = pack2_bf16(acc[a][b][0], acc[a][b][1]);
+            q[a][1] = pack2_bf16(acc[a][b][2], acc[a][b][3]);
+        }
+        // lanes g and g + 1 (g even) exchange halves, so that each has eight neighbouring columns of the 32
+        typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
+        const uint2_t lo = __builtin_amdgcn_permlane16_swap(q[0][0], q[1][0], false, false);
+        const uint2_t hi = __builtin_amdgcn_permlane16_swap(q[0][1], q[1][1], false, false);
+        const uint32_t words[4] = {lo.x, hi.x, lo.y, hi.y};
+        const int n = n0 + wn * 32 + 16 * (g & 1) + 8 * (g >> 1);
+        bf16* to = out + static_cast<size_t>(m) * stride + n;
+        if (vectors && n + 7 < N) {
+            *reinterpret_cast<uint4*>(to) = make_uint4(words[0], words[1], words[2], words[3]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 8; ++v)
+                if (n + v < N) to[v] = bf16{static_cast<uint16_t>(words[v / 2] >> (16 * (v % 2)))};
+        }
     }
 }
 
@@ -240,7 +217,7 @@ gemm_block_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* 
 // row of out to the next.  `splits` > 1: `out` is null and `partial` float32 [splits, M, N] takes the sums of the K axis's pieces.  `gated` = 1 + the
 // gate's number (with limit, slope and shift for the clamped swish): the gated product, w [2N, K], gate rows first; with the paired squared
 // relu out [M, 2N] = relu(x . w^T)^2.  K is a multiple of 64 and at least 64 * splits, x and w begin at multiples of 16 bytes and are smaller
-// than 4 GiB.  Returns 0, a HIP error code, or -1 for what it does not take.
+// than 4 GiB, and tiles times pieces are at most 256, a round.  Returns 0, a HIP error code, or -1 for what it does not take.
 WLLM_API int wllm_gemm_block(const void* x, const void* w, void* out, float* partial, int M, int N, int K, int stride, int splits, int gated,
                              float limit, float slope, float shift, int tile_m, int tile_n, hipStream_t stream) {
     if (M < 1 || N < 1 || K < kBlockKeys || K % kBlockKeys != 0 || splits < 1 || splits > K / kBlockKeys || gated < 0 || gated > kPairedGates ||
@@ -257,9 +234,8 @@ WLLM_API int wllm_gemm_block(const void* x, const void* w, void* out, float* par
     const int columns = gated ? tile_n / 2 : tile_n;
     const int m_tiles = (M - 1) / tile_m + 1, n_tiles = (N - 1) / columns + 1;
     const long long items = static_cast<long long>(m_tiles) * n_tiles * splits;
-    if (items > 0x3fffffffLL) return -1;
-    // a multiple of 8, so that a workgroup's items stay in its XCD's run
-    const int grid = items < 256 ? static_cast<int>((items + 7) / 8 * 8) : 256;
+    if (items > 256) return -1;
+    const int grid = static_cast<int>((items + 7) / 8 * 8);
     const int longest = (K / kBlockKeys + splits - 1) / splits;          // stages of an item
     const GateShape shape{limit, slope, shift};
 #define LAUNCH(TM, TN, GATED)                                                                                                     \
