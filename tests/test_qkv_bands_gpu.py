@@ -40,3 +40,29 @@ def test_halves_and_whole_bands(k, nh, nkv, d, m, tiled):
     kernels.close(got[2], want[2], dtype, "rotated queries, keys and values")
     kernels.close(got[7], want[7], dtype, "pages")
     assert (got[7] != 0).sum() == (want[7] != 0).sum(), "only the tokens' slots are written"
+
+
+# More than eight steps of 32 keys a wavefront, so that its registers are filled again: 2,080 keys are nine steps for some, 4,096 sixteen
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("k", [2080, 4096])
+def test_halves_have_the_bits_of_whole_bands(k, tiled):
+    """The first 20 heads of 34 by themselves are 88 pairs of bands, in halves; all of them 136, whole."""
+    dtype, ps, d = torch.bfloat16, 8, 128
+    torch.manual_seed(6)
+    w = (torch.randn(36 * d, k, device=DEV) / math.sqrt(k)).to(dtype)
+    x, bias = torch.randn(32, k, device=DEV).to(dtype), torch.randn(36 * d, device=DEV) * 0.3
+    inv_freq = 1.0 / (10000.0 ** (torch.arange(0, d, 2, dtype=torch.float32, device=DEV) / d))
+    positions = torch.randint(0, 3000, (32,), dtype=torch.int32, device=DEV)
+
+    def run(m, heads):
+        rows = (heads + 2) * d
+        qkv, cache = torch.zeros(m, rows, dtype=dtype, device=DEV), torch.zeros(m, 2, 1, ps * d, dtype=dtype, device=DEV)
+        part = w[:rows].contiguous()
+        ops.qkv_rope(x[:m], part, qkv, bias[:rows].contiguous(), positions[:m].contiguous(), inv_freq,
+                     torch.arange(m, dtype=torch.int32, device=DEV) * ps, cache, num_heads=heads, num_kv_heads=1, head_dim=d, page_size=ps,
+                     tiles=ops.tile_weight(part) if tiled else None)
+        return qkv
+
+    for m in (1, 16, 17, 32):
+        assert torch.equal(run(m, 20)[:, :20 * d], run(m, 34)[:, :20 * d]), f"{m} tokens"
