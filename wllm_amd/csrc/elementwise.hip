@@ -1,7 +1,7 @@
 // Embedding lookup, RMS norm with residual add, rotation with cache write, gated
 // activation.  Each is bound by memory traffic; the fusions are the ones that save
 // a pass over the residual stream or over the q/k/v rows.
-#include "common.h"
+#include "head_prepare.h"
 
 // ---- embedding: out[i] = float(table[ids[i]]) * scale ---------------------------------
 template <typename T>
@@ -391,15 +391,6 @@ __global__ void rope_cache_vec_kernel(T* __restrict__ qkv, const int* __restrict
         }
     }
 }
-
-// (`head_prepare.hip`)
-WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const float* parts, int splits,
-                               long long split_stride, const float* bias, int bias_width, const int* positions,
-                               const float* inv_freq, const int* slots, void* cache, long long num_pages, int n,
-                               int num_heads, int num_kv_heads, int head_dim, int rotary_dim, int interleaved,
-                               float norm_eps, int norm_dim, int values_are_keys, int page_size, const float* pre_q,
-                               const float* pre_k, float pre_eps, float rot_scale, float temp_coef, int temp_every,
-                               hipStream_t stream);
 
 // Few tokens with a bias or a stack of partial sums: `rope_cache_kernel` is a workgroup a token that goes to memory once for the
 // positions, once for each round of heads and once for the values; that of `head_prepare.hip` has a workgroup for every four

@@ -4,7 +4,7 @@
 // beyond the heads that only take their bias and the sum of their partial sums.  And three small
 // steps of the residual stream and of a block's output: a gate on the attention's result, a copy
 // into a band of columns, and a sum into the stream.  Everything here computes in float32.
-#include "common.h"
+#include "head_prepare.h"
 
 constexpr int kPrepareWaves = 4;
 constexpr int kPrepareMaxHead = 256;
