@@ -48,6 +48,20 @@ def test_products_and_their_rows(n, k):
     assert seen
 
 
+# the most rows that the rule has, by columns
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tile", [(3072, 2048, 192, (192, 128)), (2305, 2047, 448, (192, 128)), (6144, 1024, 128, (192, 128)), (5000, 1100, 64, (192, 128))])
+def test_products_of_many_rows(m, n, k, tile):
+    assert HipBackend.block_tile(m, n, k) == tile
+    torch.manual_seed(66)
+    w, x = (torch.randn(n, k, device=DEV) / math.sqrt(k)).bfloat16(), torch.randn(m, k, device=DEV).bfloat16()
+    out = torch.full((m + 1, n), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops.linear(x, w, out[:m])
+    exact = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -8 * exact.abs() + 1e-30        # (as above)
+    assert bool(((out[:m].double() - exact).abs() <= bound).all()) and bool((out[m] == 7.0).all())
+
+
 @pytest.mark.gpu
 def test_a_row_and_a_column_that_are_not_finite_stay_alone():
     torch.manual_seed(60)
@@ -122,7 +136,8 @@ def test_gated_products_have_the_bits_of_other_tiles(act, inter, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
-@pytest.mark.parametrize("m,inter,k", [(257, 4096, 2048), (385, 1000, 192), (512, 4096, 2048), (600, 250, 64), (1030, 778, 128)])
+@pytest.mark.parametrize("m,inter,k", [(257, 4096, 2048), (385, 1000, 192), (512, 4096, 2048), (600, 250, 64), (1030, 778, 128), (5003, 90, 320),
+                                       (16384, 32, 64), (300, 512, 3072), (700, 500, 4096)])
 def test_gated_products_of_more_rows(act, m, inter, k):
     assert HipBackend.block_gated_tile(m, inter, k) is not None
     torch.manual_seed(63)

@@ -1,5 +1,5 @@
-// out[M, N] = x[M, K] . w[N, K]^T for bfloat16 with some hundred to two thousand rows and few columns (a prompt's projections), on the matrix
-// cores, in tiles of 64 to 192 rows of x by 64 or 128 rows of w: as many as make one round of a workgroup a compute unit.
+// out[M, N] = x[M, K] . w[N, K]^T for bfloat16 with more than 64 rows and few columns (a prompt's projections), on the matrix
+// cores, in tiles of 64 to 192 rows of x by 64 or 128 rows of w: as many as make one round of a workgroup a compute unit (2,048 columns to 3,072 rows).
 // And, where one round is enough, the stack of the sums of a long K axis in pieces, and the gated form out[M, I] = act(x . Wg^T) * (x . Wu^T) with
 // w = [Wg; Wu], whose activation and product are made in the registers the sums are in: a tile's rows of w are then half gate rows, half
 // the up rows that belong to them, and a wavefront has 16 of each.
@@ -19,8 +19,9 @@
 // there.  us, weights from HBM, the library and this kernel, 2,048 keys to 2,048 columns at 100 / 256 / 508 / 1,024 / 1,500 / 2,048 rows
 // 11.3 / 12.1 / 13.2 / 16.8 / 22.4 / 24.3 and 11.1 / 11.8 / 12.0 / 16.2 / 20.5 / 22.1; to 2,560 12.1 / 13.2 / 15.4 / 23.0 / 24.4 / 29.8 and
 // 11.2 / 12.0 / 15.2 / 18.0 / 22.3 / 27.5; to 4,608 at 256 / 508 / 1,024 23.7 / 24.2 / 29.2 and 16.1 / 18.3 / 27.7; 768 keys to 2,048 at 508 / 1,500 7.8 / 10.0 and
-// 6.3 / 9.2.  Tiles of a second round find the machine half empty, and more rows are the library's (4,096 rows to 2,048 columns 34 and 41).  A
-// call of the library costs the host 19 us where a launch costs 6, and a step of a few hundred rows waits for the host.
+// 6.3 / 9.2; 2,300 / 2,560 / 3,001 rows to 2,048 columns 29 / 26 / 28 and 26 / 26 / 28; rows in whole tiles of the library's and few of these lose up to an eighth
+// (128 / 384 / 768 rows to 2,048 11.0 / 13.1 / 14.0 and 12.1 / 12.7 / 15.5).  Tiles of a second round find the machine half empty, and more rows are the library's
+// (4,096 rows to 2,048 columns 34 and 41).  A call of the library costs the host 19 us where a launch costs 6, and a step of a few hundred rows waits for the host.
 //
 // Gated, 2,048 keys to 2 x 16,384 columns at 100 / 164 / 256 rows 35.3 / 37.4 / 42.1, in tiles of 128 37.0 / 44.3 / 48.7; to 2 x 4,096 13.2 / 16.1 / 17.6 and
 // 24.1 / 23.7 / 24.6.  16,384 keys to 2,048 columns in 8 pieces at 65 / 164 rows 20.9 / 24.7 and 26.2 / 26.5.

@@ -514,7 +514,7 @@ class HipBackend:
         rounds = -(-(-(-rows // cls.WIDE_TILE) * -(-n // cls.WIDE_TILE)) // cls.COMPUTE_UNITS)
         return rows * n >= 0.6 * rounds * cls.COMPUTE_UNITS * cls.WIDE_TILE ** 2
 
-    # Tiles of the products of some hundred to two thousand rows (`gemm_block.hip`, which has the figures): rows of x, rows of w, and the time of a
+    # Tiles of the products of one round (`gemm_block.hip`, which has the figures; of 65 rows on, to 2,048 columns up to 3,072): rows of x, rows of w, and the time of a
     # launch that fills at most one round of workgroups, us and us a stage of 64 keys.  (256 rows: only the gated product has them.)
     BLOCK_TILES = ((64, 64, 2.9, 0.27), (128, 64, 3.2, 0.37), (192, 64, 3.6, 0.42), (128, 128, 4.0, 0.51), (192, 128, 4.6, 0.58), (256, 128, 4.6, 0.75))
 
@@ -537,7 +537,10 @@ class HipBackend:
         """The tile of a gated product of `columns` output columns, or None: where one round is enough, up to 256 rows, and beyond where the tiles of
         256 x 256 do not take it.  us, tiles of 128 and here, 2,048 keys to 2 x 16,384 columns at 100 / 164 / 256 rows 37.0 / 44.3 / 48.7 and 35.3 / 37.4 /
         42.1; to 2 x 4,096 24.1 / 23.7 / 24.6 and 13.2 / 16.1 / 17.6, at 300 / 512 rows the library's product with the activation's pass 27.6 / 29.2 and
-        19.7 / 23.9.  One and a half rounds lose (to 2 x 24,576 at 164 rows 57 and 64).  Up to 256 rows all have the same bits."""
+        19.7 / 23.9.  One and a half rounds lose (to 2 x 24,576 at 164 rows 57 and 64).  Beyond 256 rows and 2,048 keys few tiles are a chain of stages on a
+        part of the machine, where the library cuts the K axis (with the activation's pass, 4,096 keys to 2 x 250 columns at 300 / 1,024 / 1,200 rows 14 /
+        18 / 23 and 19 / 19 / 20, 3,072 to 2 x 128 at 1,024 / 1,200 12 / 18 and 15 / 16): from more than 64 tiles on, of more than 3,072 keys 128.
+        Up to 256 rows all have the same bits; beyond, gate and up stay float32 up to the activation, which the library rounds before it."""
         if k > 4096 or (rows > cls.WIDE_TILE and cls.wide_gated_takes(rows, columns, k)):
             return None
         found = cls._one_round(rows, columns, k, gated=True)
@@ -555,11 +558,18 @@ class HipBackend:
     @classmethod
     def block_tile(cls, rows: int, n: int, k: int):
         """The tile in which a product rounded to bfloat16 goes instead of to the library, or None: the quickest of which one round of a
-        workgroup a compute unit is enough.  A K axis of more than 3,072 keys has to fill nine tenths of the round, as the library cuts it where
-        its tiles are few (4,096 keys to 2,048 columns at 128 / 256 / 508 / 1,024 rows 12.9 / 16.2 / 22.0 / 30.6 us there, 20.3 / 20.0 / 21.3 / 28.1
-        here).  Few columns are as quick there (2,048 keys to 64 columns 8.2 and 10.0), which only shows where the step does not wait for the host:
-        at more than 512 rows they are the library's.  A launch at one side of a line or the other differs by some per cent (768 rows to 2,048
-        columns 14.6 and 15.2, to 6,144 26.6 and 27.4); none of 100 sizes within the rule lost more than 5%, most gained 5 to 15, some 30."""
+        workgroup a compute unit is enough.
+
+        Chosen by what a pass takes, not by the launch alone.  Alone (weights from HBM, us, library and here) the tiles are ahead where they fill
+        much of a round (2,048 keys to 2,048 columns at 333 / 900 / 1,200 / 1,800 / 2,300 rows 13 / 16 / 23 / 24 / 29 and 11.7 / 14.8 / 17 / 20 / 26, at
+        3,001 28 and 28) and behind by up to an eighth where the library's own are whole and these few (128 and 768 rows 11 / 14 and 12.1 / 15.5, 384 to
+        3,072 columns 14 and 15.4), by up to a third at few columns (256 rows to 64 / 16 columns 9.9 / 8.1 and 11.5 / 10.5), by more at more keys
+        (4,096 to 2,048 at 128 / 256 rows 13 / 16 and 21 / 21).  But a call of the library costs the host 19 us where a launch costs 6, and steps of up to
+        some 300 rows wait for the host.  Passes of one prompt, us, the library always / where the tiles of 64 x 64 fill less than half of the round or
+        larger ones less than four fifths / this rule: Tokuvik's 100 / 256 / 500 / 768 rows 4,690 / 4,369 / 3,508, 4,788 / 3,978 / 3,604, 5,000 / 4,632 / 4,591, 6,055 / 5,992 / 5,955,
+        Gemma-2B's 100 / 500 / 768 2,203 / 2,225 / 2,089, 3,281 / 3,249 / 3,211, 4,364 / 4,330 / 4,283; in eleven designs at 70 to 1,000 rows this rule is
+        the quickest or within 1%.  More than 512 rows to few columns, and more than 3,072 keys where the tiles fill less than nine tenths of
+        the round, are the library's, which cuts the K axis: there the pass is the GPU's."""
         if k > 4096 or (n < 1024 and rows > 512):
             return None
         found = cls._one_round(rows, n, k)

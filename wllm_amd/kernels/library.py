@@ -190,8 +190,7 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
 
     objects = []
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(names)))) as pool:
-        if os.path.samefile(source_dir, SOURCE_DIR):
-            pool.submit(build_door, verbose)
+        door_run = pool.submit(build_door, verbose) if os.path.samefile(source_dir, SOURCE_DIR) else None
         for name, obj, r in pool.map(compile_one, names):
             if r.returncode != 0:
                 raise KernelLibraryMissing(f"hipcc failed on {name}:\n{r.stderr[-4000:]}")
@@ -205,6 +204,8 @@ def build(verbose: bool = True, force: bool = True, source_dir: str = SOURCE_DIR
     os.replace(tmp, lib_path)
     with open(lib_path + ".stamp", "w", encoding="utf-8") as f:
         f.write(fingerprint)
+    if door_run is not None:
+        door_run.result()
     say(f"built {lib_path} in {time.time() - t0:.0f} s")
     return lib_path
 
