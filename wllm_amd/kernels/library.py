@@ -35,9 +35,11 @@ SOURCE_DIR = os.path.join(PACKAGE_DIR, "csrc")
 LIBRARY_NAME = "libwllm_kernels.so"
 DOOR_SOURCE, DOOR_NAME = "launch_door.cpp", "launch_door"
 ARCH = "gfx950"
-# packed float32 instructions are switched off for all device code
+# Packed float32 instructions are switched off for all device code.  The first 16 words of a kernel's arguments are in scalar registers when its wavefronts
+# start: loaded by the kernel itself they are a trip to memory in front of everything else, in each of a step's 131 to 292 launches (decode steps at Gemma-2B
+# sizes of 1 / 8 / 64 requests 1,311 / 1,401 / 2,161 to 1,293 / 1,375 / 2,113 us, Tokuvik's of 8 2,052 to 1,998, Duvozen's of 24 2,674 to 2,629).
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
-         "-packed-fp32-ops", "-fvisibility=hidden", "-Wno-unused-command-line-argument"]
+         "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-fvisibility=hidden", "-Wno-unused-command-line-argument"]
 
 
 class KernelLibraryMissing(RuntimeError):
