@@ -71,16 +71,24 @@ struct FewRowsShared {
     float row_max[4][kRowsPerTile], row_sum[4][kRowsPerTile];
 };
 
+// How a block of 32 keys lies in pages: pages of a multiple of 4 or of 8 tokens, of 16, or of a power of two from 32 on.  The last two are
+// known to hold a block in two pages, or in one: its page numbers are then the wavefront's, two scalar loads, and a lane's addresses a page's begin and its
+// own place, where the others divide, multiply and look a page up for every load.  A wavefront has a vector unit to itself in a step of few requests, so every instruction in front of the
+// loads counts (2,377 in the kernel for heads of 256 and pages of any multiple of 8, 1,184 in this one; decode steps at Gemma-2B sizes of 1 / 8 / 64 requests
+// 1,293 / 1,375 / 2,113 to 1,260 / 1,326 / 2,078 us, Tokuvik's of 8 1,998 to 1,978, Duvozen's of 24 2,629 to 2,598).  The same bits.
+enum Pages { kPagesOf4, kPagesOf8, kPagesOf16, kPagesFrom32 };
+
 // One work item, by the whole workgroup of 256 threads.
 // SPLIT: the weights of the second product keep 16 bits (rounded weight and remainder, two products).
-template <int HD, bool V16, bool SPLIT>
+template <int HD, Pages PAGES, bool SPLIT>
 __device__ __forceinline__ void
 few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
-              const int* __restrict__ block_tables, const int* __restrict__ items, const int* __restrict__ live_items,
-              const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len, const int* __restrict__ seg_ctx_len,
+              const int* __restrict__ block_tables, const int* __restrict__ items, const int* __restrict__ live_items, 
               bf16* __restrict__ out, float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
-              int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window, int q_stride, float cap_scale,
+              int num_kv_heads, int group, int page_size, int max_pages, float scale_log2e, int window, int q_stride, float cap_scale,
               float softcap, const float* __restrict__ sinks) {
+    constexpr bool V16 = PAGES != kPagesOf4, kWhole = PAGES == kPagesOf16 || PAGES == kPagesFrom32;
+    if (PAGES == kPagesOf16) page_size = 16;
     constexpr int DC = HD / 32;   // 32-wide chunks of the head for the score product
     constexpr int DT = HD / 16;   // 16-row tiles of out^T
     constexpr int kKeyStride = FewRowsShared<HD>::kKeyStride, kPartBytes = FewRowsShared<HD>::kPartBytes;
@@ -105,31 +113,32 @@ few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict_
     const int i = lane % 16, g = lane / 16;
 
     // ---- This lane's queries are asked for first: they arrive while the addresses of the keys and
-    //      values are worked out. ----
-    const int group = num_heads / num_kv_heads;
+    //      values are worked out.  (A lane without a row asks for the last one's: nothing of it is kept.) ----
     const int width = q_stride;                     // elements between two tokens' query rows
     const int total_rows = q_len * group;
     const int first_pos = ctx - q_len;
     const int seg_lo = lowest_key(first_pos, window);   // keys below may be given back
     const int row = row_begin + i;
     const bool row_valid = row < total_rows;
-    const int tok = row_valid ? row / group : 0;
-    const int head = kvh * group + (row_valid ? row % group : 0);
+    int tok = 0, in_group = min(row, total_rows - 1);
+    if (q_len > 1) {
+        tok = in_group / group;
+        in_group -= tok * group;
+    }
+    const int head = kvh * group + in_group;
     const int pos = first_pos + tok;
-    const int lo = lowest_key(pos, window);
+    const int lo = q_len > 1 ? lowest_key(pos, window) : seg_lo;
     // An item's keys lie within one aligned group of 128 (the host's chunk), so each of the four
     // wavefronts has at most one block of 32 keys and nothing is carried from block to block.
-    const int blk_first = key_begin / kKeysPerBlock;
-    const int blk_end = (key_end + kKeysPerBlock - 1) / kKeysPerBlock;
-    const int blk = blk_first + wave;
-    const bool has_block = blk < blk_end;
+    const int blk = static_cast<int>(static_cast<unsigned>(key_begin) / kKeysPerBlock) + wave;
+    const bool has_block = blk * kKeysPerBlock < key_end;
     bf16x8_t qreg[DC];
     if (has_block) {
-        const bf16* qrow = qkv + static_cast<size_t>(q_start + tok) * width + static_cast<size_t>(head) * HD;
+        const bf16* qrow = qkv + static_cast<size_t>(q_start + tok) * width + static_cast<size_t>(head) * HD + 8 * g;
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             Pack16 p;
-            p.u = row_valid ? *reinterpret_cast<const uint4*>(qrow + c * 32 + 8 * g) : make_uint4(0, 0, 0, 0);
+            p.u = *reinterpret_cast<const uint4*>(qrow + c * 32);
             qreg[c] = p.v;
         }
     }
@@ -153,40 +162,59 @@ few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict_
         // a valid page), not to the length.  A key's page and slot come from its place within the
         // block and one division a wavefront: the quotient by the page size as a float product,
         // exact for the few hundred values it is asked for here.
-        const int base_page = kbase / page_size, base_slot = kbase % page_size;     // the same for all lanes
-        const float inv_page = 1.f / static_cast<float>(page_size);
-        auto place = [&](int within, int& page_index, int& slot) {
-            const int x = base_slot + within;                                  // < page_size + 32
-            const int q = static_cast<int>((static_cast<float>(x) + 0.5f) * inv_page);
-            page_index = min(base_page + q, max_pages - 1);
-            slot = x - q * page_size;
-        };
-        const bf16* kpiece[DT];
+        if constexpr (kWhole) {
+            // (page sizes are powers of two: shifts and masks)
+            const int base_page = kbase >> __builtin_ctz(page_size), base_slot = kbase & (page_size - 1);
+            const uint32_t number0 = table[min(base_page, max_pages - 1)], number1 = PAGES == kPagesOf16 ? table[min(base_page + 1, max_pages - 1)] : 0;
+            const bf16 *page0 = cache + number0 * page_elems, *page1 = cache + number1 * page_elems;
+            // pieces of 16 bytes in the order of the rows: half of the loads in either page, or all in one
+            const uint32_t klane = lane * 8 + (PAGES == kPagesOf16 ? 0 : base_slot * HD);
 #pragma unroll
-        for (int j = 0; j < DT; ++j) {
-            // piece f of the block: key f / kPieces, its 8 elements f % kPieces; a wavefront's load
-            // covers whole consecutive rows
-            const int f = j * kWave + lane;
-            int page_index, slot;
-            place(f / kPieces, page_index, slot);
-            kpiece[j] = cache + static_cast<size_t>(table[page_index]) * page_elems + k_off +
-                        static_cast<size_t>(slot) * HD + (f % kPieces) * 8;
-        }
-        int vpage0, vslot0, vpage1 = 0, vslot1 = 0;
-        place(V16 ? 8 * g : 4 * g, vpage0, vslot0);
-        if (!V16) place(16 + 4 * g, vpage1, vslot1);
-        const bf16* vbase0 = cache + static_cast<size_t>(table[vpage0]) * page_elems + v_off + vslot0;
-        const bf16* vbase1 = cache + static_cast<size_t>(V16 ? 0 : table[vpage1]) * page_elems + v_off + vslot1;
+            for (int j = 0; j < DT; ++j) {
+                const bool second = PAGES == kPagesOf16 && j >= DT / 2;
+                kraw[j] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>((second ? page1 : page0) + k_off + klane + (second ? j - DT / 2 : j) * 512));
+            }
+            const bf16* vpage = (PAGES == kPagesOf16 && g >= 2 ? page1 : page0) + v_off;
+            const uint32_t vlane = PAGES == kPagesOf16 ? i * 16 + (g % 2) * 8 : i * page_size + base_slot + 8 * g;
+            const uint32_t vstep = PAGES == kPagesOf16 ? 256 : 16 * page_size;
 #pragma unroll
-        for (int j = 0; j < DT; ++j) kraw[j] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(kpiece[j]));
+            for (int t = 0; t < DT; ++t) va_[t].u = load_streamed(vpage + vlane + t * vstep);
+        } else {
+            const int base_page = kbase / page_size, base_slot = kbase % page_size;     // the same for all lanes
+            const float inv_page = 1.f / static_cast<float>(page_size);
+            auto place = [&](int within, int& page_index, int& slot) {
+                const int x = base_slot + within;                                  // < page_size + 32
+                const int q = static_cast<int>((static_cast<float>(x) + 0.5f) * inv_page);
+                page_index = min(base_page + q, max_pages - 1);
+                slot = x - q * page_size;
+            };
+            const bf16* kpiece[DT];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            const size_t drow = static_cast<size_t>(t * 16 + i) * page_size;
-            if (V16) {
-                va_[t].u = load_streamed(vbase0 + drow);
-            } else {
-                va_[t].half[0] = load_streamed8(vbase0 + drow);
-                va_[t].half[1] = load_streamed8(vbase1 + drow);
+            for (int j = 0; j < DT; ++j) {
+                // piece f of the block: key f / kPieces, its 8 elements f % kPieces; a wavefront's load
+                // covers whole consecutive rows
+                const int f = j * kWave + lane;
+                int page_index, slot;
+                place(f / kPieces, page_index, slot);
+                kpiece[j] = cache + static_cast<size_t>(table[page_index]) * page_elems + k_off +
+                            static_cast<size_t>(slot) * HD + (f % kPieces) * 8;
+            }
+            int vpage0, vslot0, vpage1 = 0, vslot1 = 0;
+            place(V16 ? 8 * g : 4 * g, vpage0, vslot0);
+            if (!V16) place(16 + 4 * g, vpage1, vslot1);
+            const bf16* vbase0 = cache + static_cast<size_t>(table[vpage0]) * page_elems + v_off + vslot0;
+            const bf16* vbase1 = cache + static_cast<size_t>(V16 ? 0 : table[vpage1]) * page_elems + v_off + vslot1;
+#pragma unroll
+            for (int j = 0; j < DT; ++j) kraw[j] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(kpiece[j]));
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const size_t drow = static_cast<size_t>(t * 16 + i) * page_size;
+                if (V16) {
+                    va_[t].u = load_streamed(vbase0 + drow);
+                } else {
+                    va_[t].half[0] = load_streamed8(vbase0 + drow);
+                    va_[t].half[1] = load_streamed8(vbase1 + drow);
+                }
             }
         }
         const bool edge = kbase < seg_lo || kbase + kKeysPerBlock > ctx;
@@ -222,11 +250,12 @@ few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict_
         float sv[8];
         bool ok[8];
         float tile_max = -INFINITY;
+        const int first_key = max(lo, key_begin), end_key = row_valid ? min(pos + 1, key_end) : 0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int t2 = e / 4, v = e % 4;
             const int key = kbase + (V16 ? 8 * g + 4 * t2 + v : 16 * t2 + 4 * g + v);
-            ok[e] = row_valid && key <= pos && key >= lo && key >= key_begin && key < key_end;
+            ok[e] = key >= first_key && key < end_key;
             // with a cap the score is scaled and bent here, and `scale_log2e` is log2(e) alone
             sv[e] = softcap > 0.f ? capped_score_fast(s[t2][v] * cap_scale, softcap) : s[t2][v];
             if (ok[e]) tile_max = fmaxf(tile_max, sv[e]);
@@ -252,18 +281,22 @@ few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict_
         // the row's sum over its four lanes
         l_run = sum_across(sum_across(l_run, 16), 32);
         // ---- out^T = V^T . P^T ----
+        if (edge) {
+            // keys outside the request (stale slots, pages given back) may hold anything,
+            // NaN included; 0 * NaN would poison the sum, so they are cleared
+            uint32_t keep[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = kbase + (V16 ? 8 * g + e : (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4));
+                if (key < ctx && key >= seg_lo) keep[e / 2] |= 0xffffu << (16 * (e % 2));
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+                va_[t].u = make_uint4(va_[t].u.x & keep[0], va_[t].u.y & keep[1], va_[t].u.z & keep[2], va_[t].u.w & keep[3]);
+        }
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-            Pack16 a = va_[t];
-            if (edge) {
-                // keys outside the request (stale slots, pages given back) may hold anything,
-                // NaN included; 0 * NaN would poison the sum, so they are cleared
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int key = kbase + (V16 ? 8 * g + e : (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4));
-                    if (key >= ctx || key < seg_lo) a.s[e] = 0;
-                }
-            }
+            const Pack16 a = va_[t];
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, pv.v, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             if (SPLIT) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, pr.v, acc[t], 0, 0, 0);
         }
@@ -347,19 +380,18 @@ few_rows_item(FewRowsShared<HD>& shared, uint32_t index, const bf16* __restrict_
 
 // Three workgroups a compute unit (168 registers a lane) where the kernel fits them without spilling;
 // two for the head sizes and page sizes whose staging needs more.
-template <int HD, bool V16, bool SPLIT>
-__global__ void __launch_bounds__(256, (HD <= 160 || (HD == 256 && V16)) ? 3 : 2)
-paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
-                            const int* __restrict__ block_tables, const int* __restrict__ items,
-                            const int* __restrict__ live_items, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
-                            const int* __restrict__ seg_ctx_len, bf16* __restrict__ out,
-                            float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
-                            int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window,
-                            int q_stride, float cap_scale, float softcap, const float* __restrict__ sinks) {
+template <int HD, Pages PAGES, bool SPLIT>
+__global__ void __launch_bounds__(256, (HD <= 160 || (HD == 256 && PAGES != kPagesOf4)) ? 3 : 2)
+paged_attention_mfma_kernel(const int* __restrict__ items, const int* __restrict__ live_items, const int* __restrict__ block_tables,
+                            const bf16* __restrict__ qkv, const bf16* __restrict__ cache, int group, int window, int q_stride, int max_pages,
+                            int num_kv_heads, int page_size, bf16* __restrict__ out, float* __restrict__ partial_o,
+                            float* __restrict__ partial_ml, int num_heads, float scale_log2e, float cap_scale, float softcap,
+                            const float* __restrict__ sinks) {
+    // (what stands in front of the loads is asked for first: sixteen words of arguments are in registers when a wavefront begins)
     __shared__ FewRowsShared<HD> shared;
-    few_rows_item<HD, V16, SPLIT>(shared, blockIdx.x, qkv, cache, block_tables, items, live_items, seg_q_start, seg_q_len,
-                                  seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads, page_size, max_pages,
-                                  scale_log2e, window, q_stride, cap_scale, softcap, sinks);
+    few_rows_item<HD, PAGES, SPLIT>(shared, blockIdx.x, qkv, cache, block_tables, items, live_items, out, partial_o, partial_ml,
+                                    num_heads, num_kv_heads, group, page_size, max_pages, scale_log2e, window, q_stride,
+                                    cap_scale, softcap, sinks);
 }
 
 // A step that carries both prompt portions and decoded tokens: the items of both kernels in one launch, each with the bits it
@@ -376,7 +408,7 @@ paged_attention_mfma_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
 // runs of one workgroup a unit 71.3, in two launches 78).
 template <int HD> constexpr int kRoleRun = HD == 64 ? 256 : 64;
 
-template <int HD, bool SPLIT>
+template <int HD, Pages PAGES, bool SPLIT>
 __global__ void __launch_bounds__(kPrefillThreads, 2)
 paged_attention_both_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ cache,
                             const int* __restrict__ block_tables, const int* __restrict__ portion_items, int num_portions,
@@ -384,7 +416,7 @@ paged_attention_both_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
                             const int* __restrict__ live_items, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
                             const int* __restrict__ seg_ctx_len, bf16* __restrict__ out,
                             float* __restrict__ partial_o, float* __restrict__ partial_ml, int num_heads,
-                            int num_kv_heads, int page_size, int max_pages, float scale_log2e, int window,
+                            int num_kv_heads, int group, int page_size, int max_pages, float scale_log2e, int window,
                             int q_stride, float cap_scale, float softcap, const float* __restrict__ sinks) {
     __shared__ union Either {
         PortionShared<HD> portion;
@@ -407,9 +439,9 @@ paged_attention_both_kernel(const bf16* __restrict__ qkv, const bf16* __restrict
                                 seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads, page_size, max_pages,
                                 scale_log2e, window, q_stride, cap_scale, softcap, sinks);
     else
-        few_rows_item<HD, true, SPLIT>(shared.few, index, qkv, cache, block_tables, items, live_items, seg_q_start,
-                                       seg_q_len, seg_ctx_len, out, partial_o, partial_ml, num_heads, num_kv_heads,
-                                       page_size, max_pages, scale_log2e, window, q_stride, cap_scale, softcap, sinks);
+        few_rows_item<HD, PAGES, SPLIT>(shared.few, index, qkv, cache, block_tables, items, live_items, out, partial_o, partial_ml,
+                                        num_heads, num_kv_heads, group, page_size, max_pages, scale_log2e, window, q_stride,
+                                        cap_scale, softcap, sinks);
 }
 
 // Combines the partial results of a (segment, key/value head) whose keys were split over workgroups.
@@ -558,20 +590,19 @@ struct AttentionArguments {
     hipStream_t stream;
 };
 
-template <int HD, bool V16, bool SPLIT>
+template <int HD, Pages PAGES, bool SPLIT>
 int launch_items(const AttentionArguments& a) {
-    paged_attention_mfma_kernel<HD, V16, SPLIT><<<a.num_items, 256, 0, a.stream>>>(
-        a.qkv, a.cache, a.block_tables, a.items, a.live_items, a.seg_q_start, a.seg_q_len, a.seg_ctx_len, a.out,
-        a.partial_o, a.partial_ml, a.num_heads, a.num_kv_heads, a.page_size, a.max_pages, a.scale_log2e, a.window,
-        a.q_stride, a.cap_scale, a.softcap, a.sinks);
+    paged_attention_mfma_kernel<HD, PAGES, SPLIT><<<a.num_items, 256, 0, a.stream>>>(
+        a.items, a.live_items, a.block_tables, a.qkv, a.cache, a.num_heads / a.num_kv_heads, a.window, a.q_stride, a.max_pages,
+        a.num_kv_heads, a.page_size, a.out, a.partial_o, a.partial_ml, a.num_heads, a.scale_log2e, a.cap_scale, a.softcap, a.sinks);
     return 0;
 }
 
-template <int HD, bool SPLIT>
+template <int HD, Pages PAGES, bool SPLIT>
 int launch_both(const AttentionArguments& a) {
-    paged_attention_both_kernel<HD, SPLIT><<<a.num_portions + a.num_items, kPrefillThreads, 0, a.stream>>>(
+    paged_attention_both_kernel<HD, PAGES, SPLIT><<<a.num_portions + a.num_items, kPrefillThreads, 0, a.stream>>>(
         a.qkv, a.cache, a.block_tables, a.portion_items, a.num_portions, a.items, a.num_items, a.live_items, a.seg_q_start,
-        a.seg_q_len, a.seg_ctx_len, a.out, a.partial_o, a.partial_ml, a.num_heads, a.num_kv_heads, a.page_size, a.max_pages,
+        a.seg_q_len, a.seg_ctx_len, a.out, a.partial_o, a.partial_ml, a.num_heads, a.num_kv_heads, a.num_heads / a.num_kv_heads, a.page_size, a.max_pages,
         a.scale_log2e, a.window, a.q_stride, a.cap_scale, a.softcap, a.sinks);
     return 0;
 }
@@ -580,15 +611,20 @@ template <int HD>
 int launch_all(const AttentionArguments& a) {
     if (a.num_portions > 0) {
         if constexpr (HD == 64 || HD == 128 || HD == 256) {
-            const int status = a.split_weights ? launch_both<HD, true>(a) : launch_both<HD, false>(a);
+            const int status = a.page_size == 16 ? (a.split_weights ? launch_both<HD, kPagesOf16, true>(a) : launch_both<HD, kPagesOf16, false>(a))
+                                                 : (a.split_weights ? launch_both<HD, kPagesOf8, true>(a) : launch_both<HD, kPagesOf8, false>(a));
             if (status != 0) return status;
         } else {
             return -1;
         }
     } else if (a.num_items > 0) {
-        const int status = a.page_size % 8 == 0
-            ? (a.split_weights ? launch_items<HD, true, true>(a) : launch_items<HD, true, false>(a))
-            : (a.split_weights ? launch_items<HD, false, true>(a) : launch_items<HD, false, false>(a));
+        const bool power = (a.page_size & (a.page_size - 1)) == 0;
+#define ITEMS(PAGES) (a.split_weights ? launch_items<HD, PAGES, true>(a) : launch_items<HD, PAGES, false>(a))
+        const int status = a.page_size == 16             ? ITEMS(kPagesOf16)
+                           : power && a.page_size >= 32 ? ITEMS(kPagesFrom32)
+                           : a.page_size % 8 == 0        ? ITEMS(kPagesOf8)
+                                                         : ITEMS(kPagesOf4);
+#undef ITEMS
         if (status != 0) return status;
     }
     if (a.num_reduce_items >= 64) {
