@@ -14,7 +14,8 @@ its first token among the step's tokens, first key, end key, partial slot (-1: t
 the final result), the segment's context length: what the kernel needs of the segment comes with
 the item, in the one read it begins with, and not from the segments' arrays in a second trip to memory.  A partial slot holds
 one tile of 16 rows.  A reduce item is 8 int32: segment, key/value head, first partial slot, number
-of splits, first row of the tile, slots between two splits, 2 unused.  A prefill item (long
+of splits, first row of the tile, slots between two splits, rows of the segment, the place of its first token: all that the
+combining kernel needs, in one read.  A prefill item (long
 segments, 64 rows each, for the kernel that stages keys and values through shared memory) is
 8 int32: segment, key/value head, first row, first key, end key, partial slot (-1: final), 2
 unused.  The keys of a block of rows are split over several prefill items when the step has too
@@ -210,6 +211,8 @@ def build_tile_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
     rs[..., 3] = ns[st][None, :]
     rs[..., 4] = row0[st][None, :]
     rs[..., 5] = 1
+    rs[..., 6] = rows[seg_of[st]][None, :]
+    rs[..., 7] = q_start[seg_of[st]][None, :]
     return it.reshape(-1, ITEM_INTS), rs.reshape(-1, ITEM_INTS), per_head * num_kv_heads
 
 
@@ -345,6 +348,8 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
             rs[..., 3] = ns[:, None, None]
             rs[..., 4] = tile[None, None, :] * ROWS_PER_TILE
             rs[..., 5] = 1
+            rs[..., 6] = rows[idx][:, None, None]
+            rs[..., 7] = q_start[idx][:, None, None]
             keep_r = np.broadcast_to((split_seg[:, None] & tile_live)[:, None, :], (S, num_kv_heads, T))
             reduces.append(rs[keep_r].reshape(-1, ITEM_INTS))
         slots = int((n_split_seg * num_kv_heads * rt).sum())
@@ -402,6 +407,8 @@ def build_work_items(q_len: np.ndarray, ctx_len: np.ndarray, group: int, num_kv_
             rs[..., 3] = ns[sb][None, :, None]
             rs[..., 4] = first_row[None]
             rs[..., 5] = tiles
+            rs[..., 6] = rows[seg_of[sb]][None, :, None]
+            rs[..., 7] = q_start[seg_of[sb]][None, :, None]
             reduces.append(rs[:, live].reshape(-1, ITEM_INTS))
         slots += per_head * num_kv_heads
     items = np.concatenate(items) if items else np.zeros((0, ITEM_INTS), np.int32)
