@@ -944,6 +944,44 @@ def gated_lookup(gate: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col
         call("gated_lookup", gate, ids, table, int(col0), out, activation)
 
 
+def token_side_takes(x: torch.Tensor, w_gate: torch.Tensor, w_proj: torch.Tensor, table: torch.Tensor) -> bool:
+    """Whether `token_side` has a kernel for these operands: bfloat16, at most 16 rows, a table's band of 32 or 64 columns, a
+    stream of 128 to 2,048 in multiples of 128, at aligned addresses.  Up to 16 rows every workgroup makes the small product for itself in the time that
+    the three launches wait for each other (us at 1 / 8 / 16 rows, the three 8.4 / 8.7 / 8.9, this one 5.9 / 6.7 / 7.4; with a second
+    tile of rows 9.9 and 10.4 at 32); the many-row products tile it better."""
+    n, hidden = x.shape
+    return (x.dtype == torch.bfloat16 and table.dtype == torch.bfloat16 and 1 <= n <= 16 and w_gate.shape[0] in (32, 64)
+            and 128 <= hidden <= 2048 and hidden % 128 == 0 and w_proj.shape[0] == hidden
+            and (x.data_ptr() | w_gate.data_ptr() | w_proj.data_ptr()) % 16 == 0)
+
+
+def token_side(x: torch.Tensor, w_gate: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col0: int, w_proj: torch.Tensor,
+               out: torch.Tensor, activation: str, gate_tiles: Optional[torch.Tensor] = None,
+               proj_tiles: Optional[torch.Tensor] = None) -> None:
+    """out = w_proj (act(w_gate x) * table[ids, col0 : col0 + d]): `linear`, `gated_lookup` and `linear` in one launch, with their
+    roundings, where `token_side_takes` says so.  x T [n, hidden]; w_gate T [d, hidden] and w_proj T [hidden, d] with their tile-major
+    copies, both or neither; ids int32 [n]; table T [V, D] with col0 + d <= D; out T [n, hidden]."""
+    _need(activation in ACTIVATIONS, lambda: f"activation {activation!r}: expected one of {sorted(ACTIVATIONS)}")
+    _dense(x, "x", torch.bfloat16)
+    _need(x.dim() == 2, "x: expected [n, hidden]")
+    n, hidden = x.shape
+    _dense(w_gate, "w_gate", x.dtype)
+    _need(w_gate.dim() == 2 and w_gate.shape[1] == hidden, "w_gate: expected [d, hidden]")
+    d = w_gate.shape[0]
+    _dense(w_proj, "w_proj", x.dtype, (hidden, d))
+    _dense(table, "table", x.dtype)
+    _need(table.dim() == 2 and 0 <= col0 and col0 + d <= table.shape[1], "table: expected [V, at least col0 + d]")
+    _need(token_side_takes(x, w_gate, w_proj, table), "sizes that `token_side` does not take")
+    _dense(ids, "ids", torch.int32, (n,))
+    _dense(out, "out", x.dtype, (n, hidden))
+    _need((gate_tiles is None) == (proj_tiles is None), "tile-major copies: both or neither")
+    _check_tiles(gate_tiles, w_gate, 1)
+    _check_tiles(proj_tiles, w_proj, 1)
+    if gate_tiles is not None:
+        _need((gate_tiles.data_ptr() | proj_tiles.data_ptr()) % 16 == 0, "tile-major copies: at multiples of 16 bytes")
+    call("token_side", x, w_gate, ids, table, int(col0), w_proj, out, activation, gate_tiles, proj_tiles)
+
+
 def head_linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor) -> None:
     """A product head by head: y[r, h*O + o] = sum_k x[r, h*K + k] * w[h, o, k], float32 sums in ascending
     order of k (on the matrix cores, where they take the sizes, 32 at a time).  x T [n, heads*K] and y T [n, heads*O] may be bands of wider tensors; w T [heads, O, K]."""
@@ -1705,6 +1743,21 @@ def _register_own():
                 launch=lambda fn, stream, gate, ids, table, col0, out, activation: fn(
                     p(gate), p(ids), p(table), table.shape[1], col0, p(out), int(gate.dtype == torch.bfloat16),
                     ACTIVATIONS[activation], gate.shape[0], gate.shape[1], stream))
+    def side_emulate(x, w_gate, ids, table, col0, w_proj, out, activation, gate_tiles, proj_tiles):
+        gate = x.new_empty(x.shape[0], w_gate.shape[0])
+        linear(x, w_gate, gate, gate_tiles)
+        bent = torch.empty_like(gate)
+        gated_lookup(gate, ids, table, col0, bent, activation)
+        linear(bent, w_proj, out, proj_tiles)
+
+    register_op("token_side", entry_point="wllm_token_side",
+                argtypes=[c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int,
+                          c_void_p],
+                launch=lambda fn, stream, x, w_gate, ids, table, col0, w_proj, out, activation, gate_tiles, proj_tiles: fn(
+                    p(x), p(gate_tiles if gate_tiles is not None else w_gate), p(ids), p(table), table.shape[1], col0,
+                    p(proj_tiles if proj_tiles is not None else w_proj), int(gate_tiles is not None), p(out), x.shape[0], x.shape[1],
+                    w_gate.shape[0], ACTIVATIONS[activation], stream),
+                emulate=side_emulate)
     register_op("head_linear", entry_point="wllm_head_linear",
                 argtypes=[c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int, c_int, c_void_p],
                 launch=lambda fn, stream, x, w, y: fn(

@@ -53,11 +53,15 @@ class TokenSide:
         self.w_proj, self.t_proj = load_matrix(fetch, fetch.matrix(s.proj_weight))
         self.norm.load(fetch)
 
-    def forward(self, ctx, x: torch.Tensor) -> Product:
-        """x: the stream in the activation type [n, hidden].  Returns the part's last product; the block
-        puts it under `self.norm` as it adds it."""
+    def forward(self, ctx, x: torch.Tensor):
+        """x: the stream in the activation type [n, hidden].  Returns the part's last product, or what it gave where a kernel
+        makes the whole part; the block puts it under `self.norm` as it adds it."""
         s = self.spec
         n = x.shape[0]
+        if (self.t_gate is None) == (self.t_proj is None) and ops.token_side_takes(x, self.w_gate, self.w_proj, self.table):
+            out = ctx.buffer("side_out", (n, s.hidden_size), ctx.dtype)
+            ops.token_side(x, self.w_gate, ctx.token_ids, self.table, s.offset, self.w_proj, out, s.activation, self.t_gate, self.t_proj)
+            return out
         gate = ctx.buffer("side_gate", (n, s.dim), ctx.dtype)
         ops.linear(x, self.w_gate, gate, self.t_gate)
         g = ctx.buffer("side_in", (n, s.dim), ctx.dtype)
