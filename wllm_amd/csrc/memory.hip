@@ -458,28 +458,94 @@ memory_chunk_kernel(const float* __restrict__ qk, const float* __restrict__ step
     }
 }
 
-// A workgroup owns (head, segment, 16 columns of P; the column behind the last is the normaliser's, as above).  Its four
+// A workgroup owns (head, segment, 16 columns of P; the column behind the last is the normaliser's, as above).  Its first four
 // wavefronts cut the channels, each with TILES tiles of 16: lane (i, g) holds the channels 4g .. 4g + 3 of a tile in column
 // i, which is what a product leaves and, channel by channel, what it takes (the k-th of four products takes the channels
-// 4g + k), so the memory never moves between lanes.  The wavefronts' parts of y meet in shared memory (two places in
-// turn: one barrier a chunk, which the memory's own chain does not wait for).  The operands of a chunk are asked for
-// kAhead chunks before they are used.
+// 4g + k), so the memory never moves between lanes.  They keep the memory and read it for every chunk; what is left of a chunk's results
+// (the part that its own tokens make, the sum over the wavefronts, the stores) is the other four's, a chunk and two chunks behind, beside them
+// on their SIMDs.  One barrier a chunk, two places of shared memory in turn.  The operands of a chunk are asked for kAhead chunks before they are used, while
+// the products that free their registers run.
+// What bounds it: the chain of a chunk in one wavefront, of which the products (32 clocks each, 8 TILES + TILES) should be all. (Three prompts of 3,001
+// tokens, 16 heads of 128 by 128, us: with the others' work in the same chain, and so many registers that a compute unit ran one workgroup, 157; now 115.)
 template <int TILES>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512, TILES <= 2 ? 4 : 2)
 memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride, float* __restrict__ state, long long state_stride,
                          long long n_offset, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
                          const int* __restrict__ state_slots, float* __restrict__ y, float* __restrict__ nq, int heads, int d,
                          int p_dim, int from) {
-    constexpr int C = 64 * TILES, kAhead = TILES <= 2 ? 4 : 2;
-    __shared__ memory_float4 part_s[2][4][kWave];
+    constexpr int C = 64 * TILES, kAhead = 2, kOwnAhead = 6;
+    __shared__ memory_float4 read_s[2][4][kWave], part_s[2][4][kWave];
     const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * 16;
     const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
     if (q_len < from) return;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) % 4;
+    const bool keeps = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) < 4;
     const int i = lane % 16, g = lane / 16;
     const int p = p0 + i;
     const bool norm_col = nq != nullptr && p == p_dim;
     const bool live = p < p_dim || norm_col;
+    const float* first = chunks + (static_cast<size_t>(first_place(q_start, from)) * heads + h) * chunk_floats(C);
+    const bf16* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
+    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(v_stride);
+    auto begins = [&](int c) { return min(c * kChunk, q_len - kChunk); };      // (the last chunk: the last 16 tokens)
+    const int count = (q_len + kChunk - 1) / kChunk;
+    // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
+    auto meet = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (!keeps) {
+        // wavefront w: the part of the tokens 4w .. 4w + 3 as keys; then the sums of the tokens 4g + w
+        struct Own { float n; bf16 v; };
+        const unsigned n_at = (2 * kChunk + 5) * C + i * kChunk + 4 * wave + g;
+        auto load = [&](int c) __attribute__((always_inline)) {
+            return Own{(first + static_cast<size_t>(c) * heads * chunk_floats(C))[n_at],
+                       (v_first + static_cast<size_t>(begins(c)) * v_stride)[(4 * wave + g) * row + col]};
+        };
+        auto add_own = [&](int c, const Own& now) __attribute__((always_inline)) {
+            const float x = begins(c) + 4 * wave + g >= c * kChunk ? (norm_col ? 1.f : to_float(now.v)) : 0.f;
+            part_s[c % 2][wave][lane] = add_causal_product(now.n, x, read_s[c % 2][wave][lane], i, g, [&](int q) { return 4 * wave + q; });
+        };
+        auto finish = [&](int c) __attribute__((always_inline)) {
+            const float* parts = reinterpret_cast<const float*>(&part_s[c % 2][0][lane]) + wave;
+            float o = parts[0];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
+            const int t = begins(c) + 4 * g + wave;
+            if (live && t >= c * kChunk) {
+                if (norm_col) nq[static_cast<size_t>(q_start + t) * heads + h] = o;
+                else y[static_cast<size_t>(q_start + t) * heads * p_dim + static_cast<size_t>(h) * p_dim + p] = o;
+            }
+        };
+        // (kOwnAhead chunks ahead: a wait for these loads is one for the stores in front of them, too)
+        Own ring[kOwnAhead];
+#pragma unroll
+        for (int a = 0; a < kOwnAhead; ++a) {
+            ring[a] = load(min(a, count - 1));
+            __builtin_amdgcn_sched_barrier(0);           // (in this order, which the waits of the loop count on)
+        }
+        auto step = [&](int c, int a) __attribute__((always_inline)) {
+            add_own(c + a, ring[a]);
+            __builtin_amdgcn_sched_barrier(0);
+            ring[a] = load(min(c + a + kOwnAhead, count - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            if (c + a > 0) finish(c + a - 1);
+            meet();
+        };
+        meet();                                                              // chunk 0 has read the state
+        int c = 0;
+        for (; c + kOwnAhead <= count; c += kOwnAhead) {
+#pragma unroll
+            for (int a = 0; a < kOwnAhead; ++a) step(c, a);
+        }
+#pragma unroll
+        for (int a = 0; a < kOwnAhead - 1; ++a)
+            if (c + a < count) step(c, a);
+        finish(count - 1);
+        return;
+    }
     float* request = state + static_cast<size_t>(state_slots[seg]) * state_stride;
     float* s_rows = norm_col ? request + n_offset + static_cast<size_t>(h) * d : request + static_cast<size_t>(h) * d * p_dim + p;
     const size_t s_step = norm_col ? 1 : p_dim;
@@ -494,34 +560,31 @@ memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride,
         }
     struct Operands {
         memory_float4 q[TILES], k[TILES], f[TILES];
-        float rest[TILES], n;
+        float rest[TILES];
         bf16 v[4];
     };
-    const float* first = chunks + (static_cast<size_t>(first_place(q_start, from)) * heads + h) * chunk_floats(C);
-    const bf16* v_first = v + static_cast<size_t>(q_start) * v_stride + static_cast<size_t>(h) * p_dim;
     // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
     const unsigned q_at = i * C + ch0 + 4 * g, k_at = kChunk * C + (ch0 + i) * kChunk + 4 * g, f_at = 2 * kChunk * C + ch0 + 4 * g;
-    const unsigned rest_at = (2 * kChunk + 1) * C + (ch0 + i) * 4 + g, n_at = (2 * kChunk + 5) * C + i * kChunk + 4 * wave + g;
-    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(v_stride);
-    auto begins = [&](int c) { return min(c * kChunk, q_len - kChunk); };      // (the last chunk: the last 16 tokens)
-    auto load = [&](int c) {
-        Operands o;
+    const unsigned rest_at = (2 * kChunk + 1) * C + (ch0 + i) * 4 + g;
+    // what the products read, and (asked for behind the products' results, for a copy of it would wait for it) the decays
+    auto load = [&](int c, Operands& o) __attribute__((always_inline)) {
         const float* at = first + static_cast<size_t>(c) * heads * chunk_floats(C);
+        const bf16* v_chunk = v_first + static_cast<size_t>(begins(c)) * v_stride;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[(4 * u + g) * row + col];
 #pragma unroll
         for (int j = 0; j < TILES; ++j) {
             o.q[j] = *reinterpret_cast<const memory_float4*>(at + q_at + 16 * j);
             o.k[j] = *reinterpret_cast<const memory_float4*>(at + k_at + 16 * kChunk * j);
-            o.f[j] = *reinterpret_cast<const memory_float4*>(at + f_at + 16 * j);
             o.rest[j] = at[rest_at + 64 * j];
         }
-        o.n = at[n_at];
-        const bf16* v_chunk = v_first + static_cast<size_t>(begins(c)) * v_stride;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) o.v[u] = v_chunk[(4 * u + g) * row + col];
-        return o;
     };
-    const int count = (q_len + kChunk - 1) / kChunk;
-    auto walk = [&](int c, const Operands& now) {
+    auto load_decays = [&](int c, Operands& o) __attribute__((always_inline)) {
+        const float* at = first + static_cast<size_t>(c) * heads * chunk_floats(C);
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) o.f[j] = *reinterpret_cast<const memory_float4*>(at + f_at + 16 * j);
+    };
+    auto walk = [&](int c, Operands& now) __attribute__((always_inline)) {
         memory_float4 x, read[TILES];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
@@ -542,49 +605,40 @@ memory_chunk_scan_kernel(const float* chunks, const bf16* v, long long v_stride,
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int j = 0; j < TILES; ++j) own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][u], x[u], own[j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(min(c + kAhead, count - 1), now);
+        __builtin_amdgcn_sched_barrier(0);
+        memory_float4 part = read[0];
+#pragma unroll
+        for (int j = 1; j < TILES; ++j) part += read[j];
+        read_s[c % 2][wave][lane] = part;                                    // a wavefront's part: its channels of the memory
 #pragma unroll
         for (int j = 0; j < TILES; ++j)
 #pragma unroll
             for (int u = 0; u < 4; ++u) s[j][u] = fmaf(now.f[j][u], s[j][u], own[j][u]);
-        // a wavefront's part: its channels of the memory, and four of the chunk's own tokens
-        const float mine = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
-        memory_float4 part = read[0];
-#pragma unroll
-        for (int j = 1; j < TILES; ++j) part += read[j];
-        part = add_causal_product(now.n, mine, part, i, g, [&](int q) { return 4 * wave + q; });
-        part_s[c % 2][wave][lane] = part;
-        // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        // wavefront w writes the tokens 4g + w
-        const float* parts = reinterpret_cast<const float*>(&part_s[c % 2][0][lane]) + wave;
-        float o = parts[0];
-#pragma unroll
-        for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
-        const int t = begins(c) + 4 * g + wave;
-        if (live && t >= c * kChunk) {
-            if (norm_col) nq[static_cast<size_t>(q_start + t) * heads + h] = o;
-            else y[static_cast<size_t>(q_start + t) * heads * p_dim + static_cast<size_t>(h) * p_dim + p] = o;
-        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_decays(min(c + kAhead, count - 1), now);
+        meet();
     };
     // the operands of kAhead chunks in turn (beyond the last chunk: the last's once more).  The loads stay where they are
     // written: the scratch and v may alias y as far as the compiler knows, and the empty statements touch memory.
     Operands ring[kAhead];
 #pragma unroll
-    for (int a = 0; a < kAhead; ++a) ring[a] = load(min(a, count - 1));
+    for (int a = 0; a < kAhead; ++a) {
+        load(min(a, count - 1), ring[a]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_decays(min(a, count - 1), ring[a]);
+        __builtin_amdgcn_sched_barrier(0);               // (in this order, which the waits of the loop count on)
+    }
     int c = 0;
     for (; c + kAhead <= count; c += kAhead) {
 #pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            walk(c + a, ring[a]);
-            ring[a] = load(min(c + a + kAhead, count - 1));
-            asm volatile("" ::: "memory");
-        }
+        for (int a = 0; a < kAhead; ++a) walk(c + a, ring[a]);
     }
 #pragma unroll
-    for (int a = 0; a < kAhead; ++a)
+    for (int a = 0; a < kAhead - 1; ++a)
         if (c + a < count) walk(c + a, ring[a]);
+    meet();                                                                  // the others' last sums
 #pragma unroll
     for (int j = 0; j < TILES; ++j)
 #pragma unroll
@@ -624,7 +678,7 @@ WLLM_API int wllm_memory_scan(const float* qk, const void* v, long long v_stride
         memory_chunk_kernel<R><<<chunk_grid, 256, 0, stream>>>(qk, steps, decays, seg_q_start, seg_q_len, segments, chunks, \
                                                                tokens, heads, d, row_decays, from);                    \
         if (const int err = launch_status()) return err;                                                               \
-        memory_chunk_scan_kernel<R><<<grid, 256, 0, stream>>>(chunks, static_cast<const bf16*>(v), v_stride, state,    \
+        memory_chunk_scan_kernel<R><<<grid, 512, 0, stream>>>(chunks, static_cast<const bf16*>(v), v_stride, state,    \
                                                               state_stride, n_offset, seg_q_start, seg_q_len, state_slots, y, \
                                                               steps ? nq : nullptr, heads, d, p_dim, from);            \
     } while (0)

@@ -542,7 +542,7 @@ ssm_scan_kernel(const T* __restrict__ xbc, const float* __restrict__ steps, int 
 // v_mfma_f32_16x16x4_f32 (float32 in and out), 17 of them a wavefront and chunk.  A chunk begins every 16 tokens of a
 // segment; the last one is filled with tokens that change nothing (d = 0, f = 1, B = C = 0).
 // The walk token by token is bound by its chain (0.27 us a token).  64 heads of 64 with 128 rows of state: 1,500 tokens
-// 410 us token by token, 13 and 86 us for the two kernels here (a chunk takes 1 us, of which the products are a quarter);
+// 410 us token by token, 13 and 73 us for the two kernels here (a chunk takes 0.75 us, of which the products are a third);
 // 64 tokens 21 us against 7 and 9, one line between the two ways; of more heads a group it lies further on. ----
 constexpr int kChunkHeadFloats = kChunk * kChunk + 3 * kChunk;       // N, pre, suf d, pre_16 (and padding)
 
@@ -660,29 +660,117 @@ ssm_chunk_kernel(const bf16* __restrict__ xbc, const bf16* __restrict__ dt_in, l
     }
 }
 
-// A workgroup owns (head, segment, 16 columns of P); its four wavefronts cut the rows of state, each with TILES tiles of
+// A workgroup owns (head, segment, 16 columns of P); its first four wavefronts cut the rows of state, each with TILES tiles of
 // 16: lane (i, g) holds the rows 4g .. 4g + 3 of a tile in column i, which is what a product leaves and, row by row, what
-// it takes (the k-th of four products takes the rows 4g + k), so the state never moves between lanes.  The wavefronts'
-// parts of y meet in shared memory (two places in turn: one barrier a chunk, which the state's own chain does not wait
-// for).  The operands of the next chunks are asked for kAhead chunks before they are used.
+// it takes (the k-th of four products takes the rows 4g + k), so the state never moves between lanes.  They keep the state and read it for
+// every chunk; what is left of a chunk's results (the part that its own tokens make, the sum over the wavefronts, the stores) is the other four's, a chunk
+// and two chunks behind, beside them on their SIMDs.  One barrier a chunk, two places of shared memory in turn.  The operands of a chunk are asked
+// for kAhead chunks before they are used, while the products that free their registers run.
+// What bounds it: the chain of a chunk in one wavefront, of which the products (32 clocks each, 8 TILES) should be all
+// (16 of them 0.25 us of a chunk's 0.7; with the other wavefronts' work in the same chain 83 us for 1,500 tokens of 64 heads of 64 with 128 rows of state, now
+// 73; without the loads of B and C and their conversions 52).
 struct alignas(8) SsmFour { bf16 v[4]; };
 
 template <int TILES>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512, TILES <= 2 ? 4 : 2)
 ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xbc, const float* __restrict__ d_skip,
                       float* __restrict__ state, long long state_stride, const int* __restrict__ seg_q_start,
                       const int* __restrict__ seg_q_len, const int* __restrict__ state_slots, float* __restrict__ y, int heads,
                       int groups, int n_state, int p_dim, int from) {
-    constexpr int C = 64 * TILES, kAhead = 4;
-    __shared__ ssm_float4 part_s[2][4][kWave];
+    constexpr int C = 64 * TILES, kAhead = 3, kOwnAhead = 6;
+    __shared__ ssm_float4 read_s[2][4][kWave], part_s[2][4][kWave];
     const int h = blockIdx.x, seg = blockIdx.y, p0 = blockIdx.z * 16;
     const int q_len = seg_q_len[seg], q_start = seg_q_start[seg];
     if (q_len < from) return;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) % 4;
+    const bool keeps = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) < 4;
     const int i = lane % 16, g = lane / 16;
     const int p = p0 + i;
     const bool live = p < p_dim;
     const int inner = heads * p_dim, channels = inner + 2 * groups * n_state;
+    const size_t first = static_cast<size_t>(first_place(q_start, from));
+    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), x_row = 2 * static_cast<unsigned>(channels);
+    // Where the next chunk's operands lie: addresses that are the same in all lanes, moved on by a sum a chunk (and not beyond the last chunk); a lane's
+    // offsets beside them are bytes in 32 bits.  (Worked out from the chunk's number: 76 us a scan, now 73.)
+    struct Place {
+        const char *x, *of, *rows;
+        int left;                                        // tokens from this chunk on
+    };
+    auto move_on = [&](Place& at) __attribute__((always_inline)) {
+        const bool more = at.left > kChunk;
+        at.x += more ? static_cast<size_t>(kChunk) * x_row : 0;
+        at.of += more ? static_cast<size_t>(heads) * kChunkHeadFloats * sizeof(float) : 0;
+        at.rows += more ? static_cast<size_t>(groups) * 2 * kChunk * C * sizeof(bf16) : 0;
+        at.left -= more ? kChunk : 0;
+    };
+    // (beyond the last token, that token's once more: what it is multiplied by is zero)
+    auto x_of = [&](const Place& at, unsigned row_at) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16*>(at.x + (min(row_at, static_cast<unsigned>(min(kChunk, at.left) - 1) * x_row) + 2 * col));
+    };
+    Place next = {reinterpret_cast<const char*>(xbc + static_cast<size_t>(q_start) * channels + h * p_dim),
+                  reinterpret_cast<const char*>(of_head + (first * heads + h) * kChunkHeadFloats),
+                  reinterpret_cast<const char*>(of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C), q_len};
+    const int count = (q_len + kChunk - 1) / kChunk;
+    // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
+    auto meet = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (!keeps) {
+        // wavefront w: the part of the tokens 4g + w as keys, then their sums
+        const float skip = d_skip[h];
+        float* y_first = y + static_cast<size_t>(q_start) * inner + h * p_dim;
+        struct Own { ssm_float4 pre; float n; bf16 x; };
+        const unsigned n_at = 4 * (i * kChunk + 4 * g + wave), pre_at = 4 * (kChunk * kChunk + 4 * g), x_at = (4 * g + wave) * x_row;
+        auto load = [&]() __attribute__((always_inline)) {
+            const Own o = {*reinterpret_cast<const ssm_float4*>(next.of + pre_at), *reinterpret_cast<const float*>(next.of + n_at), x_of(next, x_at)};
+            move_on(next);
+            return o;
+        };
+        float mine[2];
+        auto add_own = [&](int c, int place, const Own& now) __attribute__((always_inline)) {
+            mine[place] = c * kChunk + 4 * g + wave < q_len ? to_float(now.x) : 0.f;
+            part_s[place][wave][lane] = add_causal_product(now.n, mine[place], read_s[place][wave][lane] * now.pre, i, g, [&](int q) { return 4 * q + wave; });
+        };
+        auto finish = [&](int c, int place) __attribute__((always_inline)) {
+            const float* parts = reinterpret_cast<const float*>(&part_s[place][0][lane]) + wave;
+            float o = parts[0];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
+            const int t = 4 * g + wave;
+            if (live && c * kChunk + t < q_len)
+                (y_first + static_cast<size_t>(c) * kChunk * inner)[t * static_cast<unsigned>(inner) + col] = fmaf(skip, mine[place], o);
+        };
+        // (kOwnAhead chunks ahead: a wait for these loads is one for the stores in front of them, too)
+        Own ring[kOwnAhead];
+#pragma unroll
+        for (int a = 0; a < kOwnAhead; ++a) {
+            ring[a] = load();
+            __builtin_amdgcn_sched_barrier(0);           // (in this order, which the waits of the loop count on)
+        }
+        auto step = [&](int c, int a) __attribute__((always_inline)) {
+            add_own(c + a, a % 2, ring[a]);
+            __builtin_amdgcn_sched_barrier(0);
+            ring[a] = load();
+            __builtin_amdgcn_sched_barrier(0);
+            if (c + a > 0) finish(c + a - 1, 1 - a % 2);
+            meet();
+        };
+        meet();                                                              // chunk 0 has read the state
+        int c = 0;
+        for (; c + kOwnAhead <= count; c += kOwnAhead) {
+#pragma unroll
+            for (int a = 0; a < kOwnAhead; ++a) step(c, a);
+        }
+#pragma unroll
+        for (int a = 0; a < kOwnAhead - 1; ++a)
+            if (c + a < count) step(c, a);
+        if (count % 2) finish(count - 1, 0);
+        else finish(count - 1, 1);
+        return;
+    }
     float* s_rows = state + static_cast<size_t>(state_slots[seg]) * state_stride + static_cast<size_t>(h) * n_state * p_dim + p;
     const int n0 = wave * 16 * TILES;
     ssm_float4 s[TILES];
@@ -693,44 +781,32 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
             const int n = n0 + 16 * j + 4 * g + u;
             s[j][u] = live && n < n_state ? s_rows[static_cast<size_t>(n) * p_dim] : 0.f;
         }
-    const float skip = d_skip[h];
     struct Operands {
         SsmFour c[TILES], b[TILES];
-        ssm_float4 pre, suf;
-        float n, all;
+        ssm_float4 suf;
+        float all;
         bf16 x[4];
     };
-    const size_t first = static_cast<size_t>(first_place(q_start, from));
-    const float* head_first = of_head + (first * heads + h) * kChunkHeadFloats;
-    const bf16* group_first = of_group + (first * groups + h / (heads / groups)) * 2 * kChunk * C;
-    const bf16* x_first = xbc + static_cast<size_t>(q_start) * channels + h * p_dim;
-    float* y_first = y + static_cast<size_t>(q_start) * inner + h * p_dim;
-    // where this lane's operands lie in a chunk's (unsigned: a lane's offset beside an address that is the same in all lanes)
-    const unsigned c_at = i * C + n0 + 4 * g, b_at = kChunk * C + (n0 + i) * kChunk + 4 * g;
-    const unsigned n_at = i * kChunk + 4 * g + wave, pre_at = kChunk * kChunk + 4 * g;
-    const unsigned col = static_cast<unsigned>(min(p, p_dim - 1)), row = static_cast<unsigned>(channels);
-    auto load = [&](int c) {
+    // where this lane's operands lie in a chunk's, in bytes
+    const unsigned c_at = 2 * (i * C + n0 + 4 * g), b_at = 2 * (kChunk * C + (n0 + i) * kChunk + 4 * g), suf_at = 4 * (kChunk * kChunk + kChunk + 4 * g);
+    unsigned x_at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x_at[u] = (4 * g + u) * x_row;
+    auto load = [&]() __attribute__((always_inline)) {
         Operands o;
-        const bf16* rows = group_first + static_cast<size_t>(c) * groups * 2 * kChunk * C;
-        const float* of = head_first + static_cast<size_t>(c) * heads * kChunkHeadFloats;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o.x[u] = x_of(next, x_at[u]);
+        o.suf = *reinterpret_cast<const ssm_float4*>(next.of + suf_at);
+        o.all = *reinterpret_cast<const float*>(next.of + 4 * (kChunk * kChunk + 2 * kChunk));
 #pragma unroll
         for (int j = 0; j < TILES; ++j) {
-            o.c[j] = *reinterpret_cast<const SsmFour*>(rows + c_at + 16 * j);
-            o.b[j] = *reinterpret_cast<const SsmFour*>(rows + b_at + 16 * kChunk * j);
+            o.c[j] = *reinterpret_cast<const SsmFour*>(next.rows + c_at + 32 * j);
+            o.b[j] = *reinterpret_cast<const SsmFour*>(next.rows + b_at + 32 * kChunk * j);
         }
-        o.n = of[n_at];
-        o.pre = *reinterpret_cast<const ssm_float4*>(of + pre_at);
-        o.suf = *reinterpret_cast<const ssm_float4*>(of + pre_at + kChunk);
-        o.all = of[kChunk * kChunk + 2 * kChunk];
-        const bf16* x_chunk = x_first + static_cast<size_t>(c) * kChunk * channels;
-        const unsigned beyond = (min(kChunk, q_len - c * kChunk) - 1) * row;          // the chunk's last token
-        // (beyond it, that token's once more: what it is multiplied by is zero)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) o.x[u] = x_chunk[min((4 * g + u) * row, beyond) + col];
+        move_on(next);
         return o;
     };
-    const int count = (q_len + kChunk - 1) / kChunk;
-    auto walk = [&](int c, const Operands& now) {
+    auto walk = [&](int c, Operands& now) __attribute__((always_inline)) {
         ssm_float4 x, read[TILES];
 #pragma unroll
         for (int u = 0; u < 4; ++u) x[u] = c * kChunk + 4 * g + u < q_len ? to_float(now.x[u]) : 0.f;
@@ -743,6 +819,7 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
             for (int j = 0; j < TILES; ++j)
                 read[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.c[j].v[u]), s[j][u], read[j], 0, 0, 0);
         const ssm_float4 moved = x * now.suf;
+        const float all = now.all;
         // (the chunk's own sum first, from zero, and the state joins it with one rounding a chunk)
         ssm_float4 own[TILES];
 #pragma unroll
@@ -752,47 +829,36 @@ ssm_chunk_scan_kernel(const float* of_head, const bf16* of_group, const bf16* xb
 #pragma unroll
             for (int j = 0; j < TILES; ++j)
                 own[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(now.b[j].v[u]), moved[u], own[j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TILES; ++j)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) s[j][u] = fmaf(now.all, s[j][u], own[j][u]);
-        // a wavefront's part: its rows of the state, and the chunk's own tokens 4g + wave
-        const float mine = wave == 0 ? x[0] : wave == 1 ? x[1] : wave == 2 ? x[2] : x[3];
+        __builtin_amdgcn_sched_barrier(0);
+        now = load();
+        __builtin_amdgcn_sched_barrier(0);
         ssm_float4 part = read[0];
 #pragma unroll
         for (int j = 1; j < TILES; ++j) part += read[j];
-        part = add_causal_product(now.n, mine, part * now.pre, i, g, [&](int q) { return 4 * q + wave; });
-        part_s[c % 2][wave][lane] = part;
-        // (a barrier for what lies in shared memory alone: the operands of the chunks ahead stay on their way)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        // wavefront w writes the tokens 4g + w
-        const float* parts = reinterpret_cast<const float*>(&part_s[c % 2][0][lane]) + wave;
-        float o = parts[0];
+        read_s[c % 2][wave][lane] = part;                                    // a wavefront's part: its rows of the state
 #pragma unroll
-        for (int w = 1; w < 4; ++w) o += parts[w * 4 * kWave];
-        const int t = 4 * g + wave;
-        if (live && c * kChunk + t < q_len)
-            (y_first + static_cast<size_t>(c) * kChunk * inner)[t * static_cast<unsigned>(inner) + col] = fmaf(skip, mine, o);
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[j][u] = fmaf(all, s[j][u], own[j][u]);
+        meet();
     };
     // the operands of kAhead chunks in turn (beyond the last chunk: the last's once more).  The loads stay where they are
     // written: the scratch and xbc may alias y as far as the compiler knows, and the empty statements touch memory.
     Operands ring[kAhead];
 #pragma unroll
-    for (int d = 0; d < kAhead; ++d) ring[d] = load(min(d, count - 1));
+    for (int d = 0; d < kAhead; ++d) {
+        ring[d] = load();
+        __builtin_amdgcn_sched_barrier(0);               // (in this order, which the waits of the loop count on)
+    }
     int c = 0;
     for (; c + kAhead <= count; c += kAhead) {
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) {
-            walk(c + d, ring[d]);
-            ring[d] = load(min(c + d + kAhead, count - 1));
-            asm volatile("" ::: "memory");
-        }
+        for (int d = 0; d < kAhead; ++d) walk(c + d, ring[d]);
     }
 #pragma unroll
-    for (int d = 0; d < kAhead; ++d)
+    for (int d = 0; d < kAhead - 1; ++d)
         if (c + d < count) walk(c + d, ring[d]);
+    meet();                                                                  // the others' last sums
 #pragma unroll
     for (int j = 0; j < TILES; ++j)
 #pragma unroll
@@ -832,7 +898,7 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
             static_cast<const bf16*>(xbc), static_cast<const bf16*>(dt_in), dt_stride, dt_bias, a_log, seg_q_start, seg_q_len, \
             segments, chunks, of_group, heads, groups, n_state, p_dim, from);                                          \
         if (const int err = launch_status()) return err;                                                               \
-        ssm_chunk_scan_kernel<TILES><<<grid, 256, 0, stream>>>(                                                        \
+        ssm_chunk_scan_kernel<TILES><<<grid, 512, 0, stream>>>(                                                        \
             chunks, of_group, static_cast<const bf16*>(xbc), d_skip, state, state_stride, seg_q_start, seg_q_len, state_slots, y, \
             heads, groups, n_state, p_dim, from);                                                                      \
     } while (0)
