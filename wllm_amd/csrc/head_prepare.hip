@@ -10,6 +10,7 @@ constexpr int kPrepareWaves = 4;
 constexpr int kPrepareMaxHead = 256;
 constexpr int kPerLane = kPrepareMaxHead / kWave;
 constexpr int kRestColumns = kWave * kPrepareWaves * 4;      // columns beyond the heads that one workgroup takes
+constexpr int kValueTokens = 16;                             // tokens whose values a workgroup copies
 
 template <typename T> struct alignas(4 * sizeof(T)) Four { T v[4]; };
 
@@ -41,19 +42,44 @@ template <typename T> struct alignas(4 * sizeof(T)) Four { T v[4]; };
 // partner there.  A token's sines and cosines are worked out once a workgroup, a pair a thread, while the
 // heads are on their way: a sine of an angle of some thousand radians costs more than all else a lane
 // does (3,001 tokens of 8 heads and one key head of 256, half of the head turned: 37.6 to 29.5 us).
+// Many tokens: the first `head_rows` workgroups of a token (FOUR) walk its groups of heads, the next group's elements on their way, so that
+// its angles are worked out `head_rows` times and not once a group; and values that are only copied go to the cache
+// kValueTokens tokens at a time, a column's neighbours in a page from neighbouring lanes, where a token's workgroup writes 2 bytes of each of them
+// (us, before and now: 3,001 tokens of four groups of heads and values of their own 27.1 and 18.5, of six groups whose keys are the values 33.1 and 21.2; 1,500
+// tokens of three groups and values 13.3 and 10.5, of five groups 15.4 and 13.8).
 template <typename T, bool FOUR>
 __global__ void __launch_bounds__(kWave * kPrepareWaves)
 head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict__ parts, int splits, size_t split_stride,
                     const float* __restrict__ bias, int bias_width, const int* __restrict__ positions,
                     const float* __restrict__ inv_freq, const int* __restrict__ slots, T* __restrict__ cache,
                     long long num_pages, int num_heads, int num_kv_heads, int head_dim, int rotary_dim,
-                    int interleaved, float norm_eps, int norm_dim, int values_are_keys, int page_size, int head_pieces,
-                    const float* __restrict__ pre_q, const float* __restrict__ pre_k, float pre_eps, float rot_scale,
+                    int interleaved, float norm_eps, int norm_dim, int values_are_keys, int page_size, int head_rows, int copy_tokens,
+                    int copy_pieces, const float* __restrict__ pre_q, const float* __restrict__ pre_k, float pre_eps, float rot_scale,
                     float temp_coef, int temp_every) {
     __shared__ __align__(16) float staged[kPrepareWaves][kPrepareMaxHead];
     __shared__ float sines[kPrepareMaxHead / 2], cosines[kPrepareMaxHead / 2];
-    const int token = blockIdx.x;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int turned_heads = num_heads + num_kv_heads;
+    if (FOUR && copy_tokens > 0 && static_cast<int>(blockIdx.x) >= copy_tokens) {
+        // ---- values of their own that nothing is added to, into the cache: lane % 16 a token, four columns a lane ----
+        const int r = (static_cast<int>(blockIdx.x) - copy_tokens) * head_rows + blockIdx.y, begin = r % copy_pieces * kRestColumns;
+        const int t = r / copy_pieces * kValueTokens + threadIdx.x % kValueTokens;
+        if (t >= copy_tokens) return;
+        const int slot = slots[t];
+        const long long page = slot / page_size;
+        if (slot < 0 || page >= num_pages) return;
+        const int values = num_kv_heads * head_dim;
+        const T* from = rows + static_cast<size_t>(t) * row_width + turned_heads * head_dim;
+        T* to = cache + (static_cast<size_t>(page) * 2 + 1) * values * page_size + slot % page_size;
+        const int end = min(values, begin + kRestColumns);
+        for (int c = begin + threadIdx.x / kValueTokens * 4; c < end; c += 4 * kWave * kPrepareWaves / kValueTokens) {
+            const Four<T> v = *reinterpret_cast<const Four<T>*>(from + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) to[static_cast<size_t>(c + u) * page_size] = v.v[u];
+        }
+        return;
+    }
+    const int token = blockIdx.x;
     T* row = rows + static_cast<size_t>(token) * row_width;
     const float* prow = parts ? parts + static_cast<size_t>(token) * row_width : nullptr;
     auto value = [&](int idx) -> float {
@@ -73,12 +99,11 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
             vpage = kpage + static_cast<size_t>(num_kv_heads) * page_size * head_dim;
         }
     }
-    const int turned_heads = num_heads + num_kv_heads;
-    if (static_cast<int>(blockIdx.y) >= head_pieces) {
+    if ((!FOUR || copy_tokens == 0) && static_cast<int>(blockIdx.y) >= head_rows) {
         // ---- behind the query and key heads: value heads of their own, then the rest of the row ----
         const int begin = turned_heads * head_dim;
         const int values_end = values_are_keys ? begin : begin + num_kv_heads * head_dim;
-        const int idx0 = begin + (static_cast<int>(blockIdx.y) - head_pieces) * kRestColumns + threadIdx.x * 4;
+        const int idx0 = begin + (static_cast<int>(blockIdx.y) - head_rows) * kRestColumns + threadIdx.x * 4;
         for (int u = 0; u < 4; ++u) {
             const int idx = idx0 + u;
             if (idx >= row_width) break;
@@ -96,12 +121,11 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
         }
         return;
     }
-    const int head = static_cast<int>(blockIdx.y) * kPrepareWaves + wave;
-    const int base = head * head_dim;
-    const int kvh = head - num_heads;                 // >= 0: a key head
+    int head = static_cast<int>(blockIdx.y) * kPrepareWaves + wave;
     const int half = rotary_dim / 2;
     Four<T> loaded;                                   // FOUR: the lane's elements, asked for before the angles
-    if (FOUR && !prow && head < turned_heads && 4 * lane < head_dim) loaded = *reinterpret_cast<const Four<T>*>(row + base + 4 * lane);
+    if (FOUR && !prow && head < turned_heads && 4 * lane < head_dim)
+        loaded = *reinterpret_cast<const Four<T>*>(row + head * head_dim + 4 * lane);
     if (inv_freq) {
         if (static_cast<int>(threadIdx.x) < half) {
             float sn, cs;
@@ -112,9 +136,11 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
         __syncthreads();
     }
     if (head >= turned_heads) return;
-    float temperature = 1.f;
-    if (temp_every > 0 && kvh < 0) temperature = 1.f + temp_coef * logf(static_cast<float>((positions[token] + 1) / temp_every) + 1.f);
-    if (FOUR) {
+    float query_temperature = 1.f;
+    if (temp_every > 0) query_temperature = 1.f + temp_coef * logf(static_cast<float>((positions[token] + 1) / temp_every) + 1.f);
+    if (FOUR) for (;;) {                              // (many tokens: the wavefront's next heads)
+        const int base = head * head_dim;
+        const int kvh = head - num_heads;             // >= 0: a key head
         const int e = 4 * lane;
         float v[4] = {0.f, 0.f, 0.f, 0.f};
         const bool live = e < head_dim;
@@ -140,6 +166,8 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
             } else {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) v[u] = to_float(loaded.v[u]);
+                if (head + head_rows * kPrepareWaves < turned_heads)
+                    loaded = *reinterpret_cast<const Four<T>*>(row + base + head_rows * kPrepareWaves * head_dim + e);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -193,7 +221,7 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
             const float ss = wave_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]);
             inv = rsqrtf(ss / static_cast<float>(norm_dim) + norm_eps);
         }
-        inv *= temperature;
+        inv *= kvh < 0 ? query_temperature : 1.f;
         if (live) {
             Four<T> r;
 #pragma unroll
@@ -202,8 +230,12 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
             if (kvh >= 0 && kpage)
                 *reinterpret_cast<Four<T>*>(kpage + (static_cast<size_t>(kvh) * page_size + off) * head_dim + e) = r;
         }
-        return;
+        head += head_rows * kPrepareWaves;
+        if (head >= turned_heads) return;
     }
+    const int base = head * head_dim;
+    const int kvh = head - num_heads;                 // >= 0: a key head
+    const float temperature = kvh < 0 ? query_temperature : 1.f;
     // ---- any sizes, either pairing: the lane's elements are lane, lane + 64, ... ----
     float* mine = staged[wave];
     float v[kPerLane];
@@ -263,6 +295,9 @@ head_prepare_kernel(T* __restrict__ rows, int row_width, const float* __restrict
     }
 }
 
+// Workgroups of heads that fill the compute units, and the tokens from which on values go by columns: 32 workgroups a group of columns, where fewer would be done later than one a token.
+constexpr int kFillGroups = 2048, kCopyTokens = 512;
+
 // Returns 0, a HIP error code, or -1 for sizes the kernel does not take.  `bias` covers the first
 // `bias_width` columns of a row (0: no bias).
 WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const float* parts, int splits,
@@ -286,16 +321,22 @@ WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const flo
     const bool rest = row_width > turned && (parts != nullptr || bias_width > turned || (!values_are_keys && cache != nullptr));
     const int rest_pieces = rest ? (row_width - turned + kRestColumns - 1) / kRestColumns : 0;
     if (head_pieces + rest_pieces > 65535) return -1;
-    const dim3 grid(n, head_pieces + rest_pieces);
     const bool four = head_dim % 4 == 0 && row_width % 4 == 0 && (interleaved || rotary_dim % 8 == 0) &&
                       (parts == nullptr || split_stride % 4 == 0) &&
                       reinterpret_cast<uintptr_t>(rows) % 16 == 0 && reinterpret_cast<uintptr_t>(parts) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(cache) % 16 == 0;
+    // As many workgroups as fill the compute units (8 of four wavefronts), a group of heads each at most.
+    const int head_rows = four ? min(head_pieces, max(1, (kFillGroups + n - 1) / n)) : head_pieces;
+    // the rest of the row is copied only: by columns of a page (from kCopyTokens tokens on; of fewer a workgroup a token is done sooner)
+    const bool copies = four && n >= kCopyTokens && rest && parts == nullptr && bias_width <= turned;
+    const int copy_pieces = copies ? (num_kv_heads * head_dim + kRestColumns - 1) / kRestColumns : 1;
+    const int copy_groups = copies ? (n + kValueTokens - 1) / kValueTokens * copy_pieces : 0;
+    const dim3 grid(n + (copy_groups + head_rows - 1) / head_rows, head_rows + (copies ? 0 : rest_pieces));
 #define LAUNCH(T, FOUR)                                                                                             \
     head_prepare_kernel<T, FOUR><<<grid, kWave * kPrepareWaves, 0, stream>>>(                                       \
         static_cast<T*>(rows), row_width, parts, splits, static_cast<size_t>(split_stride), bias, bias_width, positions, \
         inv_freq, slots, static_cast<T*>(cache), num_pages, num_heads, num_kv_heads, head_dim, rotary_dim, interleaved, \
-        norm_eps, norm_dim, values_are_keys, page_size, head_pieces, pre_q, pre_k, pre_eps, rot_scale, temp_coef, \
+        norm_eps, norm_dim, values_are_keys, page_size, head_rows, copies ? n : 0, copy_pieces, pre_q, pre_k, pre_eps, rot_scale, temp_coef, \
         temp_every)
     if (is_bf16) {
         if (four) LAUNCH(bf16, true); else LAUNCH(bf16, false);
