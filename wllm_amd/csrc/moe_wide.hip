@@ -76,7 +76,10 @@ moe_wide_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, const in
         const int band = it / (kBandPairs * n_tiles), in_band = it - band * kBandPairs * n_tiles;
         const int band_rows = min(kBandPairs, m_tiles - kBandPairs * band);
         const int n_tile = in_band / band_rows;
-        const int pair = __builtin_amdgcn_readfirstlane(pairs_s[kBandPairs * band + in_band - n_tile * band_rows]);
+        // (each round of the band's items another of its tiles of rows, so that no workgroup makes tiles of one half alone, or of two: 16 experts of
+        // 4,096 behind a width of 2,048, three a token, 3,001 tokens 332 us and 314.  Tiles of one half behind all others: 357, their weights read again.)
+        const int of_band = (in_band - n_tile * band_rows + n_tile * band_rows / (static_cast<int>(gridDim.x) / 8)) % band_rows;
+        const int pair = __builtin_amdgcn_readfirstlane(pairs_s[kBandPairs * band + of_band]);
         const ExpertItem at{pair & 0x7fff, n_tile * kColumns, (pair & 0x8000) != 0};
         from.stages = K / kWideKeys;
         from.two = at.two;
