@@ -969,10 +969,69 @@ gated_group_norm_kernel(const float* __restrict__ y, const T* __restrict__ z, lo
     }
 }
 
+// The same, the same bits, for many (token, part)s of at most 256 PER columns: a wavefront each, which holds its columns in registers and adds them up as
+// the four wavefronts above do (lane by lane every 256th column, each 64 lanes by themselves, then those four sums).  No barrier, one pass over memory, and
+// all loads at once.  1,500 tokens of 8 parts of 512, bfloat16: 21.5 us and 14.0 (the bytes: 10).
+template <typename T, int PER>
+__global__ void __launch_bounds__(256)
+gated_group_norm_wave_kernel(const float* __restrict__ y, const T* __restrict__ z, long long z_stride, const float* __restrict__ weight,
+                             T* __restrict__ out, int width, int groups, float eps) {
+    const int lane = threadIdx.x % kWave, part = blockIdx.y * 4 + threadIdx.x / kWave;
+    if (part >= groups) return;
+    const size_t token = blockIdx.x;
+    const int size = width / groups, c0 = part * size;
+    const float* yr = y + token * width + c0;
+    const T* zr = z + token * z_stride + c0;
+    float yv[4][PER], v[4][PER];
+    T zv[4][PER];
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = min(64 * w + lane + 256 * j, size - 1);
+            yv[w][j] = yr[i];
+            zv[w][j] = zr[i];
+        }
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const float g = to_float(zv[w][j]);
+            v[w][j] = yv[w][j] * (g / (1.f + expf(-g)));
+            if (64 * w + lane + 256 * j < size) ss += v[w][j] * v[w][j];
+        }
+        total += wave_sum(ss);
+    }
+    const float inv = 1.f / sqrtf(total / static_cast<float>(size) + eps);
+    T* o = out + token * width + c0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = 64 * w + lane + 256 * j;
+            if (i < size) o[i] = from_float<T>(v[w][j] * inv * weight[c0 + i]);
+        }
+}
+
 WLLM_API int wllm_gated_group_norm(const float* y, const void* z, long long z_stride, const float* weight, void* out,
                                    int is_bf16, int tokens, int width, int groups, float eps, hipStream_t stream) {
     if (tokens <= 0) return 0;
     if (width <= 0 || groups <= 0 || width % groups != 0 || groups > 65535) return -1;
+    const int size = width / groups;
+    // (a wavefront a compute unit's SIMD twice over: of fewer parts the kernel with four wavefronts a part is done sooner)
+    if (size <= 1024 && static_cast<long long>(tokens) * groups >= 2048) {
+        const dim3 grid(tokens, (groups + 3) / 4);
+#define LAUNCH(T, PER)                                                                                                     \
+    gated_group_norm_wave_kernel<T, PER><<<grid, 256, 0, stream>>>(y, static_cast<const T*>(z), z_stride, weight,          \
+                                                                   static_cast<T*>(out), width, groups, eps)
+        if (size <= 256) { if (is_bf16) LAUNCH(bf16, 1); else LAUNCH(float, 1); }
+        else if (size <= 512) { if (is_bf16) LAUNCH(bf16, 2); else LAUNCH(float, 2); }
+        else { if (is_bf16) LAUNCH(bf16, 4); else LAUNCH(float, 4); }
+#undef LAUNCH
+        return launch_status();
+    }
     const dim3 grid(tokens, groups);
     if (is_bf16)
         gated_group_norm_kernel<bf16><<<grid, 256, 0, stream>>>(y, static_cast<const bf16*>(z), z_stride, weight,
