@@ -34,6 +34,53 @@ causal_conv_kernel(const T* __restrict__ in, long long in_stride, const float* _
     }
 }
 
+// The same sums for steps of a token a segment and fewer: a workgroup walks a segment's tokens in order, each thread its channels with the
+// carried rows in registers (TAPS; 0: any number, the rows in memory), and writes the new rows behind them: no launch behind this one.  A decode
+// step's chain is two launches otherwise: 8 tokens of 6,144 channels 5.0 and 4.7 us, now 4.8.
+template <typename T, int TAPS>
+__global__ void __launch_bounds__(256)
+causal_conv_segment_kernel(const T* __restrict__ in, long long in_stride, const float* __restrict__ weight,
+                           const float* __restrict__ bias, float* __restrict__ state, long long state_stride,
+                           long long carried_offset, const int* __restrict__ seg_q_start, const int* __restrict__ seg_q_len,
+                           const int* __restrict__ state_slots, T* __restrict__ out, int channels, int taps) {
+    const int seg = blockIdx.x, begin = seg_q_start[seg], len = seg_q_len[seg];
+    if (len <= 0) return;
+    float* carried = state + static_cast<size_t>(state_slots[seg]) * state_stride + carried_offset;
+    for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < channels; c += gridDim.y * blockDim.x) {
+        const float* w = weight + static_cast<size_t>(c) * taps;
+        const float b = bias[c];
+        float rows[TAPS > 1 ? TAPS - 1 : 1], by[TAPS > 0 ? TAPS : 1];
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) {
+            by[k] = w[k];
+            if (k + 1 < TAPS) rows[k] = carried[static_cast<size_t>(k) * channels + c];
+        }
+        for (int t = begin; t < begin + len; ++t) {
+            const float now = to_float(in[static_cast<size_t>(t) * in_stride + c]);
+            float acc = b;
+            if (TAPS > 0) {
+#pragma unroll
+                for (int k = 0; k + 1 < TAPS; ++k) {
+                    acc = fmaf(by[k], rows[k], acc);
+                    rows[k] = k + 2 < TAPS ? rows[k + 1] : now;
+                }
+                acc = fmaf(by[TAPS > 0 ? TAPS - 1 : 0], now, acc);
+            } else {
+                for (int k = 0; k + 1 < taps; ++k) {
+                    const float v = carried[static_cast<size_t>(k) * channels + c];
+                    acc = fmaf(w[k], v, acc);
+                    if (k > 0) carried[static_cast<size_t>(k - 1) * channels + c] = v;
+                }
+                acc = fmaf(w[taps - 1], now, acc);
+                if (taps > 1) carried[static_cast<size_t>(taps - 2) * channels + c] = now;
+            }
+            out[static_cast<size_t>(t) * channels + c] = from_float<T>(acc / (1.f + expf(-acc)));
+        }
+#pragma unroll
+        for (int k = 0; k + 1 < TAPS; ++k) carried[static_cast<size_t>(k) * channels + c] = rows[k];
+    }
+}
+
 // The same sums for the many tokens of a prompt's portion and convolutions of kSlideTaps taps: a thread takes four
 // consecutive channels and walks kSlideTokens tokens with the last inputs in registers, so a row is read once and not
 // once a tap, in 8-byte (float32: 16-byte) pieces (6,144 channels of 1,500 tokens: 62 to 17 us).
@@ -174,6 +221,16 @@ WLLM_API int wllm_causal_conv(const void* in, long long in_stride, const float* 
     if (many && !is_bf16 && in_fours<float>(in, in_stride, weight, bias, state, state_stride, carried_offset, out, channels))
         return SLIDE(float), launch_status();
 #undef SLIDE
+    if (tokens <= segments) {
+#define LAUNCH(T, TAPS)                                                                                                    \
+    causal_conv_segment_kernel<T, TAPS><<<carry_grid, 256, 0, stream>>>(                                                   \
+        static_cast<const T*>(in), in_stride, weight, bias, state, state_stride, carried_offset, seg_q_start, seg_q_len,   \
+        state_slots, static_cast<T*>(out), channels, taps)
+        if (is_bf16) { if (taps == kSlideTaps) LAUNCH(bf16, kSlideTaps); else LAUNCH(bf16, 0); }
+        else { if (taps == kSlideTaps) LAUNCH(float, kSlideTaps); else LAUNCH(float, 0); }
+#undef LAUNCH
+        return launch_status();
+    }
     if (is_bf16)
         causal_conv_kernel<bf16><<<grid, 256, 0, stream>>>(static_cast<const bf16*>(in), in_stride, weight, bias, state,
                                                            state_stride, carried_offset, token_segment, seg_q_start,
