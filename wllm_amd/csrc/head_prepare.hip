@@ -328,7 +328,7 @@ WLLM_API int wllm_head_prepare(void* rows, int is_bf16, int row_width, const flo
     // As many workgroups as fill the compute units (8 of four wavefronts), a group of heads each at most.
     const int head_rows = four ? min(head_pieces, max(1, (kFillGroups + n - 1) / n)) : head_pieces;
     // the rest of the row is copied only: by columns of a page (from kCopyTokens tokens on; of fewer a workgroup a token is done sooner)
-    const bool copies = four && n >= kCopyTokens && rest && parts == nullptr && bias_width <= turned;
+    const bool copies = four && head_rows > 0 && n >= kCopyTokens && rest && parts == nullptr && bias_width <= turned;
     const int copy_pieces = copies ? (num_kv_heads * head_dim + kRestColumns - 1) / kRestColumns : 1;
     const int copy_groups = copies ? (n + kValueTokens - 1) / kValueTokens * copy_pieces : 0;
     const dim3 grid(n + (copy_groups + head_rows - 1) / head_rows, head_rows + (copies ? 0 : rest_pieces));

@@ -941,9 +941,9 @@ WLLM_API int wllm_ssm_scan(const void* xbc, const void* dt_in, long long dt_stri
     if (segments > 65535 || (p_dim + kScanCols - 1) / kScanCols > 65535) return -1;
     const dim3 grid(heads, segments, (p_dim + kScanCols - 1) / kScanCols);
     // (a segment of `from` tokens leaves room for the others' single tokens)
-    // (what the chunks' kernels do not take goes token by token)
+    // (what the chunks' kernels do not take goes token by token: more channels than 16 rows' bytes in 32 bits allow, too)
     const bool in_chunks = from > 0 && tokens - (segments - 1) >= from && n_state <= 256 && groups <= 65535 &&
-                           static_cast<long long>(heads) * p_dim + 2LL * groups * n_state <= 0x0fffffffLL;
+                           static_cast<long long>(heads) * p_dim + 2LL * groups * n_state <= 0x07ffffffLL;
     if (in_chunks) {
         if (!is_bf16 || !chunks || from < kChunk || reinterpret_cast<uintptr_t>(chunks) % 16) return -1;
         const int places = chunk_places(tokens, from);
