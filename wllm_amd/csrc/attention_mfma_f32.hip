@@ -248,7 +248,7 @@ paged_attention_f32_kernel(const float* __restrict__ qkv, const float* __restric
 
 // Combines the partial results of a tile of rows whose keys were split over workgroups, in the order of
 // the splits.  reduce items: seg, kvh, first partial slot, number of splits, first row, slots between
-// splits, the segment's number of new tokens, the place of its first token among the step's tokens.
+// splits, the segment's rows, the place of its first token among the step's tokens (both looked up by the segment here).
 // One workgroup a (tile, four rows); a thread four consecutive elements of a row.
 template <int HD>
 __global__ void __launch_bounds__(HD)
